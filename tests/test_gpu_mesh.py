@@ -65,3 +65,19 @@ def test_gpu_fill_degenerate_faces_and_edge_cases(gpu):
     out = np.zeros((max(n.value - 1, 1), 4), np.float32)
     assert L.upf_mesh_fill(upf.ptr(f), len(f), sc, 0.01, upf.ptr(out), n.value - 1, C.byref(n)) == \
         upf._abi.UPF_ERR_RANGE
+
+
+@pytest.mark.parametrize("name,scale,spacing", [
+    ("mesh_blob.obj", (0.1, 2.0, 2.0), 0.012),    # two planes of points in x
+    ("mesh_blob.obj", (2.0, 0.1, 0.1), 0.006),    # a thin bar along x
+    ("mesh_torus.obj", (0.05, 0.12, 6.0), 0.004),  # a few points in x and y, many in z
+    ("mesh_box.obj", (1.0, 1.0, 1.0), 0.0171),    # remainders of the 4 x 4 x 4 tiles, faces along the lattice
+    ("mesh_sphere.obj", (1.0, 1.0, 1.0), 4e8),    # magnified: coordinates past the overflow bound of the face bounds
+])
+def test_gpu_fill_tile_shapes(gpu, name, scale, spacing):
+    """The lattice's 64-point tiles: thin lattices, remainders, and the form that tests every face."""
+    faces = upf.load_obj(os.path.join(GOLD, name))
+    if spacing > 1e8:
+        faces = faces * np.float32(1e11)
+    print("mesh fill tiles %s, scale %s, spacing %g" % (name, scale, spacing), flush=True)
+    assert np.array_equal(upf.mesh_fill(faces, scale, spacing), ol.mesh_fill(faces, scale, spacing))

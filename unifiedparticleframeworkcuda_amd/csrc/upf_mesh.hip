@@ -4,8 +4,9 @@
 // keeps the lattice points inside the mesh or on a face (Polygon,
 // src/cpu/Polygon.cpp).  The reader runs on the host; the point-in-mesh test of
 // every lattice point against every face -- the O(points x faces) part -- runs
-// on the GPU, one thread per lattice point over faces staged through LDS, and
-// the kept points are compacted in the reference's loop order.
+// on the GPU, one thread per lattice point over the faces that interval bounds
+// leave for its tile of 64 points, and the kept points are compacted in the
+// reference's loop order.
 //
 // Floating point: -ffp-contract=off and correctly rounded division, every
 // expression in the reference's evaluation order, so the particle set and its
@@ -92,19 +93,22 @@ int read_obj(const char* path, std::vector<F3>& tri) {
 }
 
 // ----------------------------------------------------------- face constants
-// Per face, what the crossing and touching tests read: the corners, the unit
-// normal n (Polygon::AddVertex: (v0 - v1) x (v2 - v1), vmml's normalize with
-// 1/l in double), d = -(v0 . n), the numerator -(d + o . n) of the segment
-// parameter for the common segment start o, the in-plane test's far point
-// (box minimum - 1, the box starting at the origin like the reference's), and
-// the two coordinates the in-plane test projects on.
-struct Face {
-    float4 a;  // v0, d
-    float4 b;  // v1, -(d + o . n)
-    float4 c;  // v2, index of the first projected coordinate (0 or 1)
-    float4 n;  // normal, index of the second (1 or 2)
-    float4 o;  // in-plane far point
+// Per face, what the crossing and touching tests read: the unit normal n
+// (Polygon::AddVertex: (v0 - v1) x (v2 - v1), vmml's normalize with 1/l in
+// double), d = -(v0 . n), the numerator -(d + o . n) of the segment parameter
+// for the common segment start o, and for the in-plane test the corners and
+// its far point (box minimum - 1, the box starting at the origin like the
+// reference's) projected on the two coordinates that it reads, with the side
+// of each edge that the far point lies on.  64 bytes: one scalar load.
+struct alignas(64) Face {
+    float nx, ny, nz, d;
+    float va[3], oa;  // first projected coordinate: corners, far point
+    float vb[3], ob;  // second
+    float num;
+    int code;  // 1: the first coordinate is y (else x), 2: the second is z (else y), 4 << k: side of edge k
+    int pad[2];
 };
+constexpr int FACE_Y = 1, FACE_Z = 2, FACE_SIDE = 4;
 
 inline float dot(const F3& a, const F3& b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
 
@@ -137,99 +141,232 @@ F3 face_normal(const F3* v) {
 }
 
 // ------------------------------------------------------------------ device
-__device__ __forceinline__ float pick(const float3& v, int i) { return i == 0 ? v.x : (i == 1 ? v.y : v.z); }
-
-// Polygon::ArePointsOnBothSidesOfTheLine (Polygon.cpp:73-103)
-__device__ __forceinline__ bool both_sides(int fi, int si, const float3& ls, const float3& le, const float3& p1,
-                                           const float3& p2) {
-    const float dxES = pick(le, fi) - pick(ls, fi);
-    const float dx1E = pick(p1, fi) - pick(le, fi);
-    const float dySE = pick(ls, si) - pick(le, si);
-    const float dyE1 = pick(le, si) - pick(p1, si);
-    const bool ccw1 = (dySE * dx1E) > (dyE1 * dxES);
-    const float dx2E = pick(p2, fi) - pick(le, fi);
-    const float dyE2 = pick(le, si) - pick(p2, si);
-    const bool ccw2 = (dySE * dx2E) > (dyE2 * dxES);
-    return ccw1 != ccw2;
-}
-
-// Polygon::IsPointInPlaneInside (Polygon.cpp:118-137)
-__device__ __forceinline__ bool in_plane_inside(const Face& f, const float3& pt) {
-    const int fi = (int)f.c.w, si = (int)f.n.w;
-    const float3 out = make_float3(f.o.x, f.o.y, f.o.z);
-    const float3 v[3] = {make_float3(f.a.x, f.a.y, f.a.z), make_float3(f.b.x, f.b.y, f.b.z),
-                         make_float3(f.c.x, f.c.y, f.c.z)};
+// Polygon::IsPointInPlaneInside (Polygon.cpp:118-137): the edges that the
+// segment from the far point to (pa, pb) crosses, by
+// Polygon::ArePointsOnBothSidesOfTheLine (Polygon.cpp:73-103) of the corners
+// against the segment's line (g) and of its ends against the edge's line.
+__device__ __forceinline__ bool in_plane_inside(const Face& f, float px, float py, float pz) {
+    const float pa = f.code & FACE_Y ? py : px, pb = f.code & FACE_Z ? pz : py;
+    const float dx = pa - f.oa, dy = f.ob - pb;
+    bool g[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) g[k] = (dy * (f.va[k] - pa)) > ((pb - f.vb[k]) * dx);
     bool inside = false;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        const float3& s = v[k];
-        const float3& e = v[k == 2 ? 0 : k + 1];
-        if (both_sides(fi, si, out, pt, s, e) && both_sides(fi, si, s, e, out, pt)) inside = !inside;
+        const int e = k == 2 ? 0 : k + 1;
+        const bool h = ((f.vb[k] - f.vb[e]) * (pa - f.va[e])) > ((f.vb[e] - pb) * (f.va[e] - f.va[k]));
+        inside ^= (g[k] != g[e]) && h != ((f.code & (FACE_SIDE << k)) != 0);
     }
     return inside;
 }
 
-constexpr int MF_BLOCK = 256;
-constexpr int MF_FACES = 256;  // faces per LDS stage (20 KB)
+constexpr int MF_BLOCK = 256;  // points per block of the count and emit kernels
+constexpr int MT_BLOCK = 512;  // points (threads) per block of the test
+constexpr int MT_LIST = 2048;  // faces a block holds between its two rulings
 
-// One thread per lattice point (x-major, then y, then z: the reference's loop
-// order).  For each face in file order: Polygon::DoesLineIntersect of the
-// segment from o to the point toggles the point; otherwise
-// Polygon::DoesPointTouch keeps it and ends the scan.  keep[] gets the
-// decision, counts[] the kept points of each block.
-__global__ __launch_bounds__(MF_BLOCK) void k_mesh_test(const Face* __restrict__ faces, int nf,
-                                                        const float* __restrict__ X, const float* __restrict__ Y,
-                                                        const float* __restrict__ Z, int nx, int ny, int nz, float3 o,
-                                                        uint8_t* __restrict__ keep, int* __restrict__ counts) {
-    __shared__ Face sf[MF_FACES];
-    const long long npts = (long long)nx * ny * nz;
-    const long long idx = (long long)blockIdx.x * MF_BLOCK + threadIdx.x;
-    const bool live = idx < npts;
-    float3 p = make_float3(0.f, 0.f, 0.f);
-    if (live) {
-        const int z = (int)(idx % nz);
-        const int y = (int)((idx / nz) % ny);
-        const int x = (int)(idx / ((long long)ny * nz));
-        const int par = x & 1;  // odd x: y and z start half a spacing later
-        p = make_float3(X[x], Y[par * ny + y], Z[par * nz + z]);
+// ------------------------------------------------- faces that cannot matter
+// Interval bounds of the test's own float expressions over a tile of lattice
+// points.  A rounded sum, difference, product or quotient is monotone in each
+// operand, so an expression evaluated at the right ends of its operands'
+// ranges bounds every value it takes inside them, rounding included: a face
+// that these bounds rule out neither toggles nor keeps any point of the tile.
+struct Iv {
+    float lo, hi;
+};
+__device__ __forceinline__ Iv iv_mul(const Iv& a, const Iv& b) {
+    const float p = a.lo * b.lo, q = a.lo * b.hi, r = a.hi * b.lo, s = a.hi * b.hi;
+    return {fminf(fminf(p, q), fminf(r, s)), fmaxf(fmaxf(p, q), fmaxf(r, s))};
+}
+__device__ __forceinline__ Iv iv_mul(const Iv& a, float c) {
+    const float p = a.lo * c, q = a.hi * c;
+    return {fminf(p, q), fmaxf(p, q)};
+}
+// l > r over the ranges: 1 always, 0 never, -1 undecided
+__device__ __forceinline__ int iv_greater(const Iv& l, const Iv& r) {
+    return l.lo > r.hi ? 1 : (l.hi <= r.lo ? 0 : -1);
+}
+__device__ __forceinline__ Iv iv_dot(const Iv& x, const Iv& y, const Iv& z, const float3& n) {
+    const Iv a = iv_mul(x, n.x), b = iv_mul(y, n.y), c = iv_mul(z, n.z);
+    return {a.lo + b.lo + c.lo, a.hi + b.hi + c.hi};
+}
+
+// in_plane_inside() is false for every point whose projected coordinates lie
+// in a x b: each edge toggles for all of them or for none, an even number do.
+__device__ __forceinline__ bool outside_in_plane(const Face& f, const Iv& a, const Iv& b) {
+    const Iv dy = {f.ob - b.hi, f.ob - b.lo}, dx = {a.lo - f.oa, a.hi - f.oa};
+    int g[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+        g[k] = iv_greater(iv_mul(dy, Iv{f.va[k] - a.hi, f.va[k] - a.lo}), iv_mul(Iv{b.lo - f.vb[k], b.hi - f.vb[k]}, dx));
+    bool sure = true, odd = false;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const int e = k == 2 ? 0 : k + 1;
+        const int h = iv_greater(iv_mul(Iv{a.lo - f.va[e], a.hi - f.va[e]}, f.vb[k] - f.vb[e]),
+                                 iv_mul(Iv{f.vb[e] - b.hi, f.vb[e] - b.lo}, f.va[e] - f.va[k]));
+        const int ho = f.code & (FACE_SIDE << k) ? 1 : 0;
+        const bool gsure = g[k] >= 0 && g[e] >= 0;
+        const bool never = (gsure && g[k] == g[e]) || h == ho;
+        odd ^= !never;  // always toggles, if sure
+        sure = sure && (never || (gsure && h >= 0));
     }
+    return sure && !odd;
+}
+
+// a box of lattice points and their offsets from o
+struct Box {
+    Iv x, y, z, dx, dy, dz;
+};
+
+__device__ __forceinline__ bool face_matters(const Face& f, const Box& B, const float3& o) {
+    const float3 n = make_float3(f.nx, f.ny, f.nz);
+    const Iv eq = iv_dot(B.x, B.y, B.z, n);
+    const bool touch = eq.lo + f.d <= 0.000001f && eq.hi + f.d >= -0.000001f;
+    const Iv den = iv_dot(B.dx, B.dy, B.dz, n);
+    // segment parameters in [0, 1] that the box's points can have
+    bool cross = den.hi >= 0.000001f || den.lo <= -0.000001f;
+    Iv t = {0.0f, 1.0f};
+    if (den.lo >= 0.000001f || den.hi <= -0.000001f) {  // one sign: the quotient is monotone
+        const float p = f.num / den.lo, q = f.num / den.hi;
+        const float lo = fminf(p, q), hi = fmaxf(p, q);
+        cross = !(hi < 0.0f || lo > 1.0f);
+        t = {fmaxf(lo, 0.0f), fminf(hi, 1.0f)};
+    }
+    if (!cross && !touch) return false;
+    const bool fy = f.code & FACE_Y, fz = f.code & FACE_Z;
+    const Iv pa = fy ? B.y : B.x, pb = fz ? B.z : B.y;
+    Iv a = pa, b = pb;
+    if (cross) {  // crossing points o + d t, joined with the points themselves if those can touch
+        const Iv ma = iv_mul(fy ? B.dy : B.dx, t), mb = iv_mul(fz ? B.dz : B.dy, t);
+        const float ba = fy ? o.y : o.x, bb = fz ? o.z : o.y;
+        const Iv ca = {ba + ma.lo, ba + ma.hi}, cb = {bb + mb.lo, bb + mb.hi};
+        a = touch ? Iv{fminf(pa.lo, ca.lo), fmaxf(pa.hi, ca.hi)} : ca;
+        b = touch ? Iv{fminf(pb.lo, cb.lo), fmaxf(pb.hi, cb.hi)} : cb;
+    }
+    return !outside_in_plane(f, a, b);
+}
+
+// the lattice of a launch: extents, and log2 of a block's and of a wave's box
+struct Lattice {
+    int n[3], bb[3], wb[3];
+};
+
+// the box of the points p0 .. p1 (inclusive); odd x: y and z start half a
+// spacing later, and coordinates never decrease along a row
+__device__ __forceinline__ Box lattice_box(const float* __restrict__ X, const float* __restrict__ Y,
+                                           const float* __restrict__ Z, const Lattice& L, const int* p0, const int* p1,
+                                           const float3& o) {
+    Box B;
+    B.x = {X[p0[0]], X[p1[0]]};
+    B.y = {fminf(Y[p0[1]], Y[L.n[1] + p0[1]]), fmaxf(Y[p1[1]], Y[L.n[1] + p1[1]])};
+    B.z = {fminf(Z[p0[2]], Z[L.n[2] + p0[2]]), fmaxf(Z[p1[2]], Z[L.n[2] + p1[2]])};
+    B.dx = {B.x.lo - o.x, B.x.hi - o.x};
+    B.dy = {B.y.lo - o.y, B.y.hi - o.y};
+    B.dz = {B.z.lo - o.z, B.z.hi - o.z};
+    return B;
+}
+
+// One block per box of 512 lattice points (8 x 8 x 8 unless the lattice is
+// thin), one wave per 64 of them (4 x 4 x 4).  The block rules faces out for
+// its box, one face per thread; each wave rules out what is left for its own
+// box, one face per lane; the faces left after that run in file order, one
+// lattice point per lane: Polygon::DoesLineIntersect of the segment from o to
+// the point toggles the point; otherwise Polygon::DoesPointTouch keeps it and
+// ends its scan.  keep[] gets the decision.
+// Bound by VALU.  652,228 points and 6,400 faces: 26.9 ms with every pair
+// tested, 1.03 ms now (4.0 ms with one ruling per wave over all faces staged
+// in LDS); of a wave's 6,400 faces about 360 are left, since few faces are met
+// along the segments to a small box.  A face left is one scalar load.  `cull` 0: coordinates so large that a
+// product may overflow; every face runs.
+__global__ __launch_bounds__(MT_BLOCK) void k_mesh_test(const Face* __restrict__ faces, int nf,
+                                                        const float* __restrict__ X, const float* __restrict__ Y,
+                                                        const float* __restrict__ Z, Lattice L, float3 o, int cull,
+                                                        uint8_t* __restrict__ keep) {
+    constexpr int WAVES = MT_BLOCK / 64;
+    __shared__ int list[MT_LIST];  // faces the block's box leaves, in file order
+    __shared__ int wcnt[WAVES];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    // the block's box, the wave's box in it, the lane's point
+    const int nby = ((L.n[1] - 1) >> L.bb[1]) + 1, nbz = ((L.n[2] - 1) >> L.bb[2]) + 1;
+    const int b0[3] = {(int)(blockIdx.x / (nby * nbz)) << L.bb[0], (int)(blockIdx.x / nbz % nby) << L.bb[1],
+                       (int)(blockIdx.x % nbz) << L.bb[2]};
+    const int sy = L.bb[1] - L.wb[1], sz = L.bb[2] - L.wb[2];
+    const int w0[3] = {b0[0] + ((w >> (sy + sz)) << L.wb[0]), b0[1] + (((w >> sz) & ((1 << sy) - 1)) << L.wb[1]),
+                       b0[2] + ((w & ((1 << sz) - 1)) << L.wb[2])};
+    const int x = w0[0] + (lane >> (L.wb[1] + L.wb[2])), y = w0[1] + ((lane >> L.wb[2]) & ((1 << L.wb[1]) - 1)),
+              z = w0[2] + (lane & ((1 << L.wb[2]) - 1));
+    const bool wave = w0[0] < L.n[0] && w0[1] < L.n[1] && w0[2] < L.n[2];
+    const bool live = wave && x < L.n[0] && y < L.n[1] && z < L.n[2];
+    int b1[3], w1[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        b1[a] = min(b0[a] + (1 << L.bb[a]), L.n[a]) - 1;
+        w1[a] = min(w0[a] + (1 << L.wb[a]), L.n[a]) - 1;
+    }
+    const Box bbox = lattice_box(X, Y, Z, L, b0, b1, o);
+    Box wbox = bbox;
+    if (wave) wbox = lattice_box(X, Y, Z, L, w0, w1, o);
+    float3 p = make_float3(0.f, 0.f, 0.f);
+    if (live) p = make_float3(X[x], Y[(x & 1) * L.n[1] + y], Z[(x & 1) * L.n[2] + z]);
     // segment o -> p
     const float3 dv = make_float3(p.x - o.x, p.y - o.y, p.z - o.z);
     bool add = false, done = !live;
-    for (int f0 = 0; f0 < nf; f0 += MF_FACES) {
-        const int m = min(MF_FACES, nf - f0);
+    int len = 0;  // list entries so far (the same in every thread)
+    for (int f0 = 0; f0 < nf; f0 += MT_BLOCK) {
+        const int fi = f0 + (int)threadIdx.x;
+        bool in = fi < nf;
+        if (in && cull) in = face_matters(faces[fi], bbox, o);
+        const uint64_t m = __ballot(in);
+        if (lane == 0) wcnt[w] = __popcll(m);
         __syncthreads();
-        for (int k = threadIdx.x; k < m; k += MF_BLOCK) sf[k] = faces[f0 + k];
+        int at = len;
+#pragma unroll
+        for (int k = 0; k < WAVES; ++k) {
+            const int c = wcnt[k];
+            if (k < w) at += c;
+            len += c;
+        }
+        if (in) list[at + __popcll(m & ((1ull << lane) - 1ull))] = fi;
         __syncthreads();
-        if (!done) {
-            for (int k = 0; k < m; ++k) {
-                const Face& f = sf[k];
-                const float3 n = make_float3(f.n.x, f.n.y, f.n.z);
+        if (len <= MT_LIST - MT_BLOCK && f0 + MT_BLOCK < nf) continue;  // room for another round
+        for (int g = 0; wave && g < len; g += 64) {
+            bool mine = g + lane < len;
+            const int my = mine ? list[g + lane] : 0;
+            if (mine && cull) mine = face_matters(faces[my], wbox, o);
+            for (uint64_t left = __ballot(mine); left; left &= left - 1) {
+                const Face& f = faces[__builtin_amdgcn_readlane(my, __builtin_ctzll(left))];
+                if (done) continue;
                 bool crosses = false;
-                const float den = dv.x * n.x + dv.y * n.y + dv.z * n.z;
+                const float den = dv.x * f.nx + dv.y * f.ny + dv.z * f.nz;
                 if (!(fabsf(den) < 0.000001f)) {
-                    const float dof = f.b.w / den;
-                    if (!(dof < 0.0f || dof > 1.0f)) {
-                        const float3 q = make_float3(o.x + dv.x * dof, o.y + dv.y * dof, o.z + dv.z * dof);
-                        crosses = in_plane_inside(f, q);
-                    }
+                    const float dof = f.num / den;
+                    if (!(dof < 0.0f || dof > 1.0f))
+                        crosses = in_plane_inside(f, o.x + dv.x * dof, o.y + dv.y * dof, o.z + dv.z * dof);
                 }
                 if (crosses) {
                     add = !add;
                 } else {
-                    const float eq = (p.x * n.x + p.y * n.y + p.z * n.z) + f.a.w;
-                    if (!(fabsf(eq) > 0.000001f) && in_plane_inside(f, p)) {
+                    const float eq = (p.x * f.nx + p.y * f.ny + p.z * f.nz) + f.d;
+                    if (!(fabsf(eq) > 0.000001f) && in_plane_inside(f, p.x, p.y, p.z)) {
                         add = true;
                         done = true;
-                        break;
                     }
                 }
             }
         }
-        if (__syncthreads_count(!done) == 0) break;
+        len = 0;
+        if (__syncthreads_count(!done) == 0) break;  // also: every wave is past the list
     }
-    if (live) keep[idx] = (uint8_t)add;
-    const int c = __syncthreads_count(live && add);
+    if (live) keep[((long long)x * L.n[1] + y) * L.n[2] + z] = (uint8_t)add;
+}
+
+// kept points of each block of MF_BLOCK lattice points (x-major, then y, then
+// z: the reference's loop order)
+__global__ __launch_bounds__(MF_BLOCK) void k_mesh_count(const uint8_t* __restrict__ keep, long long npts,
+                                                         int* __restrict__ counts) {
+    const long long idx = (long long)blockIdx.x * MF_BLOCK + threadIdx.x;
+    const int c = __syncthreads_count(idx < npts && keep[idx]);
     if (threadIdx.x == 0) counts[blockIdx.x] = c;
 }
 
@@ -348,20 +485,25 @@ int upf_mesh_fill(const float* faces9, int n_faces, const float scale[3], float 
         const F3& n = fn[f];
         const float d = -dot(v[0], n);
         const float num = -(d + dot(o, n));
-        int fi, si;
-        if (n.x == 0) {
-            fi = 0;
-            si = n.y == 0 ? 1 : 2;
-        } else {
-            fi = 1;
-            si = 2;
-        }
         Face& F = faces[(size_t)f];
-        F.a = make_float4(v[0].x, v[0].y, v[0].z, d);
-        F.b = make_float4(v[1].x, v[1].y, v[1].z, num);
-        F.c = make_float4(v[2].x, v[2].y, v[2].z, (float)fi);
-        F.n = make_float4(n.x, n.y, n.z, (float)si);
-        F.o = make_float4(fmn[f].x - 1.0f, fmn[f].y - 1.0f, fmn[f].z - 1.0f, 0.0f);
+        const bool fy = n.x != 0, fz = fy || n.y != 0;
+        F.nx = n.x;
+        F.ny = n.y;
+        F.nz = n.z;
+        F.d = d;
+        F.num = num;
+        F.code = (fy ? FACE_Y : 0) | (fz ? FACE_Z : 0);
+        F.oa = (fy ? fmn[f].y : fmn[f].x) - 1.0f;
+        F.ob = (fz ? fmn[f].z : fmn[f].y) - 1.0f;
+        for (int k = 0; k < 3; ++k) {
+            F.va[k] = fy ? v[k].y : v[k].x;
+            F.vb[k] = fz ? v[k].z : v[k].y;
+        }
+        for (int k = 0; k < 3; ++k) {
+            const int e = k == 2 ? 0 : k + 1;
+            if (((F.vb[k] - F.vb[e]) * (F.oa - F.va[e])) > ((F.vb[e] - F.ob) * (F.va[e] - F.va[k])))
+                F.code |= FACE_SIDE << k;
+        }
     }
     // the lattice: coordinates accumulated step by step as the reference's
     // loops do (odd x: y and z start half a spacing later)
@@ -396,6 +538,22 @@ int upf_mesh_fill(const float* faces9, int n_faces, const float scale[3], float 
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0) return UPF_ERR_NO_DEVICE;
     const int nb = (int)((npts + MF_BLOCK - 1) / MF_BLOCK);
+    // log2 extents of the boxes of 64 and 512 points: a cube bounds its faces
+    // best; an axis with fewer points hands its share to the others
+    Lattice lat = {{(int)nx, (int)ny, (int)nz}, {0, 0, 0}, {0, 0, 0}};
+    for (int k = 0; k < 9; ++k) {
+        int best = -1;
+        for (int a = 2; a >= 0; --a)
+            if (((lat.n[a] - 1) >> lat.bb[a]) && (best < 0 || lat.bb[a] < lat.bb[best])) best = a;
+        ++lat.bb[best < 0 ? 2 : best];
+        if (k == 5) std::copy(lat.bb, lat.bb + 3, lat.wb);
+    }
+    long long boxes = 1;
+    for (int a = 0; a < 3; ++a) boxes *= ((lat.n[a] - 1) >> lat.bb[a]) + 1;
+    // within these bounds no product of the interval tests overflows
+    int cull = spacing <= 1e8f && X.back() <= 1e8f && Y[(size_t)ny - 1] <= 1e8f && Y.back() <= 1e8f &&
+               Z[(size_t)nz - 1] <= 1e8f && Z.back() <= 1e8f;
+    for (size_t k = 0; k < 9 * (size_t)n_faces; ++k) cull &= std::fabs(faces9[k]) <= 1e8f;
     Face* d_faces = nullptr;
     float *d_x = nullptr, *d_y = nullptr, *d_z = nullptr;
     uint8_t* d_keep = nullptr;
@@ -416,8 +574,9 @@ int upf_mesh_fill(const float* faces9, int n_faces, const float scale[3], float 
         ok(hipMemcpyAsync(d_x, X.data(), X.size() * sizeof(float), hipMemcpyHostToDevice, st)) &&
         ok(hipMemcpyAsync(d_y, Y.data(), Y.size() * sizeof(float), hipMemcpyHostToDevice, st)) &&
         ok(hipMemcpyAsync(d_z, Z.data(), Z.size() * sizeof(float), hipMemcpyHostToDevice, st))) {
-        hipLaunchKernelGGL(k_mesh_test, dim3(nb), dim3(MF_BLOCK), 0, st, d_faces, n_faces, d_x, d_y, d_z, (int)nx,
-                           (int)ny, (int)nz, make_float3(o.x, o.y, o.z), d_keep, d_counts);
+        hipLaunchKernelGGL(k_mesh_test, dim3((unsigned)boxes), dim3(MT_BLOCK), 0, st, d_faces, n_faces, d_x, d_y, d_z,
+                           lat, make_float3(o.x, o.y, o.z), cull, d_keep);
+        hipLaunchKernelGGL(k_mesh_count, dim3(nb), dim3(MF_BLOCK), 0, st, d_keep, npts, d_counts);
         hipLaunchKernelGGL(k_mesh_scan, dim3(1), dim3(1024), 0, st, d_counts, nb, d_total);
         if (ok(hipGetLastError()) && ok(hipMemcpyAsync(&total, d_total, sizeof(int), hipMemcpyDeviceToHost, st)) &&
             ok(hipStreamSynchronize(st))) {
