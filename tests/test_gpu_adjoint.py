@@ -120,3 +120,33 @@ def test_torch_function_gives_the_adjoint_gradient(gpu):
     _, gv = r.backward(g)
     assert np.allclose(v0.grad.numpy(), gv, rtol=1e-5, atol=1e-12)
     r.close()
+
+
+@pytest.mark.parametrize("case", ["one", "two", "quads", "dense"])
+def test_lanes_and_list_forms_match_fp32_oracle(gpu, case):
+    """A particle without neighbours, a pair, a rollout past the particle
+    count at which the pair passes take quads instead of rows of lanes, and
+    query boxes with more candidates than the list build's table holds."""
+    p, pos, typ, vel, target, f = adj.differentiable_dam_break(38, 24, 32) if case == "quads" else \
+        adj.differentiable_dam_break(9, 8, 7)
+    if case in ("one", "two"):
+        n = 1 if case == "one" else 2
+        pos, typ, vel = pos[f][:n].copy(), typ[f][:n].copy(), vel[f][:n].copy()
+        target, f = pos[:, :3] + 0.01, f[f][:n]
+    if case == "dense":
+        pos[f, :3] = pos[f, :3].min(0) + (pos[f, :3] - pos[f, :3].min(0)) * np.float32(0.68)
+        p.density_error_factor *= 1e-3  # a compressed block: pressures of a normal step
+    if case == "quads":
+        assert len(typ) >= 32768
+    print("adjoint lanes %s: %d particles" % (case, len(typ)), flush=True)
+    steps, K = 3, 2
+    r = adj.Rollout(p, pos, typ, steps, K, checkpoint_every=2)
+    x, v = r.forward(vel)
+    g = (x - pos[:, :3] if case != "quads" else _dloss(x, target, f)).astype(np.float64)
+    gx, gv = r.backward(g)
+    r.close()
+    xo, vo, ox, ov = ol.diff_run(p, pos, vel, typ, steps, K, gpos=g.astype(np.float32).astype(np.float64), precision=32)
+    # the bounds of the rollout above: expf / log1pf are the only other source
+    assert np.abs(x - xo).max() < 2e-6
+    assert np.abs(v - vo).max() < 1e-4 * max(np.abs(vo).max(), 1e-3)
+    assert _rel(gv, ov) < 1e-4 and _rel(gx, ox) < 1e-4

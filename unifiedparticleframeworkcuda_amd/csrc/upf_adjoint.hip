@@ -57,10 +57,53 @@ namespace ad {
 
 constexpr int AB = 256;  // threads per block
 
+// Pair passes run LANES lanes per particle: each lane takes every LANES-th
+// neighbour, and the lanes' terms are added in list order (DPP broadcasts, one
+// addition per neighbour), so every sum has the bits of a serial loop.  One
+// lane per particle was one serial chain of gathers per wave and about one
+// wave per SIMD at 65,536 particles (density 16.7 us, pressure force 15.6,
+// their reverses 27 and 29); see lanes() for the choice.
+
+// v of lane U of this lane's group of LANES (4: the quad, 16: the DPP row)
+template <int LANES, int U>
+__device__ __forceinline__ float lane_of(float v) {
+    static_assert(LANES == 4 || LANES == 16, "a quad or a row");
+    constexpr int ctrl = LANES == 4 ? U * 0x55 : 0x150 + U;  // quad_perm [U U U U] : row_newbcast U
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xf, 0xf, true));
+}
+// acc -/+ the group's terms, lane 0's first
+template <int LANES, int U = 0>
+__device__ __forceinline__ float sub_terms(float acc, float t) {
+    if constexpr (U < LANES) return sub_terms<LANES, U + 1>(acc - lane_of<LANES, U>(t), t);
+    else return acc;
+}
+template <int LANES, int U = 0>
+__device__ __forceinline__ float add_terms(float acc, float t) {
+    if constexpr (U < LANES) return add_terms<LANES, U + 1>(acc + lane_of<LANES, U>(t), t);
+    else return acc;
+}
+
+// term(j) for this lane's neighbours of the list (none: no neighbour), then
+// add() for the group's LANES terms; the next round's list entry is loaded
+// ahead of this round's gathers
+template <int LANES, class Term, class None, class Add>
+__device__ __forceinline__ void for_pairs(const uint32_t* __restrict__ row, int cnt, int sub, Term term, None none, Add add) {
+    int j = sub < cnt ? (int)row[sub] : 0;
+    for (int k = 0; k < cnt; k += LANES) {
+        const int next = k + LANES + sub;
+        const int jn = next < cnt ? (int)row[next] : 0;
+        if (k + sub < cnt) term(j);
+        else none();
+        add();
+        j = jn;
+    }
+}
+
 struct Kern {  // closed-form kernels and their radial derivatives, FP32
-    float h, a, cs, cv;
-    __device__ explicit Kern(float sr) : h(sr) {
+    float h, a, ah, cs, cv;
+    explicit Kern(float sr) : h(sr) {
         a = 2.546479089470325472f / (sr * sr * sr);  // 8 / (pi h^3)
+        ah = a / h;
         cs = -45.0f / (3.1415926535897932384626f * sr * sr * sr * sr * sr * sr);
         cv = 45.0f / (3.1415926535897932384626f * sr * sr * sr * sr * sr * sr);
     }
@@ -74,9 +117,9 @@ struct Kern {  // closed-form kernels and their radial derivatives, FP32
     __device__ float dW(float r) const {
         if (!(r < h)) return 0.0f;
         const float s = r / h;
-        if (s < 0.5f) return a / h * (-12.0f * s + 18.0f * s * s);
+        if (s < 0.5f) return ah * (-12.0f * s + 18.0f * s * s);
         const float t = 1.0f - s;
-        return a / h * (-6.0f * t * t);
+        return ah * (-6.0f * t * t);
     }
     __device__ float G(float r) const {
         if (!(r < h) || r == 0.0f) return 0.0f;
@@ -101,9 +144,11 @@ __device__ inline float softplus(float s) {
 __device__ inline float softplus_grad(float s) { return 1.0f / (1.0f + expf(-s / kTau)); }
 
 struct Consts {
-    float m, rho0, dt, q, cvis, cp, delta, g, h;
+    Kern kn;
+    float m, rho0, dt, q, cvis, cp, delta, g;
     float fd, kb;  // wall penalty: depth and stiffness 2 F_max / d_f
     float cmin[3], cmax[3];
+    explicit Consts(float sr) : kn(sr) {}
 };
 
 // wall penalty force on a liquid particle at (x, y, z) and its diagonal derivative
@@ -124,13 +169,17 @@ __device__ inline float dot3(const float4& a, const float4& b) { return a.x * b.
 __device__ inline float ax(const float4& v, int a) { return a == 0 ? v.x : (a == 1 ? v.y : v.z); }
 
 // ---------------------------------------------------------- neighbour search
+__device__ inline void put_key(const upf_params& P, float x, float y, float z, uint32_t* key, Ctl* ctl) {
+    bool ok;
+    *key = dkey(x, y, z, P.scales, ok);
+    if (!ok) atomicOr(&ctl->err, 1u << UPF_ERR_RANGE);
+}
+
 __global__ void k_keys(int n, const float4* __restrict__ x, upf_params P, uint32_t* __restrict__ keys, Ctl* ctl) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const float4 p = x[i];
-    bool ok;
-    keys[i] = dkey(p.x, p.y, p.z, P.scales, ok);
-    if (!ok) atomicOr(&ctl->err, 1u << UPF_ERR_RANGE);
+    put_key(P, p.x, p.y, p.z, keys + i, ctl);
 }
 
 __global__ void k_clear_cells(uint2* __restrict__ cells, uint32_t nc) {
@@ -138,182 +187,309 @@ __global__ void k_clear_cells(uint2* __restrict__ cells, uint32_t nc) {
     if (c < nc) cells[c] = make_uint2(0u, 0u);
 }
 
-__global__ void k_cell_bounds(int n, const uint32_t* __restrict__ keys, uint32_t shift3, uint2* __restrict__ cells) {
+// the cell table, and the positions in sorted order with their particle in w:
+// the lists read a cell's candidates as one run
+__global__ void k_cell_bounds(int n, const uint32_t* __restrict__ keys, const uint32_t* __restrict__ perm,
+                              const float4* __restrict__ x, uint32_t shift3, uint2* __restrict__ cells,
+                              float4* __restrict__ cand) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const uint32_t c = keys[i] >> shift3;
     if (i == 0 || (keys[i - 1] >> shift3) != c) cells[c].x = (uint32_t)i;
     if (i == n - 1 || (keys[i + 1] >> shift3) != c) cells[c].y = (uint32_t)(i + 1);
+    const uint32_t j = perm[i];
+    const float4 p = x[j];
+    cand[i] = make_float4(p.x, p.y, p.z, __uint_as_float(j));
 }
 
 // neighbour ids of every fluid particle: the cells of its query box (the
-// reference's BoxQuery) in Morton order, candidates in sorted order, r < h
-__global__ void k_lists(int n, const float4* __restrict__ x, const uint32_t* __restrict__ perm,
-                        const uint2* __restrict__ cells, upf_params P, uint32_t* __restrict__ nb,
-                        int* __restrict__ cnt, Ctl* ctl) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+// reference's BoxQuery) in Morton order, candidates in sorted order, r < h.
+// Sixteen lanes per particle: each finds cells of its own, their slots go to a
+// candidate table in LDS, and the lanes test sixteen candidates at a time, the
+// passing ones appended in order through the group's ballot.  Bound by the
+// latency of table and candidate reads (267 us at 80,648 particles with one
+// lane walking the cells of each).  LIST_CAND slots hold any query box of a
+// fluid; a denser one is walked cell by cell.
+constexpr int LIST_LANES = 16;
+constexpr int LIST_CAND = 384;
+__global__ __launch_bounds__(AB) void k_lists(int n, const float4* __restrict__ x, const float4* __restrict__ cand,
+                                              const uint2* __restrict__ cells, upf_params P,
+                                              uint32_t* __restrict__ nb, int* __restrict__ cnt, Ctl* ctl) {
+    __shared__ uint32_t table[AB / LIST_LANES][LIST_CAND];
+    const int i = (int)((blockIdx.x * AB + threadIdx.x) / LIST_LANES);
+    const int sub = threadIdx.x % LIST_LANES;
     if (i >= n) return;
     const float4 xi = x[i];
-    if (!is_fluid(xi)) { cnt[i] = 0; return; }
+    if (!is_fluid(xi)) {
+        if (sub == 0) cnt[i] = 0;
+        return;
+    }
     const float h = P.support_radius, hh = h * h;
     const int cap = P.max_neighbors;
+    uint32_t* row = nb + (size_t)i * cap;
+    uint32_t* tab = table[threadIdx.x / LIST_LANES];
+    const int shift = (threadIdx.x & 63) & ~(LIST_LANES - 1);  // the group's bits of the wave's ballot
+    int c = 0;
+    // tests one candidate per lane (slot s, if any) and appends the passing ones
+    auto test = [&](bool have, const float4& xj) __attribute__((always_inline)) {
+        const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+        const uint32_t j = __float_as_uint(xj.w);
+        const bool pass = have && j != (uint32_t)i && dx * dx + dy * dy + dz * dz < hh;
+        const uint32_t m = (uint32_t)(__ballot(pass) >> shift) & 0xFFFFu;
+        const int at = c + __popc(m & ((1u << sub) - 1u));
+        if (pass && at < cap) row[at] = j;
+        c += __popc(m);
+    };
     BoxCells bc;
     bc.init(xi.x, xi.y, xi.z, h, P.scales, P.block_shift);
-    int c = 0;
-    for (int e = 0; e < bc.count(); ++e) {
-        uint32_t q[3];
-        if (!bc.cell(e, q)) continue;
-        if (q[0] >= P.grid_dim || q[1] >= P.grid_dim || q[2] >= P.grid_dim) continue;
-        const uint2 r = cells[dmorton3(q[0], q[1], q[2])];
-        for (uint32_t s = r.x; s < r.y; ++s) {
-            const int j = (int)perm[s];
-            if (j == i) continue;
-            const float4 xj = x[j];
-            const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-            if (dx * dx + dy * dy + dz * dz < hh) {
-                if (c < cap) nb[(size_t)c * n + i] = (uint32_t)j;
-                ++c;
-            }
-        }
+    // this lane's cells: enumeration indices sub, sub + 16, ... (at most 64)
+    uint2 r[4];
+    uint32_t before[4];  // candidates of the box in earlier cells
+    uint32_t total = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        r[q] = make_uint2(0u, 0u);
+        uint32_t g[3];
+        const int e = q * LIST_LANES + sub;
+        if (e < bc.count() && bc.cell(e, g) && g[0] < P.grid_dim && g[1] < P.grid_dim && g[2] < P.grid_dim)
+            r[q] = cells[dmorton3(g[0], g[1], g[2])];
     }
-    cnt[i] = c < cap ? c : cap;
-    if (c > cap) atomicOr(&ctl->err, 1u << UPF_ERR_NBR_OVERFLOW);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        uint32_t incl = r[q].y - r[q].x;
+#pragma unroll
+        for (int o = 1; o < LIST_LANES; o <<= 1) {
+            const uint32_t y = (uint32_t)__shfl_up((int)incl, o, LIST_LANES);
+            if (sub >= o) incl += y;
+        }
+        before[q] = total + incl - (r[q].y - r[q].x);
+        total += (uint32_t)__shfl((int)incl, LIST_LANES - 1, LIST_LANES);
+    }
+    if (total <= LIST_CAND) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            for (uint32_t s = r[q].x; s < r[q].y; ++s) tab[before[q] + (s - r[q].x)] = s;
+        // the group's lanes are in one wave: its LDS writes are in order before its reads
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        // four rounds' candidates are loaded together
+        for (uint32_t t = (uint32_t)sub; t - (uint32_t)sub < total; t += 4 * LIST_LANES) {
+            float4 xj[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                xj[q] = cand[tab[min(t + q * LIST_LANES, total - 1u)]];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) test(t + q * LIST_LANES < total, xj[q]);
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            for (int u = 0; u < LIST_LANES; ++u) {
+                const uint32_t s0 = (uint32_t)__shfl((int)r[q].x, u, LIST_LANES);
+                const uint32_t s1 = (uint32_t)__shfl((int)r[q].y, u, LIST_LANES);
+                for (uint32_t s = s0; s < s1; s += LIST_LANES)
+                    test(s + sub < s1, cand[min(s + (uint32_t)sub, s1 - 1u)]);
+            }
+    }
+    if (sub == 0) {
+        cnt[i] = c < cap ? c : cap;
+        if (c > cap) atomicOr(&ctl->err, 1u << UPF_ERR_NBR_OVERFLOW);
+    }
 }
 
 // --------------------------------------------------------------- forward
-__global__ void k_ext(int n, const float4* __restrict__ x, const float4* __restrict__ v, const uint32_t* __restrict__ nb,
-                      const int* __restrict__ cnt, Consts C, float4* __restrict__ F, float4* __restrict__ Fp,
-                      float* __restrict__ p) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float4 xi = x[i];
-    Fp[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    p[i] = 0.0f;
-    if (!is_fluid(xi)) { F[i] = make_float4(0.f, 0.f, 0.f, 0.f); return; }
-    const Kern kn(C.h);
-    const float4 vi = v[i];
-    float fx = 0.0f, fy = 0.0f, fz = 0.0f;
-    const int c = cnt[i];
-    for (int k = 0; k < c; ++k) {
-        const int j = (int)nb[(size_t)k * n + i];
-        const float4 xj = x[j];
-        if (!is_fluid(xj)) continue;
-        const float r = len3(xi.x - xj.x, xi.y - xj.y, xi.z - xj.z);
-        const float4 vj = v[j];
-        const float s = C.cvis * kn.L(r);
-        fx = fx - (vi.x - vj.x) * s;
-        fy = fy - (vi.y - vj.y) * s;
-        fz = fz - (vi.z - vj.z) * s;
-    }
-    fy = fy - C.m * C.g;
-    float wf[3], wg[3];
-    wall_force(C, xi.x, xi.y, xi.z, wf, wg);
-    F[i] = make_float4(fx + wf[0], fy + wf[1], fz + wf[2], 0.0f);
-}
-
 __device__ inline float clampc(float c, float mn, float mx) {
     if (c < mn) c = mn;
     if (c > mx) c = mx;
     return c;
 }
+__device__ inline bool outside(float c, int a, const Consts& C) { return c < C.cmin[a] || c > C.cmax[a]; }
 
-// prediction of iteration k: z (unclamped) to the tape, x* = clamp(z)
-__global__ void k_predict(int n, const float4* __restrict__ x, const float4* __restrict__ v, const float4* __restrict__ F,
-                          const float4* __restrict__ Fp, Consts C, float4* __restrict__ xs, float4* __restrict__ z,
-                          Ctl* ctl) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float4 xi = x[i];
-    if (!is_fluid(xi)) { xs[i] = xi; if (z) z[i] = xi; return; }
-    const float4 vi = v[i], f = F[i], fp = Fp[i];
-    const float vx = vi.x + (f.x + fp.x) * C.q, vy = vi.y + (f.y + fp.y) * C.q, vz = vi.z + (f.z + fp.z) * C.q;
-    const float4 zz = make_float4(xi.x + vx * C.dt, xi.y + vy * C.dt, xi.z + vz * C.dt, xi.w);
-    if (z) z[i] = zz;
-    xs[i] = make_float4(clampc(zz.x, C.cmin[0], C.cmax[0]), clampc(zz.y, C.cmin[1], C.cmax[1]),
-                        clampc(zz.z, C.cmin[2], C.cmax[2]), xi.w);
-    if (!(zz.x == zz.x) || !(zz.y == zz.y) || !(zz.z == zz.z)) atomicOr(&ctl->err, 1u << UPF_ERR_NAN);
+// type bits of a predicted or new position, with the axes that the clamp moved
+// above them (the reverse passes' derivative of the clamp)
+constexpr int OUT_SHIFT = 8;
+__device__ inline float type_and_out(float tw, float x, float y, float z, const Consts& C) {
+    const int out = (outside(x, 0, C) ? 1 : 0) | (outside(y, 1, C) ? 2 : 0) | (outside(z, 2, C) ? 4 : 0);
+    return __int_as_float(__float_as_int(tw) | out << OUT_SHIFT);
+}
+__device__ inline bool moved(float w, int a) { return (__float_as_int(w) >> (OUT_SHIFT + a)) & 1; }
+__device__ inline bool is_fluid_w(float w) { return (__float_as_int(w) & ((1 << OUT_SHIFT) - 1)) == UPF_LIQUID; }
+
+// prediction of an iteration: x* = clamp(z)
+__device__ inline float4 predict(const float4& xi, const float4& vi, float fx, float fy, float fz, const float4& f,
+                                 const Consts& C, Ctl* ctl) {
+    const float vx = vi.x + (f.x + fx) * C.q, vy = vi.y + (f.y + fy) * C.q, vz = vi.z + (f.z + fz) * C.q;
+    const float zx = xi.x + vx * C.dt, zy = xi.y + vy * C.dt, zz = xi.z + vz * C.dt;
+    if (!(zx == zx) || !(zy == zy) || !(zz == zz)) atomicOr(&ctl->err, 1u << UPF_ERR_NAN);
+    return make_float4(clampc(zx, C.cmin[0], C.cmax[0]), clampc(zy, C.cmin[1], C.cmax[1]),
+                       clampc(zz, C.cmin[2], C.cmax[2]), type_and_out(xi.w, zx, zy, zz, C));
 }
 
-__global__ void k_density(int n, const float4* __restrict__ xs, const uint32_t* __restrict__ nb,
-                          const int* __restrict__ cnt, Consts C, float* __restrict__ p, float* __restrict__ p_tape,
-                          float* __restrict__ rho_tape) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+// external force, and the first iteration's prediction.  Clears the cell table
+// for the next step: the lists of this one are built.
+template <int LANES>
+__global__ __launch_bounds__(AB) void k_ext(int n, const float4* __restrict__ x, const float4* __restrict__ v,
+                                            const uint32_t* __restrict__ nb, const int* __restrict__ cnt, int ld,
+                                            Consts C, float4* __restrict__ F, float* __restrict__ p,
+                                            float4* __restrict__ xs, uint2* __restrict__ cells, uint32_t nc, Ctl* ctl) {
+    const unsigned id = blockIdx.x * AB + threadIdx.x;
+    for (uint32_t c = id; c < nc; c += gridDim.x * AB) cells[c] = make_uint2(0u, 0u);
+    const int i = (int)(id / LANES), sub = (int)(id % LANES);
+    if (i >= n) return;
+    const float4 xi = x[i];
+    if (!is_fluid(xi)) {
+        if (sub == 0) {
+            F[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            p[i] = 0.0f;
+            xs[i] = xi;
+        }
+        return;
+    }
+    const float4 vi = v[i];
+    float fx = 0.0f, fy = 0.0f, fz = 0.0f, tx, ty, tz;
+    auto none = [&] { tx = ty = tz = 0.0f; };
+    for_pairs<LANES>(
+        nb + (size_t)i * ld, cnt[i], sub,
+        [&](int j) {
+            const float4 xj = x[j], vj = v[j];
+            if (!is_fluid(xj)) return none();
+            const float r = len3(xi.x - xj.x, xi.y - xj.y, xi.z - xj.z);
+            const float s = C.cvis * C.kn.L(r);
+            tx = (vi.x - vj.x) * s;
+            ty = (vi.y - vj.y) * s;
+            tz = (vi.z - vj.z) * s;
+        },
+        none,
+        [&] {
+            fx = sub_terms<LANES>(fx, tx);
+            fy = sub_terms<LANES>(fy, ty);
+            fz = sub_terms<LANES>(fz, tz);
+        });
+    if (sub != 0) return;
+    fy = fy - C.m * C.g;
+    float wf[3], wg[3];
+    wall_force(C, xi.x, xi.y, xi.z, wf, wg);
+    const float4 f = make_float4(fx + wf[0], fy + wf[1], fz + wf[2], 0.0f);
+    F[i] = f;
+    p[i] = 0.0f;
+    xs[i] = predict(xi, vi, 0.0f, 0.0f, 0.0f, f, C, ctl);
+}
+
+// density and pressure of an iteration; rec: position and pressure, the
+// pressure force's one gather per neighbour
+template <int LANES>
+__global__ __launch_bounds__(AB) void k_density(int n, const float4* __restrict__ x, const float4* __restrict__ xs,
+                                                const uint32_t* __restrict__ nb, const int* __restrict__ cnt, int ld,
+                                                Consts C, float* __restrict__ p, float4* __restrict__ rec,
+                                                float* __restrict__ p_tape, float* __restrict__ rho_tape) {
+    const unsigned id = blockIdx.x * AB + threadIdx.x;
+    const int i = (int)(id / LANES), sub = (int)(id % LANES);
     if (i >= n) return;
     const float4 xi = xs[i];
-    if (!is_fluid(xi)) { if (p_tape) { p_tape[i] = 0.0f; rho_tape[i] = 0.0f; } return; }
-    const Kern kn(C.h);
-    float r_ = C.m * kn.W(0.0f);
-    const int c = cnt[i];
-    for (int k = 0; k < c; ++k) {
-        const float4 xj = xs[nb[(size_t)k * n + i]];
-        r_ = r_ + C.m * kn.W(len3(xi.x - xj.x, xi.y - xj.y, xi.z - xj.z));
+    float rho = 0.0f, pi = 0.0f;
+    if (is_fluid_w(xi.w)) {
+        rho = C.m * C.kn.W(0.0f);
+        float t;
+        for_pairs<LANES>(
+            nb + (size_t)i * ld, cnt[i], sub,
+            [&](int j) {
+                const float4 xj = xs[j];
+                t = C.m * C.kn.W(len3(xi.x - xj.x, xi.y - xj.y, xi.z - xj.z));
+            },
+            [&] { t = -0.0f; }, [&] { rho = add_terms<LANES>(rho, t); });
+        pi = p[i] + C.delta * softplus(rho - C.rho0);
     }
-    const float pi = p[i] + C.delta * softplus(r_ - C.rho0);
+    if (sub != 0) return;
+    const float4 xc = x[i];
+    rec[i] = make_float4(xc.x, xc.y, xc.z, pi);
     p[i] = pi;
-    if (p_tape) { p_tape[i] = pi; rho_tape[i] = r_; }
+    if (p_tape) { p_tape[i] = pi; rho_tape[i] = rho; }
 }
 
-__global__ void k_pforce(int n, const float4* __restrict__ x, const uint32_t* __restrict__ nb,
-                         const int* __restrict__ cnt, Consts C, const float* __restrict__ p, float4* __restrict__ Fp) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+// pressure force of an iteration, then the next iteration's prediction (LAST:
+// the integration, and the new positions' keys for the next step's sort)
+template <int LANES, bool LAST>
+__global__ __launch_bounds__(AB) void k_pforce(int n, const float4* __restrict__ x, const float4* __restrict__ v,
+                                               const uint32_t* __restrict__ nb, const int* __restrict__ cnt, int ld,
+                                               Consts C, const float4* __restrict__ rec, const float4* __restrict__ F,
+                                               float4* __restrict__ xs, float4* __restrict__ x_new,
+                                               float4* __restrict__ v_new, float* __restrict__ y_tape, upf_params P,
+                                               uint32_t* __restrict__ keys, Ctl* ctl) {
+    const unsigned id = blockIdx.x * AB + threadIdx.x;
+    const int i = (int)(id / LANES), sub = (int)(id % LANES);
     if (i >= n) return;
     const float4 xi = x[i];
-    if (!is_fluid(xi)) return;
-    const Kern kn(C.h);
-    const float pi = p[i];
-    float fx = 0.0f, fy = 0.0f, fz = 0.0f;
-    const int c = cnt[i];
-    for (int k = 0; k < c; ++k) {
-        const int j = (int)nb[(size_t)k * n + i];
-        const float4 xj = x[j];
-        const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-        const float r = len3(dx, dy, dz);
-        const float pj = is_fluid(xj) ? p[j] : 0.0f;
-        const float s = kn.G(r) * (pi + pj) * C.cp;
-        fx = fx - dx * s;
-        fy = fy - dy * s;
-        fz = fz - dz * s;
+    float4 xn = xi, vn;
+    float yw = xi.w;
+    if (!is_fluid(xi)) {
+        if (sub != 0) return;
+        if constexpr (!LAST) {
+            xs[i] = xi;
+            return;
+        }
+        vn = v[i];
+    } else {
+        const float pi = rec[i].w;
+        float fx = 0.0f, fy = 0.0f, fz = 0.0f, tx, ty, tz;
+        for_pairs<LANES>(
+            nb + (size_t)i * ld, cnt[i], sub,
+            [&](int j) {
+                const float4 xj = rec[j];
+                const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+                const float s = C.kn.G(len3(dx, dy, dz)) * (pi + xj.w) * C.cp;
+                tx = dx * s;
+                ty = dy * s;
+                tz = dz * s;
+            },
+            [&] { tx = ty = tz = 0.0f; },
+            [&] {
+                fx = sub_terms<LANES>(fx, tx);
+                fy = sub_terms<LANES>(fy, ty);
+                fz = sub_terms<LANES>(fz, tz);
+            });
+        if (sub != 0) return;
+        const float4 vi = v[i], f = F[i];
+        if constexpr (!LAST) {
+            xs[i] = predict(xi, vi, fx, fy, fz, f, C, ctl);
+            return;
+        }
+        const float v3[3] = {vi.x + (f.x + fx) * C.q, vi.y + (f.y + fy) * C.q, vi.z + (f.z + fz) * C.q};
+        const float xo[3] = {xi.x, xi.y, xi.z};
+        float y[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) y[a] = xo[a] + v3[a] * C.dt;
+        yw = type_and_out(xi.w, y[0], y[1], y[2], C);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) y[a] = clampc(y[a], C.cmin[a], C.cmax[a]);
+        xn = make_float4(y[0], y[1], y[2], xi.w);
+        vn = make_float4(v3[0], v3[1], v3[2], 0.0f);
     }
-    Fp[i] = make_float4(fx, fy, fz, 0.0f);
-}
-
-__global__ void k_integrate(int n, float4* __restrict__ x, float4* __restrict__ v, const float4* __restrict__ F,
-                            const float4* __restrict__ Fp, Consts C, float4* __restrict__ y_tape) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float4 xi = x[i];
-    if (!is_fluid(xi)) { if (y_tape) y_tape[i] = xi; return; }
-    const float4 vi = v[i], f = F[i], fp = Fp[i];
-    const float vn[3] = {vi.x + (f.x + fp.x) * C.q, vi.y + (f.y + fp.y) * C.q, vi.z + (f.z + fp.z) * C.q};
-    const float xo[3] = {xi.x, xi.y, xi.z};
-    float y[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) y[a] = xo[a] + vn[a] * C.dt;
-    if (y_tape) y_tape[i] = make_float4(y[0], y[1], y[2], xi.w);
-#pragma unroll
-    for (int a = 0; a < 3; ++a) y[a] = clampc(y[a], C.cmin[a], C.cmax[a]);
-    x[i] = make_float4(y[0], y[1], y[2], xi.w);
-    v[i] = make_float4(vn[0], vn[1], vn[2], 0.0f);
+    x_new[i] = xn;
+    v_new[i] = vn;
+    if (y_tape) y_tape[i] = yw;
+    if (keys) put_key(P, xn.x, xn.y, xn.z, keys + i, ctl);
 }
 
 // -------------------------------------------------------------- backward
-__device__ inline bool outside(float c, int a, const Consts& C) { return c < C.cmin[a] || c > C.cmax[a]; }
-
-// reverse of the integration: (gx, gv) = dL/d(x', v') -> nx, nv, gF, gFp
-__global__ void kr_integrate(int n, const float4* __restrict__ y, const float4* __restrict__ gx,
-                             const float4* __restrict__ gv, Consts C, float4* __restrict__ nx, float4* __restrict__ nv,
-                             float4* __restrict__ gF, float4* __restrict__ gFp, float* __restrict__ gp) {
+// reverse of the integration: (gx, gv) = dL/d(x', v') -> nx, nv, gF, and gFp
+// with the last iteration's pressure in w.  Both gFp buffers are zero for
+// walls, which the pressure force's reverse reads as a neighbour's.
+__global__ void kr_integrate(int n, const float* __restrict__ y, const float4* __restrict__ gx,
+                             const float4* __restrict__ gv, Consts C, const float* __restrict__ p,
+                             float4* __restrict__ nx, float4* __restrict__ nv, float4* __restrict__ gF,
+                             float4* __restrict__ gFp, float4* __restrict__ gFp2, float* __restrict__ gp) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const float4 yi = y[i];
+    const float yi = y[i];
     const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
     gp[i] = 0.0f;
-    if (!is_fluid(yi)) { nx[i] = z4; nv[i] = z4; gF[i] = z4; gFp[i] = z4; return; }
+    if (!is_fluid_w(yi)) { nx[i] = z4; nv[i] = z4; gF[i] = z4; gFp[i] = z4; gFp2[i] = z4; return; }
     const float4 a = gx[i], b = gv[i];
     float gy[3], gvn[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        gy[k] = outside(ax(yi, k), k, C) ? 0.0f : ax(a, k);
+        gy[k] = moved(yi, k) ? 0.0f : ax(a, k);
         gvn[k] = ax(b, k);
     }
 #pragma unroll
@@ -322,89 +498,101 @@ __global__ void kr_integrate(int n, const float4* __restrict__ y, const float4* 
     nv[i] = make_float4(gvn[0], gvn[1], gvn[2], 0.0f);
     const float4 f = make_float4(gvn[0] * C.q, gvn[1] * C.q, gvn[2] * C.q, 0.0f);
     gF[i] = f;
-    gFp[i] = f;
+    gFp[i] = make_float4(f.x, f.y, f.z, p[i]);
 }
 
-// reverse of the pressure force of one iteration: dL/dp (running) and dL/dx
-__global__ void kr_pforce(int n, const float4* __restrict__ x, const uint32_t* __restrict__ nb,
-                          const int* __restrict__ cnt, Consts C, const float* __restrict__ p,
-                          const float4* __restrict__ gFp, float* __restrict__ gp, float4* __restrict__ nx) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+// reverse of the pressure force of one iteration: dL/dp (running) and dL/dx,
+// then dL/drho, which goes with the predicted position into rec, the density
+// reverse's one gather per neighbour
+template <int LANES>
+__global__ __launch_bounds__(AB) void kr_pforce(int n, const float4* __restrict__ x, const uint32_t* __restrict__ nb,
+                                                const int* __restrict__ cnt, int ld, Consts C,
+                                                const float4* __restrict__ gFp, const float4* __restrict__ xs,
+                                                const float* __restrict__ rho, float* __restrict__ gp,
+                                                float4* __restrict__ nx, float4* __restrict__ rec) {
+    const unsigned id = blockIdx.x * AB + threadIdx.x;
+    const int i = (int)(id / LANES), sub = (int)(id % LANES);
     if (i >= n) return;
-    const float4 xi = x[i];
-    if (!is_fluid(xi)) return;
-    const Kern kn(C.h);
-    const float4 gi = gFp[i];
-    const float pi = p[i];
-    float acc = 0.0f, gxx = 0.0f, gxy = 0.0f, gxz = 0.0f;
-    const int c = cnt[i];
-    for (int k = 0; k < c; ++k) {
-        const int j = (int)nb[(size_t)k * n + i];
-        const float4 xj = x[j];
-        const float4 d = make_float4(xi.x - xj.x, xi.y - xj.y, xi.z - xj.z, 0.0f);
-        const float r = len3(d.x, d.y, d.z);
-        const bool fj = is_fluid(xj);
-        const float4 gj = fj ? gFp[j] : make_float4(0.f, 0.f, 0.f, 0.f);
-        const float4 w = fj ? make_float4(gi.x - gj.x, gi.y - gj.y, gi.z - gj.z, 0.0f) : gi;
-        const float G = kn.G(r);
-        const float dw = dot3(d, w);
-        acc = acc - C.cp * G * dw;
-        const float pp = pi + (fj ? p[j] : 0.0f);
-        const float s = r > 0.0f ? kn.dG(r) / r * dw : 0.0f;
-        const float t = C.cp * pp;
-        gxx = gxx - (w.x * G + d.x * s) * t;
-        gxy = gxy - (w.y * G + d.y * s) * t;
-        gxz = gxz - (w.z * G + d.z * s) * t;
+    const float4 xi = x[i], xsi = xs[i];
+    if (!is_fluid(xi)) {
+        if (sub == 0) rec[i] = make_float4(xsi.x, xsi.y, xsi.z, 0.0f);
+        return;
     }
-    gp[i] = gp[i] + acc;
+    const float4 gi = gFp[i];
+    float acc = 0.0f, gxx = 0.0f, gxy = 0.0f, gxz = 0.0f, ta, tx, ty, tz;
+    for_pairs<LANES>(
+        nb + (size_t)i * ld, cnt[i], sub,
+        [&](int j) {
+            const float4 xj = x[j], gj = gFp[j];
+            const float4 d = make_float4(xi.x - xj.x, xi.y - xj.y, xi.z - xj.z, 0.0f);
+            const float r = len3(d.x, d.y, d.z);
+            const float4 w = make_float4(gi.x - gj.x, gi.y - gj.y, gi.z - gj.z, 0.0f);
+            const float G = C.kn.G(r);
+            const float dw = dot3(d, w);
+            ta = C.cp * G * dw;
+            const float pp = gi.w + gj.w;
+            const float s = r > 0.0f ? C.kn.dG(r) / r * dw : 0.0f;
+            const float t = C.cp * pp;
+            tx = (w.x * G + d.x * s) * t;
+            ty = (w.y * G + d.y * s) * t;
+            tz = (w.z * G + d.z * s) * t;
+        },
+        [&] { ta = tx = ty = tz = 0.0f; },
+        [&] {
+            acc = sub_terms<LANES>(acc, ta);
+            gxx = sub_terms<LANES>(gxx, tx);
+            gxy = sub_terms<LANES>(gxy, ty);
+            gxz = sub_terms<LANES>(gxz, tz);
+        });
+    if (sub != 0) return;
+    const float g = gp[i] + acc;
+    gp[i] = g;
     float4 o = nx[i];
     o.x = o.x + gxx; o.y = o.y + gxy; o.z = o.z + gxz;
     nx[i] = o;
+    rec[i] = make_float4(xsi.x, xsi.y, xsi.z, C.delta * g * softplus_grad(rho[i] - C.rho0));
 }
 
-// reverse of density, pressure update and prediction of one iteration
-__global__ void kr_density(int n, const float4* __restrict__ x, const float4* __restrict__ z,
-                           const uint32_t* __restrict__ nb, const int* __restrict__ cnt, Consts C,
-                           const float* __restrict__ rho, const float* __restrict__ gp, float4* __restrict__ nx,
-                           float4* __restrict__ nv, float4* __restrict__ gF, float4* __restrict__ gFp_prev) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+// reverse of density, pressure update and prediction of one iteration; p_prev:
+// the pressures of the iteration before (null before the first)
+template <int LANES>
+__global__ __launch_bounds__(AB) void kr_density(int n, const float4* __restrict__ xs, const float4* __restrict__ rec,
+                                                 const uint32_t* __restrict__ nb, const int* __restrict__ cnt, int ld,
+                                                 Consts C, const float* __restrict__ p_prev, float4* __restrict__ nx,
+                                                 float4* __restrict__ nv, float4* __restrict__ gF,
+                                                 float4* __restrict__ gFp_prev) {
+    const unsigned id = blockIdx.x * AB + threadIdx.x;
+    const int i = (int)(id / LANES), sub = (int)(id % LANES);
     if (i >= n) return;
-    const float4 xi = x[i];
-    if (!is_fluid(xi)) return;
-    const Kern kn(C.h);
-    const float4 zi = z[i];
-    const float xsi[3] = {clampc(zi.x, C.cmin[0], C.cmax[0]), clampc(zi.y, C.cmin[1], C.cmax[1]),
-                          clampc(zi.z, C.cmin[2], C.cmax[2])};
-    const float gri = C.delta * gp[i] * softplus_grad(rho[i] - C.rho0);
-    float gx = 0.0f, gy = 0.0f, gz = 0.0f;
-    const int c = cnt[i];
-    for (int k = 0; k < c; ++k) {
-        const int j = (int)nb[(size_t)k * n + i];
-        const float4 xj = x[j];
-        float xsj[3];
-        float grj = 0.0f;
-        if (is_fluid(xj)) {
-            const float4 zj = z[j];
-            xsj[0] = clampc(zj.x, C.cmin[0], C.cmax[0]);
-            xsj[1] = clampc(zj.y, C.cmin[1], C.cmax[1]);
-            xsj[2] = clampc(zj.z, C.cmin[2], C.cmax[2]);
-            grj = C.delta * gp[j] * softplus_grad(rho[j] - C.rho0);
-        } else {
-            xsj[0] = xj.x; xsj[1] = xj.y; xsj[2] = xj.z;
-        }
-        const float dx = xsi[0] - xsj[0], dy = xsi[1] - xsj[1], dz = xsi[2] - xsj[2];
-        const float r = len3(dx, dy, dz);
-        if (!(r < kn.h) || r == 0.0f) continue;
-        const float gr = gri + grj;
-        const float s = C.m * kn.dW(r) / r * gr;
-        gx = gx + dx * s;
-        gy = gy + dy * s;
-        gz = gz + dz * s;
-    }
+    const float w = xs[i].w;
+    if (!is_fluid_w(w)) return;
+    const float4 xi = rec[i];
+    float gx = 0.0f, gy = 0.0f, gz = 0.0f, tx, ty, tz;
+    auto none = [&] { tx = ty = tz = -0.0f; };
+    for_pairs<LANES>(
+        nb + (size_t)i * ld, cnt[i], sub,
+        [&](int j) {
+            const float4 xj = rec[j];
+            const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+            const float r = len3(dx, dy, dz);
+            if (!(r < C.kn.h) || r == 0.0f) return none();
+            const float gr = xi.w + xj.w;
+            const float s = C.m * C.kn.dW(r) / r * gr;
+            tx = dx * s;
+            ty = dy * s;
+            tz = dz * s;
+        },
+        none,
+        [&] {
+            gx = add_terms<LANES>(gx, tx);
+            gy = add_terms<LANES>(gy, ty);
+            gz = add_terms<LANES>(gz, tz);
+        });
+    if (sub != 0) return;
     const float g3[3] = {gx, gy, gz};
     float zb[3];
 #pragma unroll
-    for (int a = 0; a < 3; ++a) zb[a] = outside(ax(zi, a), a, C) ? 0.0f : g3[a];
+    for (int a = 0; a < 3; ++a) zb[a] = moved(w, a) ? 0.0f : g3[a];
     float4 o = nx[i];
     o.x = o.x + zb[0]; o.y = o.y + zb[1]; o.z = o.z + zb[2];
     nx[i] = o;
@@ -415,42 +603,55 @@ __global__ void kr_density(int n, const float4* __restrict__ x, const float4* __
     float4 of = gF[i];
     of.x = of.x + vs[0] * C.q; of.y = of.y + vs[1] * C.q; of.z = of.z + vs[2] * C.q;
     gF[i] = of;
-    gFp_prev[i] = make_float4(vs[0] * C.q, vs[1] * C.q, vs[2] * C.q, 0.0f);
+    gFp_prev[i] = make_float4(vs[0] * C.q, vs[1] * C.q, vs[2] * C.q, p_prev ? p_prev[i] : 0.0f);
 }
 
 // reverse of the viscosity force
-__global__ void kr_ext(int n, const float4* __restrict__ x, const float4* __restrict__ v, const uint32_t* __restrict__ nb,
-                       const int* __restrict__ cnt, Consts C, const float4* __restrict__ gF, float4* __restrict__ nx,
-                       float4* __restrict__ nv) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+template <int LANES>
+__global__ __launch_bounds__(AB) void kr_ext(int n, const float4* __restrict__ x, const float4* __restrict__ v,
+                                             const uint32_t* __restrict__ nb, const int* __restrict__ cnt, int ld,
+                                             Consts C, const float4* __restrict__ gF, float4* __restrict__ nx,
+                                             float4* __restrict__ nv) {
+    const unsigned id = blockIdx.x * AB + threadIdx.x;
+    const int i = (int)(id / LANES), sub = (int)(id % LANES);
     if (i >= n) return;
     const float4 xi = x[i];
     if (!is_fluid(xi)) return;
-    const Kern kn(C.h);
     const float4 vi = v[i], gi = gF[i];
     float gvx = 0.0f, gvy = 0.0f, gvz = 0.0f, gxx = 0.0f, gxy = 0.0f, gxz = 0.0f;
-    const int c = cnt[i];
-    for (int k = 0; k < c; ++k) {
-        const int j = (int)nb[(size_t)k * n + i];
-        const float4 xj = x[j];
-        if (!is_fluid(xj)) continue;
-        const float4 d = make_float4(xi.x - xj.x, xi.y - xj.y, xi.z - xj.z, 0.0f);
-        const float r = len3(d.x, d.y, d.z);
-        const float4 gj = gF[j];
-        const float4 w = make_float4(gi.x - gj.x, gi.y - gj.y, gi.z - gj.z, 0.0f);
-        const float sl = C.cvis * kn.L(r);
-        gvx = gvx - w.x * sl;
-        gvy = gvy - w.y * sl;
-        gvz = gvz - w.z * sl;
-        if (r > 0.0f) {
-            const float4 vj = v[j];
-            const float4 dv = make_float4(vi.x - vj.x, vi.y - vj.y, vi.z - vj.z, 0.0f);
-            const float s = C.cvis * kn.dL(r) / r * dot3(dv, w);
-            gxx = gxx - d.x * s;
-            gxy = gxy - d.y * s;
-            gxz = gxz - d.z * s;
-        }
-    }
+    float tvx, tvy, tvz, tx, ty, tz;
+    auto none = [&] { tvx = tvy = tvz = tx = ty = tz = 0.0f; };
+    for_pairs<LANES>(
+        nb + (size_t)i * ld, cnt[i], sub,
+        [&](int j) {
+            const float4 xj = x[j], gj = gF[j], vj = v[j];
+            if (!is_fluid(xj)) return none();
+            const float4 d = make_float4(xi.x - xj.x, xi.y - xj.y, xi.z - xj.z, 0.0f);
+            const float r = len3(d.x, d.y, d.z);
+            const float4 w = make_float4(gi.x - gj.x, gi.y - gj.y, gi.z - gj.z, 0.0f);
+            const float sl = C.cvis * C.kn.L(r);
+            tvx = w.x * sl;
+            tvy = w.y * sl;
+            tvz = w.z * sl;
+            tx = ty = tz = 0.0f;
+            if (r > 0.0f) {
+                const float4 dv = make_float4(vi.x - vj.x, vi.y - vj.y, vi.z - vj.z, 0.0f);
+                const float s = C.cvis * C.kn.dL(r) / r * dot3(dv, w);
+                tx = d.x * s;
+                ty = d.y * s;
+                tz = d.z * s;
+            }
+        },
+        none,
+        [&] {
+            gvx = sub_terms<LANES>(gvx, tvx);
+            gvy = sub_terms<LANES>(gvy, tvy);
+            gvz = sub_terms<LANES>(gvz, tvz);
+            gxx = sub_terms<LANES>(gxx, tx);
+            gxy = sub_terms<LANES>(gxy, ty);
+            gxz = sub_terms<LANES>(gxz, tz);
+        });
+    if (sub != 0) return;
     float wf[3], wg[3];
     wall_force(C, xi.x, xi.y, xi.z, wf, wg);
     gxx = gxx + gi.x * wg[0];
@@ -484,23 +685,25 @@ struct upf_adjoint {
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     float fwd_ms = 0.0f, bwd_ms = 0.0f;
     std::vector<void*> allocs;
-    // state and neighbour search
-    float4 *x = nullptr, *v = nullptr;
+    // state between steps (two buffers) and neighbour search
+    float4 *x[2] = {nullptr, nullptr}, *v[2] = {nullptr, nullptr};
     uint32_t *keys = nullptr, *skeys = nullptr, *perm = nullptr;
     uint2* cells = nullptr;
+    float4* cand = nullptr;
     uint32_t ncells = 0;
     void* sort_tmp = nullptr;
     Ctl* ctl = nullptr;
-    // forward work
-    float4 *F = nullptr, *Fp = nullptr, *xs = nullptr;
+    // forward work; rec: the pair passes' gathered records
+    float4 *F = nullptr, *xs = nullptr, *rec = nullptr;
     float* p = nullptr;
     // checkpoints (x, v) at the start of every segment
     float4 *ck_x = nullptr, *ck_v = nullptr;
-    // segment tape: per step x, v, y, lists; per iteration z, p, rho
-    float4 *t_x = nullptr, *t_v = nullptr, *t_y = nullptr, *t_z = nullptr;
+    // segment tape: per step (after the segment's first) x, v, per step y's
+    // type and clamped axes, lists; per iteration x*, p, rho
+    float4 *t_x = nullptr, *t_v = nullptr, *t_xs = nullptr;
     uint32_t* t_nb = nullptr;
     int* t_cnt = nullptr;
-    float *t_p = nullptr, *t_rho = nullptr;
+    float *t_y = nullptr, *t_p = nullptr, *t_rho = nullptr;
     // adjoint state
     float4 *gx = nullptr, *gv = nullptr, *nx = nullptr, *nv = nullptr, *gF = nullptr, *gFp = nullptr, *gFp2 = nullptr;
     float* gp = nullptr;
@@ -511,7 +714,7 @@ struct upf_adjoint {
         return e;
     }
     Consts consts() const {
-        Consts C;
+        Consts C(P.support_radius);
         C.m = P.initial_mass;
         C.rho0 = P.rest_density;
         C.dt = P.dt;
@@ -520,7 +723,6 @@ struct upf_adjoint {
         C.cp = (P.initial_mass * P.initial_mass) / (P.rest_density * P.rest_density);
         C.delta = P.density_error_factor;
         C.g = P.gravity;
-        C.h = P.support_radius;
         C.fd = P.force_distance;
         C.kb = 2.0f * P.max_boundary_force / P.force_distance;
         for (int a = 0; a < 3; ++a) {
@@ -529,66 +731,71 @@ struct upf_adjoint {
         }
         return C;
     }
-    dim3 grid() const { return dim3((unsigned)((n + AB - 1) / AB)); }
+    dim3 grid(int per = 1) const { return dim3((unsigned)(((size_t)n * per + AB - 1) / AB)); }
+    // Lanes per particle of the pair passes: a row of 16 where quads would
+    // leave the SIMDs with less than two waves each (16 lanes of a partial last
+    // round idle, and each particle's own work is repeated on all of them).
+    int lanes() const { return n < 32768 ? 16 : 4; }
     size_t nb_stride() const { return (size_t)P.max_neighbors * n; }
 };
 
-// lists of the positions in a->x into (nb, cnt)
-static void enqueue_lists(upf_adjoint* a, uint32_t* nb, int* cnt) {
-    const int n = a->n;
-    hipLaunchKernelGGL(k_keys, a->grid(), dim3(AB), 0, a->st, n, a->x, a->P, a->keys, a->ctl);
-    (void)radix_sort(a->keys, nullptr, a->skeys, a->perm, n, 30, a->sort_tmp, a->st);
+// first keys and an empty cell table for the positions x; each step leaves
+// both ready for the next
+static void enqueue_begin(upf_adjoint* a, const float4* x) {
+    hipLaunchKernelGGL(k_keys, a->grid(), dim3(AB), 0, a->st, a->n, x, a->P, a->keys, a->ctl);
     hipLaunchKernelGGL(k_clear_cells, dim3((a->ncells + AB - 1) / AB), dim3(AB), 0, a->st, a->cells, a->ncells);
-    hipLaunchKernelGGL(k_cell_bounds, a->grid(), dim3(AB), 0, a->st, n, a->skeys, 3u * a->P.block_shift, a->cells);
-    hipLaunchKernelGGL(k_lists, a->grid(), dim3(AB), 0, a->st, n, a->x, a->perm, a->cells, a->P, nb, cnt, a->ctl);
 }
 
-// one forward step of the state (a->x, a->v); with `tape` >= 0 the step's
-// lists and iteration states go to tape slot `tape`
-static void enqueue_step(upf_adjoint* a, int tape) {
-    const int n = a->n, K = a->K;
+// one forward step (x, v) -> (xn, vn); with `tape` >= 0 the step's lists and
+// iteration states go to tape slot `tape`.  more: another step follows.
+template <int LANES>
+static void enqueue_step(upf_adjoint* a, const float4* x, const float4* v, float4* xn, float4* vn, int tape, bool more) {
+    const int n = a->n, K = a->K, ld = a->P.max_neighbors;
     const Consts C = a->consts();
-    const dim3 g = a->grid();
+    const dim3 g = a->grid(LANES), b(AB);
     const bool rec = tape >= 0;
     uint32_t* nb = rec ? a->t_nb + (size_t)tape * a->nb_stride() : a->t_nb;
     int* cnt = rec ? a->t_cnt + (size_t)tape * n : a->t_cnt;
-    if (rec) {
-        (void)hipMemcpyAsync(a->t_x + (size_t)tape * n, a->x, (size_t)n * 16, hipMemcpyDeviceToDevice, a->st);
-        (void)hipMemcpyAsync(a->t_v + (size_t)tape * n, a->v, (size_t)n * 16, hipMemcpyDeviceToDevice, a->st);
-    }
-    enqueue_lists(a, nb, cnt);
-    hipLaunchKernelGGL(k_ext, g, dim3(AB), 0, a->st, n, a->x, a->v, nb, cnt, C, a->F, a->Fp, a->p);
+    auto xs = [&](int k) { return rec ? a->t_xs + ((size_t)tape * K + k) * n : a->xs; };
+    (void)radix_sort(a->keys, nullptr, a->skeys, a->perm, n, 30, a->sort_tmp, a->st);
+    hipLaunchKernelGGL(k_cell_bounds, a->grid(), b, 0, a->st, n, a->skeys, a->perm, x, 3u * a->P.block_shift, a->cells,
+                       a->cand);
+    hipLaunchKernelGGL(k_lists, a->grid(LIST_LANES), b, 0, a->st, n, x, a->cand, a->cells, a->P, nb, cnt, a->ctl);
+    hipLaunchKernelGGL(k_ext<LANES>, g, b, 0, a->st, n, x, v, nb, cnt, ld, C, a->F, a->p, xs(0), a->cells, a->ncells,
+                       a->ctl);
     for (int k = 0; k < K; ++k) {
         const size_t o = ((size_t)tape * K + k) * n;
-        hipLaunchKernelGGL(k_predict, g, dim3(AB), 0, a->st, n, a->x, a->v, a->F, a->Fp, C, a->xs,
-                           rec ? a->t_z + o : nullptr, a->ctl);
-        hipLaunchKernelGGL(k_density, g, dim3(AB), 0, a->st, n, a->xs, nb, cnt, C, a->p, rec ? a->t_p + o : nullptr,
-                           rec ? a->t_rho + o : nullptr);
-        hipLaunchKernelGGL(k_pforce, g, dim3(AB), 0, a->st, n, a->x, nb, cnt, C, a->p, a->Fp);
+        hipLaunchKernelGGL(k_density<LANES>, g, b, 0, a->st, n, x, xs(k), nb, cnt, ld, C, a->p, a->rec,
+                           rec ? a->t_p + o : nullptr, rec ? a->t_rho + o : nullptr);
+        if (k + 1 < K)
+            hipLaunchKernelGGL((k_pforce<LANES, false>), g, b, 0, a->st, n, x, v, nb, cnt, ld, C, a->rec, a->F, xs(k + 1),
+                               nullptr, nullptr, nullptr, a->P, nullptr, a->ctl);
+        else
+            hipLaunchKernelGGL((k_pforce<LANES, true>), g, b, 0, a->st, n, x, v, nb, cnt, ld, C, a->rec, a->F, nullptr, xn,
+                               vn, rec ? a->t_y + (size_t)tape * n : nullptr, a->P, more ? a->keys : nullptr, a->ctl);
     }
-    hipLaunchKernelGGL(k_integrate, g, dim3(AB), 0, a->st, n, a->x, a->v, a->F, a->Fp, C,
-                       rec ? a->t_y + (size_t)tape * n : nullptr);
 }
 
-// reverse of the step in tape slot `tape`: (gx, gv) -> (gx, gv)
-static void enqueue_step_back(upf_adjoint* a, int tape) {
-    const int n = a->n, K = a->K;
+// reverse of the step (x, v) in tape slot `tape`: (gx, gv) -> (gx, gv)
+template <int LANES>
+static void enqueue_step_back(upf_adjoint* a, const float4* x, const float4* v, int tape) {
+    const int n = a->n, K = a->K, ld = a->P.max_neighbors;
     const Consts C = a->consts();
-    const dim3 g = a->grid();
-    const float4* X = a->t_x + (size_t)tape * n;
-    const float4* V = a->t_v + (size_t)tape * n;
+    const dim3 g = a->grid(LANES), b(AB);
     const uint32_t* nb = a->t_nb + (size_t)tape * a->nb_stride();
     const int* cnt = a->t_cnt + (size_t)tape * n;
-    hipLaunchKernelGGL(kr_integrate, g, dim3(AB), 0, a->st, n, a->t_y + (size_t)tape * n, a->gx, a->gv, C, a->nx, a->nv,
-                       a->gF, a->gFp, a->gp);
+    const size_t o0 = (size_t)tape * K * n;
+    hipLaunchKernelGGL(kr_integrate, a->grid(), b, 0, a->st, n, a->t_y + (size_t)tape * n, a->gx, a->gv, C,
+                       a->t_p + o0 + (size_t)(K - 1) * n, a->nx, a->nv, a->gF, a->gFp, a->gFp2, a->gp);
     for (int k = K - 1; k >= 0; --k) {
-        const size_t o = ((size_t)tape * K + k) * n;
-        hipLaunchKernelGGL(kr_pforce, g, dim3(AB), 0, a->st, n, X, nb, cnt, C, a->t_p + o, a->gFp, a->gp, a->nx);
-        hipLaunchKernelGGL(kr_density, g, dim3(AB), 0, a->st, n, X, a->t_z + o, nb, cnt, C, a->t_rho + o, a->gp, a->nx,
-                           a->nv, a->gF, a->gFp2);
+        const size_t o = o0 + (size_t)k * n;
+        hipLaunchKernelGGL(kr_pforce<LANES>, g, b, 0, a->st, n, x, nb, cnt, ld, C, a->gFp, a->t_xs + o, a->t_rho + o,
+                           a->gp, a->nx, a->rec);
+        hipLaunchKernelGGL(kr_density<LANES>, g, b, 0, a->st, n, a->t_xs + o, a->rec, nb, cnt, ld, C,
+                           k > 0 ? a->t_p + o - n : nullptr, a->nx, a->nv, a->gF, a->gFp2);
         std::swap(a->gFp, a->gFp2);
     }
-    hipLaunchKernelGGL(kr_ext, g, dim3(AB), 0, a->st, n, X, V, nb, cnt, C, a->gF, a->nx, a->nv);
+    hipLaunchKernelGGL(kr_ext<LANES>, g, b, 0, a->st, n, x, v, nb, cnt, ld, C, a->gF, a->nx, a->nv);
     std::swap(a->gx, a->nx);
     std::swap(a->gv, a->nv);
 }
@@ -633,14 +840,16 @@ int upf_adjoint_create(const upf_params* p, int n, int steps, int iterations, in
     const size_t T = (size_t)a->ckpt;
     bool ok = hipStreamCreateWithFlags(&a->st, hipStreamNonBlocking) == hipSuccess;
     for (auto& e : a->ev) ok = ok && hipEventCreate(&e) == hipSuccess;
-    ok = ok && a->alloc(&a->x, n) == hipSuccess && a->alloc(&a->v, n) == hipSuccess &&
+    ok = ok && a->alloc(&a->x[0], n) == hipSuccess && a->alloc(&a->v[0], n) == hipSuccess &&
+         a->alloc(&a->x[1], n) == hipSuccess && a->alloc(&a->v[1], n) == hipSuccess &&
+         a->alloc(&a->cand, n) == hipSuccess &&
          a->alloc(&a->keys, n) == hipSuccess && a->alloc(&a->skeys, n) == hipSuccess &&
          a->alloc(&a->perm, n) == hipSuccess && a->alloc(&a->cells, a->ncells) == hipSuccess &&
-         a->alloc(&a->ctl, 1) == hipSuccess && a->alloc(&a->F, n) == hipSuccess && a->alloc(&a->Fp, n) == hipSuccess &&
+         a->alloc(&a->ctl, 1) == hipSuccess && a->alloc(&a->F, n) == hipSuccess && a->alloc(&a->rec, n) == hipSuccess &&
          a->alloc(&a->xs, n) == hipSuccess && a->alloc(&a->p, n) == hipSuccess &&
          a->alloc(&a->ck_x, (size_t)a->nseg * n) == hipSuccess && a->alloc(&a->ck_v, (size_t)a->nseg * n) == hipSuccess &&
          a->alloc(&a->t_x, T * n) == hipSuccess && a->alloc(&a->t_v, T * n) == hipSuccess &&
-         a->alloc(&a->t_y, T * n) == hipSuccess && a->alloc(&a->t_z, T * a->K * n) == hipSuccess &&
+         a->alloc(&a->t_y, T * n) == hipSuccess && a->alloc(&a->t_xs, T * a->K * n) == hipSuccess &&
          a->alloc(&a->t_nb, T * a->nb_stride()) == hipSuccess && a->alloc(&a->t_cnt, T * n) == hipSuccess &&
          a->alloc(&a->t_p, T * a->K * n) == hipSuccess && a->alloc(&a->t_rho, T * a->K * n) == hipSuccess &&
          a->alloc(&a->gx, n) == hipSuccess && a->alloc(&a->gv, n) == hipSuccess && a->alloc(&a->nx, n) == hipSuccess &&
@@ -674,17 +883,24 @@ int upf_adjoint_forward(upf_adjoint* a, const float* pos4, const float* vel4, co
         }
         std::memcpy(&x[4 * i + 3], &type[i], 4);
     }
-    ADCHK(hipMemcpyAsync(a->x, x.data(), (size_t)n * 16, hipMemcpyHostToDevice, a->st));
-    ADCHK(hipMemcpyAsync(a->v, v.data(), (size_t)n * 16, hipMemcpyHostToDevice, a->st));
+    // the state at the start of segment k lives in checkpoint k
+    ADCHK(hipMemcpyAsync(a->ck_x, x.data(), (size_t)n * 16, hipMemcpyHostToDevice, a->st));
+    ADCHK(hipMemcpyAsync(a->ck_v, v.data(), (size_t)n * 16, hipMemcpyHostToDevice, a->st));
     ADCHK(hipMemsetAsync(a->ctl, 0, sizeof(Ctl), a->st));
     ADCHK(hipEventRecord(a->ev[0], a->st));
+    float4 *cx = a->ck_x, *cv = a->ck_v;
+    enqueue_begin(a, cx);
     for (int s = 0; s < a->steps; ++s) {
-        if (s % a->ckpt == 0) {
-            const size_t o = (size_t)(s / a->ckpt) * n;
-            ADCHK(hipMemcpyAsync(a->ck_x + o, a->x, (size_t)n * 16, hipMemcpyDeviceToDevice, a->st));
-            ADCHK(hipMemcpyAsync(a->ck_v + o, a->v, (size_t)n * 16, hipMemcpyDeviceToDevice, a->st));
+        const bool more = s + 1 < a->steps;
+        float4 *xn = a->x[s & 1], *vn = a->v[s & 1];
+        if (more && (s + 1) % a->ckpt == 0) {
+            xn = a->ck_x + (size_t)((s + 1) / a->ckpt) * n;
+            vn = a->ck_v + (size_t)((s + 1) / a->ckpt) * n;
         }
-        enqueue_step(a, -1);
+        if (a->lanes() == 16) enqueue_step<16>(a, cx, cv, xn, vn, -1, more);
+        else enqueue_step<4>(a, cx, cv, xn, vn, -1, more);
+        cx = xn;
+        cv = vn;
     }
     ADCHK(hipEventRecord(a->ev[1], a->st));
     ADCHK(hipGetLastError());
@@ -692,8 +908,8 @@ int upf_adjoint_forward(upf_adjoint* a, const float* pos4, const float* vel4, co
     if (rc) return rc;
     ADCHK(hipEventElapsedTime(&a->fwd_ms, a->ev[0], a->ev[1]));
     if (pos_out4 || vel_out4) {
-        ADCHK(hipMemcpy(x.data(), a->x, (size_t)n * 16, hipMemcpyDeviceToHost));
-        ADCHK(hipMemcpy(v.data(), a->v, (size_t)n * 16, hipMemcpyDeviceToHost));
+        ADCHK(hipMemcpy(x.data(), cx, (size_t)n * 16, hipMemcpyDeviceToHost));
+        ADCHK(hipMemcpy(v.data(), cv, (size_t)n * 16, hipMemcpyDeviceToHost));
         for (int i = 0; i < n; ++i)
             for (int c = 0; c < 4; ++c) {
                 if (pos_out4) pos_out4[4 * i + c] = c < 3 ? x[4 * i + c] : 0.0f;
@@ -719,11 +935,21 @@ int upf_adjoint_backward(upf_adjoint* a, const float* dl_dpos4, const float* dl_
     ADCHK(hipEventRecord(a->ev[2], a->st));
     for (int seg = a->nseg - 1; seg >= 0; --seg) {
         const int s0 = seg * a->ckpt, s1 = std::min(s0 + a->ckpt, a->steps);
-        const size_t o = (size_t)seg * n;
-        ADCHK(hipMemcpyAsync(a->x, a->ck_x + o, (size_t)n * 16, hipMemcpyDeviceToDevice, a->st));
-        ADCHK(hipMemcpyAsync(a->v, a->ck_v + o, (size_t)n * 16, hipMemcpyDeviceToDevice, a->st));
-        for (int s = s0; s < s1; ++s) enqueue_step(a, s - s0);      // recompute, taping
-        for (int s = s1 - 1; s >= s0; --s) enqueue_step_back(a, s - s0);
+        // the states of the segment: its checkpoint, then tape slots 1, 2, ...;
+        // the state after its last step is not read (slot 0)
+        auto x = [&](int t) { return t == 0 ? a->ck_x + (size_t)seg * n : a->t_x + (size_t)t * n; };
+        auto v = [&](int t) { return t == 0 ? a->ck_v + (size_t)seg * n : a->t_v + (size_t)t * n; };
+        enqueue_begin(a, x(0));
+        for (int t = 0; t < s1 - s0; ++t) {  // recompute, taping
+            const bool more = t + 1 < s1 - s0;
+            float4 *xn = more ? x(t + 1) : a->t_x, *vn = more ? v(t + 1) : a->t_v;
+            if (a->lanes() == 16) enqueue_step<16>(a, x(t), v(t), xn, vn, t, more);
+            else enqueue_step<4>(a, x(t), v(t), xn, vn, t, more);
+        }
+        for (int t = s1 - s0 - 1; t >= 0; --t) {
+            if (a->lanes() == 16) enqueue_step_back<16>(a, x(t), v(t), t);
+            else enqueue_step_back<4>(a, x(t), v(t), t);
+        }
     }
     ADCHK(hipEventRecord(a->ev[3], a->st));
     ADCHK(hipGetLastError());
@@ -746,7 +972,7 @@ int upf_adjoint_timing(upf_adjoint* a, float* forward_ms, float* backward_ms, si
     if (backward_ms) *backward_ms = a->bwd_ms;
     if (device_bytes) {
         const size_t n = (size_t)a->n, T = (size_t)a->ckpt, K = (size_t)a->K;
-        *device_bytes = n * 16 * (2 + 3 + 2 * a->nseg + 3 * T + T * K + 7) + n * 4 * (4 + T + 2 * T * K) +
+        *device_bytes = n * 16 * (4 + 1 + 3 + 2 * a->nseg + 2 * T + T * K + 7) + n * 4 * (5 + 2 * T + 2 * T * K) +
                         T * a->nb_stride() * 4 + (size_t)a->ncells * 8 + radix_sort_temp_bytes(a->n);
     }
     return UPF_OK;
