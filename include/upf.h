@@ -313,7 +313,7 @@ int upf_radix_sort(int n, const uint32_t* keys_in, uint32_t* keys_out, int32_t* 
  * device pointers to n elements each (no aliasing); stream is a hipStream_t
  * (NULL: the default stream); the call enqueues the sort and returns without
  * synchronising.  The sort's working memory is a fixed array of the library
- * (about 9 MB on every device it runs on, held until the process ends),
+ * (about 11 MB on every device it runs on, held until the process ends),
  * sized for n <= UPF_NOALLOC_SORT_MAX: larger n gives UPF_ERR_ARG.  The call
  * never allocates; calls that overlap on one device share the array and
  * race, so a caller serialises them (one stream, or events).               */

@@ -42,6 +42,30 @@ def test_radix_sort_matches_stable_argsort(gpu, n):
     assert np.array_equal(out, keys[ref])
 
 
+@pytest.mark.parametrize("n", [1, 4096, 4097, 8192, 8193, 2048 * 32, 2048 * 32 + 1, 2048 * 256, 2048 * 256 + 1])
+def test_sort_forms_are_stable(gpu, n):
+    """Sizes around the sort's forms (one workgroup, tiles summed by the scatter, scanned tiles, larger tiles),
+    full 32-bit keys and the 30-bit z-index keys of a step, with runs of equal keys."""
+    rng = np.random.RandomState(n)
+    print("sort forms: n = %d" % n, flush=True)
+    keys = rng.randint(0, 1 << 32, n, dtype=np.uint64).astype(np.uint32)
+    keys[n // 3: n // 2] = 0xFFFFFFFF
+    out, perm = upf.device_radix_sort(keys)
+    want = np.argsort(keys, kind="stable")
+    assert np.array_equal(perm, want) and np.array_equal(out, keys[want])
+    p, pos, typ, _ = upf.standard_dam_break(8, 8, 8)
+    pos = np.resize(pos, (n, 4)) * np.float32(0.9)
+    pos[:, :3] += rng.uniform(0.0, 0.004, (n, 3)).astype(np.float32)
+    sim = upf.Simulation(p, n)
+    sim.upload(pos, np.full(n, upf.UPF_FROZEN, np.int32))
+    sim.sort_and_bin()
+    k, ids, _ = sim.sorted_state()
+    kin = upf.device_keys(p, pos)
+    want = np.argsort(kin, kind="stable")
+    assert np.array_equal(ids, want) and np.array_equal(k, kin[want])
+    sim.close()
+
+
 def test_radix_sort_full_32bit_and_edge_keys(gpu):
     keys = np.array([0xFFFFFFFF, 0, 0x80000000, 0xFFFFFFFF, 0, 1, 0x7FFFFFFF] * 1000, np.uint32)
     out, perm = upf.device_radix_sort(keys)

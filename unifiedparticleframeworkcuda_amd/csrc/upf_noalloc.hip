@@ -11,12 +11,10 @@
 
 namespace upf {
 
-// Working memory of one sort of up to UPF_NOALLOC_SORT_MAX keys: per-tile
-// digit counts (256 x tiles of 1024 keys), digit totals, and the ping-pong
-// (key, value) buffers of the passes.  Every device the library runs on
+// Working memory of one sort of up to UPF_NOALLOC_SORT_MAX keys (tile digit
+// counts, digit totals, ping-pong buffers).  Every device the library runs on
 // holds its own copy until the process ends.
-constexpr size_t kTiles = (UPF_NOALLOC_SORT_MAX + 1023) / 1024;
-constexpr size_t kScratchBytes = (256 * kTiles + 256) * 4 + 2 * (size_t)UPF_NOALLOC_SORT_MAX * 4;
+constexpr size_t kScratchBytes = radix_sort_temp_bytes(UPF_NOALLOC_SORT_MAX);
 __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 // The array's address on each device, looked up once per device with that
