@@ -340,3 +340,34 @@ def test_fluid_only_scene_is_the_pure_fluid_driver(gpu, method):
         sim.step(4, method)
         o.step(4, method)
         _compare(sim, o, np.ones(len(typ), bool), pcisph=False)
+
+
+@pytest.mark.parametrize("n", [1, 16384, 16385, 70001, 300001])
+def test_upload_and_download_round_trip(gpu, n):
+    """Transfers of one slice, of several and with ragged ends give back what was uploaded; a refused upload
+    (the first bad particle decides the code) leaves the state that was there."""
+    rng = np.random.RandomState(n)
+    p, pos, typ, _ = upf.standard_dam_break(8, 8, 8)
+    print("round trip: n = %d" % n, flush=True)
+    pos = np.resize(pos, (n, 4)) * np.float32(0.9)
+    pos[:, :3] += rng.uniform(0.0, 0.004, (n, 3)).astype(np.float32)
+    vel = rng.normal(size=(n, 4)).astype(np.float32)
+    typ = rng.choice([upf.UPF_LIQUID, upf.UPF_FROZEN], n).astype(np.int32)
+    sim = upf.Simulation(p, n + 3)
+    sim.upload(pos, typ, vel)
+    for code, at in (("UPF_ERR_ARG", n - 1), ("UPF_ERR_RANGE", n // 2)):
+        bad_pos, bad_typ = pos.copy(), typ.copy()
+        bad_typ[n - 1] = 17
+        if code == "UPF_ERR_RANGE":
+            bad_pos[at, 1] = -1.0
+            bad_typ[at] = upf.UPF_LIQUID
+        with pytest.raises(upf.UPFError, match=code):
+            sim.upload(bad_pos, bad_typ)
+    for _ in range(2):
+        s = sim.state()
+        assert np.array_equal(s["pos"][:, :3], pos[:, :3]) and not s["pos"][:, 3].any()
+        assert np.array_equal(s["vel"][:, :3], vel[:, :3]) and not s["vel"][:, 3].any()
+        assert np.array_equal(s["type"], typ)
+        assert (s["rho"] == p.rest_density).all() and not s["p"].any()
+        assert (s["psi"] == np.float32(p.initial_mass) / np.float32(p.rest_density)).all()
+    sim.close()

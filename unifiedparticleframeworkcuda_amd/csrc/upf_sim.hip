@@ -31,6 +31,7 @@
 #include "upf_internal.h"
 #include "upf_kernels.h"
 #include "upf_sort.h"
+#include "upf_stage.h"
 
 namespace upf {
 
@@ -2482,14 +2483,69 @@ __global__ void k_gather_keys(int n, const uint32_t* __restrict__ perm, const ui
     if (s < n) out[s] = keys[perm[s]];
 }
 
-// -------------------------------------------------------- id-order output
-__global__ void k_scatter_by_id(int n, const int* __restrict__ id, const float4* __restrict__ a4, float4* __restrict__ o4,
-                                const float* __restrict__ a1, float* __restrict__ o1) {
+// ------------------------------------------------- upload and download
+// The caller's arrays as they arrive (upload order), one after the other.
+struct RawIn {
+    const float4* pos;
+    const float4* vel;  // null: at rest
+    const int* type;
+    const float* p;    // null: 0
+    const float* rho;  // null: the rest density
+};
+
+// The state of n uploaded particles and their keys.  key0 keeps the keys by
+// upload id.
+__global__ void k_ingest(StepArgs A, RawIn in, float psi0, Slots S, Work W, uint32_t* __restrict__ key0, Ctl* ctl) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= A.n) return;
+    float4 x = in.pos[i];
+    x.w = __int_as_float(in.type[i]);
+    float4 v = in.vel ? in.vel[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    v.w = 0.0f;
+    const float rho0 = A.P.rest_density;
+    S.pos[i] = x;
+    S.vel[i] = v;
+    S.x0[i] = x;
+    S.id[i] = i;
+    S.body[i] = -1;
+    S.rel[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    S.p_last[i] = 0.0f;
+    S.p_prev[i] = 0.0f;
+    S.rho_last[i] = rho0;
+    S.psi[i] = psi0;
+    // loop arrays of the "previous step" (gathered into p_last / rho_last by the first sort)
+    W.p[i] = in.p ? in.p[i] : 0.0f;
+    W.rho[i] = in.rho ? in.rho[i] : rho0;
+    const Dom d = dom_at(A, i);
+    bool ok;
+    const uint32_t k = dkey(x.x, x.y, x.z, d.scales, ok);
+    W.keys[i] = k;
+    key0[i] = k;
+    if (!ok) set_err(ctl, UPF_ERR_RANGE);
+}
+
+// The requested arrays (null: not) in upload order.
+struct RawOut {
+    float4 *pos, *vel, *force;
+    float *rho, *p, *psi;
+    int* type;
+};
+__global__ void k_emit_state(int n, Slots S, const float4* __restrict__ force, const float* __restrict__ rho,
+                             const float* __restrict__ p, RawOut out) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= n) return;
-    const int d = id[s];
-    if (a4) o4[d] = a4[s];
-    if (a1) o1[d] = a1[s];
+    const int d = S.id[s];
+    auto xyz0 = [](const float4& a) { return make_float4(a.x, a.y, a.z, 0.0f); };
+    if (out.pos || out.type) {
+        const float4 x = S.pos[s];
+        if (out.pos) out.pos[d] = xyz0(x);
+        if (out.type) out.type[d] = ptype(x);
+    }
+    if (out.vel) out.vel[d] = xyz0(S.vel[s]);
+    if (out.force) out.force[d] = xyz0(force[s]);
+    if (out.rho) out.rho[d] = rho[s];
+    if (out.p) out.p[d] = p[s];
+    if (out.psi) out.psi[d] = S.psi[s];
 }
 
 }  // namespace upf
@@ -2626,7 +2682,8 @@ struct upf_sim {
     void* sort_tmp = nullptr;
     uint32_t ncells = 0;
     std::vector<int> k_hist;
-    std::vector<uint32_t> key0;  // z-index of every particle's uploaded position, by upload id
+    uint32_t* d_key0 = nullptr;  // z-index of every particle's uploaded position, by upload id
+    Stage stage;
     std::vector<float> rho_hist;
     std::vector<void*> allocs;
     // rigid bodies
@@ -3183,6 +3240,7 @@ static void build_bin_thresholds(float factor, float* out) {
 static int sim_alloc(upf_sim* s, int capacity, uint32_t ncells, int n_scenes) {
     const upf_params* p = &s->P;
     s->cap = capacity;
+    s->stage.expect((size_t)capacity * 64);  // a full download
     s->n_scenes = n_scenes;
     s->sps = n_scenes == 1 ? MAX_SLOTS : 16;
     s->ncells = ncells;
@@ -3205,7 +3263,10 @@ static int sim_alloc(upf_sim* s, int capacity, uint32_t ncells, int n_scenes) {
     HIPCHK(s->alloc(&W.ncount, capacity));
     // column-major (k * capacity + slot) or, for the fused build, slot-major
     // (slot * pitch + k, the pitch rounded up to four entries)
-    HIPCHK(s->alloc(&W.nbr, (size_t)capacity * ((p->max_neighbors + 3) & ~3)));
+    // -- and for uploads and downloads between steps, which pass through this
+    // memory, at most 16 words per particle
+    HIPCHK(s->alloc(&W.nbr, (size_t)capacity * std::max((p->max_neighbors + 3) & ~3, 16)));
+    HIPCHK(s->alloc(&s->d_key0, capacity));
     HIPCHK(s->alloc(&W.nbw, (size_t)capacity * ((p->max_neighbors + 7) / 8)));
     HIPCHK(s->alloc(&W.nbf, capacity));
     HIPCHK(s->alloc(&W.nbe, (size_t)capacity * NB_ESC));
@@ -3326,58 +3387,57 @@ static int upload_common(upf_sim* s, int n, const float* pos4, const float* vel4
                          const int* scene_of, const upf_params* scene_params, const float* p0 = nullptr,
                          const float* rho0 = nullptr) {
     if (!s || n <= 0 || n > s->cap || !pos4 || !type) return UPF_ERR_ARG;
-    std::vector<float> pos((size_t)4 * n), vel((size_t)4 * n, 0.0f), x0((size_t)4 * n);
-    std::vector<int> id(n), body(n, -1);
-    std::vector<uint32_t> key0(n);
-    std::vector<float> rho(n, s->P.rest_density), zero(n, 0.0f), psi(n, s->P.initial_mass / s->P.rest_density);
-    for (int i = 0; i < n; ++i) {
-        const upf_params& Q = scene_of ? scene_params[scene_of[i]] : s->P;
-        const int t = type[i];
-        if (t != UPF_LIQUID && t != UPF_FROZEN && t != UPF_RIGID) return UPF_ERR_ARG;
-        for (int a = 0; a < 3; ++a) {
-            pos[4 * i + a] = pos4[4 * i + a];
-            x0[4 * i + a] = pos4[4 * i + a];
-            if (vel4) vel[4 * i + a] = vel4[4 * i + a];
+    // everything is checked before the simulation changes; the first particle
+    // that fails decides the code
+    constexpr int PARTS = Stage::THREADS;
+    int bad[PARTS] = {};
+    Stage::split((size_t)n, 1 << 16, [&](int part, size_t beg, size_t end) {
+        for (size_t i = beg; i < end; ++i) {
+            const upf_params& Q = scene_of ? scene_params[scene_of[i]] : s->P;
+            const int t = type[i];
+            const float* x = pos4 + 4 * i;
+            uint32_t k;
+            // the query box of every particle must stay inside the grid (beyond it the
+            // reference's cell ranges overflow, src/cpu/zIndex.cpp:66)
+            if (t != UPF_LIQUID && t != UPF_FROZEN && t != UPF_RIGID) bad[part] = UPF_ERR_ARG;
+            else if (!host_key(Q, x[0], x[1], x[2], k)) bad[part] = UPF_ERR_RANGE;
+            else
+                for (int a = 0; a < 3; ++a)
+                    if (!(Q.scales[a] * (x[a] + Q.support_radius) < 1024.0f)) bad[part] = UPF_ERR_RANGE;
+            if (bad[part]) return;
         }
-        int tb = t;
-        float w;
-        std::memcpy(&w, &tb, 4);
-        pos[4 * i + 3] = w;
-        x0[4 * i + 3] = w;
-        vel[4 * i + 3] = 0.0f;
-        id[i] = i;
-        uint32_t k;
-        if (!host_key(Q, pos4[4 * i], pos4[4 * i + 1], pos4[4 * i + 2], k)) return UPF_ERR_RANGE;
-        key0[i] = k;
-        // the query box of every particle must stay inside the grid (beyond it the
-        // reference's cell ranges overflow, src/cpu/zIndex.cpp:66)
-        for (int a = 0; a < 3; ++a)
-            if (!(Q.scales[a] * (pos4[4 * i + a] + Q.support_radius) < 1024.0f)) return UPF_ERR_RANGE;
-    }
+    });
+    for (int rc : bad)
+        if (rc) return rc;
     Slots& S = s->S[0];
     s->cur = 0;
     s->n = n;
+    // the caller's arrays go side by side into the list memory, which no step
+    // has a use for before it builds its own lists
     const size_t b4 = (size_t)n * sizeof(float4), b1 = (size_t)n * sizeof(float);
-    HIPCHK(hipMemcpyAsync(S.pos, pos.data(), b4, hipMemcpyHostToDevice, s->st));
-    HIPCHK(hipMemcpyAsync(S.vel, vel.data(), b4, hipMemcpyHostToDevice, s->st));
-    HIPCHK(hipMemcpyAsync(S.x0, x0.data(), b4, hipMemcpyHostToDevice, s->st));
-    HIPCHK(hipMemcpyAsync(S.id, id.data(), (size_t)n * sizeof(int), hipMemcpyHostToDevice, s->st));
-    HIPCHK(hipMemcpyAsync(S.body, body.data(), (size_t)n * sizeof(int), hipMemcpyHostToDevice, s->st));
-    HIPCHK(hipMemsetAsync(S.rel, 0, b4, s->st));
-    HIPCHK(hipMemcpyAsync(S.p_last, zero.data(), b1, hipMemcpyHostToDevice, s->st));
-    HIPCHK(hipMemcpyAsync(S.p_prev, zero.data(), b1, hipMemcpyHostToDevice, s->st));
-    HIPCHK(hipMemcpyAsync(S.rho_last, rho.data(), b1, hipMemcpyHostToDevice, s->st));
-    HIPCHK(hipMemcpyAsync(S.psi, psi.data(), b1, hipMemcpyHostToDevice, s->st));
-    // loop arrays of the "previous step" (gathered into p_last / rho_last by the first sort)
-    HIPCHK(hipMemcpyAsync(s->W.p, p0 ? p0 : zero.data(), b1, hipMemcpyHostToDevice, s->st));
-    HIPCHK(hipMemcpyAsync(s->W.rho, rho0 ? rho0 : rho.data(), b1, hipMemcpyHostToDevice, s->st));
+    char* raw = reinterpret_cast<char*>(s->W.nbr);
+    StagePart parts[5];
+    int np = 0;
+    size_t total = 0;
+    auto add = [&](const void* host, size_t bytes) -> const char* {
+        if (!host) return nullptr;
+        parts[np++] = {const_cast<char*>(static_cast<const char*>(host)), total, bytes};
+        total += bytes;
+        return raw + total - bytes;
+    };
+    RawIn in;
+    in.pos = reinterpret_cast<const float4*>(add(pos4, b4));
+    in.vel = reinterpret_cast<const float4*>(add(vel4, b4));
+    in.type = reinterpret_cast<const int*>(add(type, b1));
+    in.p = reinterpret_cast<const float*>(add(p0, b1));
+    in.rho = reinterpret_cast<const float*>(add(rho0, b1));
+    if (!s->stage.to_device(raw, total, parts, np, s->st)) return UPF_ERR_HIP;
     HIPCHK(hipMemsetAsync(s->ctl, 0, sizeof(Ctl), s->st));
-    if (scene_of) HIPCHK(hipMemcpyAsync(s->d_scene_of, scene_of, (size_t)n * sizeof(int), hipMemcpyHostToDevice, s->st));
-    hipLaunchKernelGGL(k_keys, grid_for(n), dim3(BLOCK), 0, s->st, s->args(), S.pos, s->W.keys, s->ctl);
+    hipLaunchKernelGGL(k_ingest, grid_for(n), dim3(BLOCK), 0, s->st, s->args(), in,
+                       s->P.initial_mass / s->P.rest_density, S, s->W, s->d_key0, s->ctl);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(s->st));
     s->uploaded = true;
-    s->key0.swap(key0);
     s->psi_ready = false;
     s->k_hist.clear();
     s->rho_hist.clear();
@@ -3536,44 +3596,32 @@ int upf_download(upf_sim* s, float* pos4, float* vel4, float* rho, float* p, flo
     if (!s) return UPF_ERR_ARG;
     if (!s->uploaded) return UPF_ERR_STATE;
     const int n = s->n;
-    Slots& S = s->S[s->cur];
-    HIPCHK(hipStreamSynchronize(s->st));
-    std::vector<int> id(n);
-    HIPCHK(hipMemcpy(id.data(), S.id, (size_t)n * 4, hipMemcpyDeviceToHost));
-    std::vector<float> b4((size_t)4 * n), b1(n);
-    auto get4 = [&](const float4* src, float* dst, bool is_pos) -> int {
-        if (!dst) return UPF_OK;
-        HIPCHK(hipMemcpy(b4.data(), src, (size_t)n * 16, hipMemcpyDeviceToHost));
-        for (int k = 0; k < n; ++k) {
-            const int d = id[k];
-            for (int a = 0; a < 3; ++a) dst[4 * d + a] = b4[4 * k + a];
-            dst[4 * d + 3] = 0.0f;
-            if (is_pos && type) {
-                int t;
-                std::memcpy(&t, &b4[4 * k + 3], 4);
-                type[d] = t;
-            }
-        }
-        return UPF_OK;
+    // put in upload order on the device, side by side in the list memory
+    // (a step builds its lists anew), then copied out
+    const size_t b4 = (size_t)n * sizeof(float4), b1 = (size_t)n * sizeof(float);
+    char* raw = reinterpret_cast<char*>(s->W.nbr);
+    StagePart parts[7];
+    int np = 0;
+    size_t total = 0;
+    auto add = [&](void* host, size_t bytes) -> char* {
+        if (!host) return nullptr;
+        parts[np++] = {static_cast<char*>(host), total, bytes};
+        total += bytes;
+        return raw + total - bytes;
     };
-    auto get1 = [&](const float* src, float* dst) -> int {
-        if (!dst) return UPF_OK;
-        HIPCHK(hipMemcpy(b1.data(), src, (size_t)n * 4, hipMemcpyDeviceToHost));
-        for (int k = 0; k < n; ++k) dst[id[k]] = b1[k];
-        return UPF_OK;
-    };
+    RawOut out;
+    out.pos = reinterpret_cast<float4*>(add(pos4, b4));
+    out.vel = reinterpret_cast<float4*>(add(vel4, b4));
+    out.force = reinterpret_cast<float4*>(add(force4, b4));
+    out.rho = reinterpret_cast<float*>(add(rho, b1));
+    out.p = reinterpret_cast<float*>(add(p, b1));
+    out.psi = reinterpret_cast<float*>(add(psi, b1));
+    out.type = reinterpret_cast<int*>(add(type, b1));
     // after a step the slot arrays of the loop (W.*) are in the current slot order
-    std::vector<float> tmp4;
-    if (pos4 || type) {
-        if (!pos4) { tmp4.resize((size_t)4 * n); pos4 = tmp4.data(); }
-        if (get4(S.pos, pos4, true)) return UPF_ERR_HIP;
-    }
-    if (get4(S.vel, vel4, false)) return UPF_ERR_HIP;
-    if (get4(s->W.force, force4, false)) return UPF_ERR_HIP;
-    if (get1(s->W.rho, rho)) return UPF_ERR_HIP;
-    if (get1(sph_family(s->last_method) ? s->W.pres : s->W.p, p)) return UPF_ERR_HIP;
-    if (get1(S.psi, psi)) return UPF_ERR_HIP;
-    return UPF_OK;
+    hipLaunchKernelGGL(k_emit_state, grid_for(n), dim3(BLOCK), 0, s->st, n, s->S[s->cur], s->W.force, s->W.rho,
+                       sph_family(s->last_method) ? s->W.pres : s->W.p, out);
+    HIPCHK(hipGetLastError());
+    return s->stage.to_host(raw, total, parts, np, s->st) ? UPF_OK : UPF_ERR_HIP;
 }
 
 int upf_upload_bodies(upf_sim* s, int n_bodies, const upf_body* bodies, const int* body_id, const float* rel4) {
@@ -3668,13 +3716,15 @@ int upf_dump_cells(upf_sim* s, const char* particles_path, const char* blocks_pa
     const Slots& S = s->S[s->cur];
     std::vector<float> rec((size_t)4 * n);
     std::vector<int> id(n);
+    std::vector<uint32_t> key0(n);
     std::vector<uint2> cells(s->ncells);
+    HIPCHK(hipMemcpy(key0.data(), s->d_key0, (size_t)n * 4, hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(rec.data(), S.pos, (size_t)n * 16, hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(id.data(), S.id, (size_t)n * 4, hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(cells.data(), s->W.cells, (size_t)s->ncells * sizeof(uint2), hipMemcpyDeviceToHost));
     // w: the uploaded particle's z-index as a float (the reference uploads
     // particles_h[i].index into w and never rewrites it)
-    for (int k = 0; k < n; ++k) rec[4 * (size_t)k + 3] = (float)s->key0[id[k]];
+    for (int k = 0; k < n; ++k) rec[4 * (size_t)k + 3] = (float)key0[id[k]];
     // occupied cells as (row-major block index, first slot, count), by block index
     const uint32_t dim = s->P.grid_dim;
     std::vector<uint32_t> blocks;
@@ -3927,7 +3977,8 @@ int upf_batch_create(int n_scenes, const upf_params* scene_params, const int* co
         }
         // one scene: its domain travels in the kernel arguments
         if (n_scenes > 1 &&
-            hipMemcpy(s->d_doms, doms.data(), doms.size() * sizeof(Dom), hipMemcpyHostToDevice) != hipSuccess)
+            (hipMemcpy(s->d_doms, doms.data(), doms.size() * sizeof(Dom), hipMemcpyHostToDevice) != hipSuccess ||
+             hipMemcpy(s->d_scene_of, b->scene_of.data(), (size_t)total * sizeof(int), hipMemcpyHostToDevice) != hipSuccess))
             rc = UPF_ERR_HIP;
         // the scenes' 64-slot chunks (a chunk never straddles two scenes) for
         // the correction loop's per-iteration lists of running scenes
