@@ -1806,11 +1806,14 @@ __global__ void k_integrate(StepArgs A, Slots S, Work W, int pcisph, int pure_fl
 // P.add_wall_weight, then the pressure of physicsType 'w' (TAIT,
 // CalculatePressureWCSPH :2491-2501) or 'o' (CalculatePressureSPH
 // :2479-2489), over the lists
-// The density work of slot i (one thread) over its packed list (entries
-// carry the table bin): the density pass and the fused list build share it.
-template <bool TAIT>
+// The density work of slot i (one thread), shared by the density pass, which
+// reads column-major packed lists with the table bins in their entries, and
+// (FUSED) the fused list build, whose lists are the slot's own rows without
+// bins: it takes each pair's bin from its distance and delta-codes the list
+// for the force pass.
+template <bool TAIT, bool FUSED>
 __device__ __forceinline__ void density_wcsph_slot(const StepArgs& A, const Slots& S, const Work& W, int i,
-                                                   const float* lw) {
+                                                   const float* lw, const float2* th, Ctl* ctl) {
     const upf_params& P = A.P;
     const float4 xi = S.pos[i];
     if (ptype(xi) != UPF_LIQUID) {
@@ -1823,7 +1826,32 @@ __device__ __forceinline__ void density_wcsph_slot(const StepArgs& A, const Slot
     const float m = P.initial_mass;
     float rho = P.kernel_self * m;
     const int cnt = W.ncount[i];
-    for (int k = 0; k < cnt; ++k) rho = rho + lw[W.nbr[(size_t)k * A.stride + i] & NB_BIN_MASK] * m;
+    if constexpr (FUSED) {
+        const uint32_t* L = W.nbr + (size_t)i * A.nbr_ld;
+        ListEncoder enc(W, i, (size_t)A.stride);
+        // aligned groups of four entries, the next group's entries loaded
+        // before this group's gathers (entries past the end are not used)
+        uint4 q = cnt > 0 ? *reinterpret_cast<const uint4*>(L) : make_uint4(0u, 0u, 0u, 0u);
+        for (int k = 0; k < cnt; k += 4) {
+            const uint32_t e[4] = {q.x, q.y, q.z, q.w};
+            if (k + 4 < cnt) q = *reinterpret_cast<const uint4*>(L + k + 4);
+            float4 xj[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int j = k + u < cnt ? (int)(e[u] >> NB_SLOT_SHIFT) : i;
+                if (k + u < cnt) enc.put(k + u, (uint32_t)j, ctl);
+                xj[u] = at_u32(S.pos, j);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const float dx = xi.x - xj[u].x, dy = xi.y - xj[u].y, dz = xi.z - xj[u].z;
+                if (k + u < cnt) rho = rho + lw[bin_of_d2(dx * dx + dy * dy + dz * dz, A.lut_factor, th)] * m;
+            }
+        }
+        enc.finish();
+    } else {
+        for (int k = 0; k < cnt; ++k) rho = rho + lw[W.nbr[(size_t)k * A.stride + i] & NB_BIN_MASK] * m;
+    }
     if (P.add_wall_weight) rho = rho + wall_weight<true>(P, wall_distance(P, xi.x, xi.y, xi.z), A.lut_factor, lw);
     float pres;
     if constexpr (TAIT) {
@@ -1854,33 +1882,47 @@ __global__ __launch_bounds__(BLOCK) void k_density_wcsph(StepArgs A, Slots S, Wo
     for (int t = threadIdx.x; t < LUT_N; t += blockDim.x) lw[t] = luts[t];
     __syncthreads();
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < A.n) density_wcsph_slot<TAIT>(A, S, W, i, lw);
+    if (i < A.n) density_wcsph_slot<TAIT, false>(A, S, W, i, lw, nullptr, ctl);
 }
 
-// The list build (entries with bins) and the density pass in one kernel:
-// each lane sums the density of its own slot over the list its wave just
-// wrote (as k_nbr_build_ext does for the PCISPH external forces).
+// The list build and the density pass in one kernel: each lane sums the
+// density of its own slot over the list its wave just wrote (as
+// k_nbr_build_ext does for the PCISPH external forces).  With column-major
+// lists, whose cache lines fill over the life of a wave, and bins in the
+// entries, a root for every 64 candidates: 417 us at 1,132,556 particles, now
+// 354; the force pass takes 113 us instead of 100 for it (bins from distances).
 template <int ROUNDS, bool TAIT>
 __global__ __launch_bounds__(64) void k_nbr_build_wcsph(StepArgs A, Slots S, Work W, const float* __restrict__ luts,
                                                         Ctl* ctl) {
-    // the build's candidate table, then the density table
-    __shared__ float lw[LUT_N > CAND_CAP ? LUT_N : CAND_CAP];
-    build_wave<ROUNDS, 0, 1, 0>(A, S.pos, W.keys_sorted, W.cells, W.nbr, W.ncount, ctl,
-                                reinterpret_cast<uint32_t*>(lw));
+    // the build's candidate table, then the density table and the bin thresholds
+    __shared__ float2 tabs[2 * LUT_N];
+    static_assert(4 * LUT_N >= CAND_CAP, "candidate table");
+    build_wave<ROUNDS, 0, 0, 0, 0, UPF_LIQUID, true>(A, S.pos, W.keys_sorted, W.cells, W.nbr, W.ncount, ctl,
+                                                    reinterpret_cast<uint32_t*>(tabs));
     __syncthreads();  // the block is the wave: its lists are complete
-    for (int t = threadIdx.x; t < LUT_N; t += blockDim.x) lw[t] = luts[t];
+    float2* th = tabs;
+    float* lw = reinterpret_cast<float*>(tabs + LUT_N);
+    for (int t = threadIdx.x; t < LUT_N; t += blockDim.x) {
+        lw[t] = luts[t];
+        th[t] = reinterpret_cast<const float2*>(luts + LUT_TH_OFF)[t];
+    }
     __syncthreads();
     const int i = xblk(A.xcd) * 64 + (int)threadIdx.x;
-    if (i < A.n) density_wcsph_slot<TAIT>(A, S, W, i, lw);
+    if (i < A.n) density_wcsph_slot<TAIT, true>(A, S, W, i, lw, th, ctl);
 }
 
-// CalculateLiquidParticleForces (:3009-3083) + gravity (:2822-2824)
+// CalculateLiquidParticleForces (:3009-3083) + gravity (:2822-2824).  CODED:
+// over the delta-coded lists of the fused build, the bins from the distances
+// (the build's positions).
+template <int CODED>
 __global__ __launch_bounds__(BLOCK) void k_force_wcsph(StepArgs A, Slots S, Work W, const float* __restrict__ luts,
                                                        Ctl* ctl) {
     __shared__ float lvl[LUT_N], lpg[LUT_N];
+    __shared__ float2 th[CODED ? LUT_N : 1];
     for (int t = threadIdx.x; t < LUT_N; t += blockDim.x) {
         lvl[t] = luts[2 * LUT_N + t];
         lpg[t] = luts[LUT_N + t];
+        if constexpr (CODED != 0) th[t] = reinterpret_cast<const float2*>(luts + LUT_TH_OFF)[t];
     }
     __syncthreads();
     const upf_params& P = A.P;
@@ -1896,15 +1938,16 @@ __global__ __launch_bounds__(BLOCK) void k_force_wcsph(StepArgs A, Slots S, Work
     float fx = 0.0f, fy = 0.0f, fz = 0.0f;
     const int cnt = W.ncount[i];
     // two 16-byte records per neighbour, four neighbours' loads in flight
-    for_each_listed<0, 4>(
+    for_each_listed<CODED, 4>(
         W, i, (size_t)A.stride, cnt, [&](int j) { return PosVel{at_u32(W.xpd, j), at_u32(W.vpg, j)}; },
         [&](int, uint32_t e, const PosVel& q) __attribute__((always_inline)) {
             const float4& xj = q.x;
             if (xj.w < 0.0f) return;  // not a fluid neighbour
             const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-            const float kv = lvl[e & NB_BIN_MASK];
+            const uint32_t bin = CODED ? bin_of_d2(dx * dx + dy * dy + dz * dz, A.lut_factor, th) : (e & NB_BIN_MASK);
+            const float kv = lvl[bin];
             const float nVol = xj.w;  // m / rho_j
-            const float g = lpg[e & NB_BIN_MASK];
+            const float g = lpg[bin];
             const float grad = p_i * invD * invD + q.v.w;  // + p_j / rho_j^2
             fx = fx - (((dx * g) * grad) * m) * m;
             fy = fy - (((dy * g) * grad) * m) * m;
@@ -3161,8 +3204,9 @@ static int step_wcsph_static(upf_sim* s, bool tait) {
     const StepArgs A = s->args();
     Slots& S = s->S[s->cur];
     const dim3 g = grid_for(s->n);
-    if (s->tune.nbr_fuse && s->tune.nbr_stage == 0 && s->tune.nbr_tile == 0) {
-        // the list build (with bins) and the density pass as one kernel
+    const bool fuse = s->tune.nbr_fuse && s->tune.nbr_stage == 0 && s->tune.nbr_tile == 0 && A.code_lists;
+    if (fuse) {
+        // the list build and the density pass as one kernel
         s->prof.begin(PC_NBR_BUILD_DENSITY, s->st);
         const dim3 gb((unsigned)(((s->n + 63) / 64 + 7) / 8 * 8));  // a multiple of 8 (XCD remap)
         auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, gb, dim3(64), 0, s->st, A, S, s->W, s->luts, s->ctl); };
@@ -3185,7 +3229,8 @@ static int step_wcsph_static(upf_sim* s, bool tait) {
         s->prof.end(s->st);
     }
     s->prof.begin(PC_WCSPH_FORCE, s->st);
-    hipLaunchKernelGGL(k_force_wcsph, g, dim3(BLOCK), 0, s->st, A, S, s->W, s->luts, s->ctl);
+    if (fuse) hipLaunchKernelGGL(k_force_wcsph<1>, g, dim3(BLOCK), 0, s->st, A, S, s->W, s->luts, s->ctl);
+    else hipLaunchKernelGGL(k_force_wcsph<0>, g, dim3(BLOCK), 0, s->st, A, S, s->W, s->luts, s->ctl);
     s->prof.end(s->st);
     s->prof.begin(PC_INTEGRATE, s->st);
     hipLaunchKernelGGL(k_integrate, grid_persist(s, s->n), block_loop(s), 0, s->st, A, S, s->W, 0, 0,
