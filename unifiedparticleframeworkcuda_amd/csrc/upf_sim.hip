@@ -682,8 +682,9 @@ __device__ __forceinline__ void build_wave(const StepArgs& A, const float4* __re
     const int stride = A.stride;
     const int lane = threadIdx.x;
     // SPLIT waves share a window of 64 slots, each building the lists of the
-    // owners in its 64 / SPLIT lanes (more, shorter waves where owners are
-    // few and dense, as the rigid particles of the coupling step)
+    // owners in its 64 / SPLIT lanes (more, shorter waves where there are few
+    // windows, and where owners are few and dense, as the rigid particles of
+    // the coupling step)
     const int vb = xblk(A.xcd);
     const int base = (vb / SPLIT) * 64;
     const int part = vb % SPLIT;
@@ -702,7 +703,8 @@ __device__ __forceinline__ void build_wave(const StepArgs& A, const float4* __re
     const int my_scene = mine_valid ? scene_at(A, me) : -1;
     // owners: the slots whose lists this build writes (liquid, or the rigid
     // slots of the coupling step)
-    const bool my_owner = mine_valid && ptype(my_x) == OWNER && (SPLIT == 1 || lane / (64 / SPLIT) == part);
+    const bool my_part = mine_valid && lane / (64 / SPLIT) == part;
+    const bool my_owner = my_part && ptype(my_x) == OWNER;
     uint32_t my_blo = 0u, my_bhi = 0u;
     if (my_owner) {
         // BoxQuery of the particle in cell coordinates, clipped to the grid
@@ -921,7 +923,7 @@ __device__ __forceinline__ void build_wave(const StepArgs& A, const float4* __re
     }
     // KEEP_RIGID: rigid slots keep the counts of their own lists; a rigid-owner
     // build writes only those
-    if (OWNER == UPF_LIQUID ? mine_valid && !(KEEP_RIGID && ptype(my_x) == UPF_RIGID) : my_owner) {
+    if (OWNER == UPF_LIQUID ? my_part && !(KEEP_RIGID && ptype(my_x) == UPF_RIGID) : my_owner) {
         ncount[me] = my_cnt < cap ? my_cnt : cap;
         if (my_cnt > cap) set_err(ctl, UPF_ERR_NBR_OVERFLOW);
     }
@@ -933,6 +935,15 @@ __device__ __forceinline__ void build_wave(const StepArgs& A, const float4* __re
         for (int k = 0; k < rows; ++k)
             if (k < mine) nbr[(size_t)k * stride + me] = stage[k * 65 + lane];
     }
+}
+
+// The slot that this lane of a fused build works on after the build, or -1:
+// its wave's SPLIT-th of the window (build_wave).
+template <int SPLIT>
+__device__ __forceinline__ int split_slot(const StepArgs& A) {
+    const int vb = xblk(A.xcd), lane = threadIdx.x;
+    const int i = (vb / SPLIT) * 64 + lane;
+    return i < A.n && lane / (64 / SPLIT) == vb % SPLIT ? i : -1;
 }
 
 template <int ROUNDS, int STAGE, int BIN, int SKIP = 0>
@@ -1333,13 +1344,13 @@ __global__ __launch_bounds__(BLOCK) void k_ext_static(StepArgs A, Slots S, Work 
 // wave just wrote.  Nothing crosses waves between the two parts, so the
 // memory-bound force work of some waves overlaps the VALU-bound list work of
 // others, and the lists are read back while they are still in the cache.
-template <int ROUNDS, int SKIP, int MODE, bool SLOT_MAJOR>
+template <int ROUNDS, int SKIP, int MODE, bool SLOT_MAJOR, int SPLIT>
 __global__ __launch_bounds__(64) void k_nbr_build_ext(StepArgs A, Slots S, Work W, const float* __restrict__ luts,
                                                       Ctl* ctl) {
     // the build's candidate table, then the tables of the force pass
     __shared__ float4 tabs[LUT_N];
     static_assert(4 * LUT_N >= CAND_CAP, "candidate table");
-    build_wave<ROUNDS, 0, 0, SKIP, 0, UPF_LIQUID, SLOT_MAJOR>(A, S.pos, W.keys_sorted, W.cells, W.nbr, W.ncount, ctl,
+    build_wave<ROUNDS, 0, 0, SKIP, 0, UPF_LIQUID, SLOT_MAJOR, SPLIT>(A, S.pos, W.keys_sorted, W.cells, W.nbr, W.ncount, ctl,
                                                              reinterpret_cast<uint32_t*>(tabs));
     // the block is the wave: its lists (written by all its lanes) are complete
     // and visible to every lane after the barrier, and so are the tables
@@ -1353,8 +1364,8 @@ __global__ __launch_bounds__(64) void k_nbr_build_ext(StepArgs A, Slots S, Work 
         th[t] = reinterpret_cast<const float2*>(luts + LUT_TH_OFF)[t];
     }
     __syncthreads();
-    const int i = xblk(A.xcd) * 64 + (int)threadIdx.x;
-    if (i < A.n) ext_static_slot<MODE, SLOT_MAJOR>(A, S, W, i, lvl, lpg, th, ctl);
+    const int i = split_slot<SPLIT>(A);
+    if (i >= 0) ext_static_slot<MODE, SLOT_MAJOR>(A, S, W, i, lvl, lpg, th, ctl);
 }
 
 // ------------------------------------------------------ PCISPH iteration
@@ -1891,13 +1902,13 @@ __global__ __launch_bounds__(BLOCK) void k_density_wcsph(StepArgs A, Slots S, Wo
 // lists, whose cache lines fill over the life of a wave, and bins in the
 // entries, a root for every 64 candidates: 417 us at 1,132,556 particles, now
 // 354; the force pass takes 113 us instead of 100 for it (bins from distances).
-template <int ROUNDS, bool TAIT>
+template <int ROUNDS, bool TAIT, int SPLIT>
 __global__ __launch_bounds__(64) void k_nbr_build_wcsph(StepArgs A, Slots S, Work W, const float* __restrict__ luts,
                                                         Ctl* ctl) {
     // the build's candidate table, then the density table and the bin thresholds
     __shared__ float2 tabs[2 * LUT_N];
     static_assert(4 * LUT_N >= CAND_CAP, "candidate table");
-    build_wave<ROUNDS, 0, 0, 0, 0, UPF_LIQUID, true>(A, S.pos, W.keys_sorted, W.cells, W.nbr, W.ncount, ctl,
+    build_wave<ROUNDS, 0, 0, 0, 0, UPF_LIQUID, true, SPLIT>(A, S.pos, W.keys_sorted, W.cells, W.nbr, W.ncount, ctl,
                                                     reinterpret_cast<uint32_t*>(tabs));
     __syncthreads();  // the block is the wave: its lists are complete
     float2* th = tabs;
@@ -1907,8 +1918,8 @@ __global__ __launch_bounds__(64) void k_nbr_build_wcsph(StepArgs A, Slots S, Wor
         th[t] = reinterpret_cast<const float2*>(luts + LUT_TH_OFF)[t];
     }
     __syncthreads();
-    const int i = xblk(A.xcd) * 64 + (int)threadIdx.x;
-    if (i < A.n) density_wcsph_slot<TAIT, true>(A, S, W, i, lw, th, ctl);
+    const int i = split_slot<SPLIT>(A);
+    if (i >= 0) density_wcsph_slot<TAIT, true>(A, S, W, i, lw, th, ctl);
 }
 
 // CalculateLiquidParticleForces (:3009-3083) + gravity (:2822-2824).  CODED:
@@ -2267,13 +2278,13 @@ __global__ __launch_bounds__(BLOCK) void k_ext_coupling(StepArgs A, Slots S, Wor
 // kernel: the rigid particles' lists and boundary volumes come first (their
 // counts are kept), then a wave builds the lists of its liquid slots and each
 // lane runs the coupling work of its own slot.
-template <int ROUNDS, int MODE, bool SLOT_MAJOR>
+template <int ROUNDS, int MODE, bool SLOT_MAJOR, int SPLIT>
 __global__ __launch_bounds__(64) void k_nbr_build_coupling(StepArgs A, Slots S, Work W, const float* __restrict__ luts,
                                                            Ctl* ctl) {
     // the build's candidate table, then the tables of the coupling pass
     __shared__ float tabs[4 * LUT_N];
     static_assert(4 * LUT_N >= CAND_CAP, "candidate table");
-    build_wave<ROUNDS, 0, 1, 0, 1, UPF_LIQUID, SLOT_MAJOR>(A, S.pos, W.keys_sorted, W.cells, W.nbr, W.ncount, ctl,
+    build_wave<ROUNDS, 0, 1, 0, 1, UPF_LIQUID, SLOT_MAJOR, SPLIT>(A, S.pos, W.keys_sorted, W.cells, W.nbr, W.ncount, ctl,
                                                           reinterpret_cast<uint32_t*>(tabs));
     __syncthreads();  // the block is the wave: its lists are complete
     float* lvl = tabs;
@@ -2287,8 +2298,8 @@ __global__ __launch_bounds__(64) void k_nbr_build_coupling(StepArgs A, Slots S, 
         lad[t] = luts[4 * LUT_N + t];
     }
     __syncthreads();
-    const int i = xblk(A.xcd) * 64 + (int)threadIdx.x;
-    if (i < A.n) ext_coupling_slot<MODE, SLOT_MAJOR>(A, S, W, i, lvl, lpg, lst, lad, ctl);
+    const int i = split_slot<SPLIT>(A);
+    if (i >= 0) ext_coupling_slot<MODE, SLOT_MAJOR>(A, S, W, i, lvl, lpg, lst, lad, ctl);
 }
 
 // key of a slot for grouping rigid particles by body (non-rigid last)
@@ -2794,6 +2805,27 @@ static inline dim3 grid_persist(const upf_sim* s, int n) {
     return dim3((unsigned)((g + 7) / 8 * 8));  // a multiple of 8 (XCD remap)
 }
 
+// Waves that share a window of 64 slots in the fused builds of n slots, and
+// the grid.  A wave works through its window's cells one after the other, so
+// few windows leave most SIMDs idle behind one chain each; more waves cost a
+// set-up per cell that two of them share.  us per PCISPH / WCSPH step with 1,
+// 4 and 16 waves: 3,080 slots 159 / 110, 128 / 78, 125 / 74; 31,720 slots
+// 215 / 144, 179 / 110, 194 / 118; 143,976 slots 349 / 174, 343 / 164, 414 /
+// 230; 295,944 slots 593 / 222, 608 / 236, 774 / 382.
+static int build_split(int n) {
+    return n < 24576 ? 16 : n < 196608 ? 4 : 1;
+}
+static dim3 build_grid(int n, int split) {
+    return dim3((unsigned)(((n + 63) / 64 * split + 7) / 8 * 8));  // a multiple of 8 (XCD remap)
+}
+// f(std::integral_constant) of the split, a variant of the kernel for each
+template <class F>
+static void with_split(int split, F f) {
+    if (split == 16) f(std::integral_constant<int, 16>{});
+    else if (split == 4) f(std::integral_constant<int, 4>{});
+    else f(std::integral_constant<int, 1>{});
+}
+
 static int alloc_slots(upf_sim* s, Slots& S, int cap) {
     HIPCHK(s->alloc(&S.pos, cap));
     HIPCHK(s->alloc(&S.vel, cap));
@@ -3016,25 +3048,25 @@ static int step_static_head(upf_sim* s) {
     // without LDS staging and the delta-coded loop lists (no bins)
     if (s->tune.nbr_fuse && s->tune.nbr_stage == 0 && s->tune.nbr_tile == 0 && A.code_lists) {
         s->prof.begin(PC_NBR_BUILD_EXT, s->st);
-        const dim3 gb((unsigned)(((s->n + 63) / 64 + 7) / 8 * 8));  // a multiple of 8 (XCD remap)
+        const int split = build_split(s->n), r = s->tune.nbr_rounds, k = s->tune.nbr_skip;
+        const dim3 gb = build_grid(s->n, split);
         auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, gb, dim3(64), 0, s->st, A, S, s->W, s->luts, s->ctl); };
-        const int r = s->tune.nbr_rounds, k = s->tune.nbr_skip;
         // slot-major packed lists when only this kernel reads them (the delta-
         // coded loop lists); the chunk unions read the column-major ones
-        auto go = [&](auto sm) {
+        auto go = [&](auto mode, auto sm, auto sp) {
+            constexpr int M = decltype(mode)::value, SP = decltype(sp)::value;
             constexpr bool SM = decltype(sm)::value;
-            if (akinci) {
-                if (r == 2) k ? launch(k_nbr_build_ext<2, 1, UPF_BOUNDARY_AKINCI, SM>) : launch(k_nbr_build_ext<2, 0, UPF_BOUNDARY_AKINCI, SM>);
-                else if (r == 8) k ? launch(k_nbr_build_ext<8, 1, UPF_BOUNDARY_AKINCI, SM>) : launch(k_nbr_build_ext<8, 0, UPF_BOUNDARY_AKINCI, SM>);
-                else k ? launch(k_nbr_build_ext<4, 1, UPF_BOUNDARY_AKINCI, SM>) : launch(k_nbr_build_ext<4, 0, UPF_BOUNDARY_AKINCI, SM>);
-            } else {
-                if (r == 2) k ? launch(k_nbr_build_ext<2, 1, UPF_BOUNDARY_CPU_REF, SM>) : launch(k_nbr_build_ext<2, 0, UPF_BOUNDARY_CPU_REF, SM>);
-                else if (r == 8) k ? launch(k_nbr_build_ext<8, 1, UPF_BOUNDARY_CPU_REF, SM>) : launch(k_nbr_build_ext<8, 0, UPF_BOUNDARY_CPU_REF, SM>);
-                else k ? launch(k_nbr_build_ext<4, 1, UPF_BOUNDARY_CPU_REF, SM>) : launch(k_nbr_build_ext<4, 0, UPF_BOUNDARY_CPU_REF, SM>);
-            }
+            if (r == 2) k ? launch(k_nbr_build_ext<2, 1, M, SM, SP>) : launch(k_nbr_build_ext<2, 0, M, SM, SP>);
+            else if (r == 8) k ? launch(k_nbr_build_ext<8, 1, M, SM, SP>) : launch(k_nbr_build_ext<8, 0, M, SM, SP>);
+            else k ? launch(k_nbr_build_ext<4, 1, M, SM, SP>) : launch(k_nbr_build_ext<4, 0, M, SM, SP>);
         };
-        if (s->tune.loop_list == 1) go(std::true_type{});
-        else go(std::false_type{});
+        with_split(split, [&](auto sp) {
+            using akinci_t = std::integral_constant<int, UPF_BOUNDARY_AKINCI>;
+            using cpu_t = std::integral_constant<int, UPF_BOUNDARY_CPU_REF>;
+            const bool sm = s->tune.loop_list == 1;
+            if (akinci) sm ? go(akinci_t{}, std::true_type{}, sp) : go(akinci_t{}, std::false_type{}, sp);
+            else sm ? go(cpu_t{}, std::true_type{}, sp) : go(cpu_t{}, std::false_type{}, sp);
+        });
         s->prof.end(s->st);
     } else {
         s->static_lists = true;
@@ -3149,18 +3181,21 @@ static int step_pcisph_rigid(upf_sim* s) {
     }
     if (fuse) {
         s->prof.begin(PC_NBR_BUILD_EXT, s->st);
-        const dim3 gb((unsigned)(((s->n + 63) / 64 + 7) / 8 * 8));  // a multiple of 8 (XCD remap)
+        const int split = build_split(s->n), r = s->tune.nbr_rounds;
+        const dim3 gb = build_grid(s->n, split);
         auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, gb, dim3(64), 0, s->st, A, S, s->W, s->luts, s->ctl); };
-        const int r = s->tune.nbr_rounds;
-        if (akinci) {
-            if (r == 2) launch(k_nbr_build_coupling<2, UPF_BOUNDARY_AKINCI, true>);
-            else if (r == 8) launch(k_nbr_build_coupling<8, UPF_BOUNDARY_AKINCI, true>);
-            else launch(k_nbr_build_coupling<4, UPF_BOUNDARY_AKINCI, true>);
-        } else {
-            if (r == 2) launch(k_nbr_build_coupling<2, UPF_BOUNDARY_CPU_REF, true>);
-            else if (r == 8) launch(k_nbr_build_coupling<8, UPF_BOUNDARY_CPU_REF, true>);
-            else launch(k_nbr_build_coupling<4, UPF_BOUNDARY_CPU_REF, true>);
-        }
+        with_split(split, [&](auto sp) {
+            constexpr int SP = decltype(sp)::value;
+            if (akinci) {
+                if (r == 2) launch(k_nbr_build_coupling<2, UPF_BOUNDARY_AKINCI, true, SP>);
+                else if (r == 8) launch(k_nbr_build_coupling<8, UPF_BOUNDARY_AKINCI, true, SP>);
+                else launch(k_nbr_build_coupling<4, UPF_BOUNDARY_AKINCI, true, SP>);
+            } else {
+                if (r == 2) launch(k_nbr_build_coupling<2, UPF_BOUNDARY_CPU_REF, true, SP>);
+                else if (r == 8) launch(k_nbr_build_coupling<8, UPF_BOUNDARY_CPU_REF, true, SP>);
+                else launch(k_nbr_build_coupling<4, UPF_BOUNDARY_CPU_REF, true, SP>);
+            }
+        });
         s->prof.end(s->st);
     } else {
         s->prof.begin(PC_NBR_EXT, s->st);
@@ -3208,18 +3243,21 @@ static int step_wcsph_static(upf_sim* s, bool tait) {
     if (fuse) {
         // the list build and the density pass as one kernel
         s->prof.begin(PC_NBR_BUILD_DENSITY, s->st);
-        const dim3 gb((unsigned)(((s->n + 63) / 64 + 7) / 8 * 8));  // a multiple of 8 (XCD remap)
+        const int split = build_split(s->n), r = s->tune.nbr_rounds;
+        const dim3 gb = build_grid(s->n, split);
         auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, gb, dim3(64), 0, s->st, A, S, s->W, s->luts, s->ctl); };
-        const int r = s->tune.nbr_rounds;
-        if (tait) {
-            if (r == 2) launch(k_nbr_build_wcsph<2, true>);
-            else if (r == 8) launch(k_nbr_build_wcsph<8, true>);
-            else launch(k_nbr_build_wcsph<4, true>);
-        } else {
-            if (r == 2) launch(k_nbr_build_wcsph<2, false>);
-            else if (r == 8) launch(k_nbr_build_wcsph<8, false>);
-            else launch(k_nbr_build_wcsph<4, false>);
-        }
+        with_split(split, [&](auto sp) {
+            constexpr int SP = decltype(sp)::value;
+            if (tait) {
+                if (r == 2) launch(k_nbr_build_wcsph<2, true, SP>);
+                else if (r == 8) launch(k_nbr_build_wcsph<8, true, SP>);
+                else launch(k_nbr_build_wcsph<4, true, SP>);
+            } else {
+                if (r == 2) launch(k_nbr_build_wcsph<2, false, SP>);
+                else if (r == 8) launch(k_nbr_build_wcsph<8, false, SP>);
+                else launch(k_nbr_build_wcsph<4, false, SP>);
+            }
+        });
         s->prof.end(s->st);
     } else {
         build_lists(s, A);
