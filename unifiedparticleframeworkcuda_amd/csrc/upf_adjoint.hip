@@ -50,6 +50,7 @@
 #include "upf_device.h"
 #include "upf_internal.h"
 #include "upf_kernels.h"
+#include "upf_lanes.h"
 #include "upf_sort.h"
 
 namespace upf {
@@ -57,47 +58,10 @@ namespace ad {
 
 constexpr int AB = 256;  // threads per block
 
-// Pair passes run LANES lanes per particle: each lane takes every LANES-th
-// neighbour, and the lanes' terms are added in list order (DPP broadcasts, one
-// addition per neighbour), so every sum has the bits of a serial loop.  One
-// lane per particle was one serial chain of gathers per wave and about one
-// wave per SIMD at 65,536 particles (density 16.7 us, pressure force 15.6,
-// their reverses 27 and 29); see lanes() for the choice.
-
-// v of lane U of this lane's group of LANES (4: the quad, 16: the DPP row)
-template <int LANES, int U>
-__device__ __forceinline__ float lane_of(float v) {
-    static_assert(LANES == 4 || LANES == 16, "a quad or a row");
-    constexpr int ctrl = LANES == 4 ? U * 0x55 : 0x150 + U;  // quad_perm [U U U U] : row_newbcast U
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xf, 0xf, true));
-}
-// acc -/+ the group's terms, lane 0's first
-template <int LANES, int U = 0>
-__device__ __forceinline__ float sub_terms(float acc, float t) {
-    if constexpr (U < LANES) return sub_terms<LANES, U + 1>(acc - lane_of<LANES, U>(t), t);
-    else return acc;
-}
-template <int LANES, int U = 0>
-__device__ __forceinline__ float add_terms(float acc, float t) {
-    if constexpr (U < LANES) return add_terms<LANES, U + 1>(acc + lane_of<LANES, U>(t), t);
-    else return acc;
-}
-
-// term(j) for this lane's neighbours of the list (none: no neighbour), then
-// add() for the group's LANES terms; the next round's list entry is loaded
-// ahead of this round's gathers
-template <int LANES, class Term, class None, class Add>
-__device__ __forceinline__ void for_pairs(const uint32_t* __restrict__ row, int cnt, int sub, Term term, None none, Add add) {
-    int j = sub < cnt ? (int)row[sub] : 0;
-    for (int k = 0; k < cnt; k += LANES) {
-        const int next = k + LANES + sub;
-        const int jn = next < cnt ? (int)row[next] : 0;
-        if (k + sub < cnt) term(j);
-        else none();
-        add();
-        j = jn;
-    }
-}
+// Pair passes run LANES lanes per particle (upf_lanes.h).  One lane per particle
+// was one serial chain of gathers per wave and about one wave per SIMD at
+// 65,536 particles (density 16.7 us, pressure force 15.6, their reverses 27 and
+// 29; 10.3, 9.9, 12 and 14 now); see lanes() for the choice.
 
 struct Kern {  // closed-form kernels and their radial derivatives, FP32
     float h, a, ah, cs, cv;

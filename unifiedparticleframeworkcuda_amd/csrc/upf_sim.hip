@@ -30,6 +30,7 @@
 #include "upf_device.h"
 #include "upf_internal.h"
 #include "upf_kernels.h"
+#include "upf_lanes.h"
 #include "upf_sort.h"
 #include "upf_stage.h"
 
@@ -945,6 +946,13 @@ __device__ __forceinline__ int split_slot(const StepArgs& A) {
     const int i = (vb / SPLIT) * 64 + lane;
     return i < A.n && lane / (64 / SPLIT) == vb % SPLIT ? i : -1;
 }
+// The same with SPLIT lanes per slot of the wave's 64 / SPLIT.
+template <int SPLIT>
+__device__ __forceinline__ int split_slot_lanes(const StepArgs& A) {
+    const int vb = xblk(A.xcd);
+    const int i = (vb / SPLIT) * 64 + (vb % SPLIT) * (64 / SPLIT) + (int)threadIdx.x / SPLIT;
+    return i < A.n ? i : -1;
+}
 
 template <int ROUNDS, int STAGE, int BIN, int SKIP = 0>
 __global__ __launch_bounds__(64) void k_nbr_build(StepArgs A, const float4* __restrict__ pos,
@@ -1323,6 +1331,88 @@ __device__ __forceinline__ void ext_static_slot(const StepArgs& A, const Slots& 
     W.xs[i] = predict(xi, vi, F, make_float4(0.f, 0.f, 0.f, 0.f), A, d, ctl);
 }
 
+// The external-force work of slot i with LANES lanes (lane sub of them), over
+// the slot's row of packed lists without bins; the correction loop reads the
+// same rows (k_density_lanes, k_force_lanes).
+template <int MODE, int LANES>
+__device__ __forceinline__ void ext_static_lanes(const StepArgs& A, const Slots& S, const Work& W, int i, int sub,
+                                                 const float* lvl, const float* lpg, const float2* th, Ctl* ctl) {
+    const upf_params& P = A.P;
+    const uint32_t* row = W.nbr + (size_t)i * A.nbr_ld;
+    const int cnt = W.ncount[i];
+    const uint32_t e0 = first_entry(row, cnt, sub);
+    const float4 xi = S.pos[i];
+    const int ti = ptype(xi);
+    const float own_psi = S.psi[i], own_rho = S.rho_last[i];
+    if (sub == 0) {
+        W.p[i] = 0.0f;
+        W.xpd[i] = make_float4(xi.x, xi.y, xi.z, pressure_record_w<MODE>(ti, own_psi, P.rest_density));
+        W.fp[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        W.rho[i] = own_rho;
+    }
+    if (ti != UPF_LIQUID) {
+        if (sub == 0) {
+            W.xs[i] = boundary_xs<MODE>((ti == UPF_RIGID && !P.rigid_predicted_current) ? S.x0[i] : xi, own_psi,
+                                        P.rest_density);
+            W.force[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        return;
+    }
+    const float4 vi = S.vel[i];
+    const float h = P.support_radius;
+    const float rv = A.rest_vol, visc = P.visc_const;
+    const float own_p = MODE == UPF_BOUNDARY_CPU_REF ? S.p_prev[i] : S.p_last[i];
+    const float inv = 1.0f / own_rho;
+    const float pg = own_p * inv * inv;
+    float fx = 0.0f, fy = 0.0f, fz = 0.0f, tx, ty, tz;
+    auto none = [&] { tx = ty = tz = 0.0f; };
+    // the terms of ext_static_slot's pair, all subtracted (x + -t is x - t)
+    for_pairs<LANES>(
+        row, cnt, sub, e0,
+        [&](uint32_t e) __attribute__((always_inline)) {
+            const int j = (int)(e >> NB_SLOT_SHIFT);
+            const float4 xj = at_u32(S.pos, j), vj = at_u32(S.vel, j);
+            const int tj = ptype(xj);
+            const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+            none();
+            if (tj == UPF_LIQUID) {
+                const float kv = lvl[bin_of_d2(dx * dx + dy * dy + dz * dz, A.lut_factor, th)];
+                const float vx = vi.x - vj.x, vy = vi.y - vj.y, vz = vi.z - vj.z;
+                tx = vx * rv * rv * visc * kv;
+                ty = vy * rv * rv * visc * kv;
+                tz = vz * rv * rv * visc * kv;
+            } else if (tj == UPF_FROZEN) {
+                float g, wv;
+                if (MODE == UPF_BOUNDARY_CPU_REF) {
+                    g = 0.0f;
+                    wv = own_psi;
+                } else {
+                    const float dist = sqrtf(dx * dx + dy * dy + dz * dz);
+                    uint32_t dl = (uint32_t)(dist * 300.0f / h);
+                    dl = dl > 300u ? 300u : dl;
+                    g = lpg[dl];
+                    wv = S.psi[j];
+                }
+                tx = ((((dx * g) * pg) * P.initial_mass) * P.rest_density) * wv;
+                ty = ((((dy * g) * pg) * P.initial_mass) * P.rest_density) * wv;
+                tz = ((((dz * g) * pg) * P.initial_mass) * P.rest_density) * wv;
+            }
+        },
+        none,
+        [&] {
+            fx = sub_terms<LANES>(fx, tx);
+            fy = sub_terms<LANES>(fy, ty);
+            fz = sub_terms<LANES>(fz, tz);
+        });
+    if (sub != 0) return;
+    fy = fy - P.initial_mass * P.gravity;
+    const Dom d = dom_at(A, i);
+    if (P.add_boundary_force) box_force_static(P, d, xi, fx, fy, fz);
+    const float4 F = make_float4(fx, fy, fz, 0.0f);
+    W.force[i] = F;
+    W.xs[i] = predict(xi, vi, F, make_float4(0.f, 0.f, 0.f, 0.f), A, d, ctl);
+}
+
 template <int MODE>
 __global__ __launch_bounds__(BLOCK) void k_ext_static(StepArgs A, Slots S, Work W, const float* __restrict__ luts,
                                                       Ctl* ctl) {
@@ -1344,7 +1434,8 @@ __global__ __launch_bounds__(BLOCK) void k_ext_static(StepArgs A, Slots S, Work 
 // wave just wrote.  Nothing crosses waves between the two parts, so the
 // memory-bound force work of some waves overlaps the VALU-bound list work of
 // others, and the lists are read back while they are still in the cache.
-template <int ROUNDS, int SKIP, int MODE, bool SLOT_MAJOR, int SPLIT>
+// LANES: SPLIT lanes per slot in the second part, and no delta-coded lists.
+template <int ROUNDS, int SKIP, int MODE, bool SLOT_MAJOR, int SPLIT, bool LANES = false>
 __global__ __launch_bounds__(64) void k_nbr_build_ext(StepArgs A, Slots S, Work W, const float* __restrict__ luts,
                                                       Ctl* ctl) {
     // the build's candidate table, then the tables of the force pass
@@ -1364,8 +1455,13 @@ __global__ __launch_bounds__(64) void k_nbr_build_ext(StepArgs A, Slots S, Work 
         th[t] = reinterpret_cast<const float2*>(luts + LUT_TH_OFF)[t];
     }
     __syncthreads();
-    const int i = split_slot<SPLIT>(A);
-    if (i >= 0) ext_static_slot<MODE, SLOT_MAJOR>(A, S, W, i, lvl, lpg, th, ctl);
+    if constexpr (LANES) {
+        const int i = split_slot_lanes<SPLIT>(A);
+        if (i >= 0) ext_static_lanes<MODE, SPLIT>(A, S, W, i, (int)threadIdx.x % SPLIT, lvl, lpg, th, ctl);
+    } else {
+        const int i = split_slot<SPLIT>(A);
+        if (i >= 0) ext_static_slot<MODE, SLOT_MAJOR>(A, S, W, i, lvl, lpg, th, ctl);
+    }
 }
 
 // ------------------------------------------------------ PCISPH iteration
@@ -1759,6 +1855,124 @@ __global__ __launch_bounds__(BLOCK) void k_force(int t, StepArgs A, Slots S, Wor
     }
 }
 
+// The two iteration passes of one scene with LANES lanes per particle over the
+// packed slot-major lists (k_nbr_build_ext with LANES): k_density's and
+// k_force's expressions.  Few particles leave one chain of list rows and
+// gathers per wave, and the chip mostly idle (9.5 and 9.0 us per launch from
+// 3,080 to 80,648 particles with one lane each); LANES_FIG
+template <int MODE, int LANES>
+__global__ __launch_bounds__(BLOCK) void k_density_lanes(int t, StepArgs A, Work W, const float* __restrict__ luts,
+                                                         Ctl* ctl) {
+    if (t >= __atomic_load_n(&ctl->want_any, __ATOMIC_RELAXED)) return;
+    __shared__ float lw[LUT_N];
+    __shared__ float2 th[LUT_N];
+    __shared__ float wmax[BLOCK / 64];
+    const upf_params& P = A.P;
+    const unsigned id = (unsigned)xblk_down(A.xcd) * BLOCK + threadIdx.x;
+    const int i = (int)(id / LANES), sub = (int)(id % LANES);
+    const bool in = i < A.n;
+    // the list's first entries are on their way while the tables load
+    const float4 xi = in ? W.xs[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const uint32_t* row = W.nbr + (size_t)(in ? i : 0) * A.nbr_ld;
+    const int cnt = in ? W.ncount[i] : 0;
+    const uint32_t e0 = first_entry(row, cnt, sub);
+    for (int k = threadIdx.x; k < LUT_N; k += BLOCK) {
+        lw[k] = k < 300 ? luts[k] : 0.0f;  // bin 300 (dist >= h) weighs 0, as in lut_at
+        th[k] = reinterpret_cast<const float2*>(luts + LUT_TH_OFF)[k];
+    }
+    __syncthreads();
+    float mine = 0.0f;
+    if (in && ptype(xi) == UPF_LIQUID) {
+        const float m = P.initial_mass;
+        const float T = P.support_radius_sq_limit;
+        float rho = P.kernel_self * m;
+        if (P.add_wall_weight)
+            rho = rho + wall_weight<false>(P, wall_distance(P, xi.x, xi.y, xi.z), A.lut_factor, lw);
+        float term;
+        for_pairs<LANES>(
+            row, cnt, sub, e0,
+            [&](uint32_t e) __attribute__((always_inline)) {
+                const float4 xj = at_u32(W.xs, (int)(e >> NB_SLOT_SHIFT));
+                const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+                const float d2 = dx * dx + dy * dy + dz * dz;
+                const float w = lw[bin_of_d2(d2, A.lut_factor, th)];
+                // a pair at d2 >= T adds +0, which leaves rho > 0 as it is
+                const float mj = MODE == UPF_BOUNDARY_AKINCI && ptype(xj) != UPF_LIQUID ? -xj.w : m;
+                term = d2 < T ? w * mj : 0.0f;
+            },
+            [&] { term = 0.0f; }, [&] { rho = add_terms<LANES>(rho, term); });
+        if (sub == 0) {
+            const float err = fmax_ref(rho - P.rest_density, 0.0f);
+            const float p = W.p[i] + fmax_ref(err * P.density_error_factor, 0.0f);
+            W.p[i] = p;
+            reinterpret_cast<float*>(W.xpd)[4 * (size_t)i + 3] = p / (P.rest_density * P.rest_density);
+            W.rho[i] = rho;
+        }
+        mine = rho;
+    }
+    mine = wave_max(mine);
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = mine;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        float b = wmax[0];
+        for (int k = 1; k < BLOCK / 64; ++k) b = fmaxf(b, wmax[k]);
+        if (b > 0.0f) atomicMax(&A.max_slots[(blockIdx.x % A.slots_per_scene) * 32], __float_as_uint(b));
+    }
+}
+
+template <int MODE, int LANES>
+__global__ __launch_bounds__(BLOCK) void k_force_lanes(int t, StepArgs A, Slots S, Work W,
+                                                       const float* __restrict__ luts, Ctl* ctl) {
+    if (t >= __atomic_load_n(&ctl->want_any, __ATOMIC_RELAXED)) return;
+    if (blockIdx.x == 0 && threadIdx.x < 64) loop_test(A, 0, t, threadIdx.x, ctl);
+    __shared__ float lpg[LUT_N];
+    __shared__ float2 th[LUT_N];
+    const upf_params& P = A.P;
+    const unsigned id = (unsigned)xblk(A.xcd) * BLOCK + threadIdx.x;
+    const int i = (int)(id / LANES), sub = (int)(id % LANES);
+    const bool in = i < A.n;
+    const float4 xr = in ? W.xpd[i] : make_float4(0.f, 0.f, 0.f, -0.0f);
+    const uint32_t* row = W.nbr + (size_t)(in ? i : 0) * A.nbr_ld;
+    const int cnt = in ? W.ncount[i] : 0;
+    const uint32_t e0 = first_entry(row, cnt, sub);
+    for (int k = threadIdx.x; k < LUT_N; k += BLOCK) {
+        lpg[k] = luts[LUT_N + k];
+        th[k] = reinterpret_cast<const float2*>(luts + LUT_TH_OFF)[k];
+    }
+    __syncthreads();
+    if (__builtin_signbit(xr.w)) return;  // not liquid
+    const float m = P.initial_mass;
+    float fx = 0.0f, fy = 0.0f, fz = 0.0f, tx, ty, tz;
+    for_pairs<LANES>(
+        row, cnt, sub, e0,
+        [&](uint32_t e) __attribute__((always_inline)) {
+            const float4 xj = at_u32(W.xpd, (int)(e >> NB_SLOT_SHIFT));
+            const float dx = xr.x - xj.x, dy = xr.y - xj.y, dz = xr.z - xj.z;
+            const float g = lpg[bin_of_d2(dx * dx + dy * dy + dz * dz, A.lut_factor, th)];
+            float pd = xj.w, mj = m;
+            if (MODE == UPF_BOUNDARY_AKINCI && __builtin_signbit(xj.w)) {  // boundary: p_j = 0, mass rho0 psi_j
+                mj = -xj.w;
+                pd = 0.0f;
+            }
+            const float grad = xr.w + pd;
+            tx = (((dx * g) * grad) * m) * mj;
+            ty = (((dy * g) * grad) * m) * mj;
+            tz = (((dz * g) * grad) * m) * mj;
+        },
+        [&] { tx = ty = tz = 0.0f; },
+        [&] {
+            fx = sub_terms<LANES>(fx, tx);
+            fy = sub_terms<LANES>(fy, ty);
+            fz = sub_terms<LANES>(fz, tz);
+        });
+    if (sub != 0) return;
+    const float4 Fp = make_float4(fx, fy, fz, 0.0f);
+    // written when this iteration may be the scene's last (k_force)
+    if (t + 1 >= __atomic_load_n(&A.sctl[0].want, __ATOMIC_RELAXED)) W.fp[i] = Fp;
+    const float4 xi = make_float4(xr.x, xr.y, xr.z, __int_as_float(UPF_LIQUID));
+    W.xs[i] = predict(xi, S.vel[i], W.force[i], Fp, A, A.dom0, ctl);
+}
+
 // ------------------------------------------------------------ integration
 // UpdateLiquidParticlePosVelSphCPU (:3705-3742) + BoundaryHandlingBoxPerParticleOMP
 // (:3940-3970) / BoundaryHandlingPureFluidOMP (:3972-3998): symplectic Euler,
@@ -1817,6 +2031,42 @@ __global__ void k_integrate(StepArgs A, Slots S, Work W, int pcisph, int pure_fl
 // P.add_wall_weight, then the pressure of physicsType 'w' (TAIT,
 // CalculatePressureWCSPH :2491-2501) or 'o' (CalculatePressureSPH
 // :2479-2489), over the lists
+// Slot i's density, pressure and records from its sum over the list.
+template <bool TAIT>
+__device__ __forceinline__ void finish_density_wcsph(const StepArgs& A, const Slots& S, const Work& W, int i,
+                                                     const float4& xi, float rho, const float* lw) {
+    const upf_params& P = A.P;
+    if (ptype(xi) != UPF_LIQUID) {
+        W.rho[i] = 0.0f;
+        W.pres[i] = 0.0f;
+        W.force[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        W.xpd[i] = make_float4(xi.x, xi.y, xi.z, -1.0f);  // w < 0: not a fluid neighbour
+        return;
+    }
+    const float m = P.initial_mass;
+    if (P.add_wall_weight) rho = rho + wall_weight<true>(P, wall_distance(P, xi.x, xi.y, xi.z), A.lut_factor, lw);
+    float pres;
+    if constexpr (TAIT) {
+        const float gamma = 7.0f;
+        const float b = P.rest_density * P.gas_const_wcsph / gamma;
+        const float frac = rho / P.rest_density;
+        const float pg = powf(frac, gamma);
+        pres = fmax_ref(0.0f, b * (pg - 1.0f));
+    } else {  // gamma = 1: p = k (rho - rho0) written as the reference writes it
+        const float b = P.rest_density * P.gas_const_sph / 1.0f;
+        const float frac = rho / P.rest_density;
+        pres = fmax_ref(0.0f, b * (frac - 1.0f));
+    }
+    W.rho[i] = rho;
+    W.pres[i] = pres;
+    // what the force pass needs of this particle as a neighbour, in two
+    // 16-byte records: (position, m / rho) and (velocity, p / rho^2) -- the
+    // same expressions it would evaluate per pair
+    const float4 vi = S.vel[i];
+    W.xpd[i] = make_float4(xi.x, xi.y, xi.z, m / rho);
+    W.vpg[i] = make_float4(vi.x, vi.y, vi.z, pres / (rho * rho));
+}
+
 // The density work of slot i (one thread), shared by the density pass, which
 // reads column-major packed lists with the table bins in their entries, and
 // (FUSED) the fused list build, whose lists are the slot's own rows without
@@ -1827,16 +2077,9 @@ __device__ __forceinline__ void density_wcsph_slot(const StepArgs& A, const Slot
                                                    const float* lw, const float2* th, Ctl* ctl) {
     const upf_params& P = A.P;
     const float4 xi = S.pos[i];
-    if (ptype(xi) != UPF_LIQUID) {
-        W.rho[i] = 0.0f;
-        W.pres[i] = 0.0f;
-        W.force[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        W.xpd[i] = make_float4(xi.x, xi.y, xi.z, -1.0f);  // w < 0: not a fluid neighbour
-        return;
-    }
     const float m = P.initial_mass;
     float rho = P.kernel_self * m;
-    const int cnt = W.ncount[i];
+    const int cnt = W.ncount[i];  // 0 unless liquid
     if constexpr (FUSED) {
         const uint32_t* L = W.nbr + (size_t)i * A.nbr_ld;
         ListEncoder enc(W, i, (size_t)A.stride);
@@ -1863,27 +2106,28 @@ __device__ __forceinline__ void density_wcsph_slot(const StepArgs& A, const Slot
     } else {
         for (int k = 0; k < cnt; ++k) rho = rho + lw[W.nbr[(size_t)k * A.stride + i] & NB_BIN_MASK] * m;
     }
-    if (P.add_wall_weight) rho = rho + wall_weight<true>(P, wall_distance(P, xi.x, xi.y, xi.z), A.lut_factor, lw);
-    float pres;
-    if constexpr (TAIT) {
-        const float gamma = 7.0f;
-        const float b = P.rest_density * P.gas_const_wcsph / gamma;
-        const float frac = rho / P.rest_density;
-        const float pg = powf(frac, gamma);
-        pres = fmax_ref(0.0f, b * (pg - 1.0f));
-    } else {  // gamma = 1: p = k (rho - rho0) written as the reference writes it
-        const float b = P.rest_density * P.gas_const_sph / 1.0f;
-        const float frac = rho / P.rest_density;
-        pres = fmax_ref(0.0f, b * (frac - 1.0f));
-    }
-    W.rho[i] = rho;
-    W.pres[i] = pres;
-    // what the force pass needs of this particle as a neighbour, in two
-    // 16-byte records: (position, m / rho) and (velocity, p / rho^2) -- the
-    // same expressions it would evaluate per pair
-    const float4 vi = S.vel[i];
-    W.xpd[i] = make_float4(xi.x, xi.y, xi.z, m / rho);
-    W.vpg[i] = make_float4(vi.x, vi.y, vi.z, pres / (rho * rho));
+    finish_density_wcsph<TAIT>(A, S, W, i, xi, rho, lw);
+}
+
+// The same with LANES lanes (lane sub of them) over the slot's row; the force
+// pass reads the rows too (k_force_wcsph_lanes).
+template <bool TAIT, int LANES>
+__device__ __forceinline__ void density_wcsph_lanes(const StepArgs& A, const Slots& S, const Work& W, int i, int sub,
+                                                    const float* lw, const float2* th) {
+    const upf_params& P = A.P;
+    const uint32_t* row = W.nbr + (size_t)i * A.nbr_ld;
+    const int cnt = W.ncount[i];
+    const float4 xi = S.pos[i];
+    float rho = P.kernel_self * P.initial_mass, term;
+    for_pairs<LANES>(
+        row, cnt, sub,
+        [&](uint32_t e) __attribute__((always_inline)) {
+            const float4 xj = at_u32(S.pos, (int)(e >> NB_SLOT_SHIFT));
+            const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+            term = lw[bin_of_d2(dx * dx + dy * dy + dz * dz, A.lut_factor, th)] * P.initial_mass;
+        },
+        [&] { term = -0.0f; }, [&] { rho = add_terms<LANES>(rho, term); });
+    if (sub == 0) finish_density_wcsph<TAIT>(A, S, W, i, xi, rho, lw);
 }
 
 template <bool TAIT>
@@ -1902,7 +2146,8 @@ __global__ __launch_bounds__(BLOCK) void k_density_wcsph(StepArgs A, Slots S, Wo
 // lists, whose cache lines fill over the life of a wave, and bins in the
 // entries, a root for every 64 candidates: 417 us at 1,132,556 particles, now
 // 354; the force pass takes 113 us instead of 100 for it (bins from distances).
-template <int ROUNDS, bool TAIT, int SPLIT>
+// LANES as in k_nbr_build_ext.
+template <int ROUNDS, bool TAIT, int SPLIT, bool LANES = false>
 __global__ __launch_bounds__(64) void k_nbr_build_wcsph(StepArgs A, Slots S, Work W, const float* __restrict__ luts,
                                                         Ctl* ctl) {
     // the build's candidate table, then the density table and the bin thresholds
@@ -1918,8 +2163,13 @@ __global__ __launch_bounds__(64) void k_nbr_build_wcsph(StepArgs A, Slots S, Wor
         th[t] = reinterpret_cast<const float2*>(luts + LUT_TH_OFF)[t];
     }
     __syncthreads();
-    const int i = split_slot<SPLIT>(A);
-    if (i >= 0) density_wcsph_slot<TAIT, true>(A, S, W, i, lw, th, ctl);
+    if constexpr (LANES) {
+        const int i = split_slot_lanes<SPLIT>(A);
+        if (i >= 0) density_wcsph_lanes<TAIT, SPLIT>(A, S, W, i, (int)threadIdx.x % SPLIT, lw, th);
+    } else {
+        const int i = split_slot<SPLIT>(A);
+        if (i >= 0) density_wcsph_slot<TAIT, true>(A, S, W, i, lw, th, ctl);
+    }
 }
 
 // CalculateLiquidParticleForces (:3009-3083) + gravity (:2822-2824).  CODED:
@@ -1968,6 +2218,64 @@ __global__ __launch_bounds__(BLOCK) void k_force_wcsph(StepArgs A, Slots S, Work
             fy = fy - vy * pVol * nVol * P.visc_const * kv;
             fz = fz - vz * pVol * nVol * P.visc_const * kv;
         });
+    if (P.add_boundary_force) box_force_static(P, dom_at(A, i), xi, fx, fy, fz);
+    fy = fy - P.initial_mass * P.gravity;
+    W.force[i] = make_float4(fx, fy, fz, 0.0f);
+}
+
+// The force pass with LANES lanes per particle over the slot-major lists.
+template <int LANES>
+__global__ __launch_bounds__(BLOCK) void k_force_wcsph_lanes(StepArgs A, Slots S, Work W,
+                                                             const float* __restrict__ luts, Ctl* ctl) {
+    __shared__ float lvl[LUT_N], lpg[LUT_N];
+    __shared__ float2 th[LUT_N];
+    const upf_params& P = A.P;
+    const unsigned id = blockIdx.x * BLOCK + threadIdx.x;
+    const int i = (int)(id / LANES), sub = (int)(id % LANES);
+    const bool in = i < A.n;
+    const float4 xi = in ? S.pos[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const uint32_t* row = W.nbr + (size_t)(in ? i : 0) * A.nbr_ld;
+    const int cnt = in ? W.ncount[i] : 0;
+    const uint32_t e0 = first_entry(row, cnt, sub);
+    for (int t = threadIdx.x; t < LUT_N; t += BLOCK) {
+        lvl[t] = luts[2 * LUT_N + t];
+        lpg[t] = luts[LUT_N + t];
+        th[t] = reinterpret_cast<const float2*>(luts + LUT_TH_OFF)[t];
+    }
+    __syncthreads();
+    if (!in || ptype(xi) != UPF_LIQUID) return;
+    const float m = P.initial_mass;
+    const float p_i = W.pres[i];
+    const float invD = (float)(1.0 / (double)W.rho[i]);
+    const float pVol = m * invD;
+    const float4 vi = S.vel[i];
+    float fx = 0.0f, fy = 0.0f, fz = 0.0f, gx, gy, gz, ux, uy, uz;
+    auto none = [&] { gx = gy = gz = ux = uy = uz = 0.0f; };
+    for_pairs<LANES>(
+        row, cnt, sub, e0,
+        [&](uint32_t e) __attribute__((always_inline)) {
+            const int j = (int)(e >> NB_SLOT_SHIFT);
+            const float4 xj = at_u32(W.xpd, j), vj = at_u32(W.vpg, j);
+            if (xj.w < 0.0f) return none();  // not a fluid neighbour
+            const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+            const uint32_t bin = bin_of_d2(dx * dx + dy * dy + dz * dz, A.lut_factor, th);
+            const float kv = lvl[bin], g = lpg[bin];
+            const float grad = p_i * invD * invD + vj.w;
+            gx = (((dx * g) * grad) * m) * m;
+            gy = (((dy * g) * grad) * m) * m;
+            gz = (((dz * g) * grad) * m) * m;
+            const float vx = vi.x - vj.x, vy = vi.y - vj.y, vz = vi.z - vj.z;
+            ux = vx * pVol * xj.w * P.visc_const * kv;
+            uy = vy * pVol * xj.w * P.visc_const * kv;
+            uz = vz * pVol * xj.w * P.visc_const * kv;
+        },
+        none,
+        [&] {  // per neighbour the pressure term, then the viscosity term
+            fx = sub_terms2<LANES>(fx, gx, ux);
+            fy = sub_terms2<LANES>(fy, gy, uy);
+            fz = sub_terms2<LANES>(fz, gz, uz);
+        });
+    if (sub != 0) return;
     if (P.add_boundary_force) box_force_static(P, dom_at(A, i), xi, fx, fy, fz);
     fy = fy - P.initial_mass * P.gravity;
     W.force[i] = make_float4(fx, fy, fz, 0.0f);
@@ -2699,6 +3007,7 @@ struct upf_sim {
     int n_bodies = 0;
     int last_method = UPF_PCISPH_STATIC;
     bool union_ready = false;  // this step's union lists are built (static PCISPH)
+    int lanes = 0;             // lanes per particle of this step's pair passes over slot-major lists (0: coded lists)
     hipStream_t st = nullptr;
     Slots S[2];
     Work W;
@@ -2815,8 +3124,19 @@ static inline dim3 grid_persist(const upf_sim* s, int n) {
 static int build_split(int n) {
     return n < 24576 ? 16 : n < 196608 ? 4 : 1;
 }
+static dim3 lanes_grid(int n, int lanes) {
+    return dim3((unsigned)((((size_t)n * lanes + BLOCK - 1) / BLOCK + 7) / 8 * 8));  // a multiple of 8 (XCD remap)
+}
 static dim3 build_grid(int n, int split) {
     return dim3((unsigned)(((n + 63) / 64 * split + 7) / 8 * 8));  // a multiple of 8 (XCD remap)
+}
+// Lanes per particle of the pair passes after a fused build, 0 for one lane and
+// the delta-coded lists: the build's split, where the launch shapes are the
+// default ones (their variants exist for one wave per window) and the scene is
+// not one of a batch, whose passes run over chunks of slots.
+static int pair_lanes(const upf_sim* s, int split) {
+    const upf_tuning& t = s->tune;
+    return split > 1 && s->n_scenes == 1 && t.loop_list == 1 && t.nbr_rounds == 4 && !t.nbr_skip ? split : 0;
 }
 // f(std::integral_constant) of the split, a variant of the kernel for each
 template <class F>
@@ -2913,14 +3233,25 @@ static void enqueue_iteration(upf_sim* s, const StepArgs& A, int t) {
     const int lw = s->tune.loop_width, ll = s->tune.loop_list;
     // the iteration passes are timed by their own dispatches when profiling
     // (their device time is the figure the roofline is quoted on)
-#define UPF_PASS(KERNEL, CLS)                                                                               \
-    do {                                                                                                   \
-        hipEvent_t e0, e1;                                                                                 \
-        if (s->prof.span(CLS, e0, e1))                                                                     \
-            hipExtLaunchKernelGGL(KERNEL, g, b, 0, s->st, e0, e1, 0, t, A, S, s->W, s->luts, s->ctl);      \
-        else                                                                                               \
-            hipLaunchKernelGGL(KERNEL, g, b, 0, s->st, t, A, S, s->W, s->luts, s->ctl);                    \
-    } while (0)
+    auto pass = [&](int cls, dim3 grid, dim3 block, auto kernel, auto... args) {
+        hipEvent_t e0, e1;
+        if (s->prof.span(cls, e0, e1))
+            hipExtLaunchKernelGGL(kernel, grid, block, 0, s->st, e0, e1, 0, t, A, args..., s->W, s->luts, s->ctl);
+        else
+            hipLaunchKernelGGL(kernel, grid, block, 0, s->st, t, A, args..., s->W, s->luts, s->ctl);
+    };
+#define UPF_PASS(KERNEL, CLS) pass(CLS, g, b, KERNEL, S)
+    if (s->lanes) {
+        with_split(s->lanes, [&](auto lanes) {
+            constexpr int L = decltype(lanes)::value;
+            if constexpr (L > 1) {
+                const dim3 gl = lanes_grid(s->n, L), bl(BLOCK);
+                pass(PC_DENSITY, gl, bl, k_density_lanes<MODE, L>);
+                pass(PC_FORCE, gl, bl, k_force_lanes<MODE, L>, S);
+            }
+        });
+        return;
+    }
     // union lists (the step built them): both passes read their neighbours'
     // records from LDS; the Akinci density needs boundary volumes by slot and
     // keeps the delta-coded lists
@@ -3044,11 +3375,13 @@ static int step_static_head(upf_sim* s) {
         s->prof.end(s->st);
         s->psi_ready = true;
     }
+    s->lanes = 0;
     // the fused list build + external forces needs the cell-by-cell build
     // without LDS staging and the delta-coded loop lists (no bins)
     if (s->tune.nbr_fuse && s->tune.nbr_stage == 0 && s->tune.nbr_tile == 0 && A.code_lists) {
         s->prof.begin(PC_NBR_BUILD_EXT, s->st);
         const int split = build_split(s->n), r = s->tune.nbr_rounds, k = s->tune.nbr_skip;
+        s->lanes = pair_lanes(s, split);
         const dim3 gb = build_grid(s->n, split);
         auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, gb, dim3(64), 0, s->st, A, S, s->W, s->luts, s->ctl); };
         // slot-major packed lists when only this kernel reads them (the delta-
@@ -3063,7 +3396,15 @@ static int step_static_head(upf_sim* s) {
         with_split(split, [&](auto sp) {
             using akinci_t = std::integral_constant<int, UPF_BOUNDARY_AKINCI>;
             using cpu_t = std::integral_constant<int, UPF_BOUNDARY_CPU_REF>;
+            constexpr int SP = decltype(sp)::value;
             const bool sm = s->tune.loop_list == 1;
+            if constexpr (SP > 1) {
+                if (s->lanes) {
+                    if (akinci) launch(k_nbr_build_ext<4, 0, UPF_BOUNDARY_AKINCI, true, SP, true>);
+                    else launch(k_nbr_build_ext<4, 0, UPF_BOUNDARY_CPU_REF, true, SP, true>);
+                    return;
+                }
+            }
             if (akinci) sm ? go(akinci_t{}, std::true_type{}, sp) : go(akinci_t{}, std::false_type{}, sp);
             else sm ? go(cpu_t{}, std::true_type{}, sp) : go(cpu_t{}, std::false_type{}, sp);
         });
@@ -3136,6 +3477,7 @@ static int step_pcisph_rigid(upf_sim* s) {
     int rc = sort_and_bin(s);
     if (rc) return rc;
     s->union_ready = false;  // the coupling loop reads the delta-coded lists
+    s->lanes = 0;
     const StepArgs A = s->args();
     Slots& S = s->S[s->cur];
     const dim3 g = grid_for(s->n);
@@ -3240,14 +3582,23 @@ static int step_wcsph_static(upf_sim* s, bool tait) {
     Slots& S = s->S[s->cur];
     const dim3 g = grid_for(s->n);
     const bool fuse = s->tune.nbr_fuse && s->tune.nbr_stage == 0 && s->tune.nbr_tile == 0 && A.code_lists;
+    s->lanes = 0;
     if (fuse) {
         // the list build and the density pass as one kernel
         s->prof.begin(PC_NBR_BUILD_DENSITY, s->st);
         const int split = build_split(s->n), r = s->tune.nbr_rounds;
+        s->lanes = pair_lanes(s, split);
         const dim3 gb = build_grid(s->n, split);
         auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, gb, dim3(64), 0, s->st, A, S, s->W, s->luts, s->ctl); };
         with_split(split, [&](auto sp) {
             constexpr int SP = decltype(sp)::value;
+            if constexpr (SP > 1) {
+                if (s->lanes) {
+                    if (tait) launch(k_nbr_build_wcsph<4, true, SP, true>);
+                    else launch(k_nbr_build_wcsph<4, false, SP, true>);
+                    return;
+                }
+            }
             if (tait) {
                 if (r == 2) launch(k_nbr_build_wcsph<2, true, SP>);
                 else if (r == 8) launch(k_nbr_build_wcsph<8, true, SP>);
@@ -3267,7 +3618,14 @@ static int step_wcsph_static(upf_sim* s, bool tait) {
         s->prof.end(s->st);
     }
     s->prof.begin(PC_WCSPH_FORCE, s->st);
-    if (fuse) hipLaunchKernelGGL(k_force_wcsph<1>, g, dim3(BLOCK), 0, s->st, A, S, s->W, s->luts, s->ctl);
+    if (s->lanes)
+        with_split(s->lanes, [&](auto lanes) {
+            constexpr int L = decltype(lanes)::value;
+            if constexpr (L > 1)
+                hipLaunchKernelGGL(k_force_wcsph_lanes<L>, lanes_grid(s->n, L), dim3(BLOCK), 0, s->st, A, S, s->W, s->luts,
+                                   s->ctl);
+        });
+    else if (fuse) hipLaunchKernelGGL(k_force_wcsph<1>, g, dim3(BLOCK), 0, s->st, A, S, s->W, s->luts, s->ctl);
     else hipLaunchKernelGGL(k_force_wcsph<0>, g, dim3(BLOCK), 0, s->st, A, S, s->W, s->luts, s->ctl);
     s->prof.end(s->st);
     s->prof.begin(PC_INTEGRATE, s->st);
