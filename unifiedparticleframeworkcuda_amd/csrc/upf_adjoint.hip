@@ -61,7 +61,7 @@ constexpr int AB = 256;  // threads per block
 // Pair passes run LANES lanes per particle (upf_lanes.h).  One lane per particle
 // was one serial chain of gathers per wave and about one wave per SIMD at
 // 65,536 particles (density 16.7 us, pressure force 15.6, their reverses 27 and
-// 29; 10.3, 9.9, 12 and 14 now); see lanes() for the choice.
+// 29; 8.9, 8.7, 10 and 14 now); see lanes() for the choice.
 
 struct Kern {  // closed-form kernels and their radial derivatives, FP32
     float h, a, ah, cs, cv;
@@ -311,25 +311,16 @@ __global__ __launch_bounds__(AB) void k_ext(int n, const float4* __restrict__ x,
         return;
     }
     const float4 vi = v[i];
-    float fx = 0.0f, fy = 0.0f, fz = 0.0f, tx, ty, tz;
-    auto none = [&] { tx = ty = tz = 0.0f; };
+    float fx = 0.0f, fy = 0.0f, fz = 0.0f;
     for_pairs<LANES>(
-        nb + (size_t)i * ld, cnt[i], sub,
-        [&](int j) {
-            const float4 xj = x[j], vj = v[j];
-            if (!is_fluid(xj)) return none();
-            const float r = len3(xi.x - xj.x, xi.y - xj.y, xi.z - xj.z);
+        nb + (size_t)i * ld, cnt[i], sub, [&](uint32_t j) { return Pair4{x[j], v[j]}; },
+        [&](const Pair4& q, bool have) {
+            if (!have || !is_fluid(q.a)) return Term3{0.0f, 0.0f, 0.0f};
+            const float r = len3(xi.x - q.a.x, xi.y - q.a.y, xi.z - q.a.z);
             const float s = C.cvis * C.kn.L(r);
-            tx = (vi.x - vj.x) * s;
-            ty = (vi.y - vj.y) * s;
-            tz = (vi.z - vj.z) * s;
+            return Term3{(vi.x - q.b.x) * s, (vi.y - q.b.y) * s, (vi.z - q.b.z) * s};
         },
-        none,
-        [&] {
-            fx = sub_terms<LANES>(fx, tx);
-            fy = sub_terms<LANES>(fy, ty);
-            fz = sub_terms<LANES>(fz, tz);
-        });
+        [&](const Term3& t) { sub_terms<LANES>(fx, fy, fz, t); });
     if (sub != 0) return;
     fy = fy - C.m * C.g;
     float wf[3], wg[3];
@@ -354,14 +345,12 @@ __global__ __launch_bounds__(AB) void k_density(int n, const float4* __restrict_
     float rho = 0.0f, pi = 0.0f;
     if (is_fluid_w(xi.w)) {
         rho = C.m * C.kn.W(0.0f);
-        float t;
         for_pairs<LANES>(
-            nb + (size_t)i * ld, cnt[i], sub,
-            [&](int j) {
-                const float4 xj = xs[j];
-                t = C.m * C.kn.W(len3(xi.x - xj.x, xi.y - xj.y, xi.z - xj.z));
+            nb + (size_t)i * ld, cnt[i], sub, [&](uint32_t j) { return xs[j]; },
+            [&](const float4& xj, bool have) {
+                return have ? C.m * C.kn.W(len3(xi.x - xj.x, xi.y - xj.y, xi.z - xj.z)) : -0.0f;
             },
-            [&] { t = -0.0f; }, [&] { rho = add_terms<LANES>(rho, t); });
+            [&](float t) { rho = add_terms<LANES>(rho, t); });
         pi = p[i] + C.delta * softplus(rho - C.rho0);
     }
     if (sub != 0) return;
@@ -395,23 +384,15 @@ __global__ __launch_bounds__(AB) void k_pforce(int n, const float4* __restrict__
         vn = v[i];
     } else {
         const float pi = rec[i].w;
-        float fx = 0.0f, fy = 0.0f, fz = 0.0f, tx, ty, tz;
+        float fx = 0.0f, fy = 0.0f, fz = 0.0f;
         for_pairs<LANES>(
-            nb + (size_t)i * ld, cnt[i], sub,
-            [&](int j) {
-                const float4 xj = rec[j];
+            nb + (size_t)i * ld, cnt[i], sub, [&](uint32_t j) { return rec[j]; },
+            [&](const float4& xj, bool have) {
                 const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
                 const float s = C.kn.G(len3(dx, dy, dz)) * (pi + xj.w) * C.cp;
-                tx = dx * s;
-                ty = dy * s;
-                tz = dz * s;
+                return have ? Term3{dx * s, dy * s, dz * s} : Term3{0.0f, 0.0f, 0.0f};
             },
-            [&] { tx = ty = tz = 0.0f; },
-            [&] {
-                fx = sub_terms<LANES>(fx, tx);
-                fy = sub_terms<LANES>(fy, ty);
-                fz = sub_terms<LANES>(fz, tz);
-            });
+            [&](const Term3& t) { sub_terms<LANES>(fx, fy, fz, t); });
         if (sub != 0) return;
         const float4 vi = v[i], f = F[i];
         if constexpr (!LAST) {
@@ -483,30 +464,29 @@ __global__ __launch_bounds__(AB) void kr_pforce(int n, const float4* __restrict_
         return;
     }
     const float4 gi = gFp[i];
-    float acc = 0.0f, gxx = 0.0f, gxy = 0.0f, gxz = 0.0f, ta, tx, ty, tz;
+    float acc = 0.0f, gxx = 0.0f, gxy = 0.0f, gxz = 0.0f;
+    struct Terms {
+        float a;
+        Term3 g;
+    };
     for_pairs<LANES>(
-        nb + (size_t)i * ld, cnt[i], sub,
-        [&](int j) {
-            const float4 xj = x[j], gj = gFp[j];
+        nb + (size_t)i * ld, cnt[i], sub, [&](uint32_t j) { return Pair4{x[j], gFp[j]}; },
+        [&](const Pair4& q, bool have) {
+            const float4 &xj = q.a, &gj = q.b;
+            if (!have) return Terms{0.0f, {0.0f, 0.0f, 0.0f}};
             const float4 d = make_float4(xi.x - xj.x, xi.y - xj.y, xi.z - xj.z, 0.0f);
             const float r = len3(d.x, d.y, d.z);
             const float4 w = make_float4(gi.x - gj.x, gi.y - gj.y, gi.z - gj.z, 0.0f);
             const float G = C.kn.G(r);
             const float dw = dot3(d, w);
-            ta = C.cp * G * dw;
             const float pp = gi.w + gj.w;
             const float s = r > 0.0f ? C.kn.dG(r) / r * dw : 0.0f;
             const float t = C.cp * pp;
-            tx = (w.x * G + d.x * s) * t;
-            ty = (w.y * G + d.y * s) * t;
-            tz = (w.z * G + d.z * s) * t;
+            return Terms{C.cp * G * dw, {(w.x * G + d.x * s) * t, (w.y * G + d.y * s) * t, (w.z * G + d.z * s) * t}};
         },
-        [&] { ta = tx = ty = tz = 0.0f; },
-        [&] {
-            acc = sub_terms<LANES>(acc, ta);
-            gxx = sub_terms<LANES>(gxx, tx);
-            gxy = sub_terms<LANES>(gxy, ty);
-            gxz = sub_terms<LANES>(gxz, tz);
+        [&](const Terms& t) {
+            acc = sub_terms<LANES>(acc, t.a);
+            sub_terms<LANES>(gxx, gxy, gxz, t.g);
         });
     if (sub != 0) return;
     const float g = gp[i] + acc;
@@ -531,27 +511,18 @@ __global__ __launch_bounds__(AB) void kr_density(int n, const float4* __restrict
     const float w = xs[i].w;
     if (!is_fluid_w(w)) return;
     const float4 xi = rec[i];
-    float gx = 0.0f, gy = 0.0f, gz = 0.0f, tx, ty, tz;
-    auto none = [&] { tx = ty = tz = -0.0f; };
+    float gx = 0.0f, gy = 0.0f, gz = 0.0f;
     for_pairs<LANES>(
-        nb + (size_t)i * ld, cnt[i], sub,
-        [&](int j) {
-            const float4 xj = rec[j];
+        nb + (size_t)i * ld, cnt[i], sub, [&](uint32_t j) { return rec[j]; },
+        [&](const float4& xj, bool have) {
             const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
             const float r = len3(dx, dy, dz);
-            if (!(r < C.kn.h) || r == 0.0f) return none();
+            if (!have || !(r < C.kn.h) || r == 0.0f) return Term3{-0.0f, -0.0f, -0.0f};
             const float gr = xi.w + xj.w;
             const float s = C.m * C.kn.dW(r) / r * gr;
-            tx = dx * s;
-            ty = dy * s;
-            tz = dz * s;
+            return Term3{dx * s, dy * s, dz * s};
         },
-        none,
-        [&] {
-            gx = add_terms<LANES>(gx, tx);
-            gy = add_terms<LANES>(gy, ty);
-            gz = add_terms<LANES>(gz, tz);
-        });
+        [&](const Term3& t) { add_terms<LANES>(gx, gy, gz, t); });
     if (sub != 0) return;
     const float g3[3] = {gx, gy, gz};
     float zb[3];
@@ -583,37 +554,33 @@ __global__ __launch_bounds__(AB) void kr_ext(int n, const float4* __restrict__ x
     if (!is_fluid(xi)) return;
     const float4 vi = v[i], gi = gF[i];
     float gvx = 0.0f, gvy = 0.0f, gvz = 0.0f, gxx = 0.0f, gxy = 0.0f, gxz = 0.0f;
-    float tvx, tvy, tvz, tx, ty, tz;
-    auto none = [&] { tvx = tvy = tvz = tx = ty = tz = 0.0f; };
+    struct Rec {
+        float4 x, g, v;
+    };
+    struct Terms {
+        Term3 v, x;
+    };
     for_pairs<LANES>(
-        nb + (size_t)i * ld, cnt[i], sub,
-        [&](int j) {
-            const float4 xj = x[j], gj = gF[j], vj = v[j];
-            if (!is_fluid(xj)) return none();
+        nb + (size_t)i * ld, cnt[i], sub, [&](uint32_t j) { return Rec{x[j], gF[j], v[j]}; },
+        [&](const Rec& q, bool have) {
+            const float4 &xj = q.x, &gj = q.g, &vj = q.v;
+            Terms t = {{0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}};
+            if (!have || !is_fluid(xj)) return t;
             const float4 d = make_float4(xi.x - xj.x, xi.y - xj.y, xi.z - xj.z, 0.0f);
             const float r = len3(d.x, d.y, d.z);
             const float4 w = make_float4(gi.x - gj.x, gi.y - gj.y, gi.z - gj.z, 0.0f);
             const float sl = C.cvis * C.kn.L(r);
-            tvx = w.x * sl;
-            tvy = w.y * sl;
-            tvz = w.z * sl;
-            tx = ty = tz = 0.0f;
+            t.v = {w.x * sl, w.y * sl, w.z * sl};
             if (r > 0.0f) {
                 const float4 dv = make_float4(vi.x - vj.x, vi.y - vj.y, vi.z - vj.z, 0.0f);
                 const float s = C.cvis * C.kn.dL(r) / r * dot3(dv, w);
-                tx = d.x * s;
-                ty = d.y * s;
-                tz = d.z * s;
+                t.x = {d.x * s, d.y * s, d.z * s};
             }
+            return t;
         },
-        none,
-        [&] {
-            gvx = sub_terms<LANES>(gvx, tvx);
-            gvy = sub_terms<LANES>(gvy, tvy);
-            gvz = sub_terms<LANES>(gvz, tvz);
-            gxx = sub_terms<LANES>(gxx, tx);
-            gxy = sub_terms<LANES>(gxy, ty);
-            gxz = sub_terms<LANES>(gxz, tz);
+        [&](const Terms& t) {
+            sub_terms<LANES>(gvx, gvy, gvz, t.v);
+            sub_terms<LANES>(gxx, gxy, gxz, t.x);
         });
     if (sub != 0) return;
     float wf[3], wg[3];

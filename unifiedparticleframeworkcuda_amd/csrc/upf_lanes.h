@@ -42,31 +42,55 @@ __device__ __forceinline__ float sub_terms2(float acc, float t, float u) {
     else return acc;
 }
 
-// This lane's first entry of the list row (0 past its end).
-__device__ __forceinline__ uint32_t first_entry(const uint32_t* __restrict__ row, int cnt, int sub) {
-    return sub < cnt ? row[sub] : 0u;
+// Entry k of the list row (0 past its end).
+__device__ __forceinline__ uint32_t entry_at(const uint32_t* __restrict__ row, int cnt, int k) {
+    return k < cnt ? row[k] : 0u;
 }
 
-// term(entry) for this lane's entries of the list (none(): it has no entry in
-// this round), then add() for the group's LANES terms; the next round's entry
-// is loaded ahead of this round's gathers.  e: first_entry().
-template <int LANES, class Term, class None, class Add>
-__device__ __forceinline__ void for_pairs(const uint32_t* __restrict__ row, int cnt, int sub, uint32_t e, Term term,
-                                          None none, Add add) {
-    for (int k = 0; k < cnt; k += LANES) {
-        const int next = k + LANES + sub;
-        const uint32_t en = next < cnt ? row[next] : 0u;
-        if (k + sub < cnt) term(e);
-        else none();
-        add();
-        e = en;
+// Walks this lane's entries of the list row: load(entry) for the lane's next
+// two, then for each term(record, whether the lane has that entry) and, per
+// LANES neighbours, add(the lane's term).  An entry past the list's end reads
+// slot 0's records, for a term that changes no sum.  The next entries are
+// loaded ahead of the gathers of this round.  e: entry_at().
+template <int LANES, class Load, class Term, class Add>
+__device__ __forceinline__ void for_pairs(const uint32_t* __restrict__ row, int cnt, int sub, uint32_t e, Load load,
+                                          Term term, Add add) {
+    uint32_t f = entry_at(row, cnt, sub + LANES);
+    for (int k = sub; k - sub < cnt; k += 2 * LANES) {
+        const auto r = load(e);
+        const auto s = load(f);
+        e = entry_at(row, cnt, k + 2 * LANES);
+        f = entry_at(row, cnt, k + 3 * LANES);
+        add(term(r, k < cnt));
+        if (k - sub + LANES < cnt) add(term(s, k + LANES < cnt));
     }
 }
-template <int LANES, class Term, class None, class Add>
-__device__ __forceinline__ void for_pairs(const uint32_t* __restrict__ row, int cnt, int sub, Term term, None none,
+template <int LANES, class Load, class Term, class Add>
+__device__ __forceinline__ void for_pairs(const uint32_t* __restrict__ row, int cnt, int sub, Load load, Term term,
                                           Add add) {
-    for_pairs<LANES>(row, cnt, sub, first_entry(row, cnt, sub), term, none, add);
+    for_pairs<LANES>(row, cnt, sub, entry_at(row, cnt, sub), load, term, add);
 }
+
+// three sums' terms, and their subtraction or addition
+struct Term3 {
+    float x, y, z;
+};
+template <int LANES>
+__device__ __forceinline__ void sub_terms(float& x, float& y, float& z, const Term3& t) {
+    x = sub_terms<LANES>(x, t.x);
+    y = sub_terms<LANES>(y, t.y);
+    z = sub_terms<LANES>(z, t.z);
+}
+template <int LANES>
+__device__ __forceinline__ void add_terms(float& x, float& y, float& z, const Term3& t) {
+    x = add_terms<LANES>(x, t.x);
+    y = add_terms<LANES>(y, t.y);
+    z = add_terms<LANES>(z, t.z);
+}
+// two 16-byte records of a neighbour
+struct Pair4 {
+    float4 a, b;
+};
 
 }  // namespace upf
 

@@ -1340,7 +1340,7 @@ __device__ __forceinline__ void ext_static_lanes(const StepArgs& A, const Slots&
     const upf_params& P = A.P;
     const uint32_t* row = W.nbr + (size_t)i * A.nbr_ld;
     const int cnt = W.ncount[i];
-    const uint32_t e0 = first_entry(row, cnt, sub);
+    const uint32_t e0 = entry_at(row, cnt, sub);
     const float4 xi = S.pos[i];
     const int ti = ptype(xi);
     const float own_psi = S.psi[i], own_rho = S.rho_last[i];
@@ -1364,23 +1364,27 @@ __device__ __forceinline__ void ext_static_lanes(const StepArgs& A, const Slots&
     const float own_p = MODE == UPF_BOUNDARY_CPU_REF ? S.p_prev[i] : S.p_last[i];
     const float inv = 1.0f / own_rho;
     const float pg = own_p * inv * inv;
-    float fx = 0.0f, fy = 0.0f, fz = 0.0f, tx, ty, tz;
-    auto none = [&] { tx = ty = tz = 0.0f; };
+    float fx = 0.0f, fy = 0.0f, fz = 0.0f;
+    struct Rec {
+        float4 x, v;
+        int j;
+    };
     // the terms of ext_static_slot's pair, all subtracted (x + -t is x - t)
     for_pairs<LANES>(
         row, cnt, sub, e0,
         [&](uint32_t e) __attribute__((always_inline)) {
             const int j = (int)(e >> NB_SLOT_SHIFT);
-            const float4 xj = at_u32(S.pos, j), vj = at_u32(S.vel, j);
-            const int tj = ptype(xj);
+            return Rec{at_u32(S.pos, j), at_u32(S.vel, j), j};
+        },
+        [&](const Rec& q, bool have) __attribute__((always_inline)) {
+            const float4 &xj = q.x, &vj = q.v;
+            const int tj = have ? ptype(xj) : UPF_RIGID;  // no term
+            Term3 t = {0.0f, 0.0f, 0.0f};
             const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-            none();
             if (tj == UPF_LIQUID) {
                 const float kv = lvl[bin_of_d2(dx * dx + dy * dy + dz * dz, A.lut_factor, th)];
                 const float vx = vi.x - vj.x, vy = vi.y - vj.y, vz = vi.z - vj.z;
-                tx = vx * rv * rv * visc * kv;
-                ty = vy * rv * rv * visc * kv;
-                tz = vz * rv * rv * visc * kv;
+                t = {vx * rv * rv * visc * kv, vy * rv * rv * visc * kv, vz * rv * rv * visc * kv};
             } else if (tj == UPF_FROZEN) {
                 float g, wv;
                 if (MODE == UPF_BOUNDARY_CPU_REF) {
@@ -1391,19 +1395,15 @@ __device__ __forceinline__ void ext_static_lanes(const StepArgs& A, const Slots&
                     uint32_t dl = (uint32_t)(dist * 300.0f / h);
                     dl = dl > 300u ? 300u : dl;
                     g = lpg[dl];
-                    wv = S.psi[j];
+                    wv = S.psi[q.j];
                 }
-                tx = ((((dx * g) * pg) * P.initial_mass) * P.rest_density) * wv;
-                ty = ((((dy * g) * pg) * P.initial_mass) * P.rest_density) * wv;
-                tz = ((((dz * g) * pg) * P.initial_mass) * P.rest_density) * wv;
+                t = {((((dx * g) * pg) * P.initial_mass) * P.rest_density) * wv,
+                     ((((dy * g) * pg) * P.initial_mass) * P.rest_density) * wv,
+                     ((((dz * g) * pg) * P.initial_mass) * P.rest_density) * wv};
             }
+            return t;
         },
-        none,
-        [&] {
-            fx = sub_terms<LANES>(fx, tx);
-            fy = sub_terms<LANES>(fy, ty);
-            fz = sub_terms<LANES>(fz, tz);
-        });
+        [&](const Term3& t) { sub_terms<LANES>(fx, fy, fz, t); });
     if (sub != 0) return;
     fy = fy - P.initial_mass * P.gravity;
     const Dom d = dom_at(A, i);
@@ -1859,7 +1859,8 @@ __global__ __launch_bounds__(BLOCK) void k_force(int t, StepArgs A, Slots S, Wor
 // packed slot-major lists (k_nbr_build_ext with LANES): k_density's and
 // k_force's expressions.  Few particles leave one chain of list rows and
 // gathers per wave, and the chip mostly idle (9.5 and 9.0 us per launch from
-// 3,080 to 80,648 particles with one lane each); LANES_FIG
+// 3,080 to 80,648 particles with one lane each; now 5.4 and 4.7 at 3,080, 7.8
+// and 7.9 at 80,648).
 template <int MODE, int LANES>
 __global__ __launch_bounds__(BLOCK) void k_density_lanes(int t, StepArgs A, Work W, const float* __restrict__ luts,
                                                          Ctl* ctl) {
@@ -1875,7 +1876,7 @@ __global__ __launch_bounds__(BLOCK) void k_density_lanes(int t, StepArgs A, Work
     const float4 xi = in ? W.xs[i] : make_float4(0.f, 0.f, 0.f, 0.f);
     const uint32_t* row = W.nbr + (size_t)(in ? i : 0) * A.nbr_ld;
     const int cnt = in ? W.ncount[i] : 0;
-    const uint32_t e0 = first_entry(row, cnt, sub);
+    const uint32_t e0 = entry_at(row, cnt, sub);
     for (int k = threadIdx.x; k < LUT_N; k += BLOCK) {
         lw[k] = k < 300 ? luts[k] : 0.0f;  // bin 300 (dist >= h) weighs 0, as in lut_at
         th[k] = reinterpret_cast<const float2*>(luts + LUT_TH_OFF)[k];
@@ -1888,19 +1889,17 @@ __global__ __launch_bounds__(BLOCK) void k_density_lanes(int t, StepArgs A, Work
         float rho = P.kernel_self * m;
         if (P.add_wall_weight)
             rho = rho + wall_weight<false>(P, wall_distance(P, xi.x, xi.y, xi.z), A.lut_factor, lw);
-        float term;
         for_pairs<LANES>(
-            row, cnt, sub, e0,
-            [&](uint32_t e) __attribute__((always_inline)) {
-                const float4 xj = at_u32(W.xs, (int)(e >> NB_SLOT_SHIFT));
+            row, cnt, sub, e0, [&](uint32_t e) { return at_u32(W.xs, (int)(e >> NB_SLOT_SHIFT)); },
+            [&](const float4& xj, bool have) __attribute__((always_inline)) {
                 const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
                 const float d2 = dx * dx + dy * dy + dz * dz;
                 const float w = lw[bin_of_d2(d2, A.lut_factor, th)];
                 // a pair at d2 >= T adds +0, which leaves rho > 0 as it is
                 const float mj = MODE == UPF_BOUNDARY_AKINCI && ptype(xj) != UPF_LIQUID ? -xj.w : m;
-                term = d2 < T ? w * mj : 0.0f;
+                return have && d2 < T ? w * mj : 0.0f;
             },
-            [&] { term = 0.0f; }, [&] { rho = add_terms<LANES>(rho, term); });
+            [&](float t) { rho = add_terms<LANES>(rho, t); });
         if (sub == 0) {
             const float err = fmax_ref(rho - P.rest_density, 0.0f);
             const float p = W.p[i] + fmax_ref(err * P.density_error_factor, 0.0f);
@@ -1934,7 +1933,7 @@ __global__ __launch_bounds__(BLOCK) void k_force_lanes(int t, StepArgs A, Slots 
     const float4 xr = in ? W.xpd[i] : make_float4(0.f, 0.f, 0.f, -0.0f);
     const uint32_t* row = W.nbr + (size_t)(in ? i : 0) * A.nbr_ld;
     const int cnt = in ? W.ncount[i] : 0;
-    const uint32_t e0 = first_entry(row, cnt, sub);
+    const uint32_t e0 = entry_at(row, cnt, sub);
     for (int k = threadIdx.x; k < LUT_N; k += BLOCK) {
         lpg[k] = luts[LUT_N + k];
         th[k] = reinterpret_cast<const float2*>(luts + LUT_TH_OFF)[k];
@@ -1942,11 +1941,10 @@ __global__ __launch_bounds__(BLOCK) void k_force_lanes(int t, StepArgs A, Slots 
     __syncthreads();
     if (__builtin_signbit(xr.w)) return;  // not liquid
     const float m = P.initial_mass;
-    float fx = 0.0f, fy = 0.0f, fz = 0.0f, tx, ty, tz;
+    float fx = 0.0f, fy = 0.0f, fz = 0.0f;
     for_pairs<LANES>(
-        row, cnt, sub, e0,
-        [&](uint32_t e) __attribute__((always_inline)) {
-            const float4 xj = at_u32(W.xpd, (int)(e >> NB_SLOT_SHIFT));
+        row, cnt, sub, e0, [&](uint32_t e) { return at_u32(W.xpd, (int)(e >> NB_SLOT_SHIFT)); },
+        [&](const float4& xj, bool have) __attribute__((always_inline)) {
             const float dx = xr.x - xj.x, dy = xr.y - xj.y, dz = xr.z - xj.z;
             const float g = lpg[bin_of_d2(dx * dx + dy * dy + dz * dz, A.lut_factor, th)];
             float pd = xj.w, mj = m;
@@ -1955,16 +1953,10 @@ __global__ __launch_bounds__(BLOCK) void k_force_lanes(int t, StepArgs A, Slots 
                 pd = 0.0f;
             }
             const float grad = xr.w + pd;
-            tx = (((dx * g) * grad) * m) * mj;
-            ty = (((dy * g) * grad) * m) * mj;
-            tz = (((dz * g) * grad) * m) * mj;
+            return have ? Term3{(((dx * g) * grad) * m) * mj, (((dy * g) * grad) * m) * mj, (((dz * g) * grad) * m) * mj}
+                        : Term3{0.0f, 0.0f, 0.0f};
         },
-        [&] { tx = ty = tz = 0.0f; },
-        [&] {
-            fx = sub_terms<LANES>(fx, tx);
-            fy = sub_terms<LANES>(fy, ty);
-            fz = sub_terms<LANES>(fz, tz);
-        });
+        [&](const Term3& t) { sub_terms<LANES>(fx, fy, fz, t); });
     if (sub != 0) return;
     const float4 Fp = make_float4(fx, fy, fz, 0.0f);
     // written when this iteration may be the scene's last (k_force)
@@ -2118,15 +2110,15 @@ __device__ __forceinline__ void density_wcsph_lanes(const StepArgs& A, const Slo
     const uint32_t* row = W.nbr + (size_t)i * A.nbr_ld;
     const int cnt = W.ncount[i];
     const float4 xi = S.pos[i];
-    float rho = P.kernel_self * P.initial_mass, term;
+    float rho = P.kernel_self * P.initial_mass;
     for_pairs<LANES>(
-        row, cnt, sub,
-        [&](uint32_t e) __attribute__((always_inline)) {
-            const float4 xj = at_u32(S.pos, (int)(e >> NB_SLOT_SHIFT));
+        row, cnt, sub, [&](uint32_t e) { return at_u32(S.pos, (int)(e >> NB_SLOT_SHIFT)); },
+        [&](const float4& xj, bool have) __attribute__((always_inline)) {
             const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-            term = lw[bin_of_d2(dx * dx + dy * dy + dz * dz, A.lut_factor, th)] * P.initial_mass;
+            const float w = lw[bin_of_d2(dx * dx + dy * dy + dz * dz, A.lut_factor, th)];
+            return have ? w * P.initial_mass : -0.0f;
         },
-        [&] { term = -0.0f; }, [&] { rho = add_terms<LANES>(rho, term); });
+        [&](float t) { rho = add_terms<LANES>(rho, t); });
     if (sub == 0) finish_density_wcsph<TAIT>(A, S, W, i, xi, rho, lw);
 }
 
@@ -2236,7 +2228,7 @@ __global__ __launch_bounds__(BLOCK) void k_force_wcsph_lanes(StepArgs A, Slots S
     const float4 xi = in ? S.pos[i] : make_float4(0.f, 0.f, 0.f, 0.f);
     const uint32_t* row = W.nbr + (size_t)(in ? i : 0) * A.nbr_ld;
     const int cnt = in ? W.ncount[i] : 0;
-    const uint32_t e0 = first_entry(row, cnt, sub);
+    const uint32_t e0 = entry_at(row, cnt, sub);
     for (int t = threadIdx.x; t < LUT_N; t += BLOCK) {
         lvl[t] = luts[2 * LUT_N + t];
         lpg[t] = luts[LUT_N + t];
@@ -2249,31 +2241,33 @@ __global__ __launch_bounds__(BLOCK) void k_force_wcsph_lanes(StepArgs A, Slots S
     const float invD = (float)(1.0 / (double)W.rho[i]);
     const float pVol = m * invD;
     const float4 vi = S.vel[i];
-    float fx = 0.0f, fy = 0.0f, fz = 0.0f, gx, gy, gz, ux, uy, uz;
-    auto none = [&] { gx = gy = gz = ux = uy = uz = 0.0f; };
+    float fx = 0.0f, fy = 0.0f, fz = 0.0f;
+    struct Terms {
+        Term3 g, u;
+    };
     for_pairs<LANES>(
         row, cnt, sub, e0,
         [&](uint32_t e) __attribute__((always_inline)) {
             const int j = (int)(e >> NB_SLOT_SHIFT);
-            const float4 xj = at_u32(W.xpd, j), vj = at_u32(W.vpg, j);
-            if (xj.w < 0.0f) return none();  // not a fluid neighbour
+            return Pair4{at_u32(W.xpd, j), at_u32(W.vpg, j)};
+        },
+        [&](const Pair4& q, bool have) __attribute__((always_inline)) {
+            const float4 &xj = q.a, &vj = q.b;
+            // not a fluid neighbour, or none
+            if (!have || xj.w < 0.0f) return Terms{{0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}};
             const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
             const uint32_t bin = bin_of_d2(dx * dx + dy * dy + dz * dz, A.lut_factor, th);
             const float kv = lvl[bin], g = lpg[bin];
             const float grad = p_i * invD * invD + vj.w;
-            gx = (((dx * g) * grad) * m) * m;
-            gy = (((dy * g) * grad) * m) * m;
-            gz = (((dz * g) * grad) * m) * m;
             const float vx = vi.x - vj.x, vy = vi.y - vj.y, vz = vi.z - vj.z;
-            ux = vx * pVol * xj.w * P.visc_const * kv;
-            uy = vy * pVol * xj.w * P.visc_const * kv;
-            uz = vz * pVol * xj.w * P.visc_const * kv;
+            return Terms{{(((dx * g) * grad) * m) * m, (((dy * g) * grad) * m) * m, (((dz * g) * grad) * m) * m},
+                         {vx * pVol * xj.w * P.visc_const * kv, vy * pVol * xj.w * P.visc_const * kv,
+                          vz * pVol * xj.w * P.visc_const * kv}};
         },
-        none,
-        [&] {  // per neighbour the pressure term, then the viscosity term
-            fx = sub_terms2<LANES>(fx, gx, ux);
-            fy = sub_terms2<LANES>(fy, gy, uy);
-            fz = sub_terms2<LANES>(fz, gz, uz);
+        [&](const Terms& t) {  // per neighbour the pressure term, then the viscosity term
+            fx = sub_terms2<LANES>(fx, t.g.x, t.u.x);
+            fy = sub_terms2<LANES>(fy, t.g.y, t.u.y);
+            fz = sub_terms2<LANES>(fz, t.g.z, t.u.z);
         });
     if (sub != 0) return;
     if (P.add_boundary_force) box_force_static(P, dom_at(A, i), xi, fx, fy, fz);
