@@ -66,6 +66,47 @@ def test_sort_forms_are_stable(gpu, n):
     sim.close()
 
 
+# cell tables of one tile, of tiles summed by the scan, of summed blocks, of
+# several tiles per block, and one too sparse for the counting (sorted by key);
+# particles in random order, in key order, and piled into few cells
+@pytest.mark.parametrize("grid,n", [(2, 1), (8, 63), (16, 65), (32, 4097), (64, 70001), (128, 30011), (256, 1600000),
+                                    (256, 1000)])
+@pytest.mark.parametrize("order", ["random", "sorted", "piled"])
+def test_cell_bins_are_a_stable_sort(gpu, grid, n, order):
+    print("cell bins: grid %d, n %d, %s" % (grid, n, order), flush=True)
+    p, _, _, _ = upf.standard_dam_break(8, 8, 8)
+    p.grid_dim, p.block_size = grid, 1024 // grid
+    p.block_shift = p.block_size.bit_length() - 1
+    width = 1.02 * p.support_radius
+    for a in range(3):
+        p.scales[a] = p.block_size / width
+        p.vbox_max[a] = grid * width
+    rng = np.random.RandomState(grid + n)
+    pos = np.zeros((n, 4), np.float32)
+    top = (grid - 1.01) * width
+    pos[:, :3] = rng.uniform(0.0, top, (n, 3)).astype(np.float32)
+    if order == "piled":
+        pos[n // 4:, :3] = top / 2 + rng.randint(0, 3, (n - n // 4, 3)) * (width / 7)
+        pos = pos[:100000]  # ranking costs a cell's count per particle
+        n = len(pos)
+    key = upf.device_keys(p, pos)
+    if order == "sorted":
+        pos = pos[np.argsort(key, kind="stable")]
+        key = np.sort(key)
+    sim = upf.Simulation(p, n)
+    for _ in range(2):  # the counts are left at zero
+        sim.upload(pos, np.full(n, upf.UPF_FROZEN, np.int32))
+        sim.sort_and_bin()
+        k, ids, cells = sim.sorted_state()
+        want = np.argsort(key, kind="stable")
+        assert np.array_equal(ids, want) and np.array_equal(k, key[want])
+        code = k >> np.uint32(3 * p.block_shift)
+        first = np.flatnonzero(np.r_[True, code[1:] != code[:-1]])
+        ref = np.stack([code[first], first, np.r_[first[1:], n]], 1).astype(np.uint32)
+        assert np.array_equal(cells, ref)
+    sim.close()
+
+
 def test_radix_sort_full_32bit_and_edge_keys(gpu):
     keys = np.array([0xFFFFFFFF, 0, 0x80000000, 0xFFFFFFFF, 0, 1, 0x7FFFFFFF] * 1000, np.uint32)
     out, perm = upf.device_radix_sort(keys)

@@ -47,6 +47,7 @@
 #include <vector>
 
 #include "upf.h"
+#include "upf_bins.h"
 #include "upf_device.h"
 #include "upf_internal.h"
 #include "upf_kernels.h"
@@ -164,6 +165,18 @@ __global__ void k_cell_bounds(int n, const uint32_t* __restrict__ keys, const ui
     const uint32_t j = perm[i];
     const float4 p = x[j];
     cand[i] = make_float4(p.x, p.y, p.z, __uint_as_float(j));
+}
+
+// the same positions from the particles' places cell by cell (upf_bins.h)
+__global__ __launch_bounds__(AB) void k_rank_cand(int n, CellMap map, const uint64_t* __restrict__ place,
+                                                  const uint2* __restrict__ cells, const float4* __restrict__ x,
+                                                  float4* __restrict__ cand) {
+    const int t = blockIdx.x * AB + threadIdx.x;
+    if (t >= n) return;
+    const uint64_t v = place[t];
+    const uint32_t j = (uint32_t)v;
+    const float4 p = x[j];
+    cand[bin_slot(place, v, cells[map((uint32_t)(v >> 32), t)])] = make_float4(p.x, p.y, p.z, __uint_as_float(j));
 }
 
 // neighbour ids of every fluid particle: the cells of its query box (the
@@ -290,8 +303,8 @@ __device__ inline float4 predict(const float4& xi, const float4& vi, float fx, f
                        clampc(zz, C.cmin[2], C.cmax[2]), type_and_out(xi.w, zx, zy, zz, C));
 }
 
-// external force, and the first iteration's prediction.  Clears the cell table
-// for the next step: the lists of this one are built.
+// external force, and the first iteration's prediction.  Clears nc cells of the
+// table for the next step: the lists of this one are built.
 template <int LANES>
 __global__ __launch_bounds__(AB) void k_ext(int n, const float4* __restrict__ x, const float4* __restrict__ v,
                                             const uint32_t* __restrict__ nb, const int* __restrict__ cnt, int ld,
@@ -622,7 +635,8 @@ struct upf_adjoint {
     uint2* cells = nullptr;
     float4* cand = nullptr;
     uint32_t ncells = 0;
-    void* sort_tmp = nullptr;
+    Bins bins = {};            // count null: sorted by key instead (bins_apply)
+    void* sort_tmp = nullptr;  // the key sort's arrays: skeys, perm, sort_tmp
     Ctl* ctl = nullptr;
     // forward work; rec: the pair passes' gathered records
     float4 *F = nullptr, *xs = nullptr, *rec = nullptr;
@@ -674,7 +688,8 @@ struct upf_adjoint {
 // both ready for the next
 static void enqueue_begin(upf_adjoint* a, const float4* x) {
     hipLaunchKernelGGL(k_keys, a->grid(), dim3(AB), 0, a->st, a->n, x, a->P, a->keys, a->ctl);
-    hipLaunchKernelGGL(k_clear_cells, dim3((a->ncells + AB - 1) / AB), dim3(AB), 0, a->st, a->cells, a->ncells);
+    if (!a->bins.count)
+        hipLaunchKernelGGL(k_clear_cells, dim3((a->ncells + AB - 1) / AB), dim3(AB), 0, a->st, a->cells, a->ncells);
 }
 
 // one forward step (x, v) -> (xn, vn); with `tape` >= 0 the step's lists and
@@ -688,12 +703,17 @@ static void enqueue_step(upf_adjoint* a, const float4* x, const float4* v, float
     uint32_t* nb = rec ? a->t_nb + (size_t)tape * a->nb_stride() : a->t_nb;
     int* cnt = rec ? a->t_cnt + (size_t)tape * n : a->t_cnt;
     auto xs = [&](int k) { return rec ? a->t_xs + ((size_t)tape * K + k) * n : a->xs; };
-    (void)radix_sort(a->keys, nullptr, a->skeys, a->perm, n, 30, a->sort_tmp, a->st);
-    hipLaunchKernelGGL(k_cell_bounds, a->grid(), b, 0, a->st, n, a->skeys, a->perm, x, 3u * a->P.block_shift, a->cells,
-                       a->cand);
+    const CellMap map{3u * a->P.block_shift, nullptr, nullptr};
+    if (a->bins.count) {
+        (void)cell_bins(a->keys, n, map, a->bins, a->st);
+        hipLaunchKernelGGL(k_rank_cand, a->grid(), b, 0, a->st, n, map, a->bins.place, a->cells, x, a->cand);
+    } else {
+        (void)radix_sort(a->keys, nullptr, a->skeys, a->perm, n, 30, a->sort_tmp, a->st);
+        hipLaunchKernelGGL(k_cell_bounds, a->grid(), b, 0, a->st, n, a->skeys, a->perm, x, map.shift3, a->cells, a->cand);
+    }
     hipLaunchKernelGGL(k_lists, a->grid(LIST_LANES), b, 0, a->st, n, x, a->cand, a->cells, a->P, nb, cnt, a->ctl);
-    hipLaunchKernelGGL(k_ext<LANES>, g, b, 0, a->st, n, x, v, nb, cnt, ld, C, a->F, a->p, xs(0), a->cells, a->ncells,
-                       a->ctl);
+    hipLaunchKernelGGL(k_ext<LANES>, g, b, 0, a->st, n, x, v, nb, cnt, ld, C, a->F, a->p, xs(0), a->cells,
+                       a->bins.count ? 0u : a->ncells, a->ctl);
     for (int k = 0; k < K; ++k) {
         const size_t o = ((size_t)tape * K + k) * n;
         hipLaunchKernelGGL(k_density<LANES>, g, b, 0, a->st, n, x, xs(k), nb, cnt, ld, C, a->p, a->rec,
@@ -774,8 +794,7 @@ int upf_adjoint_create(const upf_params* p, int n, int steps, int iterations, in
     ok = ok && a->alloc(&a->x[0], n) == hipSuccess && a->alloc(&a->v[0], n) == hipSuccess &&
          a->alloc(&a->x[1], n) == hipSuccess && a->alloc(&a->v[1], n) == hipSuccess &&
          a->alloc(&a->cand, n) == hipSuccess &&
-         a->alloc(&a->keys, n) == hipSuccess && a->alloc(&a->skeys, n) == hipSuccess &&
-         a->alloc(&a->perm, n) == hipSuccess && a->alloc(&a->cells, a->ncells) == hipSuccess &&
+         a->alloc(&a->keys, n) == hipSuccess && a->alloc(&a->cells, a->ncells) == hipSuccess &&
          a->alloc(&a->ctl, 1) == hipSuccess && a->alloc(&a->F, n) == hipSuccess && a->alloc(&a->rec, n) == hipSuccess &&
          a->alloc(&a->xs, n) == hipSuccess && a->alloc(&a->p, n) == hipSuccess &&
          a->alloc(&a->ck_x, (size_t)a->nseg * n) == hipSuccess && a->alloc(&a->ck_v, (size_t)a->nseg * n) == hipSuccess &&
@@ -786,9 +805,16 @@ int upf_adjoint_create(const upf_params* p, int n, int steps, int iterations, in
          a->alloc(&a->gx, n) == hipSuccess && a->alloc(&a->gv, n) == hipSuccess && a->alloc(&a->nx, n) == hipSuccess &&
          a->alloc(&a->nv, n) == hipSuccess && a->alloc(&a->gF, n) == hipSuccess && a->alloc(&a->gFp, n) == hipSuccess &&
          a->alloc(&a->gFp2, n) == hipSuccess && a->alloc(&a->gp, n) == hipSuccess;
-    if (ok) {
+    if (ok && bins_apply(n, a->ncells)) {
+        a->bins.cells = a->cells;
+        a->bins.ncells = a->ncells;
+        ok = a->alloc(&a->bins.at, n) == hipSuccess && a->alloc(&a->bins.place, n) == hipSuccess &&
+             a->alloc(&a->bins.sums, BIN_BLOCKS) == hipSuccess && a->alloc(&a->bins.count, a->ncells) == hipSuccess &&
+             hipMemset(a->bins.count, 0, (size_t)a->ncells * sizeof(uint32_t)) == hipSuccess;
+    } else if (ok) {
         void* tmp = nullptr;
-        ok = hipMalloc(&tmp, radix_sort_temp_bytes(n)) == hipSuccess;
+        ok = a->alloc(&a->skeys, n) == hipSuccess && a->alloc(&a->perm, n) == hipSuccess &&
+             hipMalloc(&tmp, radix_sort_temp_bytes(n)) == hipSuccess;
         if (ok) { a->sort_tmp = tmp; a->allocs.push_back(tmp); }
     }
     if (!ok) {
@@ -903,8 +929,10 @@ int upf_adjoint_timing(upf_adjoint* a, float* forward_ms, float* backward_ms, si
     if (backward_ms) *backward_ms = a->bwd_ms;
     if (device_bytes) {
         const size_t n = (size_t)a->n, T = (size_t)a->ckpt, K = (size_t)a->K;
-        *device_bytes = n * 16 * (4 + 1 + 3 + 2 * a->nseg + 2 * T + T * K + 7) + n * 4 * (5 + 2 * T + 2 * T * K) +
-                        T * a->nb_stride() * 4 + (size_t)a->ncells * 8 + radix_sort_temp_bytes(a->n);
+        *device_bytes = n * 16 * (4 + 1 + 3 + 2 * a->nseg + 2 * T + T * K + 7) + n * 4 * (3 + 2 * T + 2 * T * K) +
+                        T * a->nb_stride() * 4 + (size_t)a->ncells * 8;
+        *device_bytes += a->bins.count ? n * 12 + (size_t)a->ncells * 4 + BIN_BLOCKS * 4
+                                       : n * 8 + radix_sort_temp_bytes(a->n);
     }
     return UPF_OK;
 }

@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "upf.h"
+#include "upf_bins.h"
 #include "upf_device.h"
 #include "upf_internal.h"
 #include "upf_kernels.h"
@@ -168,23 +169,65 @@ __global__ void k_keys(StepArgs A, const float4* __restrict__ pos, uint32_t* __r
 // CopySortedParticleValuesKernel* (src/gpu/particles_kernel.cu:544-654):
 // the persistent particle state follows the sort permutation.  Pressures of
 // the finished loop move one generation back (p_last -> p_prev).
-__global__ void k_gather(int n, const uint32_t* __restrict__ perm, Slots src, Slots dst, const float* __restrict__ p_work,
-                         const float* __restrict__ rho_work, int rigid) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const int o = (int)perm[s];
-    dst.pos[s] = src.pos[o];
-    dst.vel[s] = src.vel[o];
-    dst.id[s] = src.id[o];
-    dst.p_prev[s] = src.p_last[o];
-    dst.p_last[s] = p_work[o];
-    dst.rho_last[s] = rho_work[o];
-    dst.psi[s] = src.psi[o];
-    if (rigid) {
-        dst.x0[s] = src.x0[o];
-        dst.body[s] = src.body[o];
-        dst.rel[s] = src.rel[o];
+// Slot o of src as slot at() of dst; at() runs while the state is on its way.
+// (Values of the vector extension: as float4 the compiler keeps them in LDS,
+// with a read of the dispatch packet in host memory per wave for it.)
+template <bool RIGID, class At>
+__device__ __forceinline__ int move_slot(const Slots& src, const Slots& dst, int o, const float* __restrict__ p_work,
+                                         const float* __restrict__ rho_work, At at) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    auto vec = [](float4* p) { return reinterpret_cast<f4*>(p); };
+    const f4 pos = vec(src.pos)[o], vel = vec(src.vel)[o];
+    const int id = src.id[o];
+    const float p_prev = src.p_last[o], p_last = p_work[o], rho = rho_work[o], psi = src.psi[o];
+    f4 x0, rel;
+    int body;
+    if constexpr (RIGID) {
+        x0 = vec(src.x0)[o];
+        rel = vec(src.rel)[o];
+        body = src.body[o];
     }
+    const int s = at();
+    vec(dst.pos)[s] = pos;
+    vec(dst.vel)[s] = vel;
+    dst.id[s] = id;
+    dst.p_prev[s] = p_prev;
+    dst.p_last[s] = p_last;
+    dst.rho_last[s] = rho;
+    dst.psi[s] = psi;
+    if constexpr (RIGID) {
+        vec(dst.x0)[s] = x0;
+        vec(dst.rel)[s] = rel;
+        dst.body[s] = body;
+    }
+    return s;
+}
+
+template <bool RIGID>
+__global__ __launch_bounds__(BLOCK) void k_gather(int n, const uint32_t* __restrict__ perm, Slots src, Slots dst,
+                                                  const float* __restrict__ p_work,
+                                                  const float* __restrict__ rho_work) {
+    const int s = blockIdx.x * BLOCK + threadIdx.x;
+    if (s >= n) return;
+    move_slot<RIGID>(src, dst, (int)perm[s], p_work, rho_work, [&] { return s; });
+}
+
+// The same from the particles' places cell by cell (upf_bins.h): the slot is
+// the rank within the cell, counted while the state is on its way.
+template <bool RIGID>
+__global__ __launch_bounds__(BLOCK) void k_rank_gather(int n, CellMap map, const uint64_t* __restrict__ place,
+                                                       const uint2* __restrict__ cells, Slots src, Slots dst,
+                                                       const float* __restrict__ p_work,
+                                                       const float* __restrict__ rho_work,
+                                                       uint32_t* __restrict__ keys_sorted) {
+    const int t = blockIdx.x * BLOCK + threadIdx.x;
+    if (t >= n) return;
+    const uint64_t v = place[t];
+    const uint32_t key = (uint32_t)(v >> 32);
+    const uint2 r = cells[map(key, t)];
+    const int s = move_slot<RIGID>(src, dst, (int)(uint32_t)v, p_work, rho_work,
+                                   [&] { return (int)bin_slot(place, v, r); });
+    keys_sorted[s] = key;
 }
 
 // ------------------------------------------------------------ cell table
@@ -3038,6 +3081,7 @@ struct upf_sim {
     float* luts = nullptr;  // 5 * 301
     void* sort_tmp = nullptr;
     uint32_t ncells = 0;
+    Bins bins = {};  // count null: the cell table is too sparse for it (bins_apply)
     std::vector<int> k_hist;
     uint32_t* d_key0 = nullptr;  // z-index of every particle's uploaded position, by upload id
     Stage stage;
@@ -3159,6 +3203,20 @@ static int sort_and_bin(upf_sim* s) {
     const int n = s->n;
     Work& W = s->W;
     s->prof.begin(PC_SORT, s->st);
+    const int nxt = 1 - s->cur;
+    if (s->bins.count) {
+        const CellMap map{3u * s->P.block_shift, s->n_scenes > 1 ? s->d_doms : nullptr,
+                          s->n_scenes > 1 ? s->d_scene_of : nullptr};
+        HIPCHK(cell_bins(W.keys, n, map, s->bins, s->st));
+        s->prof.end(s->st);
+        s->prof.begin(PC_GATHER, s->st);
+        hipLaunchKernelGGL(s->rigid ? k_rank_gather<true> : k_rank_gather<false>, grid_for(n), dim3(BLOCK), 0, s->st, n,
+                           map, s->bins.place, W.cells, s->S[s->cur], s->S[nxt], W.p, W.rho, W.keys_sorted);
+        s->prof.end(s->st);
+        s->cur = nxt;
+        HIPCHK(hipGetLastError());
+        return UPF_OK;
+    }
     if (s->n_scenes == 1) {
         HIPCHK(radix_sort(W.keys, nullptr, W.keys_sorted, W.perm, n, 30, s->sort_tmp, s->st));
     } else {
@@ -3171,10 +3229,9 @@ static int sort_and_bin(upf_sim* s) {
         hipLaunchKernelGGL(k_gather_keys, grid_for(n), dim3(BLOCK), 0, s->st, n, W.perm, W.keys, W.keys_sorted);
     }
     s->prof.end(s->st);
-    const int nxt = 1 - s->cur;
     s->prof.begin(PC_GATHER, s->st);
-    hipLaunchKernelGGL(k_gather, grid_for(n), dim3(BLOCK), 0, s->st, n, W.perm, s->S[s->cur], s->S[nxt], W.p, W.rho,
-                       s->rigid ? 1 : 0);
+    hipLaunchKernelGGL(s->rigid ? k_gather<true> : k_gather<false>, grid_for(n), dim3(BLOCK), 0, s->st, n, W.perm,
+                       s->S[s->cur], s->S[nxt], W.p, W.rho);
     s->prof.end(s->st);
     s->cur = nxt;
     s->prof.begin(PC_CELLS, s->st);
@@ -3710,6 +3767,15 @@ static int sim_alloc(upf_sim* s, int capacity, uint32_t ncells, int n_scenes) {
     HIPCHK(s->alloc(&W.uslots, nchunks * UNION_CAP));
     HIPCHK(s->alloc(&W.un, nchunks));
     HIPCHK(s->alloc(&W.cells, ncells));
+    if (bins_apply(capacity, ncells)) {
+        s->bins.cells = W.cells;
+        s->bins.ncells = ncells;
+        HIPCHK(s->alloc(&s->bins.at, capacity));
+        HIPCHK(s->alloc(&s->bins.place, capacity));
+        HIPCHK(s->alloc(&s->bins.sums, BIN_BLOCKS));
+        HIPCHK(s->alloc(&s->bins.count, ncells));
+        HIPCHK(hipMemset(s->bins.count, 0, (size_t)ncells * sizeof(uint32_t)));
+    }
     HIPCHK(s->alloc(&s->luts, LUT_TOTAL));
     HIPCHK(s->alloc(&s->ctl, 1));
     HIPCHK(s->alloc(&s->sctl, n_scenes));
