@@ -119,7 +119,14 @@ struct StepArgs {
 };
 
 __device__ inline int scene_at(const StepArgs& A, int i) { return A.scene_of ? A.scene_of[i] : 0; }
-__device__ inline Dom dom_at(const StepArgs& A, int i) { return A.scene_of ? A.doms[A.scene_of[i]] : A.dom0; }
+// Scene sc's domain, by value in both cases: a choice between two addresses
+// would put a copy of dom0 in scratch memory and load each field through it.
+__device__ __forceinline__ Dom scene_dom(const StepArgs& A, int sc) {
+    Dom d = A.dom0;
+    if (A.scene_of) d = A.doms[sc];
+    return d;
+}
+__device__ __forceinline__ Dom dom_at(const StepArgs& A, int i) { return scene_dom(A, A.scene_of ? A.scene_of[i] : 0); }
 __device__ inline int gstride() { return gridDim.x * blockDim.x; }
 
 // Batched form, iteration t: true when the block's slots [i0, i0 + blockDim.x)
@@ -492,11 +499,11 @@ struct ListDecoder {
     size_t st;
     uint32_t j;
     int esc = 0;
-    __device__ ListDecoder(const Work& W, int i, size_t stride)
-        : rows(W.nbw + i), e(W.nbe + i), st(stride), j(W.nbf[i]) {}
+    __device__ ListDecoder(const Work& W, int i, size_t stride, uint32_t first)
+        : rows(W.nbw + i), e(W.nbe + i), st(stride), j(first) {}
     // the 16-byte word of entries k0 .. k0 + 7 (k0 a multiple of 8)
-    __device__ void load(int k0, uint64_t& lo, uint64_t& hi) const {
-        const uint4 r = rows[(size_t)(k0 >> 3) * st];
+    __device__ uint4 load(int k0) const { return rows[(size_t)(k0 >> 3) * st]; }
+    __device__ static void words(const uint4& r, uint64_t& lo, uint64_t& hi) {
         lo = (uint64_t)r.x | ((uint64_t)r.y << 32);
         hi = (uint64_t)r.z | ((uint64_t)r.w << 32);
     }
@@ -513,10 +520,6 @@ struct ListDecoder {
     }
 };
 
-// Visits the list of slot i in order: load(j) for G neighbours is issued
-// together, then use(j, entry, value) runs for them in list order.  CODED:
-// the delta-coded lists (entry = 0; eight entries per list load), else the
-// packed 32-bit lists (entry = (slot << 9) | bin).
 // base[j] addressed with a 32-bit byte offset (slots < 2^23, records <= 16
 // bytes), which lets the load take its base from scalar registers
 template <class T>
@@ -524,9 +527,29 @@ __device__ __forceinline__ T at_u32(const T* __restrict__ base, int j) {
     return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + (uint32_t)j * (uint32_t)sizeof(T));
 }
 
+// What a pass needs of slot i's list before its first gathers: loaded at the
+// start of a pass, beside the tables and the slot's record, so that a wave
+// waits for memory once there and not three times in a row (predicted density of
+// 1,132,556 particles 41.5 -> 40.5 us, WCSPH forces 113 -> 111.5).
+struct ListHead {
+    int cnt;
+    uint32_t first;  // CODED == 1: the first slot and the first row
+    uint4 row;
+};
+template <int CODED>
+__device__ __forceinline__ ListHead list_head(const Work& W, int i) {
+    if constexpr (CODED == 1) return ListHead{W.ncount[i], W.nbf[i], W.nbw[i]};
+    else return ListHead{W.ncount[i], 0u, make_uint4(0u, 0u, 0u, 0u)};
+}
+
+// Visits the list of slot i in order: load(j) for G neighbours is issued
+// together, then use(j, entry, value) runs for them in list order.  CODED:
+// the delta-coded lists (entry = 0; eight entries per list load), else the
+// packed 32-bit lists (entry = (slot << 9) | bin).
 template <int CODED, int G, class Load, class Use>
-__device__ __forceinline__ void for_each_listed(const Work& W, int i, size_t st, int cnt, Load load, Use use) {
+__device__ __forceinline__ void for_each_listed(const Work& W, int i, size_t st, const ListHead& head, Load load, Use use) {
     using V = decltype(load(0));
+    const int cnt = head.cnt;
     if (CODED == 2) {
         // union indices: eight 16-bit entries per row, each the neighbour's
         // place in the chunk's union (load(u) reads it from LDS)
@@ -556,14 +579,14 @@ __device__ __forceinline__ void for_each_listed(const Work& W, int i, size_t st,
             }
         }
     } else if (CODED) {
-        ListDecoder dec(W, i, st);
+        ListDecoder dec(W, i, st, head.first);
         int k0 = 0;
         // full rows: the next row's load is issued before this row's gathers
-        uint64_t lo = 0, hi = 0;
-        if (cnt > 0) dec.load(0, lo, hi);
+        uint64_t lo, hi;
+        ListDecoder::words(head.row, lo, hi);
         for (; k0 + 8 <= cnt; k0 += 8) {
             uint64_t nlo = 0, nhi = 0;
-            if (k0 + 8 < cnt) dec.load(k0 + 8, nlo, nhi);
+            if (k0 + 8 < cnt) ListDecoder::words(dec.load(k0 + 8), nlo, nhi);
             int j[8];
 #pragma unroll
             for (int u = 0; u < 8; ++u) j[u] = dec.next(k0, u, lo, hi);
@@ -734,6 +757,18 @@ __global__ __launch_bounds__(UNION_CHUNK) void k_union(StepArgs A, Work W) {
     if (tid == 0) W.un[c] = U;
 }
 
+// Inclusive sum over the wave's lanes, through DPP: shifts within the rows of 16,
+// then row ends broadcast to the rows after them.
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);  // row_shr:1, 2, 4, 8
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);  // row_bcast:15 to rows 1 and 3
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast:31 to rows 2 and 3
+    return v;
+}
+
 // GetNeighbors (src/cpu/UnifiedPhysics.cpp:2242-2295) for every slot of type
 // OWNER (liquid; rigid for the coupling step's rigid lists), one wave per 64
 // consecutive slots.  For each cell met in its slots the wave lists the
@@ -796,7 +831,7 @@ __device__ __forceinline__ void build_wave(const StepArgs& A, const float4* __re
     uint32_t my_blo = 0u, my_bhi = 0u;
     if (my_owner) {
         // BoxQuery of the particle in cell coordinates, clipped to the grid
-        const Dom dm = A.scene_of ? A.doms[my_scene] : A.dom0;
+        const Dom dm = scene_dom(A, my_scene);
         const float xv[3] = {my_x.x, my_x.y, my_x.z};
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
@@ -817,23 +852,31 @@ __device__ __forceinline__ void build_wave(const StepArgs& A, const float4* __re
     uint32_t my_seg = my_key;
     if constexpr (OWNER == UPF_RIGID) {
         if (my_owner) {
-            const Dom dm = A.scene_of ? A.doms[my_scene] : A.dom0;
+            const Dom dm = scene_dom(A, my_scene);
             bool ok;
             my_seg = dkey(my_x.x, my_x.y, my_x.z, dm.scales, ok);
         }
     }
     const uint64_t owners = wballot(my_owner);
     int my_cnt = 0;  // this lane's slot: list length so far
+    // the cells' grid, in scalar registers (of the scene met last, in a batch)
+    uint32_t block_shift = A.dom0.block_shift, G = A.dom0.grid_dim, cell_off = 0;
+    int grid_of = A.scene_of ? -1 : 0;
     int s = base;
     while (s < wend) {
         const int sl = s - base;
         // the cell's values are the same on every lane: read from lane sl into
         // scalar registers, so that the cell's set-up runs on the scalar unit
         const int sc = __builtin_amdgcn_readlane(my_scene, sl);
-        const Dom d = A.scene_of ? A.doms[sc] : A.dom0;  // the cell's scene
-        const uint32_t shift3 = 3u * d.block_shift;
-        const uint32_t G = d.grid_dim;
-        const uint2* T3 = cells + d.cell_off;
+        if (sc != grid_of) {
+            const Dom& d = A.doms[sc];
+            block_shift = (uint32_t)__builtin_amdgcn_readfirstlane((int)d.block_shift);
+            G = (uint32_t)__builtin_amdgcn_readfirstlane((int)d.grid_dim);
+            cell_off = (uint32_t)__builtin_amdgcn_readfirstlane((int)d.cell_off);
+            grid_of = sc;
+        }
+        const uint32_t shift3 = 3u * block_shift;
+        const uint2* T3 = cells + cell_off;
         const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)my_seg, sl) >> shift3;
         // end of the cell within the wave: first later slot of another cell or scene
         const uint64_t other = wballot(mine_valid && me > s && ((my_seg >> shift3) != c || my_scene != sc));
@@ -877,11 +920,7 @@ __device__ __forceinline__ void build_wave(const StepArgs& A, const float4* __re
         const int nr = __popcll(vm);
         const int rank = __popcll(vm & lt);
         // prefix of the occupied cells' lengths in rank (= lane) order
-        uint32_t incl = valid ? rl : 0u;
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t y = (uint32_t)__shfl_up((int)incl, o, 64);
-            if (lane >= o) incl += y;
-        }
+        const uint32_t incl = wave_scan(valid ? rl : 0u);
         if (valid) { r_start[rank] = rs; r_cell[rank] = rcell; r_pref[rank + 1] = incl; }
         if (lane == 0) r_pref[0] = 0;
         __syncthreads();
@@ -1592,13 +1631,13 @@ __global__ __launch_bounds__(BLOCK) void k_density(int t, StepArgs A, Slots S, W
     const int sps = A.slots_per_scene;
     // the predicted density of slot i (this iteration's pressure, the
     // force pass's record), or 0 with sc = -1 when the slot has none
-    auto density_of = [&](int i, int un, float& mine, int& sc) __attribute__((always_inline)) {
+    auto density_of = [&](int i, int un, const float4& xi, const ListHead& head, float& mine, int& sc)
+                          __attribute__((always_inline)) {
         mine = 0.0f;
         sc = scene_at(A, i);
-        // batched: a converged scene's slot stops before its record is
-        // read (one scene runs iteration t: the kernel's entry test decided it)
+        // batched: a converged scene's slot has no density (one scene runs
+        // iteration t: the kernel's entry test decided it)
         const bool runs = !A.scene_of || t < A.sctl[sc].want;
-        const float4 xi = runs ? W.xs[i] : make_float4(0.f, 0.f, 0.f, 0.f);
         if (!(runs && ptype(xi) == UPF_LIQUID)) {
             sc = -1;
             return;
@@ -1608,7 +1647,6 @@ __global__ __launch_bounds__(BLOCK) void k_density(int t, StepArgs A, Slots S, W
         float rho = P.kernel_self * m;
         if (P.add_wall_weight)  // the GPU path's order: walls before neighbours
             rho = rho + wall_weight<false>(P, wall_distance(P, xi.x, xi.y, xi.z), A.lut_factor, lw);
-        const int cnt = W.ncount[i];
         const size_t st = (size_t)A.stride;
         // G neighbours per round: their loads are issued together,
         // the sum still runs in list order
@@ -1632,10 +1670,10 @@ __global__ __launch_bounds__(BLOCK) void k_density(int t, StepArgs A, Slots S, W
         };
         auto from_global = [&](int j) { return at_u32(W.xs, j); };
         if constexpr (CODED == 2) {
-            if (un >= 0) for_each_listed<2, G>(W, i, st, cnt, [&](int u) { return urec[u]; }, use);
-            else for_each_listed<1, G>(W, i, st, cnt, from_global, use);
+            if (un >= 0) for_each_listed<2, G>(W, i, st, head, [&](int u) { return urec[u]; }, use);
+            else for_each_listed<1, G>(W, i, st, list_head<1>(W, i), from_global, use);
         } else {
-            for_each_listed<CODED, G>(W, i, st, cnt, from_global, use);
+            for_each_listed<CODED, G>(W, i, st, head, from_global, use);
         }
         const float err = fmax_ref(rho - P.rest_density, 0.0f);
         const float delta = A.scene_of ? A.doms[sc].delta : P.density_error_factor;
@@ -1649,6 +1687,13 @@ __global__ __launch_bounds__(BLOCK) void k_density(int t, StepArgs A, Slots S, W
         W.rho[i] = rho;
         mine = rho;
     };
+    auto load_tables = [&] {
+        for (int k = threadIdx.x; k < LUT_N; k += blockDim.x) {
+            lw[k] = k < 300 ? luts[k] : 0.0f;  // bin 300 (dist >= h) weighs 0, as in lut_at
+            th[k] = reinterpret_cast<const float2*>(luts + LUT_TH_OFF)[k];
+        }
+        __syncthreads();
+    };
     if constexpr (CODED != 2) {
         if (A.act) {
             // batched: one wave per chunk of this iteration's list
@@ -1660,18 +1705,28 @@ __global__ __launch_bounds__(BLOCK) void k_density(int t, StepArgs A, Slots S, W
             const int wpb = blockDim.x >> 6;
             const int w0 = (int)blockIdx.x * wpb;
             if (w0 >= cnt) return;  // nothing for this block: no tables
-            for (int k = threadIdx.x; k < LUT_N; k += blockDim.x) {
-                lw[k] = k < 300 ? luts[k] : 0.0f;  // bin 300 (dist >= h) weighs 0, as in lut_at
-                th[k] = reinterpret_cast<const float2*>(luts + LUT_TH_OFF)[k];
-            }
-            __syncthreads();
             const int* list = A.act + (size_t)(t & 1) * A.n_chunks;
-            for (int q = w0 + (int)(threadIdx.x >> 6); q < cnt; q += (int)gridDim.x * wpb) {
+            // entry q's slot of this lane (-1: none), its record and list
+            int i = -1;
+            float4 xi = make_float4(0.f, 0.f, 0.f, 0.f);
+            ListHead head = {};
+            auto begin = [&](int q) __attribute__((always_inline)) {
                 const int c = all ? q : list[q];
-                const int i = A.chunk_begin[c] + lane;
+                i = A.chunk_begin[c] + lane;
+                if (i < A.chunk_end[c]) {
+                    xi = W.xs[i];
+                    head = list_head<CODED>(W, i);
+                } else {
+                    i = -1;
+                }
+            };
+            int q = w0 + (int)(threadIdx.x >> 6);
+            if (q < cnt) begin(q);
+            load_tables();
+            for (; q < cnt; q += (int)gridDim.x * wpb, q < cnt ? begin(q) : void()) {
                 float mine = 0.0f;
                 int sc = -1;
-                if (i < A.chunk_end[c]) density_of(i, -1, mine, sc);
+                if (i >= 0) density_of(i, -1, xi, head, mine, sc);
                 // a chunk holds one scene: one maximum per wave
                 const uint64_t act = wballot(sc >= 0);
                 if (act == 0ull) continue;
@@ -1682,23 +1737,25 @@ __global__ __launch_bounds__(BLOCK) void k_density(int t, StepArgs A, Slots S, W
             return;
         }
     }
-    for (int k = threadIdx.x; k < LUT_N; k += blockDim.x) {
-        lw[k] = k < 300 ? luts[k] : 0.0f;  // bin 300 (dist >= h) weighs 0, as in lut_at
-        th[k] = reinterpret_cast<const float2*>(luts + LUT_TH_OFF)[k];
-    }
-    __syncthreads();
     float run = 0.0f;  // single scene: running max over the thread's slots
     // top down (the list build and the force pass walk upwards), so that the
     // previous kernel's last slots come first, while they are in L2
     const int n_round = (A.n + gstride() - 1) / gstride();
     for (int r = n_round - 1; r >= 0; --r) {
         const int i = r * gstride() + xblk_down(A.xcd) * blockDim.x + threadIdx.x;
+        float4 xi = make_float4(0.f, 0.f, 0.f, 0.f);
+        ListHead head = {};
+        if (i < A.n) {
+            xi = W.xs[i];
+            head = list_head<CODED>(W, i);
+        }
+        if (r == n_round - 1) load_tables();
         if (block_idle(A, i - (int)threadIdx.x, t)) continue;
         int un = -1;
         if constexpr (CODED == 2) un = stage_union(A, W, W.xs, urec, (i - (int)threadIdx.x) / UNION_CHUNK);
         float mine = 0.0f;
         int sc = -1;
-        if (i < A.n) density_of(i, un, mine, sc);
+        if (i < A.n) density_of(i, un, xi, head, mine, sc);
         if (A.scene_of == nullptr) {
             run = fmaxf(run, mine);
             continue;
@@ -1832,15 +1889,17 @@ __global__ __launch_bounds__(BLOCK) void k_force(int t, StepArgs A, Slots S, Wor
         if (A.scene_of && t >= A.sctl[A.scene_of[i]].want) return;
         // the slot's own record: current position and p / rho0^2 -- the density
         // pass's p / (rho0 rho0), the same division as W.p[i] / dens_sq -- with
-        // the sign bit set for a non-liquid particle
+        // the sign bit set for a non-liquid particle.  (Loaded before the tables
+        // with the list's head, as the density pass does, it costs registers and
+        // 0.6 us a pass.)
         const float4 xr = W.xpd[i];
         if (__builtin_signbit(xr.w)) return;
         const float4 xi = make_float4(xr.x, xr.y, xr.z, __int_as_float(UPF_LIQUID));
         const float m = P.initial_mass;
         const float pi_d = xr.w;
         float fx = 0.0f, fy = 0.0f, fz = 0.0f;
-        const int cnt = W.ncount[i];
         const size_t st = (size_t)A.stride;
+        const ListHead head = list_head<CODED>(W, i);
         // every listed pair is closer than h at these (current) positions, so the
         // reference's `dist < h` test holds; the table bin is the one the list
         // build computed from the same positions (carried by the packed entry,
@@ -1868,11 +1927,11 @@ __global__ __launch_bounds__(BLOCK) void k_force(int t, StepArgs A, Slots S, Wor
         auto from_global = [&](int j) { return at_u32(W.xpd, j); };
         if constexpr (CODED == 2) {
             if (un >= 0)
-                for_each_listed<2, G>(W, i, st, cnt, [&](int u) { return urec[u]; }, use);
+                for_each_listed<2, G>(W, i, st, head, [&](int u) { return urec[u]; }, use);
             else
-                for_each_listed<1, G>(W, i, st, cnt, from_global, use);
+                for_each_listed<1, G>(W, i, st, list_head<1>(W, i), from_global, use);
         } else {
-            for_each_listed<CODED, G>(W, i, st, cnt, from_global, use);
+            for_each_listed<CODED, G>(W, i, st, head, from_global, use);
         }
         const float4 Fp = make_float4(fx, fy, fz, 0.0f);
         // only the last iteration's pressure force is read (by the integration):
@@ -2239,27 +2298,33 @@ __global__ __launch_bounds__(BLOCK) void k_force_wcsph(StepArgs A, Slots S, Work
                                                        Ctl* ctl) {
     __shared__ float lvl[LUT_N], lpg[LUT_N];
     __shared__ float2 th[CODED ? LUT_N : 1];
+    const upf_params& P = A.P;
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool in = i < A.n;
+    float4 xi = make_float4(0.f, 0.f, 0.f, 0.f), vi = xi;
+    float rho_i = 1.0f, p_i = 0.0f;
+    ListHead head = {};
+    if (in) {
+        xi = S.pos[i];
+        vi = S.vel[i];
+        rho_i = W.rho[i];
+        p_i = W.pres[i];
+        head = list_head<CODED>(W, i);
+    }
     for (int t = threadIdx.x; t < LUT_N; t += blockDim.x) {
         lvl[t] = luts[2 * LUT_N + t];
         lpg[t] = luts[LUT_N + t];
         if constexpr (CODED != 0) th[t] = reinterpret_cast<const float2*>(luts + LUT_TH_OFF)[t];
     }
     __syncthreads();
-    const upf_params& P = A.P;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= A.n) return;
-    const float4 xi = S.pos[i];
-    if (ptype(xi) != UPF_LIQUID) return;
+    if (!in || ptype(xi) != UPF_LIQUID) return;
     const float m = P.initial_mass;
-    const float rho_i = W.rho[i], p_i = W.pres[i];
     const float invD = (float)(1.0 / (double)rho_i);
     const float pVol = m * invD;
-    const float4 vi = S.vel[i];
     float fx = 0.0f, fy = 0.0f, fz = 0.0f;
-    const int cnt = W.ncount[i];
     // two 16-byte records per neighbour, four neighbours' loads in flight
     for_each_listed<CODED, 4>(
-        W, i, (size_t)A.stride, cnt, [&](int j) { return PosVel{at_u32(W.xpd, j), at_u32(W.vpg, j)}; },
+        W, i, (size_t)A.stride, head, [&](int j) { return PosVel{at_u32(W.xpd, j), at_u32(W.vpg, j)}; },
         [&](int, uint32_t e, const PosVel& q) __attribute__((always_inline)) {
             const float4& xj = q.x;
             if (xj.w < 0.0f) return;  // not a fluid neighbour
