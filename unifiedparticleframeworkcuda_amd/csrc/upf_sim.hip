@@ -859,7 +859,11 @@ __device__ __forceinline__ void build_wave(const StepArgs& A, const float4* __re
     }
     const uint64_t owners = wballot(my_owner);
     int my_cnt = 0;  // this lane's slot: list length so far
-    // the cells' grid, in scalar registers (of the scene met last, in a batch)
+    // the cells' grid, in scalar registers (of the scene met last, in a batch):
+    // so the stencil of a cell is set up on the scalar unit.  Through a choice of
+    // addresses it took vector instructions and three dependent loads from
+    // scratch per cell (WCSPH build of 1,132,556 particles 350 -> 335 us, PCISPH
+    // 326 -> 319, rigid lists 160 -> 148).
     uint32_t block_shift = A.dom0.block_shift, G = A.dom0.grid_dim, cell_off = 0;
     int grid_of = A.scene_of ? -1 : 0;
     int s = base;
