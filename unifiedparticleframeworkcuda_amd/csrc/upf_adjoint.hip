@@ -181,18 +181,15 @@ __global__ __launch_bounds__(AB) void k_rank_cand(int n, CellMap map, const uint
 
 // neighbour ids of every fluid particle: the cells of its query box (the
 // reference's BoxQuery) in Morton order, candidates in sorted order, r < h.
-// Sixteen lanes per particle: each finds cells of its own, their slots go to a
-// candidate table in LDS, and the lanes test sixteen candidates at a time, the
-// passing ones appended in order through the group's ballot.  Bound by the
-// latency of table and candidate reads (267 us at 80,648 particles with one
-// lane walking the cells of each).  LIST_CAND slots hold any query box of a
-// fluid; a denser one is walked cell by cell.
-constexpr int LIST_LANES = 16;
-constexpr int LIST_CAND = 384;
+// Sixteen lanes per particle test sixteen candidates at a time, the passing ones
+// appended in order through the group's ballot.  Bound by the latency of table
+// and candidate reads (267 us at 80,648 particles with one lane walking the cells
+// of each, now 37).
+constexpr int LIST_LANES = BOX_LANES;
 __global__ __launch_bounds__(AB) void k_lists(int n, const float4* __restrict__ x, const float4* __restrict__ cand,
                                               const uint2* __restrict__ cells, upf_params P,
                                               uint32_t* __restrict__ nb, int* __restrict__ cnt, Ctl* ctl) {
-    __shared__ uint32_t table[AB / LIST_LANES][LIST_CAND];
+    __shared__ uint32_t table[AB / LIST_LANES][BOX_CAND];
     const int i = (int)((blockIdx.x * AB + threadIdx.x) / LIST_LANES);
     const int sub = threadIdx.x % LIST_LANES;
     if (i >= n) return;
@@ -204,11 +201,10 @@ __global__ __launch_bounds__(AB) void k_lists(int n, const float4* __restrict__ 
     const float h = P.support_radius, hh = h * h;
     const int cap = P.max_neighbors;
     uint32_t* row = nb + (size_t)i * cap;
-    uint32_t* tab = table[threadIdx.x / LIST_LANES];
     const int shift = (threadIdx.x & 63) & ~(LIST_LANES - 1);  // the group's bits of the wave's ballot
     int c = 0;
-    // tests one candidate per lane (slot s, if any) and appends the passing ones
-    auto test = [&](bool have, const float4& xj) __attribute__((always_inline)) {
+    // tests one candidate per lane (if any) and appends the passing ones
+    auto test = [&](bool have, uint32_t, const float4& xj) __attribute__((always_inline)) {
         const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
         const uint32_t j = __float_as_uint(xj.w);
         const bool pass = have && j != (uint32_t)i && dx * dx + dy * dy + dz * dz < hh;
@@ -217,58 +213,8 @@ __global__ __launch_bounds__(AB) void k_lists(int n, const float4* __restrict__ 
         if (pass && at < cap) row[at] = j;
         c += __popc(m);
     };
-    BoxCells bc;
-    bc.init(xi.x, xi.y, xi.z, h, P.scales, P.block_shift);
-    // this lane's cells: enumeration indices sub, sub + 16, ... (at most 64)
-    uint2 r[4];
-    uint32_t before[4];  // candidates of the box in earlier cells
-    uint32_t total = 0;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        r[q] = make_uint2(0u, 0u);
-        uint32_t g[3];
-        const int e = q * LIST_LANES + sub;
-        if (e < bc.count() && bc.cell(e, g) && g[0] < P.grid_dim && g[1] < P.grid_dim && g[2] < P.grid_dim)
-            r[q] = cells[dmorton3(g[0], g[1], g[2])];
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        uint32_t incl = r[q].y - r[q].x;
-#pragma unroll
-        for (int o = 1; o < LIST_LANES; o <<= 1) {
-            const uint32_t y = (uint32_t)__shfl_up((int)incl, o, LIST_LANES);
-            if (sub >= o) incl += y;
-        }
-        before[q] = total + incl - (r[q].y - r[q].x);
-        total += (uint32_t)__shfl((int)incl, LIST_LANES - 1, LIST_LANES);
-    }
-    if (total <= LIST_CAND) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            for (uint32_t s = r[q].x; s < r[q].y; ++s) tab[before[q] + (s - r[q].x)] = s;
-        // the group's lanes are in one wave: its LDS writes are in order before its reads
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        // four rounds' candidates are loaded together
-        for (uint32_t t = (uint32_t)sub; t - (uint32_t)sub < total; t += 4 * LIST_LANES) {
-            float4 xj[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                xj[q] = cand[tab[min(t + q * LIST_LANES, total - 1u)]];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) test(t + q * LIST_LANES < total, xj[q]);
-        }
-    } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            for (int u = 0; u < LIST_LANES; ++u) {
-                const uint32_t s0 = (uint32_t)__shfl((int)r[q].x, u, LIST_LANES);
-                const uint32_t s1 = (uint32_t)__shfl((int)r[q].y, u, LIST_LANES);
-                for (uint32_t s = s0; s < s1; s += LIST_LANES)
-                    test(s + sub < s1, cand[min(s + (uint32_t)sub, s1 - 1u)]);
-            }
-    }
+    for_each_in_box(xi.x, xi.y, xi.z, h, P.scales, P.block_shift, P.grid_dim, cells, sub,
+                    table[threadIdx.x / LIST_LANES], [&](uint32_t s) { return cand[s]; }, test);
     if (sub == 0) {
         cnt[i] = c < cap ? c : cap;
         if (c > cap) atomicOr(&ctl->err, 1u << UPF_ERR_NBR_OVERFLOW);

@@ -13,6 +13,8 @@
 
 #include <cstdint>
 
+#include "upf_device.h"
+
 namespace upf {
 
 // v of lane U of this lane's group of LANES (4: the quad, 16: the DPP row)
@@ -91,6 +93,79 @@ __device__ __forceinline__ void add_terms(float& x, float& y, float& z, const Te
 struct Pair4 {
     float4 a, b;
 };
+
+// Visits the candidates of the query box of (x, y, z) (the reference's BoxQuery)
+// in ascending slot order with BOX_LANES lanes (lane sub of them): per round,
+// load(slot) and then test(whether the lane has a candidate, slot, record).
+// Each lane finds cells of its own, their slots go to a candidate table in LDS
+// (tab, BOX_CAND entries per group), and four rounds' records are loaded
+// together.  BOX_CAND slots hold any query box of a fluid; a denser one is
+// walked cell by cell.
+constexpr int BOX_LANES = 16;
+constexpr int BOX_CAND = 384;
+template <class Load, class Test>
+__device__ __forceinline__ void for_each_in_box(float x, float y, float z, float h, const float* scales,
+                                                uint32_t block_shift, uint32_t grid_dim,
+                                                const uint2* __restrict__ cells, int sub, uint32_t* tab, Load load,
+                                                Test test) {
+    using V = decltype(load(0u));
+    BoxCells bc;
+    bc.init(x, y, z, h, scales, block_shift);
+    // this lane's cells: enumeration indices sub, sub + 16, ... (at most 64)
+    uint2 r[4];
+    uint32_t before[4];  // candidates of the box in earlier cells
+    uint32_t total = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        r[q] = make_uint2(0u, 0u);
+        uint32_t g[3];
+        const int e = q * BOX_LANES + sub;
+        if (e < bc.count() && bc.cell(e, g) && g[0] < grid_dim && g[1] < grid_dim && g[2] < grid_dim)
+            r[q] = cells[dmorton3(g[0], g[1], g[2])];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        uint32_t incl = r[q].y - r[q].x;
+#pragma unroll
+        for (int o = 1; o < BOX_LANES; o <<= 1) {
+            const uint32_t y = (uint32_t)__shfl_up((int)incl, o, BOX_LANES);
+            if (sub >= o) incl += y;
+        }
+        before[q] = total + incl - (r[q].y - r[q].x);
+        total += (uint32_t)__shfl((int)incl, BOX_LANES - 1, BOX_LANES);
+    }
+    if (total <= BOX_CAND) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            for (uint32_t s = r[q].x; s < r[q].y; ++s) tab[before[q] + (s - r[q].x)] = s;
+        // the group's lanes are in one wave: its LDS writes are in order before its reads
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        for (uint32_t t = (uint32_t)sub; t - (uint32_t)sub < total; t += 4 * BOX_LANES) {
+            uint32_t s[4];
+            V v[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                s[q] = tab[min(t + q * BOX_LANES, total - 1u)];
+                v[q] = load(s[q]);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) test(t + q * BOX_LANES < total, s[q], v[q]);
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            for (int u = 0; u < BOX_LANES; ++u) {
+                const uint32_t s0 = (uint32_t)__shfl((int)r[q].x, u, BOX_LANES);
+                const uint32_t s1 = (uint32_t)__shfl((int)r[q].y, u, BOX_LANES);
+                for (uint32_t t = s0; t < s1; t += BOX_LANES) {
+                    const uint32_t s = min(t + (uint32_t)sub, s1 - 1u);
+                    test(t + sub < s1, s, load(s));
+                }
+            }
+    }
+}
 
 }  // namespace upf
 

@@ -320,32 +320,37 @@ __device__ __forceinline__ void for_each_candidate(const float4& x, float h, con
 
 // --------------------------------------------------- boundary volume (Psi)
 // CalculateWeightedVolume (src/cpu/UnifiedPhysics.cpp:2703-2746): Psi_b = 1 / sum_b W
-__global__ void k_psi(StepArgs A, const float4* __restrict__ pos, const uint2* __restrict__ cells,
+// Sixteen lanes per boundary particle: one lane each walked 27 cells one candidate
+// at a time (89 us at 3,080 particles, 417 at 2.4M).
+__global__ __launch_bounds__(BLOCK) void k_psi(StepArgs A, const float4* __restrict__ pos, const uint2* __restrict__ cells,
                       const float* __restrict__ luts, float* __restrict__ psi, Ctl* ctl) {
     __shared__ float lw[LUT_N];
-    for (int t = threadIdx.x; t < LUT_N; t += blockDim.x) lw[t] = luts[t];
+    __shared__ uint32_t table[BLOCK / BOX_LANES][BOX_CAND];
+    for (int t = threadIdx.x; t < LUT_N; t += BLOCK) lw[t] = luts[t];
     __syncthreads();
     const upf_params& P = A.P;
     const float lut_factor = A.lut_factor;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = (int)((blockIdx.x * BLOCK + threadIdx.x) / BOX_LANES), sub = (int)threadIdx.x % BOX_LANES;
     if (i >= A.n) return;
-    const Dom d = dom_at(A, i);
     const float4 xi = pos[i];
     const int ti = ptype(xi);
     if (ti != UPF_FROZEN && ti != UPF_RIGID) return;
+    const Dom d = dom_at(A, i);
     const float T = P.support_radius_sq_limit;
     // Akinci et al. 2012 eq. 4 sums over the boundary neighbourhood including the
     // particle itself (W(0) = the table's entry 0); the CPU path excludes it
     float inv = P.boundary_pressure_mode == UPF_BOUNDARY_AKINCI ? lw[0] : 0.0f;
-    for_each_candidate(xi, P.support_radius, d, cells, [&](int j) __attribute__((always_inline)) {
-        if (j == i) return;
-        const float4 xj = pos[j];
-        const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-        const float d2 = dx * dx + dy * dy + dz * dz;
-        if (!(d2 < T)) return;
-        const int tj = ptype(xj);
-        if (tj == UPF_FROZEN || tj == UPF_RIGID) inv += lut_at(lw, sqrtf(d2), lut_factor);
-    });
+    for_each_in_box(
+        xi.x, xi.y, xi.z, P.support_radius, d.scales, d.block_shift, d.grid_dim, cells + d.cell_off, sub,
+        table[threadIdx.x / BOX_LANES], [&](uint32_t j) { return pos[j]; },
+        [&](bool have, uint32_t j, const float4& xj) __attribute__((always_inline)) {
+            const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+            const float d2 = dx * dx + dy * dy + dz * dz;
+            const int tj = ptype(xj);
+            const bool pass = have && (int)j != i && d2 < T && (tj == UPF_FROZEN || tj == UPF_RIGID);
+            inv = add_terms<BOX_LANES>(inv, pass ? lut_at(lw, sqrtf(d2), lut_factor) : -0.0f);
+        });
+    if (sub != 0) return;
     // CPU path: 1 / sum W (:2735); Akinci mode: the GPU path's factor 0.7
     // (src/gpu/particles_kernel.cu:5927-5946) on the self-inclusive sum
     if (inv != 0.0f) psi[i] = P.boundary_pressure_mode == UPF_BOUNDARY_AKINCI ? (float)(0.7 / (double)inv) : (float)(1.0 / (double)inv);
@@ -3535,7 +3540,7 @@ static int step_static_head(upf_sim* s) {
     const bool akinci = s->P.boundary_pressure_mode == UPF_BOUNDARY_AKINCI;
     if (!s->psi_ready) {
         s->prof.begin(PC_PSI, s->st);
-        hipLaunchKernelGGL(k_psi, g, dim3(BLOCK), 0, s->st, A, S.pos, s->W.cells, s->luts, S.psi, s->ctl);
+        hipLaunchKernelGGL(k_psi, lanes_grid(s->n, BOX_LANES), dim3(BLOCK), 0, s->st, A, S.pos, s->W.cells, s->luts, S.psi, s->ctl);
         s->prof.end(s->st);
         s->psi_ready = true;
     }
@@ -3677,7 +3682,7 @@ static int step_pcisph_rigid(upf_sim* s) {
     if (akinci) {
         s->prof.begin(PC_PSI, s->st);
         if (!s->psi_ready) {  // walls: once (they do not move)
-            hipLaunchKernelGGL(k_psi, g, dim3(BLOCK), 0, s->st, A, S.pos, s->W.cells, s->luts, S.psi, s->ctl);
+            hipLaunchKernelGGL(k_psi, lanes_grid(s->n, BOX_LANES), dim3(BLOCK), 0, s->st, A, S.pos, s->W.cells, s->luts, S.psi, s->ctl);
             s->psi_ready = true;
         }
         hipLaunchKernelGGL(k_psi_rigid, g, dim3(BLOCK), 0, s->st, s->n, S.pos, s->W.nbr, fuse ? 1 : A.stride,
