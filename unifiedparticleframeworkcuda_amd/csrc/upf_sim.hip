@@ -3021,6 +3021,21 @@ __global__ void k_ingest(StepArgs A, RawIn in, float psi0, Slots S, Work W, uint
     if (!ok) set_err(ctl, UPF_ERR_RANGE);
 }
 
+// Body index, offset and volume of every slot from the caller's arrays (upload
+// order).  A rigid particle's weighted_volume_ = its mass / rest density
+// (UnifiedParticle.cpp:24).
+__global__ __launch_bounds__(BLOCK) void k_attach_bodies(int n, const int* __restrict__ body_id,
+                                                         const float4* __restrict__ rel4, float rest_density, Slots S) {
+    const int i = blockIdx.x * BLOCK + threadIdx.x;
+    if (i >= n) return;
+    const int u = S.id[i];
+    const int b = body_id[u];
+    const float4 r = rel4[u];
+    S.body[i] = b;
+    S.rel[i] = r;
+    if (b >= 0) S.psi[i] = r.w / rest_density;
+}
+
 // The requested arrays (null: not) in upload order.
 struct RawOut {
     float4 *pos, *vel, *force;
@@ -3187,6 +3202,7 @@ struct upf_sim {
     std::vector<void*> allocs;
     // rigid bodies
     upf_body* d_bodies = nullptr;
+    int body_cap = 0;  // bodies that d_bodies and d_body_start hold
     int* d_body_start = nullptr;       // first member slot of each body (n_bodies + 1, -1 when empty)
     uint32_t* d_body_keys = nullptr;   // scratch: body key per slot
     uint32_t* d_body_keys2 = nullptr;
@@ -4250,50 +4266,48 @@ int upf_upload_bodies(upf_sim* s, int n_bodies, const upf_body* bodies, const in
     if (!s || n_bodies <= 0 || n_bodies >= 0xFFFF || !bodies || !body_id || !rel4) return UPF_ERR_ARG;
     if (!s->uploaded) return UPF_ERR_STATE;
     const int n = s->n;
-    // per-particle body data in the current slot order (slots are still in
-    // upload order unless a step ran, so scatter through the ids), checked on
-    // the host before anything on the device changes
-    std::vector<int> id(n), bid(n);
-    std::vector<float> rel((size_t)4 * n), psi(n);
+    // checked before anything on the device changes
+    int bad[Stage::THREADS] = {};
+    Stage::split((size_t)n, 1 << 16, [&](int part, size_t beg, size_t end) {
+        for (size_t i = beg; i < end; ++i)
+            if (body_id[i] < -1 || body_id[i] >= n_bodies) bad[part] = 1;
+    });
+    for (int b : bad)
+        if (b) return UPF_ERR_ARG;
     Slots& S = s->S[s->cur];
-    HIPCHK(hipMemcpy(id.data(), S.id, (size_t)n * 4, hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(psi.data(), S.psi, (size_t)n * 4, hipMemcpyDeviceToHost));
-    for (int k = 0; k < n; ++k) {
-        const int u = id[k];
-        bid[k] = body_id[u];
-        if (bid[k] < -1 || bid[k] >= n_bodies) return UPF_ERR_ARG;
-        for (int a = 0; a < 4; ++a) rel[4 * k + a] = rel4[4 * u + a];
-        // a rigid particle's weighted_volume_ = its mass / rest density (UnifiedParticle.cpp:24)
-        if (bid[k] >= 0) psi[k] = rel4[4 * u + 3] / s->P.rest_density;
-    }
     // the previous bodies are dropped first: after a failure below the
     // simulation has none (a rigid step returns UPF_ERR_STATE), never a body
     // count that disagrees with the device arrays
     s->rigid = false;
     s->n_bodies = 0;
-    if (s->d_bodies) (void)hipFree(s->d_bodies);
-    if (s->d_body_start) (void)hipFree(s->d_body_start);
-    s->d_bodies = nullptr;
-    s->d_body_start = nullptr;
-    upf_body* d_b = nullptr;
-    int* d_start = nullptr;
-    bool ok = hipMalloc((void**)&d_b, (size_t)n_bodies * sizeof(upf_body)) == hipSuccess &&
-              hipMalloc((void**)&d_start, (size_t)(n_bodies + 1) * sizeof(int)) == hipSuccess;
-    if (ok && !s->d_body_keys)
-        ok = s->alloc(&s->d_body_keys, s->cap) == hipSuccess && s->alloc(&s->d_body_keys2, s->cap) == hipSuccess &&
-             s->alloc(&s->d_body_members, s->cap) == hipSuccess &&
-             s->alloc(&s->d_body_terms, (size_t)7 * s->cap) == hipSuccess;
-    ok = ok && hipMemcpy(d_b, bodies, (size_t)n_bodies * sizeof(upf_body), hipMemcpyHostToDevice) == hipSuccess &&
-         hipMemcpy(S.body, bid.data(), (size_t)n * 4, hipMemcpyHostToDevice) == hipSuccess &&
-         hipMemcpy(S.rel, rel.data(), (size_t)n * 16, hipMemcpyHostToDevice) == hipSuccess &&
-         hipMemcpy(S.psi, psi.data(), (size_t)n * 4, hipMemcpyHostToDevice) == hipSuccess;
-    if (!ok) {
-        if (d_b) (void)hipFree(d_b);
-        if (d_start) (void)hipFree(d_start);
-        return UPF_ERR_HIP;
+    if (n_bodies > s->body_cap) {
+        if (s->d_bodies) (void)hipFree(s->d_bodies);
+        if (s->d_body_start) (void)hipFree(s->d_body_start);
+        s->d_bodies = nullptr;
+        s->d_body_start = nullptr;
+        s->body_cap = 0;
+        HIPCHK(hipMalloc((void**)&s->d_bodies, (size_t)n_bodies * sizeof(upf_body)));
+        HIPCHK(hipMalloc((void**)&s->d_body_start, (size_t)(n_bodies + 1) * sizeof(int)));
+        s->body_cap = n_bodies;
     }
-    s->d_bodies = d_b;
-    s->d_body_start = d_start;
+    if (!s->d_body_terms) {  // the last of them
+        HIPCHK(s->alloc(&s->d_body_keys, s->cap));
+        HIPCHK(s->alloc(&s->d_body_keys2, s->cap));
+        HIPCHK(s->alloc(&s->d_body_members, s->cap));
+        HIPCHK(s->alloc(&s->d_body_terms, (size_t)7 * s->cap));
+    }
+    // the caller's arrays go side by side into the list memory (a step builds
+    // its lists anew), through pinned slices; one kernel brings them into slot order
+    char* raw = reinterpret_cast<char*>(s->W.nbr);
+    const size_t br = (size_t)n * 16, bi = (size_t)n * 4;
+    const StagePart parts[2] = {{reinterpret_cast<char*>(const_cast<float*>(rel4)), 0, br},
+                                {reinterpret_cast<char*>(const_cast<int*>(body_id)), br, bi}};
+    HIPCHK(hipMemcpy(s->d_bodies, bodies, (size_t)n_bodies * sizeof(upf_body), hipMemcpyHostToDevice));
+    if (!s->stage.to_device(raw, br + bi, parts, 2, s->st)) return UPF_ERR_HIP;
+    hipLaunchKernelGGL(k_attach_bodies, grid_for(n), dim3(BLOCK), 0, s->st, n, reinterpret_cast<const int*>(raw + br),
+                       reinterpret_cast<const float4*>(raw), s->P.rest_density, S);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(s->st));
     s->n_bodies = n_bodies;
     s->rigid = true;
     return UPF_OK;
@@ -4364,7 +4378,7 @@ int upf_dump_cells(upf_sim* s, const char* particles_path, const char* blocks_pa
 
 int upf_download_bodies(upf_sim* s, upf_body* out) {
     if (!s || !out) return UPF_ERR_ARG;
-    if (!s->d_bodies) return UPF_ERR_STATE;
+    if (s->n_bodies == 0) return UPF_ERR_STATE;
     HIPCHK(hipStreamSynchronize(s->st));
     HIPCHK(hipMemcpy(out, s->d_bodies, (size_t)s->n_bodies * sizeof(upf_body), hipMemcpyDeviceToHost));
     return UPF_OK;
