@@ -1332,6 +1332,19 @@ __device__ __forceinline__ float4 boundary_xs(float4 x, float psi, float rho0) {
     return x;
 }
 
+// Its position: the initial one for a rigid particle of the CPU path (component
+// by component: a choice between S.x0[i] and xi puts xi in scratch memory).
+__device__ __forceinline__ float4 predicted_boundary(const upf_params& P, const Slots& S, int i, int ti, float4 xi) {
+    if (ti == UPF_RIGID && !P.rigid_predicted_current) {
+        const float* x0 = reinterpret_cast<const float*>(S.x0 + i);
+        xi.x = x0[0];
+        xi.y = x0[1];
+        xi.z = x0[2];
+        xi.w = x0[3];
+    }
+    return xi;
+}
+
 // The external-force work of slot i (one thread), shared by the
 // external-force pass and the fused list build: per-step records of the slot,
 // and for a liquid slot the forces over its list, the first predicted
@@ -1348,8 +1361,7 @@ __device__ __forceinline__ void ext_static_slot(const StepArgs& A, const Slots& 
     W.fp[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     W.rho[i] = S.rho_last[i];
     if (ti != UPF_LIQUID) {
-        W.xs[i] = boundary_xs<MODE>((ti == UPF_RIGID && !P.rigid_predicted_current) ? S.x0[i] : xi, S.psi[i],
-                                    P.rest_density);
+        W.xs[i] = boundary_xs<MODE>(predicted_boundary(P, S, i, ti, xi), S.psi[i], P.rest_density);
         W.force[i] = make_float4(0.f, 0.f, 0.f, 0.f);
         return;
     }
@@ -1487,8 +1499,7 @@ __device__ __forceinline__ void ext_static_lanes(const StepArgs& A, const Slots&
     }
     if (ti != UPF_LIQUID) {
         if (sub == 0) {
-            W.xs[i] = boundary_xs<MODE>((ti == UPF_RIGID && !P.rigid_predicted_current) ? S.x0[i] : xi, own_psi,
-                                        P.rest_density);
+            W.xs[i] = boundary_xs<MODE>(predicted_boundary(P, S, i, ti, xi), own_psi, P.rest_density);
             W.force[i] = make_float4(0.f, 0.f, 0.f, 0.f);
         }
         return;
