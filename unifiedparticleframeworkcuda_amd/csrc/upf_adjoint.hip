@@ -260,7 +260,10 @@ __global__ __launch_bounds__(AB) void k_ext(int n, const float4* __restrict__ x,
     for (uint32_t c = id; c < nc; c += gridDim.x * AB) cells[c] = make_uint2(0u, 0u);
     const int i = (int)(id / LANES), sub = (int)(id % LANES);
     if (i >= n) return;
-    const float4 xi = x[i];
+    float4 xi = x[i], vi = v[i];
+    const uint32_t* row = nb + (size_t)i * ld;
+    RowHead head = row_head<LANES>(row, ld, cnt + i, sub);
+    together(xi, vi, head);
     if (!is_fluid(xi)) {
         if (sub == 0) {
             F[i] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -269,10 +272,9 @@ __global__ __launch_bounds__(AB) void k_ext(int n, const float4* __restrict__ x,
         }
         return;
     }
-    const float4 vi = v[i];
     float fx = 0.0f, fy = 0.0f, fz = 0.0f;
     for_pairs<LANES>(
-        nb + (size_t)i * ld, cnt[i], sub, [&](uint32_t j) { return Pair4{x[j], v[j]}; },
+        row, head, sub, [&](uint32_t j) { return Pair4{x[j], v[j]}; },
         [&](const Pair4& q, bool have) {
             if (!have || !is_fluid(q.a)) return Term3{0.0f, 0.0f, 0.0f};
             const float r = len3(xi.x - q.a.x, xi.y - q.a.y, xi.z - q.a.z);
@@ -300,12 +302,15 @@ __global__ __launch_bounds__(AB) void k_density(int n, const float4* __restrict_
     const unsigned id = blockIdx.x * AB + threadIdx.x;
     const int i = (int)(id / LANES), sub = (int)(id % LANES);
     if (i >= n) return;
-    const float4 xi = xs[i];
+    float4 xi = xs[i];
+    const uint32_t* row = nb + (size_t)i * ld;
+    RowHead head = row_head<LANES>(row, ld, cnt + i, sub);
+    together(xi, head);
     float rho = 0.0f, pi = 0.0f;
     if (is_fluid_w(xi.w)) {
         rho = C.m * C.kn.W(0.0f);
         for_pairs<LANES>(
-            nb + (size_t)i * ld, cnt[i], sub, [&](uint32_t j) { return xs[j]; },
+            row, head, sub, [&](uint32_t j) { return xs[j]; },
             [&](const float4& xj, bool have) {
                 return have ? C.m * C.kn.W(len3(xi.x - xj.x, xi.y - xj.y, xi.z - xj.z)) : -0.0f;
             },
@@ -331,7 +336,11 @@ __global__ __launch_bounds__(AB) void k_pforce(int n, const float4* __restrict__
     const unsigned id = blockIdx.x * AB + threadIdx.x;
     const int i = (int)(id / LANES), sub = (int)(id % LANES);
     if (i >= n) return;
-    const float4 xi = x[i];
+    float4 xi = x[i];
+    float pi = rec[i].w;
+    const uint32_t* row = nb + (size_t)i * ld;
+    RowHead head = row_head<LANES>(row, ld, cnt + i, sub);
+    together(xi, pi, head);
     float4 xn = xi, vn;
     float yw = xi.w;
     if (!is_fluid(xi)) {
@@ -342,10 +351,9 @@ __global__ __launch_bounds__(AB) void k_pforce(int n, const float4* __restrict__
         }
         vn = v[i];
     } else {
-        const float pi = rec[i].w;
         float fx = 0.0f, fy = 0.0f, fz = 0.0f;
         for_pairs<LANES>(
-            nb + (size_t)i * ld, cnt[i], sub, [&](uint32_t j) { return rec[j]; },
+            row, head, sub, [&](uint32_t j) { return rec[j]; },
             [&](const float4& xj, bool have) {
                 const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
                 const float s = C.kn.G(len3(dx, dy, dz)) * (pi + xj.w) * C.cp;
@@ -417,19 +425,21 @@ __global__ __launch_bounds__(AB) void kr_pforce(int n, const float4* __restrict_
     const unsigned id = blockIdx.x * AB + threadIdx.x;
     const int i = (int)(id / LANES), sub = (int)(id % LANES);
     if (i >= n) return;
-    const float4 xi = x[i], xsi = xs[i];
+    float4 xi = x[i], xsi = xs[i], gi = gFp[i];
+    const uint32_t* row = nb + (size_t)i * ld;
+    RowHead head = row_head<LANES>(row, ld, cnt + i, sub);
+    together(xi, xsi, gi, head);
     if (!is_fluid(xi)) {
         if (sub == 0) rec[i] = make_float4(xsi.x, xsi.y, xsi.z, 0.0f);
         return;
     }
-    const float4 gi = gFp[i];
     float acc = 0.0f, gxx = 0.0f, gxy = 0.0f, gxz = 0.0f;
     struct Terms {
         float a;
         Term3 g;
     };
     for_pairs<LANES>(
-        nb + (size_t)i * ld, cnt[i], sub, [&](uint32_t j) { return Pair4{x[j], gFp[j]}; },
+        row, head, sub, [&](uint32_t j) { return Pair4{x[j], gFp[j]}; },
         [&](const Pair4& q, bool have) {
             const float4 &xj = q.a, &gj = q.b;
             if (!have) return Terms{0.0f, {0.0f, 0.0f, 0.0f}};
@@ -467,12 +477,15 @@ __global__ __launch_bounds__(AB) void kr_density(int n, const float4* __restrict
     const unsigned id = blockIdx.x * AB + threadIdx.x;
     const int i = (int)(id / LANES), sub = (int)(id % LANES);
     if (i >= n) return;
-    const float w = xs[i].w;
+    float w = xs[i].w;
+    float4 xi = rec[i];
+    const uint32_t* row = nb + (size_t)i * ld;
+    RowHead head = row_head<LANES>(row, ld, cnt + i, sub);
+    together(w, xi, head);
     if (!is_fluid_w(w)) return;
-    const float4 xi = rec[i];
     float gx = 0.0f, gy = 0.0f, gz = 0.0f;
     for_pairs<LANES>(
-        nb + (size_t)i * ld, cnt[i], sub, [&](uint32_t j) { return rec[j]; },
+        row, head, sub, [&](uint32_t j) { return rec[j]; },
         [&](const float4& xj, bool have) {
             const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
             const float r = len3(dx, dy, dz);
@@ -509,9 +522,11 @@ __global__ __launch_bounds__(AB) void kr_ext(int n, const float4* __restrict__ x
     const unsigned id = blockIdx.x * AB + threadIdx.x;
     const int i = (int)(id / LANES), sub = (int)(id % LANES);
     if (i >= n) return;
-    const float4 xi = x[i];
+    float4 xi = x[i], vi = v[i], gi = gF[i];
+    const uint32_t* row = nb + (size_t)i * ld;
+    RowHead head = row_head<LANES>(row, ld, cnt + i, sub);
+    together(xi, vi, gi, head);
     if (!is_fluid(xi)) return;
-    const float4 vi = v[i], gi = gF[i];
     float gvx = 0.0f, gvy = 0.0f, gvz = 0.0f, gxx = 0.0f, gxy = 0.0f, gxz = 0.0f;
     struct Rec {
         float4 x, g, v;
@@ -520,7 +535,7 @@ __global__ __launch_bounds__(AB) void kr_ext(int n, const float4* __restrict__ x
         Term3 v, x;
     };
     for_pairs<LANES>(
-        nb + (size_t)i * ld, cnt[i], sub, [&](uint32_t j) { return Rec{x[j], gF[j], v[j]}; },
+        row, head, sub, [&](uint32_t j) { return Rec{x[j], gF[j], v[j]}; },
         [&](const Rec& q, bool have) {
             const float4 &xj = q.x, &gj = q.g, &vj = q.v;
             Terms t = {{0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}};

@@ -49,15 +49,41 @@ __device__ __forceinline__ uint32_t entry_at(const uint32_t* __restrict__ row, i
     return k < cnt ? row[k] : 0u;
 }
 
+// A list's length and this lane's first two entries, which do not wait for the
+// length: rows of ld words are there whole, and for_pairs ignores what lies past
+// the list's end.  Loaded with the particle's own records, so that the first
+// gathers come one trip to memory after a pass starts, not three or four.
+struct RowHead {
+    int cnt;
+    uint32_t e, f;
+};
+template <int LANES>
+__device__ __forceinline__ RowHead row_head(const uint32_t* __restrict__ row, int ld, const int* __restrict__ cnt, int sub) {
+    return RowHead{*cnt, row[min(sub, ld - 1)], row[min(sub + LANES, ld - 1)]};
+}
+// Values that are to be on their way together: the compiler moves no load of
+// theirs past this, where the first use of any of them waits.
+__device__ __forceinline__ void together(int& v) { asm volatile("" : "+v"(v)); }
+__device__ __forceinline__ void together(uint32_t& v) { asm volatile("" : "+v"(v)); }
+__device__ __forceinline__ void together(float& v) { asm volatile("" : "+v"(v)); }
+__device__ __forceinline__ void together(float4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
+__device__ __forceinline__ void together(RowHead& v) { asm volatile("" : "+v"(v.cnt), "+v"(v.e), "+v"(v.f)); }
+template <class T, class... More>
+__device__ __forceinline__ void together(T& v, More&... more) {
+    together(v);
+    together(more...);
+}
+
 // Walks this lane's entries of the list row: load(entry) for the lane's next
 // two, then for each term(record, whether the lane has that entry) and, per
 // LANES neighbours, add(the lane's term).  An entry past the list's end reads
 // slot 0's records, for a term that changes no sum.  The next entries are
-// loaded ahead of the gathers of this round.  e: entry_at().
+// loaded ahead of the gathers of this round.
 template <int LANES, class Load, class Term, class Add>
-__device__ __forceinline__ void for_pairs(const uint32_t* __restrict__ row, int cnt, int sub, uint32_t e, Load load,
+__device__ __forceinline__ void for_pairs(const uint32_t* __restrict__ row, const RowHead& head, int sub, Load load,
                                           Term term, Add add) {
-    uint32_t f = entry_at(row, cnt, sub + LANES);
+    const int cnt = head.cnt;
+    uint32_t e = sub < cnt ? head.e : 0u, f = sub + LANES < cnt ? head.f : 0u;
     for (int k = sub; k - sub < cnt; k += 2 * LANES) {
         const auto r = load(e);
         const auto s = load(f);
@@ -66,11 +92,6 @@ __device__ __forceinline__ void for_pairs(const uint32_t* __restrict__ row, int 
         add(term(r, k < cnt));
         if (k - sub + LANES < cnt) add(term(s, k + LANES < cnt));
     }
-}
-template <int LANES, class Load, class Term, class Add>
-__device__ __forceinline__ void for_pairs(const uint32_t* __restrict__ row, int cnt, int sub, Load load, Term term,
-                                          Add add) {
-    for_pairs<LANES>(row, cnt, sub, entry_at(row, cnt, sub), load, term, add);
 }
 
 // three sums' terms, and their subtraction or addition

@@ -1486,11 +1486,12 @@ __device__ __forceinline__ void ext_static_lanes(const StepArgs& A, const Slots&
                                                  const float* lvl, const float* lpg, const float2* th, Ctl* ctl) {
     const upf_params& P = A.P;
     const uint32_t* row = W.nbr + (size_t)i * A.nbr_ld;
-    const int cnt = W.ncount[i];
-    const uint32_t e0 = entry_at(row, cnt, sub);
-    const float4 xi = S.pos[i];
+    RowHead head = row_head<LANES>(row, A.nbr_ld, W.ncount + i, sub);
+    float4 xi = S.pos[i], vi = S.vel[i];
+    float own_psi = S.psi[i], own_rho = S.rho_last[i];
+    float own_p = MODE == UPF_BOUNDARY_CPU_REF ? S.p_prev[i] : S.p_last[i];
+    together(head, xi, vi, own_psi, own_rho, own_p);
     const int ti = ptype(xi);
-    const float own_psi = S.psi[i], own_rho = S.rho_last[i];
     if (sub == 0) {
         W.p[i] = 0.0f;
         W.xpd[i] = make_float4(xi.x, xi.y, xi.z, pressure_record_w<MODE>(ti, own_psi, P.rest_density));
@@ -1504,10 +1505,8 @@ __device__ __forceinline__ void ext_static_lanes(const StepArgs& A, const Slots&
         }
         return;
     }
-    const float4 vi = S.vel[i];
     const float h = P.support_radius;
     const float rv = A.rest_vol, visc = P.visc_const;
-    const float own_p = MODE == UPF_BOUNDARY_CPU_REF ? S.p_prev[i] : S.p_last[i];
     const float inv = 1.0f / own_rho;
     const float pg = own_p * inv * inv;
     float fx = 0.0f, fy = 0.0f, fz = 0.0f;
@@ -1517,7 +1516,7 @@ __device__ __forceinline__ void ext_static_lanes(const StepArgs& A, const Slots&
     };
     // the terms of ext_static_slot's pair, all subtracted (x + -t is x - t)
     for_pairs<LANES>(
-        row, cnt, sub, e0,
+        row, head, sub,
         [&](uint32_t e) __attribute__((always_inline)) {
             const int j = (int)(e >> NB_SLOT_SHIFT);
             return Rec{at_u32(S.pos, j), at_u32(S.vel, j), j};
@@ -2001,33 +2000,54 @@ __global__ __launch_bounds__(BLOCK) void k_force(int t, StepArgs A, Slots S, Wor
     }
 }
 
+// A table of the kernel tables, and the bin thresholds, into LDS by a block of
+// BLOCK threads: all loads on their way before the first is stored.
+__device__ __forceinline__ void load_tables(const float* __restrict__ luts, float* __restrict__ a, int ta,
+                                            float2* __restrict__ th, float* __restrict__ b = nullptr, int tb = 0) {
+    static_assert(BLOCK < LUT_N && LUT_N <= 2 * BLOCK, "two entries per thread");
+    const int k = threadIdx.x, l = min(k + BLOCK, LUT_N - 1);
+    const float2* t = reinterpret_cast<const float2*>(luts + LUT_TH_OFF);
+    const float a0 = luts[ta * LUT_N + k], a1 = luts[ta * LUT_N + l];
+    const float b0 = b ? luts[tb * LUT_N + k] : 0.0f, b1 = b ? luts[tb * LUT_N + l] : 0.0f;
+    const float2 t0 = t[k], t1 = t[l];
+    a[k] = a0;
+    th[k] = t0;
+    if (b) b[k] = b0;
+    if (k + BLOCK < LUT_N) {
+        a[l] = a1;
+        th[l] = t1;
+        if (b) b[l] = b1;
+    }
+}
+
 // The two iteration passes of one scene with LANES lanes per particle over the
 // packed slot-major lists (k_nbr_build_ext with LANES): k_density's and
 // k_force's expressions.  Few particles leave one chain of list rows and
 // gathers per wave, and the chip mostly idle (9.5 and 9.0 us per launch from
-// 3,080 to 80,648 particles with one lane each; now 5.4 and 4.7 at 3,080, 7.8
-// and 7.9 at 80,648).
+// 3,080 to 80,648 particles with one lane each; now 4.5 and 4.4 at 3,080, 6.9
+// and 7.8 at 80,648).
 template <int MODE, int LANES>
 __global__ __launch_bounds__(BLOCK) void k_density_lanes(int t, StepArgs A, Work W, const float* __restrict__ luts,
                                                          Ctl* ctl) {
-    if (t >= __atomic_load_n(&ctl->want_any, __ATOMIC_RELAXED)) return;
+    // whether the iteration runs: tested after the tables, on its way with all else
+    const int want = __atomic_load_n(&ctl->want_any, __ATOMIC_RELAXED);
     __shared__ float lw[LUT_N];
     __shared__ float2 th[LUT_N];
     __shared__ float wmax[BLOCK / 64];
     const upf_params& P = A.P;
     const unsigned id = (unsigned)xblk_down(A.xcd) * BLOCK + threadIdx.x;
     const int i = (int)(id / LANES), sub = (int)(id % LANES);
+    // the slot's records and the list's first entries are on their way while the
+    // tables load (a lane past the last slot loads that one's)
     const bool in = i < A.n;
-    // the list's first entries are on their way while the tables load
-    const float4 xi = in ? W.xs[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const uint32_t* row = W.nbr + (size_t)(in ? i : 0) * A.nbr_ld;
-    const int cnt = in ? W.ncount[i] : 0;
-    const uint32_t e0 = entry_at(row, cnt, sub);
-    for (int k = threadIdx.x; k < LUT_N; k += BLOCK) {
-        lw[k] = k < 300 ? luts[k] : 0.0f;  // bin 300 (dist >= h) weighs 0, as in lut_at
-        th[k] = reinterpret_cast<const float2*>(luts + LUT_TH_OFF)[k];
-    }
+    const int at = min(i, A.n - 1);
+    const float4 xi = W.xs[at];
+    const float p_before = W.p[at];
+    const uint32_t* row = W.nbr + (size_t)at * A.nbr_ld;
+    const RowHead head = row_head<LANES>(row, A.nbr_ld, W.ncount + at, sub);
+    load_tables(luts, lw, 0, th);  // (entry 300, dist >= h, is 0 in every table)
     __syncthreads();
+    if (t >= want) return;
     float mine = 0.0f;
     if (in && ptype(xi) == UPF_LIQUID) {
         const float m = P.initial_mass;
@@ -2036,7 +2056,7 @@ __global__ __launch_bounds__(BLOCK) void k_density_lanes(int t, StepArgs A, Work
         if (P.add_wall_weight)
             rho = rho + wall_weight<false>(P, wall_distance(P, xi.x, xi.y, xi.z), A.lut_factor, lw);
         for_pairs<LANES>(
-            row, cnt, sub, e0, [&](uint32_t e) { return at_u32(W.xs, (int)(e >> NB_SLOT_SHIFT)); },
+            row, head, sub, [&](uint32_t e) { return at_u32(W.xs, (int)(e >> NB_SLOT_SHIFT)); },
             [&](const float4& xj, bool have) __attribute__((always_inline)) {
                 const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
                 const float d2 = dx * dx + dy * dy + dz * dz;
@@ -2048,7 +2068,7 @@ __global__ __launch_bounds__(BLOCK) void k_density_lanes(int t, StepArgs A, Work
             [&](float t) { rho = add_terms<LANES>(rho, t); });
         if (sub == 0) {
             const float err = fmax_ref(rho - P.rest_density, 0.0f);
-            const float p = W.p[i] + fmax_ref(err * P.density_error_factor, 0.0f);
+            const float p = p_before + fmax_ref(err * P.density_error_factor, 0.0f);
             W.p[i] = p;
             reinterpret_cast<float*>(W.xpd)[4 * (size_t)i + 3] = p / (P.rest_density * P.rest_density);
             W.rho[i] = rho;
@@ -2068,28 +2088,25 @@ __global__ __launch_bounds__(BLOCK) void k_density_lanes(int t, StepArgs A, Work
 template <int MODE, int LANES>
 __global__ __launch_bounds__(BLOCK) void k_force_lanes(int t, StepArgs A, Slots S, Work W,
                                                        const float* __restrict__ luts, Ctl* ctl, Publish pub) {
-    if (t >= __atomic_load_n(&ctl->want_any, __ATOMIC_RELAXED)) return;
-    if (blockIdx.x == 0 && threadIdx.x < 64) loop_test(A, 0, t, threadIdx.x, ctl, pub);
+    const int want = __atomic_load_n(&ctl->want_any, __ATOMIC_RELAXED);  // as in k_density_lanes
     __shared__ float lpg[LUT_N];
     __shared__ float2 th[LUT_N];
     const upf_params& P = A.P;
     const unsigned id = (unsigned)xblk(A.xcd) * BLOCK + threadIdx.x;
     const int i = (int)(id / LANES), sub = (int)(id % LANES);
-    const bool in = i < A.n;
-    const float4 xr = in ? W.xpd[i] : make_float4(0.f, 0.f, 0.f, -0.0f);
-    const uint32_t* row = W.nbr + (size_t)(in ? i : 0) * A.nbr_ld;
-    const int cnt = in ? W.ncount[i] : 0;
-    const uint32_t e0 = entry_at(row, cnt, sub);
-    for (int k = threadIdx.x; k < LUT_N; k += BLOCK) {
-        lpg[k] = luts[LUT_N + k];
-        th[k] = reinterpret_cast<const float2*>(luts + LUT_TH_OFF)[k];
-    }
+    const int at = min(i, A.n - 1);
+    const float4 xr = W.xpd[at], vel = S.vel[at], ext = W.force[at];
+    const uint32_t* row = W.nbr + (size_t)at * A.nbr_ld;
+    const RowHead head = row_head<LANES>(row, A.nbr_ld, W.ncount + at, sub);
+    load_tables(luts, lpg, 1, th);
     __syncthreads();
-    if (__builtin_signbit(xr.w)) return;  // not liquid
+    if (t >= want) return;
+    if (blockIdx.x == 0 && threadIdx.x < 64) loop_test(A, 0, t, threadIdx.x, ctl, pub);
+    if (i >= A.n || __builtin_signbit(xr.w)) return;  // not liquid
     const float m = P.initial_mass;
     float fx = 0.0f, fy = 0.0f, fz = 0.0f;
     for_pairs<LANES>(
-        row, cnt, sub, e0, [&](uint32_t e) { return at_u32(W.xpd, (int)(e >> NB_SLOT_SHIFT)); },
+        row, head, sub, [&](uint32_t e) { return at_u32(W.xpd, (int)(e >> NB_SLOT_SHIFT)); },
         [&](const float4& xj, bool have) __attribute__((always_inline)) {
             const float dx = xr.x - xj.x, dy = xr.y - xj.y, dz = xr.z - xj.z;
             const float g = lpg[bin_of_d2(dx * dx + dy * dy + dz * dz, A.lut_factor, th)];
@@ -2108,7 +2125,7 @@ __global__ __launch_bounds__(BLOCK) void k_force_lanes(int t, StepArgs A, Slots 
     // written when this iteration may be the scene's last (k_force)
     if (t + 1 >= __atomic_load_n(&A.sctl[0].want, __ATOMIC_RELAXED)) W.fp[i] = Fp;
     const float4 xi = make_float4(xr.x, xr.y, xr.z, __int_as_float(UPF_LIQUID));
-    W.xs[i] = predict(xi, S.vel[i], W.force[i], Fp, A, A.dom0, ctl);
+    W.xs[i] = predict(xi, vel, ext, Fp, A, A.dom0, ctl);
 }
 
 // ------------------------------------------------------------ integration
@@ -2254,11 +2271,11 @@ __device__ __forceinline__ void density_wcsph_lanes(const StepArgs& A, const Slo
                                                     const float* lw, const float2* th) {
     const upf_params& P = A.P;
     const uint32_t* row = W.nbr + (size_t)i * A.nbr_ld;
-    const int cnt = W.ncount[i];
+    const RowHead head = row_head<LANES>(row, A.nbr_ld, W.ncount + i, sub);
     const float4 xi = S.pos[i];
     float rho = P.kernel_self * P.initial_mass;
     for_pairs<LANES>(
-        row, cnt, sub, [&](uint32_t e) { return at_u32(S.pos, (int)(e >> NB_SLOT_SHIFT)); },
+        row, head, sub, [&](uint32_t e) { return at_u32(S.pos, (int)(e >> NB_SLOT_SHIFT)); },
         [&](const float4& xj, bool have) __attribute__((always_inline)) {
             const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
             const float w = lw[bin_of_d2(dx * dx + dy * dy + dz * dz, A.lut_factor, th)];
@@ -2376,29 +2393,23 @@ __global__ __launch_bounds__(BLOCK) void k_force_wcsph_lanes(StepArgs A, Slots S
     const upf_params& P = A.P;
     const unsigned id = blockIdx.x * BLOCK + threadIdx.x;
     const int i = (int)(id / LANES), sub = (int)(id % LANES);
-    const bool in = i < A.n;
-    const float4 xi = in ? S.pos[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const uint32_t* row = W.nbr + (size_t)(in ? i : 0) * A.nbr_ld;
-    const int cnt = in ? W.ncount[i] : 0;
-    const uint32_t e0 = entry_at(row, cnt, sub);
-    for (int t = threadIdx.x; t < LUT_N; t += BLOCK) {
-        lvl[t] = luts[2 * LUT_N + t];
-        lpg[t] = luts[LUT_N + t];
-        th[t] = reinterpret_cast<const float2*>(luts + LUT_TH_OFF)[t];
-    }
+    const int at = min(i, A.n - 1);
+    const float4 xi = S.pos[at], vi = S.vel[at];
+    const float p_i = W.pres[at], rho_i = W.rho[at];
+    const uint32_t* row = W.nbr + (size_t)at * A.nbr_ld;
+    const RowHead head = row_head<LANES>(row, A.nbr_ld, W.ncount + at, sub);
+    load_tables(luts, lvl, 2, th, lpg, 1);
     __syncthreads();
-    if (!in || ptype(xi) != UPF_LIQUID) return;
+    if (i >= A.n || ptype(xi) != UPF_LIQUID) return;
     const float m = P.initial_mass;
-    const float p_i = W.pres[i];
-    const float invD = (float)(1.0 / (double)W.rho[i]);
+    const float invD = (float)(1.0 / (double)rho_i);
     const float pVol = m * invD;
-    const float4 vi = S.vel[i];
     float fx = 0.0f, fy = 0.0f, fz = 0.0f;
     struct Terms {
         Term3 g, u;
     };
     for_pairs<LANES>(
-        row, cnt, sub, e0,
+        row, head, sub,
         [&](uint32_t e) __attribute__((always_inline)) {
             const int j = (int)(e >> NB_SLOT_SHIFT);
             return Pair4{at_u32(W.xpd, j), at_u32(W.vpg, j)};
