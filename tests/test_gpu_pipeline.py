@@ -66,6 +66,18 @@ def test_sort_forms_are_stable(gpu, n):
     sim.close()
 
 
+def _grid(grid):
+    """Parameters with a z-index grid of `grid` cells per axis, and the cells' width."""
+    p, _, _, _ = upf.standard_dam_break(8, 8, 8)
+    p.grid_dim, p.block_size = grid, 1024 // grid
+    p.block_shift = p.block_size.bit_length() - 1
+    width = 1.02 * p.support_radius
+    for a in range(3):
+        p.scales[a] = p.block_size / width
+        p.vbox_max[a] = grid * width
+    return p, width
+
+
 # cell tables of one tile, of tiles summed by the scan, of summed blocks, of
 # several tiles per block, and one too sparse for the counting (sorted by key);
 # particles in random order, in key order, and piled into few cells
@@ -74,13 +86,7 @@ def test_sort_forms_are_stable(gpu, n):
 @pytest.mark.parametrize("order", ["random", "sorted", "piled"])
 def test_cell_bins_are_a_stable_sort(gpu, grid, n, order):
     print("cell bins: grid %d, n %d, %s" % (grid, n, order), flush=True)
-    p, _, _, _ = upf.standard_dam_break(8, 8, 8)
-    p.grid_dim, p.block_size = grid, 1024 // grid
-    p.block_shift = p.block_size.bit_length() - 1
-    width = 1.02 * p.support_radius
-    for a in range(3):
-        p.scales[a] = p.block_size / width
-        p.vbox_max[a] = grid * width
+    p, width = _grid(grid)
     rng = np.random.RandomState(grid + n)
     pos = np.zeros((n, 4), np.float32)
     top = (grid - 1.01) * width
@@ -104,6 +110,28 @@ def test_cell_bins_are_a_stable_sort(gpu, grid, n, order):
         first = np.flatnonzero(np.r_[True, code[1:] != code[:-1]])
         ref = np.stack([code[first], first, np.r_[first[1:], n]], 1).astype(np.uint32)
         assert np.array_equal(cells, ref)
+    sim.close()
+
+
+# every cell of a grid, its edges and corners among them, as the centre of a stencil
+@pytest.mark.parametrize("grid", [2, 4, 8, 16])
+def test_lists_over_a_full_grid(gpu, grid):
+    print("lists: grid %d" % grid, flush=True)
+    p, width = _grid(grid)
+    n = 6 * grid ** 3
+    pos = np.zeros((n, 4), np.float32)
+    pos[:, :3] = np.random.RandomState(grid).uniform(0.0, grid * width - 1.01 * p.support_radius, (n, 3))
+    sim = upf.Simulation(p, n)
+    sim.upload(pos, np.full(n, upf.UPF_LIQUID, np.int32))
+    counts, flat = sim.neighbors()
+    _, ids, _ = sim.sorted_state()
+    x = pos[ids, :3]
+    first = np.cumsum(counts) - counts
+    for i in range(n):
+        d = x[i] - x
+        d2 = d[:, 0] * d[:, 0] + d[:, 1] * d[:, 1] + d[:, 2] * d[:, 2]
+        want = np.flatnonzero(d2 < np.float32(p.support_radius_sq_limit))
+        assert np.array_equal(flat[first[i]: first[i] + counts[i]], want[want != i]), i
     sim.close()
 
 

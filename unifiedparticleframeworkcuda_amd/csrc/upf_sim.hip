@@ -833,11 +833,20 @@ __device__ __forceinline__ void build_wave(const StepArgs& A, const float4* __re
     // slots of the coupling step)
     const bool my_part = mine_valid && lane / (64 / SPLIT) == part;
     const bool my_owner = my_part && ptype(my_x) == OWNER;
-    uint32_t my_blo = 0u, my_bhi = 0u;
+    // the key whose cell centres a slot's stencil: its sort key, or for a
+    // rigid owner -- keyed at its position before the last rigid update -- the
+    // key of its current position, whose cell's stencil holds its query box
+    uint32_t my_seg = my_key;
+    // all ones where the particle's query box (BoxQuery, in cell coordinates,
+    // clipped to the grid) ends before the next lower / higher cell of an axis
+    uint32_t no_below[3] = {0u, 0u, 0u}, no_above[3] = {0u, 0u, 0u};
     if (my_owner) {
-        // BoxQuery of the particle in cell coordinates, clipped to the grid
         const Dom dm = scene_dom(A, my_scene);
         const float xv[3] = {my_x.x, my_x.y, my_x.z};
+        if constexpr (OWNER == UPF_RIGID) {
+            bool ok;
+            my_seg = dkey(my_x.x, my_x.y, my_x.z, dm.scales, ok);
+        }
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
             float lo_f = dm.scales[a] * (xv[a] - h);
@@ -847,28 +856,18 @@ __device__ __forceinline__ void build_wave(const StepArgs& A, const float4* __re
             const uint32_t l = ((uint32_t)(unsigned short)lo_f) >> dm.block_shift;
             uint32_t u = ((uint32_t)(unsigned short)hi_f) >> dm.block_shift;
             u = u < dm.grid_dim ? u : dm.grid_dim - 1;  // cells lie below G <= 512
-            my_blo |= l << (10 * a);
-            my_bhi |= u << (10 * a);
-        }
-    }
-    // the key whose cell centres a slot's stencil: its sort key, or for a
-    // rigid owner -- keyed at its position before the last rigid update -- the
-    // key of its current position, whose cell's stencil holds its query box
-    uint32_t my_seg = my_key;
-    if constexpr (OWNER == UPF_RIGID) {
-        if (my_owner) {
-            const Dom dm = scene_dom(A, my_scene);
-            bool ok;
-            my_seg = dkey(my_x.x, my_x.y, my_x.z, dm.scales, ok);
+            const uint32_t own = compact10((my_seg >> (3u * dm.block_shift)) >> a);
+            no_below[a] = l < own ? 0u : ~0u;
+            no_above[a] = u > own ? 0u : ~0u;
         }
     }
     const uint64_t owners = wballot(my_owner);
     int my_cnt = 0;  // this lane's slot: list length so far
-    // the cells' grid, in scalar registers (of the scene met last, in a batch):
-    // so the stencil of a cell is set up on the scalar unit.  Through a choice of
-    // addresses it took vector instructions and three dependent loads from
-    // scratch per cell (WCSPH build of 1,132,556 particles 350 -> 335 us, PCISPH
-    // 326 -> 319, rigid lists 160 -> 148).
+    // the cells' grid, in scalar registers (of the scene met last, in a batch).
+    // Setting up a cell's stencil took about as many instructions as its tests,
+    // vector and scalar ones at the same rate; as masks of lanes (below) it takes
+    // half of them (1,132,556 particles, from before both: WCSPH build 350 -> 275
+    // us, PCISPH 326 -> 288; rigid lists of the 524k coupling scene 160 -> 126).
     uint32_t block_shift = A.dom0.block_shift, G = A.dom0.grid_dim, cell_off = 0;
     int grid_of = A.scene_of ? -1 : 0;
     int s = base;
@@ -897,76 +896,84 @@ __device__ __forceinline__ void build_wave(const StepArgs& A, const float4* __re
             s = pe;
             continue;
         }
-        const uint32_t cc[3] = {compact10(c), compact10(c >> 1), compact10(c >> 2)};
-        // stencil cells in Morton order: lane e names enumeration index e
-        BoxCells bc;
+        // The 3x3x3 stencil in Morton order, one cell per lane.  Of an axis' three
+        // coordinates v - 1, v, v + 1, v's pair by the lowest bit shares all higher
+        // ones; the third differs from the pair first at bit key (in the code).  So
+        // lanes count through three high bits, the axes' keys in order (sh: the
+        // axis' bit), then the three lowest bits; a third coordinate has no partner
+        // (skip).  All of it is the same on every lane: masks of lanes in scalar
+        // registers.
+        uint32_t code = 0u, cls = 0u;  // the lane's cell; bit a / 3 + a: below / above along axis a
+        uint64_t skip = 0ull;
         {
-            // a degenerate "box" whose cells are the clipped 3x3x3 stencil
-            int nn[3];
-            uint32_t lo[3];
+            uint32_t key[3];
 #pragma unroll
             for (int a = 0; a < 3; ++a) {
-                lo[a] = cc[a] > 0 ? cc[a] - 1 : 0;
-                const uint32_t hi = cc[a] + 1 < G ? cc[a] + 1 : G - 1;
-                nn[a] = (int)(hi - lo[a]) + 1;
+                const uint32_t ma = 0x09249249u << a, ca = c & ma;
+                const uint32_t third = (c >> a) & 1u ? ((ca | ~ma) + 1u) & ma : ca;
+                key[a] = third ? (uint32_t)__builtin_ctz(third) : 32u + a;
             }
-            bc.init_cells(lo, nn);
-        }
-        uint32_t rs = 0, rl = 0, rcell = 0;
-        bool valid = false;
-        if (lane < bc.count()) {
-            uint32_t q[3];
-            if (bc.cell(lane, q)) {
-                const uint2 r = T3[dmorton3(q[0], q[1], q[2])];
-                valid = r.y > r.x;
-                rs = r.x;
-                rl = r.y - r.x;
-                rcell = q[0] | (q[1] << 10) | (q[2] << 20);
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                const int b1 = (a + 1) % 3, b2 = (a + 2) % 3;
+                const int sh = (key[b1] < key[a] ? 1 : 0) + (key[b2] < key[a] ? 1 : 0);
+                const uint64_t hb = sh == 0 ? 0xFF00FF00FF00FF00ull
+                                            : (sh == 1 ? 0xFFFF0000FFFF0000ull : 0xFFFFFFFF00000000ull);
+                const uint64_t lb = a == 0 ? 0xAAAAAAAAAAAAAAAAull
+                                           : (a == 1 ? 0xCCCCCCCCCCCCCCCCull : 0xF0F0F0F0F0F0F0F0ull);
+                const uint32_t ma = 0x09249249u << a, ca = c & ma;
+                const bool odd = (c >> a) & 1u;
+                const uint32_t dn = (ca - 1u) & ma, up = ((ca | ~ma) + 1u) & ma;
+                // even: v - 1 | v, v + 1; odd: v - 1, v | v + 1
+                const uint64_t below = odd ? ~hb & ~lb : ~hb, above = odd ? hb : hb & lb;
+                skip |= lb & (odd ? hb : ~hb);
+                if (ca == 0u) skip |= below;
+                if (ca == (ma & (G * G * G - 1u))) skip |= above;
+                const bool l1 = __builtin_amdgcn_inverse_ballot_w64(lb);
+                code |= __builtin_amdgcn_inverse_ballot_w64(hb) ? (l1 ? up : (odd ? up : ca)) : (l1 ? (odd ? ca : dn) : dn);
+                cls |= (__builtin_amdgcn_inverse_ballot_w64(below) ? 1u << a : 0u) |
+                       (__builtin_amdgcn_inverse_ballot_w64(above) ? 8u << a : 0u);
             }
         }
-        const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+        uint32_t rs = 0, rl = 0;
+        if (__builtin_amdgcn_inverse_ballot_w64(~skip)) {
+            const uint2 r = T3[code];
+            rs = r.x;
+            rl = r.y - r.x;
+        }
+        const bool valid = rl != 0u;
         const uint64_t vm = wballot(valid);
         const int nr = __popcll(vm);
-        const int rank = __popcll(vm & lt);
+        const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(vm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)vm, 0u));
         // prefix of the occupied cells' lengths in rank (= lane) order
-        const uint32_t incl = wave_scan(valid ? rl : 0u);
-        if (valid) { r_start[rank] = rs; r_cell[rank] = rcell; r_pref[rank + 1] = incl; }
+        const uint32_t incl = wave_scan(rl);
+        if (valid) { r_start[rank] = rs; r_cell[rank] = cls; r_pref[rank + 1] = incl; }
         if (lane == 0) r_pref[0] = 0;
         __syncthreads();
-        const int M = (int)r_pref[nr];
+        const int M = __builtin_amdgcn_readlane((int)incl, 63);
+        // lanes k and k + 32: the occupied cell of rank k
+        const int k5 = lane & 31;
+        const uint32_t k_cls = k5 < nr ? r_cell[k5] : 0u;
         // candidate table (cand, CAND_CAP entries of LDS): slot << 5 | cell rank
-        // of every candidate, written by the lanes of the occupied cells, so
+        // of every candidate, written by two lanes per occupied cell, so
         // that each round reads its candidates at once; a stencil with more
         // candidates finds their cells by a walk over the prefix sums
         const bool table = M <= CAND_CAP;
         if (table) {
-            const uint32_t len = valid ? rl : 0u;
-            const int beg = (int)(incl - len);  // r_pref[rank] of a valid lane
-            for (uint32_t t = 0; wballot(t < len) != 0ull; ++t)
-                if (t < len) cand[beg + (int)t] = ((rs + t) << 5) | (uint32_t)rank;
+            const uint32_t beg = r_pref[k5], len = k5 < nr ? r_pref[k5 + 1] - beg : 0u, k_rs = r_start[k5];
+            for (uint32_t t = (uint32_t)lane >> 5; wballot(t < len) != 0ull; t += 2)
+                if (t < len) cand[beg + t] = ((k_rs + t) << 5) | (uint32_t)k5;
             __syncthreads();
         }
         // Which occupied stencil cells (bit k: rank k) lie in the query box of
         // this lane's particle -- the box test of every candidate of the cell,
-        // done once per cell: lane k < nr holds rank k's cell; per axis, the
-        // ranks one below, at and one above the cell's own coordinate, and the
-        // lane's box (blo .. bhi per field) keeps those of each class it meets.
-        uint32_t in_box;
-        {
-            const uint32_t qk = lane < nr ? r_cell[lane] : 0u;
-            in_box = (1u << nr) - 1u;  // nr <= 27
+        // done once per cell: the box holds the particle's own cell, and the
+        // ranks below or above it along an axis as far as it reaches there
+        uint32_t in_box = (1u << nr) - 1u;  // nr <= 27
 #pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                const uint32_t qa = (qk >> (10 * a)) & 0x3FFu;
-                const uint32_t below = (uint32_t)wballot(lane < nr && qa < cc[a]);
-                const uint32_t above = (uint32_t)wballot(lane < nr && qa > cc[a]);
-                const uint32_t at = (uint32_t)wballot(lane < nr && qa == cc[a]);
-                const uint32_t l = (my_blo >> (10 * a)) & 0x3FFu, u = (my_bhi >> (10 * a)) & 0x3FFu;
-                // stencil coordinates are cc - 1, cc, cc + 1 (cc - 1 only when cc > 0)
-                if (!(cc[a] > 0 && l <= cc[a] - 1 && cc[a] - 1 <= u)) in_box &= ~below;
-                if (!(l <= cc[a] && cc[a] <= u)) in_box &= ~at;
-                if (!(l <= cc[a] + 1 && cc[a] + 1 <= u)) in_box &= ~above;
-            }
+        for (int a = 0; a < 3; ++a) {
+            const uint32_t below = (uint32_t)wballot((k_cls >> a) & 1u), above = (uint32_t)wballot((k_cls >> (3 + a)) & 1u);
+            in_box &= ~((no_below[a] & below) | (no_above[a] & above));
         }
         for (int c0 = 0; c0 < M; c0 += NB_CHUNK) {
             // this lane's candidates of the chunk; a lane past the end holds
