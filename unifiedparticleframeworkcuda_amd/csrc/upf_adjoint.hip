@@ -184,7 +184,7 @@ __global__ __launch_bounds__(AB) void k_rank_cand(int n, CellMap map, const uint
 // Sixteen lanes per particle test sixteen candidates at a time, the passing ones
 // appended in order through the group's ballot.  Bound by the latency of table
 // and candidate reads (267 us at 80,648 particles with one lane walking the cells
-// of each, now 37).
+// of each, 37 with BoxCells' enumeration per lane, now 32).
 constexpr int LIST_LANES = BOX_LANES;
 __global__ __launch_bounds__(AB) void k_lists(int n, const float4* __restrict__ x, const float4* __restrict__ cand,
                                               const uint2* __restrict__ cells, upf_params P,

@@ -130,19 +130,52 @@ __device__ __forceinline__ void for_each_in_box(float x, float y, float z, float
                                                 const uint2* __restrict__ cells, int sub, uint32_t* tab, Load load,
                                                 Test test) {
     using V = decltype(load(0u));
-    BoxCells bc;
-    bc.init(x, y, z, h, scales, block_shift);
-    // this lane's cells: enumeration indices sub, sub + 16, ... (at most 64)
+    // This lane's cells: numbers sub, sub + 16, ... of the 3x3x3 stencil around
+    // (x, y, z) in Morton order.  Of an axis' three coordinates two share all but
+    // the lowest bit, the third differs from them first at bit key of the cell code;
+    // the numbers count through three high bits, the axes' keys in order, then the
+    // lowest bits.  The box reaches at most one cell either way (a cell is wider
+    // than h).
+    bool in_grid;
+    const uint32_t c = dkey(x, y, z, scales, in_grid) >> (3u * block_shift);
+    uint32_t key[3], v0[3], v1[3];  // the axis' part of the code for a high bit of 0 / 1
+    bool ok0[3], ok1[3];
+    const float xv[3] = {x, y, z};
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const uint32_t ma = 0x09249249u << a, ca = c & ma;
+        const bool odd = (c >> a) & 1u, lb = (sub >> a) & 1;
+        const uint32_t dn = (ca - 1u) & ma, up = ((ca | ~ma) + 1u) & ma, third = odd ? up : ca;
+        key[a] = third ? (uint32_t)__ffs((int)third) : 33u + a;
+        v0[a] = lb && odd ? ca : dn;
+        v1[a] = lb || odd ? up : ca;
+        // BoxQuery along the axis
+        bool in;
+        const uint32_t own = dgrid(scales[a] * xv[a], in) >> block_shift;
+        const float lo_f = scales[a] * (xv[a] - h), hi_f = scales[a] * (xv[a] + h);
+        const uint32_t l = ((uint32_t)(unsigned short)(lo_f >= 0.0f ? lo_f : 0.0f)) >> block_shift;
+        const uint32_t u = ((uint32_t)(unsigned short)(hi_f <= 1024.0f ? hi_f : 1024.0f)) >> block_shift;
+        const bool below = l < own, above = u > own && own + 1 < grid_dim;
+        ok0[a] = odd ? lb || below : !lb && below;
+        ok1[a] = odd ? !lb && above : !lb || above;
+    }
     uint2 r[4];
     uint32_t before[4];  // candidates of the box in earlier cells
     uint32_t total = 0;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
+        uint32_t code = 0;
+        bool ok = true;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const int b = (a + 1) % 3, d = (a + 2) % 3;
+            const int sh = (key[b] < key[a] ? 1 : 0) + (key[d] < key[a] ? 1 : 0);  // the axis' high bit
+            const bool hb = sh == 0 ? (sub >> 3) & 1 : (sh == 1 ? q & 1 : q >> 1);
+            code |= hb ? v1[a] : v0[a];
+            ok = ok && (hb ? ok1[a] : ok0[a]);
+        }
         r[q] = make_uint2(0u, 0u);
-        uint32_t g[3];
-        const int e = q * BOX_LANES + sub;
-        if (e < bc.count() && bc.cell(e, g) && g[0] < grid_dim && g[1] < grid_dim && g[2] < grid_dim)
-            r[q] = cells[dmorton3(g[0], g[1], g[2])];
+        if (ok) r[q] = cells[code];
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
