@@ -266,7 +266,9 @@ int upf_upload_bodies(upf_sim* s, int n_bodies, const upf_body* bodies,
                       const int* body_id, const float* rel4);
 
 /* One or more full time steps of `method` (UPF_*), equivalent to calling the
- * reference's per-frame driver nsteps times.                              */
+ * reference's per-frame driver nsteps times.  A step that fails ends the
+ * call with its code; a WCSPH or SPH step's failure is seen when the next
+ * step has been enqueued, which then runs as well.                         */
 int upf_step(upf_sim* s, int nsteps, int method);
 
 /* CopyParticlesCUDA (src/gpu/particles.cu:62-72) in upload (id) order.  Any
