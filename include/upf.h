@@ -267,8 +267,9 @@ int upf_upload_bodies(upf_sim* s, int n_bodies, const upf_body* bodies,
 
 /* One or more full time steps of `method` (UPF_*), equivalent to calling the
  * reference's per-frame driver nsteps times.  A step that fails ends the
- * call with its code; a WCSPH or SPH step's failure is seen when the next
- * step has been enqueued, which then runs as well.                         */
+ * call with its code, and the state is that step's.  A particle that a
+ * PCISPH or coupling step's integration carries out of the z-index grid is
+ * found by the next step, or at the end of the call.                       */
 int upf_step(upf_sim* s, int nsteps, int method);
 
 /* CopyParticlesCUDA (src/gpu/particles.cu:62-72) in upload (id) order.  Any

@@ -161,3 +161,113 @@ def test_set_params_keeps_the_domain(gpu):
     q = p.copy()
     q.dt = 0.0008
     sim.set_params(q)
+
+
+def _same_state(a, b):
+    return all(np.array_equal(a[k], b[k], equal_nan=a[k].dtype.kind == "f") for k in a)
+
+
+def _everything(sim):
+    keys, ids, cells = sim.sorted_state()
+    return dict(sim.state(), K=np.array(sim.stats()[0]), keys=keys, ids=ids, cells=cells)
+
+
+def _leaves_the_grid(p, pos, typ, speed):
+    """The scene with a liquid particle that its integration carries past the top of the z-index grid."""
+    p.collision_max[1] = p.vbox_max[1] * 1.5
+    x = np.float32([[0.5 * (p.collision_min[0] + p.collision_max[0]), p.vbox_max[1] - p.support_radius - 0.001,
+                     0.5 * (p.collision_min[2] + p.collision_max[2]), 0.0]])
+    pos, typ = np.vstack([pos, x]), np.r_[typ, np.int32(upf.UPF_LIQUID)].astype(np.int32)
+    vel = np.zeros_like(pos)
+    vel[-1, 1] = speed
+    return pos, typ, vel
+
+
+@pytest.mark.parametrize("n", [8, 30])  # 16 and 4 lanes per particle
+@pytest.mark.parametrize("method", [upf.UPF_WCSPH_STATIC, upf.UPF_SPH_STATIC, upf.UPF_PCISPH_STATIC])
+def test_failed_step_ends_a_call_of_several(gpu, method, n):
+    """A call of six steps whose second fails (a particle leaves the grid in its integration): WCSPH and SPH end
+    with the state of that step, PCISPH with that of the next, whose sort finds it -- as one call per step does."""
+    p, pos, typ, nf = scenes.dam_break(n)
+    # past the top (0.021 m up) in the second step
+    pos, typ, vel = _leaves_the_grid(p, pos, typ, 0.7 * (p.support_radius + 0.001) / p.dt)
+    print("failed step: method %d, %d particles" % (method, len(typ)), flush=True)
+    runs = []
+    for calls in ((6,), (1, 1) if method != upf.UPF_PCISPH_STATIC else (1, 1, 1)):
+        sim = upf.Simulation(p, len(typ))
+        sim.upload(pos, typ, vel)
+        code = []
+        for steps in calls:
+            try:
+                sim.step(steps, method)
+                code.append(0)
+            except upf.UPFError as e:
+                code.append(e.code)
+        assert code[-1] == upf._abi.UPF_ERR_RANGE, code
+        runs.append(_everything(sim))
+        sim.close()
+    assert len(runs[0]["K"]) == len(runs[1]["K"]) and _same_state(*runs)
+
+
+def _overflowing(n, rigid=False):
+    if rigid:
+        p, pos, typ, bid, rel, bodies, _ = upf.standard_rigid_scene(n, n, 2 * n, 4)
+        return p, pos, typ, (bodies, bid, rel)
+    p = upf.make_params(0.01, 0.001)
+    pos, typ, nf = upf.dam_break(p, n, n, n, (0.02 * n, 0.01 * n, 0.01 * n), lattice_rel=0.95)
+    upf.density_error_factor(p)
+    return p, pos, typ, None
+
+
+@pytest.mark.parametrize("n,rigid", [(10, False), (32, False), (12, True)])
+def test_nan_of_the_last_force_pass_ends_the_step(gpu, n, rigid):
+    """Pressures beyond the floats give NaN forces in the one iteration of a step: the call of five steps ends
+    with that step, every time."""
+    method = upf.UPF_PCISPH_RIGID if rigid else upf.UPF_PCISPH_STATIC
+    p, pos, typ, bodies = _overflowing(n, rigid)
+    print("nan in the last pass: %d particles, rigid %d" % (len(typ), rigid), flush=True)
+    runs = []
+    for steps in (1, 5, 5):
+        sim = upf.Simulation(p, len(typ))
+        sim.upload(pos, typ)
+        if rigid:
+            sim.upload_bodies(*bodies)
+        sim.step(2, method)
+        q = p.copy()
+        q.min_loops = q.max_loops = 1
+        q.density_error_factor = 3e38
+        sim.set_params(q)
+        with pytest.raises(upf.UPFError) as e:
+            sim.step(steps, method)
+        assert e.value.code == upf._abi.UPF_ERR_NAN
+        runs.append(_everything(sim))
+        sim.close()
+    assert len(runs[0]["K"]) == 3
+    assert _same_state(runs[0], runs[1]) and _same_state(runs[0], runs[2])
+
+
+@pytest.mark.parametrize("n", [10, 32])
+def test_nan_ends_the_loop_after_the_enqueued_iterations(gpu, n):
+    """Pressures that overflow after some iterations: the loop ends behind the enqueued ones, whose number is the
+    tuning's (three, then `speculate` at a time)."""
+    p, pos, typ, _ = _overflowing(n)
+    p.min_loops, p.max_loops = 3, 50
+    p.density_error_factor = 4e32
+    K = {}
+    for spec in (1, 4, 4, 8):
+        sim = upf.Simulation(p, len(typ))
+        t = sim.tuning()
+        t.speculate = spec
+        sim.set_tuning(t)
+        sim.upload(pos, typ)
+        with pytest.raises(upf.UPFError) as e:
+            sim.step(1, upf.UPF_PCISPH_STATIC)
+        assert e.value.code == upf._abi.UPF_ERR_NAN
+        k = int(sim.stats()[0][0])
+        assert K.setdefault(spec, k) == k
+        sim.close()
+    print("iterations wanted when the loop ended: %s" % K, flush=True)
+    done = K[1] - 1  # iterations run when the NaN was found: the loop wanted one more
+    assert 3 < done < 50
+    for spec in (4, 8):
+        assert K[spec] == min(3 + -(-(done - 3) // spec) * spec, 50) + 1

@@ -28,7 +28,7 @@ struct Ctl {              // whole simulation
     int want_any;        // largest number of iterations any scene's loop must run
     uint32_t err;        // bit (1 << UPF_ERR_*) set on failures
     uint32_t step;       // steps recorded in the per-scene statistics
-    uint32_t pad;
+    uint32_t late;       // the same of the last integration; in err from the next sort on
 };
 
 struct SceneCtl {         // one scene's PCISPH loop
@@ -53,6 +53,7 @@ struct Dom {
 struct Slots {
     float4* pos;        // xyz, w = particle type (int bits)
     float4* vel;
+    uint32_t* key;      // z-index key that the slot was sorted by
     int* id;            // upload index
     float* p_last;      // correction pressure at the end of the previous step's loop
     float* p_prev;      // the one before (previous_correction_pressure_ of the CPU path)
@@ -65,7 +66,6 @@ struct Slots {
 
 struct Work {           // per-step arrays, slot order
     uint32_t* keys;     // keys of the slot order before sorting (written by integration)
-    uint32_t* keys_sorted;
     uint32_t* perm;     // sorted slot -> previous slot
     float4* force;      // external force, after integration force + pressure force
     float4* fp;         // correction pressure force

@@ -86,6 +86,8 @@ __device__ inline int ptype(const float4& x) { return __float_as_int(x.w); }
 __device__ __forceinline__ uint64_t wballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
 
 __device__ inline void set_err(Ctl* ctl, int code) { atomicOr(&ctl->err, 1u << code); }
+// a failure of the step's integration (Ctl::late)
+__device__ inline void set_late_err(Ctl* ctl, int code) { atomicOr(&ctl->late, 1u << code); }
 
 struct StepArgs {
     upf_params P;        // physics shared by all scenes
@@ -167,7 +169,8 @@ struct CtlMirror {
     Ctl ctl;
     SceneCtl scene0;
     uint32_t seq;
-    uint32_t pad[3];
+    uint32_t pad;
+    uint64_t fail;  // failures << 32 | sequence number
 };
 struct Publish {
     CtlMirror* m;  // null: nothing to publish
@@ -181,9 +184,15 @@ __device__ inline void publish(const Publish& pub, const Ctl& ctl, const SceneCt
     *(volatile uint32_t*)&pub.m->seq = pub.seq;
 }
 
-// Start of a step (block 0 of the kernel that moves the state): the errors so
-// far for the host, if it asked for them, and every scene's correction loop runs
-// iteration 0 (the CPU loop starts with density_error_too_large_ = true) unless
+// Failures alone, in one store: nothing waits for it (the fence above takes as
+// long as a small kernel).
+__device__ inline void publish_failures(const Publish& pub, uint32_t err) {
+    *(volatile uint64_t*)&pub.m->fail = (uint64_t)err << 32 | pub.seq;
+}
+
+// Start of a step (block 0 of the kernel that moves the state): the failures of
+// the step before, its integration's among them, for the host, if it asked for
+// them, and every scene's correction loop runs iteration 0 (the CPU loop starts with density_error_too_large_ = true) unless
 // its limits are zero.  As a kernel of its own this took 4 us a step.
 struct StepBegin {
     SceneCtl* sctl;
@@ -195,10 +204,16 @@ struct StepBegin {
 };
 __device__ inline void begin_step(const StepBegin& B) {
     if (blockIdx.x != 0) return;
-    if (threadIdx.x == 0 && B.pub.m) publish(B.pub, *B.ctl, B.sctl[0]);
+    if (threadIdx.x == 0) {
+        Ctl c = *B.ctl;
+        c.err |= c.late;
+        c.late = 0u;
+        if (B.pub.m) publish_failures(B.pub, c.err);
+        c.want_any = B.want;
+        *B.ctl = c;
+    }
     for (int sc = threadIdx.x; sc < B.n_scenes; sc += blockDim.x) B.sctl[sc] = SceneCtl{B.want, 1, 0.0f, 0};
     if (threadIdx.x == 0) {
-        B.ctl->want_any = B.want;
         if (B.act_n) B.act_n[0] = -B.n_chunks;  // iteration 0: every chunk
     }
 }
@@ -268,8 +283,7 @@ template <bool RIGID>
 __global__ __launch_bounds__(BLOCK) void k_rank_gather(int n, CellMap map, const uint64_t* __restrict__ place,
                                                        const uint2* __restrict__ cells, Slots src, Slots dst,
                                                        const float* __restrict__ p_work,
-                                                       const float* __restrict__ rho_work,
-                                                       uint32_t* __restrict__ keys_sorted, StepBegin begin) {
+                                                       const float* __restrict__ rho_work, StepBegin begin) {
     begin_step(begin);
     const int t = blockIdx.x * BLOCK + threadIdx.x;
     if (t >= n) return;
@@ -278,7 +292,7 @@ __global__ __launch_bounds__(BLOCK) void k_rank_gather(int n, CellMap map, const
     const uint2 r = cells[map(key, t)];
     const int s = move_slot<RIGID>(src, dst, (int)(uint32_t)v, p_work, rho_work,
                                    [&] { return (int)bin_slot(place, v, r); });
-    keys_sorted[s] = key;
+    dst.key[s] = key;
 }
 
 // ------------------------------------------------------------ cell table
@@ -1640,7 +1654,7 @@ __global__ __launch_bounds__(64) void k_nbr_build_ext(StepArgs A, Slots S, Work 
     // the build's candidate table, then the tables of the force pass
     __shared__ float4 tabs[LUT_N];
     static_assert(4 * LUT_N >= CAND_CAP, "candidate table");
-    build_wave<ROUNDS, 0, 0, SKIP, 0, UPF_LIQUID, SLOT_MAJOR, SPLIT>(A, S.pos, W.keys_sorted, W.cells, W.nbr, W.ncount, ctl,
+    build_wave<ROUNDS, 0, 0, SKIP, 0, UPF_LIQUID, SLOT_MAJOR, SPLIT>(A, S.pos, S.key, W.cells, W.nbr, W.ncount, ctl,
                                                              reinterpret_cast<uint32_t*>(tabs));
     // the block is the wave: its lists (written by all its lanes) are complete
     // and visible to every lane after the barrier, and so are the tables
@@ -1682,6 +1696,19 @@ __device__ inline int stage_union(const StepArgs& A, const Work& W, const float4
     return un;
 }
 
+// The host enqueues further iterations (gate: the first of them) while the last
+// force pass before them still runs.  A NaN found by then ends the loop instead:
+// the first density pass publishes it in the decision's place and makes every
+// later pass return at once.
+__device__ inline bool stopped_by_nan(const Publish& gate, const StepArgs& A, int t, Ctl* ctl) {
+    if (!gate.m || !(__atomic_load_n(&ctl->err, __ATOMIC_RELAXED) & (1u << UPF_ERR_NAN))) return false;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        publish(gate, *ctl, A.sctl[0]);
+        __atomic_store_n(&ctl->want_any, t, __ATOMIC_RELAXED);
+    }
+    return true;
+}
+
 // ComputePredictedDensityAndPressure (:5456-5491) + the max reduction of the
 // predicted density per scene: maxima fold into a few padded slots per scene
 // (atomics spread over cache lines).  Persistent grid-stride kernel; iteration
@@ -1689,9 +1716,9 @@ __device__ inline int stage_union(const StepArgs& A, const Work& W, const float4
 // when no scene runs iteration t.
 template <int MODE, int CODED, int G>
 __global__ __launch_bounds__(BLOCK) void k_density(int t, StepArgs A, Slots S, Work W, const float* __restrict__ luts,
-                                                   Ctl* ctl) {
+                                                   Ctl* ctl, Publish gate) {
     static_assert(!(MODE == UPF_BOUNDARY_AKINCI && CODED == 2), "the Akinci density reads boundary volumes by slot");
-    if (t >= __atomic_load_n(&ctl->want_any, __ATOMIC_RELAXED)) return;
+    if (t >= __atomic_load_n(&ctl->want_any, __ATOMIC_RELAXED) || stopped_by_nan(gate, A, t, ctl)) return;
     __shared__ float lw[LUT_N];
     __shared__ float2 th[LUT_N];
     __shared__ float wmax[BLOCK / 64];  // blockDim.x <= BLOCK
@@ -1866,7 +1893,8 @@ __global__ __launch_bounds__(BLOCK) void k_density(int t, StepArgs A, Slots S, W
 // number also raises ctl->want_any.  Every scene's count only grows during a
 // step, so want_any needs no reset between iterations.  With pub (one scene) the
 // host learns the decision from here, while the force pass of the iteration runs
-// on: it enqueues the rest of the step meanwhile.  (Read back after that pass by
+// on: it enqueues the rest of the step meanwhile.  Failures are published later,
+// when the pass is over (stopped_by_nan, k_integrate).  (Read back after that pass by
 // a kernel of its own, and the loop started by another, a step of 80,648
 // particles took 198 us, now 184; of 3,080 83 and 78.)
 __device__ inline void loop_test(const StepArgs& A, int sc, int t, int lane, Ctl* ctl, const Publish& pub) {
@@ -1894,8 +1922,7 @@ __device__ inline void loop_test(const StepArgs& A, int sc, int t, int lane, Ctl
         C.want = want;
         atomicMax(&ctl->want_any, want);
         if (pub.m && (!next || pub.last)) {
-            const uint32_t err = __atomic_load_n(&ctl->err, __ATOMIC_RELAXED);
-            publish(pub, Ctl{want, err, ctl->step, 0u}, SceneCtl{want, too_large, mx, 0});
+            publish(pub, Ctl{want, 0u, ctl->step, 0u}, SceneCtl{want, too_large, mx, 0});
         }
     }
     // batched: a scene that runs iteration t + 1 puts its chunks on that
@@ -2082,7 +2109,7 @@ __device__ __forceinline__ void load_tables(const float* __restrict__ luts, floa
 // and 7.8 at 80,648).
 template <int MODE, int LANES>
 __global__ __launch_bounds__(BLOCK) void k_density_lanes(int t, StepArgs A, Work W, const float* __restrict__ luts,
-                                                         Ctl* ctl) {
+                                                         Ctl* ctl, Publish gate) {
     // whether the iteration runs: tested after the tables, on its way with all else
     const int want = __atomic_load_n(&ctl->want_any, __ATOMIC_RELAXED);
     __shared__ float lw[LUT_N];
@@ -2101,7 +2128,7 @@ __global__ __launch_bounds__(BLOCK) void k_density_lanes(int t, StepArgs A, Work
     const RowHead head = row_head<LANES>(row, A.nbr_ld, W.ncount + at, sub);
     load_tables(luts, lw, 0, th);  // (entry 300, dist >= h, is 0 in every table)
     __syncthreads();
-    if (t >= want) return;
+    if (t >= want || stopped_by_nan(gate, A, t, ctl)) return;
     float mine = 0.0f;
     if (in && ptype(xi) == UPF_LIQUID) {
         const float m = P.initial_mass;
@@ -2185,9 +2212,12 @@ __global__ __launch_bounds__(BLOCK) void k_force_lanes(int t, StepArgs A, Slots 
 // ------------------------------------------------------------ integration
 // UpdateLiquidParticlePosVelSphCPU (:3705-3742) + BoundaryHandlingBoxPerParticleOMP
 // (:3940-3970) / BoundaryHandlingPureFluidOMP (:3972-3998): symplectic Euler,
-// box clamp with damping -0.5, new z-index key of every particle.
-__global__ void k_integrate(StepArgs A, Slots S, Work W, int pcisph, int pure_fluid_clamp, int has_bodies, Ctl* ctl) {
+// box clamp with damping -0.5, new z-index key of every particle.  pub: the
+// failures of the passes before it, which this kernel's own do not join.
+__global__ void k_integrate(StepArgs A, Slots S, Work W, int pcisph, int pure_fluid_clamp, int has_bodies, Ctl* ctl,
+                            Publish pub) {
     const upf_params& P = A.P;
+    if (pub.m && blockIdx.x == 0 && threadIdx.x == 0) publish_failures(pub, ctl->err);
     for (int i = xblk(A.xcd) * blockDim.x + threadIdx.x; i < A.n; i += gstride()) {
     float4 x = S.pos[i];
     const int ti = ptype(x);
@@ -2195,7 +2225,7 @@ __global__ void k_integrate(StepArgs A, Slots S, Work W, int pcisph, int pure_fl
     if (ti == UPF_FROZEN) {
         bool ok;
         W.keys[i] = dkey(x.x, x.y, x.z, d.scales, ok);
-        if (!ok) set_err(ctl, UPF_ERR_RANGE);
+        if (!ok) set_late_err(ctl, UPF_ERR_RANGE);
         continue;
     }
     float4 v = S.vel[i];
@@ -2231,7 +2261,7 @@ __global__ void k_integrate(StepArgs A, Slots S, Work W, int pcisph, int pure_fl
     }
     bool ok;
     W.keys[i] = dkey(x.x, x.y, x.z, d.scales, ok);
-    if (!ok) set_err(ctl, UPF_ERR_RANGE);
+    if (!ok) set_late_err(ctl, UPF_ERR_RANGE);
     }
 }
 
@@ -2362,7 +2392,7 @@ __global__ __launch_bounds__(64) void k_nbr_build_wcsph(StepArgs A, Slots S, Wor
     // the build's candidate table, then the density table and the bin thresholds
     __shared__ float2 tabs[2 * LUT_N];
     static_assert(4 * LUT_N >= CAND_CAP, "candidate table");
-    build_wave<ROUNDS, 0, 0, 0, 0, UPF_LIQUID, true, SPLIT>(A, S.pos, W.keys_sorted, W.cells, W.nbr, W.ncount, ctl,
+    build_wave<ROUNDS, 0, 0, 0, 0, UPF_LIQUID, true, SPLIT>(A, S.pos, S.key, W.cells, W.nbr, W.ncount, ctl,
                                                     reinterpret_cast<uint32_t*>(tabs));
     __syncthreads();  // the block is the wave: its lists are complete
     float2* th = tabs;
@@ -2803,7 +2833,7 @@ __global__ __launch_bounds__(64) void k_nbr_build_coupling(StepArgs A, Slots S, 
     // the build's candidate table, then the tables of the coupling pass
     __shared__ float tabs[4 * LUT_N];
     static_assert(4 * LUT_N >= CAND_CAP, "candidate table");
-    build_wave<ROUNDS, 0, 1, 0, 1, UPF_LIQUID, SLOT_MAJOR, SPLIT>(A, S.pos, W.keys_sorted, W.cells, W.nbr, W.ncount, ctl,
+    build_wave<ROUNDS, 0, 1, 0, 1, UPF_LIQUID, SLOT_MAJOR, SPLIT>(A, S.pos, S.key, W.cells, W.nbr, W.ncount, ctl,
                                                           reinterpret_cast<uint32_t*>(tabs));
     __syncthreads();  // the block is the wave: its lists are complete
     float* lvl = tabs;
@@ -3377,6 +3407,7 @@ static void with_split(int split, F f) {
 static int alloc_slots(upf_sim* s, Slots& S, int cap) {
     HIPCHK(s->alloc(&S.pos, cap));
     HIPCHK(s->alloc(&S.vel, cap));
+    HIPCHK(s->alloc(&S.key, cap));
     HIPCHK(s->alloc(&S.id, cap));
     HIPCHK(s->alloc(&S.p_last, cap));
     HIPCHK(s->alloc(&S.p_prev, cap));
@@ -3386,6 +3417,16 @@ static int alloc_slots(upf_sim* s, Slots& S, int cap) {
     HIPCHK(s->alloc(&S.body, cap));
     HIPCHK(s->alloc(&S.rel, cap));
     return UPF_OK;
+}
+
+// The cell table of the current slots.
+static void cell_table(upf_sim* s) {
+    s->prof.begin(PC_CELLS, s->st);
+    hipLaunchKernelGGL(k_fill_cells, dim3((s->ncells + BLOCK - 1) / BLOCK), dim3(BLOCK), 0, s->st, s->W.cells, s->ncells);
+    s->prof.end(s->st);
+    s->prof.begin(PC_CELLS, s->st);
+    hipLaunchKernelGGL(k_cell_bounds, grid_for(s->n), dim3(BLOCK), 0, s->st, s->args(), s->S[s->cur].key, s->W.cells);
+    s->prof.end(s->st);
 }
 
 // sort + gather + cell table (the first part of every step)
@@ -3403,14 +3444,14 @@ static int sort_and_bin(upf_sim* s, const Publish& pub = Publish{}) {
         s->prof.end(s->st);
         s->prof.begin(PC_GATHER, s->st);
         hipLaunchKernelGGL(s->rigid ? k_rank_gather<true> : k_rank_gather<false>, grid_for(n), dim3(BLOCK), 0, s->st, n,
-                           map, s->bins.place, W.cells, s->S[s->cur], s->S[nxt], W.p, W.rho, W.keys_sorted, begin);
+                           map, s->bins.place, W.cells, s->S[s->cur], s->S[nxt], W.p, W.rho, begin);
         s->prof.end(s->st);
         s->cur = nxt;
         HIPCHK(hipGetLastError());
         return UPF_OK;
     }
     if (s->n_scenes == 1) {
-        HIPCHK(radix_sort(W.keys, nullptr, W.keys_sorted, W.perm, n, 30, s->sort_tmp, s->st));
+        HIPCHK(radix_sort(W.keys, nullptr, s->S[nxt].key, W.perm, n, 30, s->sort_tmp, s->st));
     } else {
         // stable sort by (scene, key): keys first, then the scene as the most
         // significant digit; scenes keep their slot ranges
@@ -3418,7 +3459,7 @@ static int sort_and_bin(upf_sim* s, const Publish& pub = Publish{}) {
         hipLaunchKernelGGL(k_scene_keys, grid_for(n), dim3(BLOCK), 0, s->st, n, s->b_perm1, s->d_scene_of, s->b_sk);
         const int sbits = s->n_scenes <= 256 ? 8 : 16;
         HIPCHK(radix_sort(s->b_sk, s->b_perm1, s->b_sk2, W.perm, n, sbits, s->sort_tmp, s->st));
-        hipLaunchKernelGGL(k_gather_keys, grid_for(n), dim3(BLOCK), 0, s->st, n, W.perm, W.keys, W.keys_sorted);
+        hipLaunchKernelGGL(k_gather_keys, grid_for(n), dim3(BLOCK), 0, s->st, n, W.perm, W.keys, s->S[nxt].key);
     }
     s->prof.end(s->st);
     s->prof.begin(PC_GATHER, s->st);
@@ -3426,49 +3467,19 @@ static int sort_and_bin(upf_sim* s, const Publish& pub = Publish{}) {
                        s->S[s->cur], s->S[nxt], W.p, W.rho, begin);
     s->prof.end(s->st);
     s->cur = nxt;
-    s->prof.begin(PC_CELLS, s->st);
-    hipLaunchKernelGGL(k_fill_cells, dim3((s->ncells + BLOCK - 1) / BLOCK), dim3(BLOCK), 0, s->st, W.cells, s->ncells);
-    s->prof.end(s->st);
-    s->prof.begin(PC_CELLS, s->st);
-    hipLaunchKernelGGL(k_cell_bounds, grid_for(n), dim3(BLOCK), 0, s->st, s->args(), W.keys_sorted, W.cells);
-    s->prof.end(s->st);
+    cell_table(s);
     HIPCHK(hipGetLastError());
     return UPF_OK;
 }
 
-// Where the device publishes its loop state next (two places in turn).
-static Publish next_publish(upf_sim* s, int last) {
-    ++s->mirror_seq;
-    return Publish{s->mirror_dev + (s->mirror_seq & 1u), s->mirror_seq, last};
-}
-// Waits for the state published under the last sequence number: the host spins
-// on it (a blocking stream synchronisation wakes the host up later than the GPU
-// finishes, and the GPU idles meanwhile).
-static int wait_published(upf_sim* s) {
-    const uint32_t seq = s->mirror_seq;
-    const CtlMirror* m = s->mirror + (seq & 1u);
-    const volatile uint32_t* flag = &m->seq;
-    for (uint64_t spins = 1; *flag != seq; ++spins) {
-        if ((spins & 4095u) == 0) {
-            const hipError_t e = hipStreamQuery(s->st);
-            if (e == hipSuccess) {
-                if (*flag == seq) break;
-                return UPF_ERR_HIP;  // the stream drained without the mirror update
-            }
-            if (e != hipErrorNotReady) return UPF_ERR_HIP;
-        }
-    }
-    std::atomic_thread_fence(std::memory_order_acquire);
-    *s->h_ctl = m->ctl;
-    *s->h_sctl = m->scene0;
-    s->prof.collect();
-    return UPF_OK;
-}
-// The loop state after all work enqueued so far.
-static int read_ctl(upf_sim* s) {
-    hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, s->st, s->ctl, s->sctl, next_publish(s, 1));
+// Takes back the sort_and_bin that was enqueued behind a step which failed: the
+// state from before it is untouched in the other buffer.
+static int unsort(upf_sim* s) {
+    s->cur = 1 - s->cur;
+    cell_table(s);
     HIPCHK(hipGetLastError());
-    return wait_published(s);
+    HIPCHK(hipStreamSynchronize(s->st));
+    return UPF_OK;
 }
 
 static int err_code(uint32_t bits) {
@@ -3478,8 +3489,59 @@ static int err_code(uint32_t bits) {
     return UPF_OK;
 }
 
+// Where the device publishes its loop state or the failures next (two places in turn).
+static Publish next_publish(upf_sim* s, int last) {
+    ++s->mirror_seq;
+    return Publish{s->mirror_dev + (s->mirror_seq & 1u), s->mirror_seq, last};
+}
+// Waits until there(): the host spins on it (a blocking stream synchronisation
+// wakes the host up later than the GPU finishes, and the GPU idles meanwhile).
+template <class There>
+static int spin(upf_sim* s, There there) {
+    for (uint64_t spins = 1; !there(); ++spins) {
+        if ((spins & 4095u) == 0) {
+            const hipError_t e = hipStreamQuery(s->st);
+            if (e == hipSuccess) {
+                if (there()) break;
+                return UPF_ERR_HIP;  // the stream drained without the mirror update
+            }
+            if (e != hipErrorNotReady) return UPF_ERR_HIP;
+        }
+    }
+    std::atomic_thread_fence(std::memory_order_acquire);
+    return UPF_OK;
+}
+// Waits for the state published under the last sequence number.
+static int wait_published(upf_sim* s) {
+    const uint32_t seq = s->mirror_seq;
+    const CtlMirror* m = s->mirror + (seq & 1u);
+    const int rc = spin(s, [&] { return *(const volatile uint32_t*)&m->seq == seq; });
+    if (rc) return rc;
+    *s->h_ctl = m->ctl;
+    *s->h_sctl = m->scene0;
+    s->prof.collect();
+    return UPF_OK;
+}
+// Waits for the failures published under it: their code.
+static int wait_failures(upf_sim* s, int* code) {
+    const uint32_t seq = s->mirror_seq;
+    const CtlMirror* m = s->mirror + (seq & 1u);
+    uint64_t v = 0;
+    const int rc = spin(s, [&] { return (uint32_t)(v = *(const volatile uint64_t*)&m->fail) == seq; });
+    if (rc) return rc;
+    *code = err_code((uint32_t)(v >> 32));
+    return UPF_OK;
+}
+// The loop state after all work enqueued so far.
+static int read_ctl(upf_sim* s) {
+    hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, s->st, s->ctl, s->sctl, next_publish(s, 1));
+    HIPCHK(hipGetLastError());
+    return wait_published(s);
+}
+
 template <int MODE>
-static void enqueue_iteration(upf_sim* s, const StepArgs& A, int t, const Publish& pub = Publish{}) {
+static void enqueue_iteration(upf_sim* s, const StepArgs& A, int t, const Publish& pub = Publish{},
+                              const Publish& gate = Publish{}) {
     const dim3 g = grid_persist(s, s->n), b = block_loop(s);
     Slots& S = s->S[s->cur];
     const int lw = s->tune.loop_width, ll = s->tune.loop_list;
@@ -3492,14 +3554,14 @@ static void enqueue_iteration(upf_sim* s, const StepArgs& A, int t, const Publis
         else
             hipLaunchKernelGGL(kernel, grid, block, 0, s->st, t, A, args...);
     };
-#define UPF_DENSITY(...) pass(PC_DENSITY, g, b, __VA_ARGS__, S, s->W, s->luts, s->ctl)
+#define UPF_DENSITY(...) pass(PC_DENSITY, g, b, __VA_ARGS__, S, s->W, s->luts, s->ctl, gate)
 #define UPF_FORCE(...) pass(PC_FORCE, g, b, __VA_ARGS__, S, s->W, s->luts, s->ctl, pub)
     if (s->lanes) {
         with_split(s->lanes, [&](auto lanes) {
             constexpr int L = decltype(lanes)::value;
             if constexpr (L > 1) {
                 const dim3 gl = lanes_grid(s->n, L), bl(BLOCK);
-                pass(PC_DENSITY, gl, bl, k_density_lanes<MODE, L>, s->W, s->luts, s->ctl);
+                pass(PC_DENSITY, gl, bl, k_density_lanes<MODE, L>, s->W, s->luts, s->ctl, gate);
                 pass(PC_FORCE, gl, bl, k_force_lanes<MODE, L>, S, s->W, s->luts, s->ctl, pub);
             }
         });
@@ -3531,7 +3593,8 @@ static void enqueue_iteration(upf_sim* s, const StepArgs& A, int t, const Publis
 // PredictionCorrectionStep (:5367-5424).  The loop test runs on the device;
 // the host enqueues iterations ahead (as many as the previous step needed)
 // and reads the decision back once the enqueued ones are done.  Iterations
-// beyond the device's decision return at their first instruction.
+// beyond the device's decision return at their first instruction.  A NaN in the
+// enqueued ones ends a loop that would go on.
 template <int MODE>
 static int pcisph_loop(upf_sim* s, const StepArgs& A) {
     const int maxl = std::max(s->P.max_loops, 1);
@@ -3549,9 +3612,11 @@ static int pcisph_loop(upf_sim* s, const StepArgs& A) {
     int t = 0;
     auto enqueue = [&](int stop) {
         Publish pub = own ? next_publish(s, 0) : Publish{};
+        Publish gate = t > 0 ? pub : Publish{};
         for (; t < stop; ++t) {
             pub.last = t + 1 == stop;
-            enqueue_iteration<MODE>(s, A, t, pub);
+            enqueue_iteration<MODE>(s, A, t, pub, gate);
+            gate = Publish{};
         }
     };
     enqueue(ahead);
@@ -3581,7 +3646,7 @@ static void build_lists(upf_sim* s, const StepArgs& A) {
     s->prof.begin(PC_NBR_BUILD, s->st);
     const dim3 g((unsigned)(((s->n + 63) / 64 + 7) / 8 * 8));  // a multiple of 8 (XCD remap)
     auto launch = [&](auto kern) {
-        hipLaunchKernelGGL(kern, g, dim3(64), 0, s->st, A, S.pos, s->W.keys_sorted, s->W.cells, s->W.nbr, s->W.ncount,
+        hipLaunchKernelGGL(kern, g, dim3(64), 0, s->st, A, S.pos, S.key, s->W.cells, s->W.nbr, s->W.ncount,
                            s->ctl);
     };
     const int r = s->tune.nbr_rounds;
@@ -3617,14 +3682,12 @@ static void build_lists(upf_sim* s, const StepArgs& A) {
     s->prof.end(s->st);
 }
 
-// The parts of a static-boundary step: the head (sort, cell table, boundary
+// The parts of a static-boundary step after its sort: the head (boundary
 // volumes on the first step, lists, external forces and first prediction)
 // and the tail (integration, per-scene record).  The correction loop runs
 // between them; its iterations only touch the slot buffer the head sorted
 // into, so a batch captures head, loop chunks and tail as separate graphs.
 static int step_static_head(upf_sim* s) {
-    int rc = sort_and_bin(s);
-    if (rc) return rc;
     const StepArgs A = s->args();
     Slots& S = s->S[s->cur];
     const dim3 g = grid_for(s->n);
@@ -3702,12 +3765,12 @@ static void step_static_iterations(upf_sim* s, int t0, int t1) {
     }
 }
 
-static int step_static_tail(upf_sim* s) {
+static int step_static_tail(upf_sim* s, const Publish& pub = Publish{}) {
     const StepArgs A = s->args();
     Slots& S = s->S[s->cur];
     s->prof.begin(PC_INTEGRATE, s->st);
     hipLaunchKernelGGL(k_integrate, grid_persist(s, s->n), block_loop(s), 0, s->st, A, S, s->W, 1, 0,
-                       s->rigid ? 1 : 0, s->ctl);
+                       s->rigid ? 1 : 0, s->ctl, pub);
     s->prof.end(s->st);
     if (s->d_kstat)
         hipLaunchKernelGGL(k_record, dim3(1), dim3(256), 0, s->st, A, s->ctl, s->d_kstat, s->d_rstat, s->stat_cap);
@@ -3717,7 +3780,8 @@ static int step_static_tail(upf_sim* s) {
 
 // CpuParticlePhysicsStaticBoundariesPCISPH (src/cpu/UnifiedPhysics.cpp:4220-4238).
 // device_loop: the loop decision stays on the device and every iteration up
-// to max_loops is enqueued; otherwise the host reads the decision back.
+// to max_loops is enqueued; otherwise the host reads the decision back, and the
+// integration publishes the failures before it.
 static int step_pcisph_static(upf_sim* s, bool device_loop) {
     int rc = step_static_head(s);
     if (rc) return rc;
@@ -3730,13 +3794,11 @@ static int step_pcisph_static(upf_sim* s, bool device_loop) {
         rc = akinci ? pcisph_loop<UPF_BOUNDARY_AKINCI>(s, A) : pcisph_loop<UPF_BOUNDARY_CPU_REF>(s, A);
         if (rc) return rc;
     }
-    return step_static_tail(s);
+    return step_static_tail(s, device_loop ? Publish{} : next_publish(s, 1));
 }
 
 // CpuParticlePhysicsVersatileCouplingPCISPH (src/cpu/UnifiedPhysics.cpp:4991-5024)
 static int step_pcisph_rigid(upf_sim* s) {
-    int rc = sort_and_bin(s);
-    if (rc) return rc;
     s->union_ready = false;  // the coupling loop reads the delta-coded lists
     s->lanes = 0;
     const StepArgs A = s->args();
@@ -3752,7 +3814,7 @@ static int step_pcisph_rigid(upf_sim* s) {
         // RIGID_SPLIT waves per window of 64 slots, a multiple of 8 (XCD remap)
         const dim3 gb((unsigned)(((s->n + 63) / 64 * RIGID_SPLIT + 7) / 8 * 8));
         auto launch = [&](auto kern) {
-            hipLaunchKernelGGL(kern, gb, dim3(64), 0, s->st, A, S.pos, s->W.keys_sorted, s->W.cells, s->W.nbr,
+            hipLaunchKernelGGL(kern, gb, dim3(64), 0, s->st, A, S.pos, S.key, s->W.cells, s->W.nbr,
                                s->W.ncount, s->ctl);
         };
         const int r = s->tune.nbr_rounds;
@@ -3808,11 +3870,11 @@ static int step_pcisph_rigid(upf_sim* s) {
             hipLaunchKernelGGL(k_ext_coupling<UPF_BOUNDARY_CPU_REF>, g, dim3(BLOCK), 0, s->st, A, S, s->W, s->luts, s->ctl);
         s->prof.end(s->st);
     }
-    rc = s->P.boundary_pressure_mode == UPF_BOUNDARY_AKINCI ? pcisph_loop<UPF_BOUNDARY_AKINCI>(s, A)
-                                                            : pcisph_loop<UPF_BOUNDARY_CPU_REF>(s, A);
+    const int rc = akinci ? pcisph_loop<UPF_BOUNDARY_AKINCI>(s, A) : pcisph_loop<UPF_BOUNDARY_CPU_REF>(s, A);
     if (rc) return rc;
     s->prof.begin(PC_INTEGRATE, s->st);
-    hipLaunchKernelGGL(k_integrate, grid_persist(s, s->n), block_loop(s), 0, s->st, A, S, s->W, 1, 1, 1, s->ctl);
+    hipLaunchKernelGGL(k_integrate, grid_persist(s, s->n), block_loop(s), 0, s->st, A, S, s->W, 1, 1, 1, s->ctl,
+                       next_publish(s, 1));
     s->prof.end(s->st);
     // rigid bodies: members grouped by body in slot order, one thread per body
     s->prof.begin(PC_RIGID, s->st);
@@ -3836,10 +3898,7 @@ static int step_pcisph_rigid(upf_sim* s) {
 // The methods whose pressure is the state pressure W.pres (no correction loop).
 static inline bool sph_family(int method) { return method == UPF_WCSPH_STATIC || method == UPF_SPH_STATIC; }
 
-// pub: the errors of the steps before, published as this one starts
-static int step_wcsph_static(upf_sim* s, bool tait, const Publish& pub) {
-    int rc = sort_and_bin(s, pub);
-    if (rc) return rc;
+static int step_wcsph_static(upf_sim* s, bool tait) {
     const StepArgs A = s->args();
     Slots& S = s->S[s->cur];
     const dim3 g = grid_for(s->n);
@@ -3892,7 +3951,7 @@ static int step_wcsph_static(upf_sim* s, bool tait, const Publish& pub) {
     s->prof.end(s->st);
     s->prof.begin(PC_INTEGRATE, s->st);
     hipLaunchKernelGGL(k_integrate, grid_persist(s, s->n), block_loop(s), 0, s->st, A, S, s->W, 0, 0,
-                       s->rigid ? 1 : 0, s->ctl);
+                       s->rigid ? 1 : 0, s->ctl, Publish{});
     s->prof.end(s->st);
     HIPCHK(hipGetLastError());
     s->k_hist.push_back(0);
@@ -3950,7 +4009,6 @@ static int sim_alloc(upf_sim* s, int capacity, uint32_t ncells, int n_scenes) {
     Work& W = s->W;
     const size_t nslots = (size_t)n_scenes * s->sps * 32;
     HIPCHK(s->alloc(&W.keys, capacity));
-    HIPCHK(s->alloc(&W.keys_sorted, capacity));
     HIPCHK(s->alloc(&W.perm, capacity));
     HIPCHK(s->alloc(&W.force, capacity));
     HIPCHK(s->alloc(&W.fp, capacity));
@@ -4168,30 +4226,36 @@ int upf_step(upf_sim* s, int nsteps, int method) {
     if (!s->uploaded) return UPF_ERR_STATE;
     if (method == UPF_PCISPH_RIGID && !s->rigid) return UPF_ERR_STATE;
     if (method == UPF_PCISPH_RIGID && s->P.add_wall_weight) return UPF_ERR_ARG;
+    const bool sph = sph_family(method);
+    if (nsteps > 0 && !sph && method != UPF_PCISPH_STATIC && method != UPF_PCISPH_RIGID) return UPF_ERR_ARG;
     for (int k = 0; k < nsteps; ++k) {
-        int rc;
-        if (method == UPF_PCISPH_STATIC) rc = step_pcisph_static(s, false);
-        else if (sph_family(method)) {
-            // no decision to wait for: a step is enqueued while the one before
-            // runs, and that one's errors come from its start
-            const Publish pub = k > 0 ? next_publish(s, 1) : Publish{};
-            rc = step_wcsph_static(s, method == UPF_WCSPH_STATIC, pub);
-            if (!rc && k > 0) rc = wait_published(s);
-        } else if (method == UPF_PCISPH_RIGID) rc = step_pcisph_rigid(s);
-        else return UPF_ERR_ARG;
+        // The sort is enqueued while the step before still runs, then the host
+        // waits for that step's failures: a WCSPH or SPH step's come from the
+        // start of this one's gather, a PCISPH step's (without its integration's,
+        // which the next step reports) from its integration.  After a failure the
+        // sort is taken back: the call ends with the state of the step that failed.
+        int rc = sort_and_bin(s, k > 0 && sph ? next_publish(s, 1) : Publish{});
+        if (!rc && k > 0) {
+            int e = UPF_OK;
+            rc = wait_failures(s, &e);
+            if (e) {
+                rc = unsort(s);
+                return rc ? rc : e;
+            }
+        }
+        if (rc) return rc;
+        if (sph) rc = step_wcsph_static(s, method == UPF_WCSPH_STATIC);
+        else if (method == UPF_PCISPH_STATIC) rc = step_pcisph_static(s, false);
+        else rc = step_pcisph_rigid(s);
         s->last_method = method;
         if (rc) return rc;
-        if (k == 0 && sph_family(method)) continue;
-        const int e = err_code(s->h_ctl->err);
-        if (e) return e;
     }
     if (nsteps > 0) {
-        // the loop's decision comes before the last force pass and the
-        // integration (a WCSPH step's errors at the start of the next): the last
-        // step's errors are read once more here, so that this call reports them
+        // the last step's failures, its integration's too
         const int rc = read_ctl(s);
         if (rc) return rc;
-        return err_code(s->h_ctl->err);
+        const int e = sph ? UPF_OK : err_code(s->h_ctl->err);
+        return e ? e : err_code(s->h_ctl->err | s->h_ctl->late);
     }
     HIPCHK(hipStreamSynchronize(s->st));
     return UPF_OK;
@@ -4249,7 +4313,7 @@ int upf_sort_and_bin(upf_sim* s) {
     int rc = sort_and_bin(s);
     if (rc) return rc;
     // the state is now in key order: its keys are the sorted ones
-    HIPCHK(hipMemcpyAsync(s->W.keys, s->W.keys_sorted, (size_t)s->n * 4, hipMemcpyDeviceToDevice, s->st));
+    HIPCHK(hipMemcpyAsync(s->W.keys, s->S[s->cur].key, (size_t)s->n * 4, hipMemcpyDeviceToDevice, s->st));
     // loop arrays follow the new order too (identity gather for the next sort)
     Slots& S = s->S[s->cur];
     HIPCHK(hipMemcpyAsync(s->W.p, S.p_last, (size_t)s->n * 4, hipMemcpyDeviceToDevice, s->st));
@@ -4279,14 +4343,14 @@ int upf_download_neighbors(upf_sim* s, int* counts, int32_t* flat, int cap) {
     }
     Ctl h;
     if (hipMemcpy(&h, s->ctl, sizeof(Ctl), hipMemcpyDeviceToHost) != hipSuccess) return -UPF_ERR_HIP;
-    const int e = err_code(h.err);
+    const int e = err_code(h.err | h.late);
     return e ? -e : w;
 }
 
 int upf_download_sorted(upf_sim* s, uint32_t* keys, int32_t* ids, uint32_t* cells, int* n_cells) {
     if (!s) return UPF_ERR_ARG;
     const int n = s->n;
-    if (keys) HIPCHK(hipMemcpy(keys, s->W.keys_sorted, (size_t)n * 4, hipMemcpyDeviceToHost));
+    if (keys) HIPCHK(hipMemcpy(keys, s->S[s->cur].key, (size_t)n * 4, hipMemcpyDeviceToHost));
     if (ids) HIPCHK(hipMemcpy(ids, s->S[s->cur].id, (size_t)n * 4, hipMemcpyDeviceToHost));
     if (n_cells) {
         std::vector<uint2> t(s->ncells);
@@ -4564,7 +4628,8 @@ static int capture_step(upf_sim* s, int cur, hipGraphExec_t* out) {
     int rc = UPF_OK;
     if (hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal) != hipSuccess) rc = UPF_ERR_HIP;
     if (!rc) {
-        rc = step_pcisph_static(s, true);
+        rc = sort_and_bin(s);
+        if (!rc) rc = step_pcisph_static(s, true);
         const hipError_t e = hipStreamEndCapture(s->st, &g);
         if (!rc && e != hipSuccess) rc = UPF_ERR_HIP;
     }
@@ -4597,7 +4662,8 @@ static int capture_split(upf_batch* b) {
     for (int c = 0; c < 2 && !rc; ++c) {
         s->cur = c;
         rc = capture_graph(s, &b->head[c], [&] {
-            const int r = step_static_head(s);  // sorts into buffer 1 - c
+            int r = sort_and_bin(s);  // into buffer 1 - c
+            if (!r) r = step_static_head(s);
             if (r) return r;
             step_static_iterations(s, 0, std::min(LOOP_CHUNK, maxl));
             return (int)UPF_OK;
@@ -4748,10 +4814,12 @@ int upf_batch_step(upf_batch* b, int nsteps, int use_graph) {
     int k = 0;
     // the first step also computes the boundary volumes: eager
     for (; k < nsteps && (!use_graph || !s->psi_ready); ++k) {
-        int rc = step_pcisph_static(s, false);
+        int rc = sort_and_bin(s);
+        if (!rc) rc = step_pcisph_static(s, false);
+        int e = UPF_OK;
+        if (!rc) rc = wait_failures(s, &e);
         if (rc) return rc;
         ++s->steps_done;
-        const int e = err_code(s->h_ctl->err);
         if (e) return e;
     }
     // the graphs bake in the launch shapes and the physics (every kernel's
@@ -4818,7 +4886,7 @@ int upf_batch_step(upf_batch* b, int nsteps, int use_graph) {
     }
     int rc = read_ctl(s);
     if (rc) return rc;
-    return err_code(s->h_ctl->err);
+    return err_code(s->h_ctl->err | s->h_ctl->late);
 }
 
 int upf_batch_download(upf_batch* b, float* pos4, float* vel4, float* rho) {
