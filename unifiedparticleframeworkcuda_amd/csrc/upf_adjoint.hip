@@ -771,7 +771,7 @@ int upf_adjoint_create(const upf_params* p, int n, int steps, int iterations, in
         a->bins.ncells = a->ncells;
         ok = a->alloc(&a->bins.at, n) == hipSuccess && a->alloc(&a->bins.place, n) == hipSuccess &&
              a->alloc(&a->bins.sums, BIN_BLOCKS) == hipSuccess && a->alloc(&a->bins.count, a->ncells) == hipSuccess &&
-             hipMemset(a->bins.count, 0, (size_t)a->ncells * sizeof(uint32_t)) == hipSuccess;
+             hipMemsetAsync(a->bins.count, 0, (size_t)a->ncells * sizeof(uint32_t), a->st) == hipSuccess;
     } else if (ok) {
         void* tmp = nullptr;
         ok = a->alloc(&a->skeys, n) == hipSuccess && a->alloc(&a->perm, n) == hipSuccess &&

@@ -4041,7 +4041,7 @@ static int sim_alloc(upf_sim* s, int capacity, uint32_t ncells, int n_scenes) {
         HIPCHK(s->alloc(&s->bins.place, capacity));
         HIPCHK(s->alloc(&s->bins.sums, BIN_BLOCKS));
         HIPCHK(s->alloc(&s->bins.count, ncells));
-        HIPCHK(hipMemset(s->bins.count, 0, (size_t)ncells * sizeof(uint32_t)));
+        HIPCHK(hipMemsetAsync(s->bins.count, 0, (size_t)ncells * sizeof(uint32_t), s->st));
     }
     HIPCHK(s->alloc(&s->luts, LUT_TOTAL));
     HIPCHK(s->alloc(&s->ctl, 1));
@@ -4065,7 +4065,7 @@ static int sim_alloc(upf_sim* s, int capacity, uint32_t ncells, int n_scenes) {
         // below 2 thr[300] (above it both are 300)
         unsigned long long* bad = nullptr;
         HIPCHK(s->alloc(&bad, 1));
-        HIPCHK(hipMemset(bad, 0, sizeof(unsigned long long)));
+        HIPCHK(hipMemsetAsync(bad, 0, sizeof(unsigned long long), s->st));
         const float top = 2.0f * L[LUT_TH_OFF + 2 * 300];
         uint32_t top_bits;
         std::memcpy(&top_bits, &top, 4);
@@ -4078,9 +4078,9 @@ static int sim_alloc(upf_sim* s, int capacity, uint32_t ncells, int n_scenes) {
             return UPF_ERR_HIP;
         }
     }
-    HIPCHK(hipMemset(s->ctl, 0, sizeof(Ctl)));
-    HIPCHK(hipMemset(s->sctl, 0, (size_t)n_scenes * sizeof(SceneCtl)));
-    HIPCHK(hipMemset(W.max_slots, 0, nslots * sizeof(uint32_t)));
+    HIPCHK(hipMemsetAsync(s->ctl, 0, sizeof(Ctl), s->st));
+    HIPCHK(hipMemsetAsync(s->sctl, 0, (size_t)n_scenes * sizeof(SceneCtl), s->st));
+    HIPCHK(hipMemsetAsync(W.max_slots, 0, nslots * sizeof(uint32_t), s->st));
     if (n_scenes > 1) {
         HIPCHK(s->alloc(&s->d_doms, n_scenes));
         HIPCHK(s->alloc(&s->d_scene_of, capacity));
@@ -4544,7 +4544,7 @@ int upf_keys(const upf_params* p, int n, const float* pos4, uint32_t* keys) {
         if (hipMalloc((void**)&d_pos, (size_t)n * 16) != hipSuccess) break;
         if (hipMalloc((void**)&d_keys, (size_t)n * 4) != hipSuccess) break;
         if (hipMalloc((void**)&ctl, sizeof(Ctl)) != hipSuccess) break;
-        if (hipMemset(ctl, 0, sizeof(Ctl)) != hipSuccess) break;
+        if (hipMemsetAsync(ctl, 0, sizeof(Ctl), nullptr) != hipSuccess) break;
         if (hipMemcpy(d_pos, pos4, (size_t)n * 16, hipMemcpyHostToDevice) != hipSuccess) break;
         upf_sim tmp;
         tmp.P = *p;
@@ -4780,7 +4780,7 @@ int upf_batch_create(int n_scenes, const upf_params* scene_params, const int* co
                 hipMemcpy(s->d_chunk_end, ce.data(), ce.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess ||
                 hipMemcpy(s->d_sc_chunk0, c0.data(), c0.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess ||
                 hipMemcpy(s->d_sc_nchunks, nc.data(), nc.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess ||
-                hipMemset(s->d_act_n, 0, 2 * sizeof(int)) != hipSuccess)
+                hipMemsetAsync(s->d_act_n, 0, 2 * sizeof(int), s->st) != hipSuccess)
                 rc = UPF_ERR_HIP;
         }
     }
