@@ -150,3 +150,28 @@ def test_lanes_and_list_forms_match_fp32_oracle(gpu, case):
     assert np.abs(x - xo).max() < 2e-6
     assert np.abs(v - vo).max() < 1e-4 * max(np.abs(vo).max(), 1e-3)
     assert _rel(gv, ov) < 1e-4 and _rel(gx, ox) < 1e-4
+
+
+def test_crowded_cell_leaves_the_gradient(gpu):
+    """A pile of wall particles far from the fluid: its cell is ranked by blocks, and the fluid's rollout and
+    gradient are those of the scene without it, bit for bit."""
+    import scenes
+    p, pos, typ, vel, target, f = adj.differentiable_dam_break(9, 8, 7)
+    pos2, typ2 = scenes.with_pile(p, pos, typ, 7000)
+    # the particles of the plain scene in the piled one, by position
+    where = {tuple(x): i for i, x in enumerate(map(tuple, pos2[:, :3]))}
+    at = np.array([where[tuple(x)] for x in map(tuple, pos[:, :3])])
+    print("crowded rollout: %d particles" % len(typ2), flush=True)
+    vel2 = np.zeros((len(typ2), vel.shape[1]), np.float32)
+    vel2[at] = vel
+    out = []
+    for q, t, v, i in ((pos, typ, vel, np.arange(len(typ))), (pos2, typ2, vel2, at)):
+        r = adj.Rollout(p, q, t, 5, 2, checkpoint_every=2)
+        x, _ = r.forward(v)
+        g = np.zeros((len(t), 3), np.float32)
+        g[i[f]] = x[i[f]] - target[f]
+        gx, gv = r.backward(g)
+        r.close()
+        out.append([a[i] for a in (x, gx, gv)])
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)

@@ -162,3 +162,28 @@ def test_batch_graph_follows_set_params(gpu):
         assert np.array_equal(a["pos"], g["pos"]) and np.array_equal(a["vel"], g["vel"])
         assert np.array_equal(Ka, Kg) and np.array_equal(ra, rg)
     assert Ka[2:].max() <= 7
+
+
+@pytest.mark.parametrize("use_graph", [1, 0, 2])
+def test_batch_with_a_crowded_cell_equals_plain(gpu, use_graph):
+    """A pile of wall particles in one scene's cell: the sort by blocks of the first call, graphs captured with it
+    and graphs captured again with the radix sort give the plain per-scene runs."""
+    import scenes as sc
+    some = _scenes(n_scenes=3, seed=4)
+    some[1] = (some[1][0],) + sc.with_pile(*some[1][:3], 7000)
+    print("crowded batch: counts %s, graph %s" % ([len(s[2]) for s in some], use_graph), flush=True)
+    b = upf.Batch.from_scenes(some)
+    for steps in (2, 2, 3):
+        b.step(steps, use_graph=use_graph)
+    st = b.state()
+    b.close()
+    off = 0
+    for p, pos, typ in (s[:3] for s in some):
+        sim = upf.Simulation(p, len(typ))
+        sim.upload(pos, typ)
+        sim.step(7, upf.UPF_PCISPH_STATIC)
+        r = sim.state()
+        sim.close()
+        for k in ("pos", "vel", "rho"):
+            assert np.array_equal(st[k][off:off + len(typ)], r[k]), k
+        off += len(typ)

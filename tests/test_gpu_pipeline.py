@@ -440,3 +440,70 @@ def test_upload_and_download_round_trip(gpu, n):
         assert (s["rho"] == p.rest_density).all() and not s["p"].any()
         assert (s["psi"] == np.float32(p.initial_mass) / np.float32(p.rest_density)).all()
     sim.close()
+
+
+def _piled(p, width, sizes, one_key, rng):
+    """Frozen particles piled into cells of the given sizes, at one place each or over the cell, in random order."""
+    cell = np.repeat(np.arange(len(sizes)), sizes)
+    base = (np.stack([3 + 2 * cell, 4 + cell % 3, 5 + cell % 2], 1) + 0.25) * width
+    x = base if one_key else base + rng.uniform(0.0, 0.5 * width, base.shape)
+    pos = np.zeros((len(cell), 4), np.float32)
+    pos[:, :3] = x[rng.permutation(len(cell))]
+    return pos
+
+
+# cells around the size from which blocks rank them, and around multiples of a block's share
+@pytest.mark.parametrize("one_key", [True, False])
+@pytest.mark.parametrize("sizes", [(2048, 6144), (6145,), (6143, 1, 6146, 8192), (8193, 300, 20011, 6145), (300007,)])
+def test_crowded_cells_are_a_stable_sort(gpu, sizes, one_key):
+    print("crowded cells: %s, one key %d" % (sizes, one_key), flush=True)
+    rng = np.random.RandomState(len(sizes))
+    p, width = _grid(32)
+    pos = _piled(p, width, sizes, one_key, rng)
+    key = upf.device_keys(p, pos)
+    want = np.argsort(key, kind="stable")
+    sim = upf.Simulation(p, len(pos))
+    for _ in range(2):
+        sim.upload(pos, np.full(len(pos), upf.UPF_FROZEN, np.int32))
+        sim.sort_and_bin()
+        k, ids, cells = sim.sorted_state()
+        assert np.array_equal(ids, want) and np.array_equal(k, key[want])
+        code, first = np.unique(k >> np.uint32(3 * p.block_shift), return_index=True)
+        assert np.array_equal(cells, np.stack([code, first, np.r_[first[1:], len(k)]], 1))
+    sim.close()
+
+
+def test_crowded_cells_take_no_square(gpu):
+    """A million particles in one cell: ranked against each other one by one they took 464 ms."""
+    import time
+    p, width = _grid(32)
+    pos = _piled(p, width, (1000000,), False, np.random.RandomState(0))
+    sim = upf.Simulation(p, len(pos))
+    took = []
+    for _ in range(3):
+        sim.upload(pos, np.full(len(pos), upf.UPF_FROZEN, np.int32))
+        t = time.perf_counter()
+        sim.sort_and_bin()
+        took.append(time.perf_counter() - t)
+    sim.close()
+    print("sorts of a million particles in one cell: %s s" % took, flush=True)
+    assert min(took) < 0.1
+
+
+@pytest.mark.parametrize("method", [upf.UPF_PCISPH_STATIC, upf.UPF_SPH_STATIC])
+def test_steps_over_a_crowded_cell(gpu, method):
+    """A pile of wall particles beside a dam break: the sort by blocks of the first step and the radix sort of the
+    next ones, in one call and in several, against the oracle."""
+    p, pos, typ, _ = upf.standard_dam_break(16, 16, 16, dt=0.000253)
+    p.boundary_pressure_mode = upf.UPF_BOUNDARY_AKINCI
+    pos, typ = scenes.with_pile(p, pos, typ, 7000)
+    print("crowded step: method %d, %d particles" % (method, len(typ)), flush=True)
+    o = ol.OracleSim(p, pos, None, typ)
+    o.step(4, method)
+    for calls in ((4,), (1, 1, 1, 1)):
+        sim = upf.Simulation(p, len(typ))
+        sim.upload(pos, typ)
+        for steps in calls:
+            sim.step(steps, method)
+        _compare(sim, o, typ == upf.UPF_LIQUID, pcisph=method == upf.UPF_PCISPH_STATIC)
+        sim.close()

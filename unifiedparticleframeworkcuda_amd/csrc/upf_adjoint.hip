@@ -168,15 +168,15 @@ __global__ void k_cell_bounds(int n, const uint32_t* __restrict__ keys, const ui
 }
 
 // the same positions from the particles' places cell by cell (upf_bins.h)
-__global__ __launch_bounds__(AB) void k_rank_cand(int n, CellMap map, const uint64_t* __restrict__ place,
+__global__ __launch_bounds__(AB, 8) void k_rank_cand(int n, CellMap map, const uint64_t* __restrict__ place,
                                                   const uint2* __restrict__ cells, const float4* __restrict__ x,
-                                                  float4* __restrict__ cand) {
-    const int t = blockIdx.x * AB + threadIdx.x;
-    if (t >= n) return;
-    const uint64_t v = place[t];
-    const uint32_t j = (uint32_t)v;
-    const float4 p = x[j];
-    cand[bin_slot(place, v, cells[map((uint32_t)(v >> 32), t)])] = make_float4(p.x, p.y, p.z, __uint_as_float(j));
+                                                  float4* __restrict__ cand, Ctl* ctl) {
+    static_assert(AB == BLOCK, "move_ranked");
+    move_ranked(n, map, place, cells, &ctl->crowded, [&](uint64_t v, auto slot) __attribute__((always_inline)) {
+        const uint32_t j = (uint32_t)v;
+        const float4 p = x[j];
+        cand[slot()] = make_float4(p.x, p.y, p.z, __uint_as_float(j));
+    });
 }
 
 // neighbour ids of every fluid particle: the cells of its query box (the
@@ -667,7 +667,7 @@ static void enqueue_step(upf_adjoint* a, const float4* x, const float4* v, float
     const CellMap map{3u * a->P.block_shift, nullptr, nullptr};
     if (a->bins.count) {
         (void)cell_bins(a->keys, n, map, a->bins, a->st);
-        hipLaunchKernelGGL(k_rank_cand, a->grid(), b, 0, a->st, n, map, a->bins.place, a->cells, x, a->cand);
+        hipLaunchKernelGGL(k_rank_cand, a->grid(), b, 0, a->st, n, map, a->bins.place, a->cells, x, a->cand, a->ctl);
     } else {
         (void)radix_sort(a->keys, nullptr, a->skeys, a->perm, n, 30, a->sort_tmp, a->st);
         hipLaunchKernelGGL(k_cell_bounds, a->grid(), b, 0, a->st, n, a->skeys, a->perm, x, map.shift3, a->cells, a->cand);

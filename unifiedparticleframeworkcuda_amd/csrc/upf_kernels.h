@@ -29,6 +29,7 @@ struct Ctl {              // whole simulation
     uint32_t err;        // bit (1 << UPF_ERR_*) set on failures
     uint32_t step;       // steps recorded in the per-scene statistics
     uint32_t late;       // the same of the last integration; in err from the next sort on
+    uint32_t crowded;    // a cell of more than BIN_CROWD particles was met (upf_bins.h)
 };
 
 struct SceneCtl {         // one scene's PCISPH loop

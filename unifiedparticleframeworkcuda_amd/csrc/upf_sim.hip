@@ -185,9 +185,10 @@ __device__ inline void publish(const Publish& pub, const Ctl& ctl, const SceneCt
 }
 
 // Failures alone, in one store: nothing waits for it (the fence above takes as
-// long as a small kernel).
-__device__ inline void publish_failures(const Publish& pub, uint32_t err) {
-    *(volatile uint64_t*)&pub.m->fail = (uint64_t)err << 32 | pub.seq;
+// long as a small kernel).  CROWDED among them: Ctl::crowded.
+constexpr uint32_t CROWDED = 1u << 31;
+__device__ inline void publish_failures(const Publish& pub, uint32_t err, uint32_t crowded) {
+    *(volatile uint64_t*)&pub.m->fail = (uint64_t)(err | (crowded ? CROWDED : 0u)) << 32 | pub.seq;
 }
 
 // Start of a step (block 0 of the kernel that moves the state): the failures of
@@ -205,12 +206,11 @@ struct StepBegin {
 __device__ inline void begin_step(const StepBegin& B) {
     if (blockIdx.x != 0) return;
     if (threadIdx.x == 0) {
-        Ctl c = *B.ctl;
-        c.err |= c.late;
-        c.late = 0u;
-        if (B.pub.m) publish_failures(B.pub, c.err);
-        c.want_any = B.want;
-        *B.ctl = c;
+        const uint32_t err = B.ctl->err | B.ctl->late;
+        B.ctl->err = err;
+        B.ctl->late = 0u;
+        if (B.pub.m) publish_failures(B.pub, err, B.ctl->crowded);
+        B.ctl->want_any = B.want;
     }
     for (int sc = threadIdx.x; sc < B.n_scenes; sc += blockDim.x) B.sctl[sc] = SceneCtl{B.want, 1, 0.0f, 0};
     if (threadIdx.x == 0) {
@@ -280,19 +280,15 @@ __global__ __launch_bounds__(BLOCK) void k_gather(int n, const uint32_t* __restr
 // The same from the particles' places cell by cell (upf_bins.h): the slot is
 // the rank within the cell, counted while the state is on its way.
 template <bool RIGID>
-__global__ __launch_bounds__(BLOCK) void k_rank_gather(int n, CellMap map, const uint64_t* __restrict__ place,
+__global__ __launch_bounds__(BLOCK, 8) void k_rank_gather(int n, CellMap map, const uint64_t* __restrict__ place,
                                                        const uint2* __restrict__ cells, Slots src, Slots dst,
                                                        const float* __restrict__ p_work,
                                                        const float* __restrict__ rho_work, StepBegin begin) {
     begin_step(begin);
-    const int t = blockIdx.x * BLOCK + threadIdx.x;
-    if (t >= n) return;
-    const uint64_t v = place[t];
-    const uint32_t key = (uint32_t)(v >> 32);
-    const uint2 r = cells[map(key, t)];
-    const int s = move_slot<RIGID>(src, dst, (int)(uint32_t)v, p_work, rho_work,
-                                   [&] { return (int)bin_slot(place, v, r); });
-    dst.key[s] = key;
+    move_ranked(n, map, place, cells, &begin.ctl->crowded, [&](uint64_t v, auto slot) __attribute__((always_inline)) {
+        const int s = move_slot<RIGID>(src, dst, (int)(uint32_t)v, p_work, rho_work, [&] { return (int)slot(); });
+        dst.key[s] = (uint32_t)(v >> 32);
+    });
 }
 
 // ------------------------------------------------------------ cell table
@@ -1922,7 +1918,7 @@ __device__ inline void loop_test(const StepArgs& A, int sc, int t, int lane, Ctl
         C.want = want;
         atomicMax(&ctl->want_any, want);
         if (pub.m && (!next || pub.last)) {
-            publish(pub, Ctl{want, 0u, ctl->step, 0u}, SceneCtl{want, too_large, mx, 0});
+            publish(pub, Ctl{want, 0u, ctl->step, 0u, 0u}, SceneCtl{want, too_large, mx, 0});
         }
     }
     // batched: a scene that runs iteration t + 1 puts its chunks on that
@@ -2217,7 +2213,7 @@ __global__ __launch_bounds__(BLOCK) void k_force_lanes(int t, StepArgs A, Slots 
 __global__ void k_integrate(StepArgs A, Slots S, Work W, int pcisph, int pure_fluid_clamp, int has_bodies, Ctl* ctl,
                             Publish pub) {
     const upf_params& P = A.P;
-    if (pub.m && blockIdx.x == 0 && threadIdx.x == 0) publish_failures(pub, ctl->err);
+    if (pub.m && blockIdx.x == 0 && threadIdx.x == 0) publish_failures(pub, ctl->err, ctl->crowded);
     for (int i = xblk(A.xcd) * blockDim.x + threadIdx.x; i < A.n; i += gstride()) {
     float4 x = S.pos[i];
     const int ti = ptype(x);
@@ -3301,6 +3297,7 @@ struct upf_sim {
     void* sort_tmp = nullptr;
     uint32_t ncells = 0;
     Bins bins = {};  // count null: the cell table is too sparse for it (bins_apply)
+    bool crowded = false;  // a cell was ranked by blocks since the upload: the radix sort from then on
     std::vector<int> k_hist;
     uint32_t* d_key0 = nullptr;  // z-index of every particle's uploaded position, by upload id
     Stage stage;
@@ -3437,7 +3434,7 @@ static int sort_and_bin(upf_sim* s, const Publish& pub = Publish{}) {
     Work& W = s->W;
     s->prof.begin(PC_SORT, s->st);
     const int nxt = 1 - s->cur;
-    if (s->bins.count) {
+    if (s->bins.count && !s->crowded) {
         const CellMap map{3u * s->P.block_shift, s->n_scenes > 1 ? s->d_doms : nullptr,
                           s->n_scenes > 1 ? s->d_scene_of : nullptr};
         HIPCHK(cell_bins(W.keys, n, map, s->bins, s->st));
@@ -3530,13 +3527,16 @@ static int wait_failures(upf_sim* s, int* code) {
     const int rc = spin(s, [&] { return (uint32_t)(v = *(const volatile uint64_t*)&m->fail) == seq; });
     if (rc) return rc;
     *code = err_code((uint32_t)(v >> 32));
+    s->crowded = s->crowded || (v >> 32) & CROWDED;
     return UPF_OK;
 }
 // The loop state after all work enqueued so far.
 static int read_ctl(upf_sim* s) {
     hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, s->st, s->ctl, s->sctl, next_publish(s, 1));
     HIPCHK(hipGetLastError());
-    return wait_published(s);
+    const int rc = wait_published(s);
+    if (!rc) s->crowded = s->crowded || s->h_ctl->crowded;
+    return rc;
 }
 
 template <int MODE>
@@ -4206,6 +4206,7 @@ static int upload_common(upf_sim* s, int n, const float* pos4, const float* vel4
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(s->st));
     s->uploaded = true;
+    s->crowded = false;
     s->psi_ready = false;
     s->k_hist.clear();
     s->rho_hist.clear();
@@ -4602,6 +4603,7 @@ struct upf_batch {
     int last_k = 0;                                 // split form: iterations of the previous step
     upf_tuning captured{};                          // launch shapes baked into the graphs
     upf_params captured_p{};                        // physics baked into the graphs (StepArgs, loop bounds)
+    bool captured_crowded = false;                  // the sort baked into the graphs (upf_sim::crowded)
 
     void drop_graphs() {
         for (auto& g : gexec)
@@ -4824,9 +4826,10 @@ int upf_batch_step(upf_batch* b, int nsteps, int use_graph) {
     }
     // the graphs bake in the launch shapes and the physics (every kernel's
     // StepArgs, the number of loop iterations): recapture when upf_set_tuning
-    // or upf_set_params (through upf_batch_sim) changed either
+    // or upf_set_params (through upf_batch_sim) changed either, or the sort has
     if ((b->gexec[0] || b->head[0]) && (std::memcmp(&b->captured, &s->tune, sizeof(upf_tuning)) != 0 ||
-                                        std::memcmp(&b->captured_p, &s->P, sizeof(upf_params)) != 0))
+                                        std::memcmp(&b->captured_p, &s->P, sizeof(upf_params)) != 0 ||
+                                        b->captured_crowded != s->crowded))
         b->drop_graphs();
     if (use_graph == 2) {
         // split form: head graph, then chunk graphs while the device's loop
@@ -4834,6 +4837,7 @@ int upf_batch_step(upf_batch* b, int nsteps, int use_graph) {
         if (k < nsteps && !b->head[0]) {
             b->captured = s->tune;
             b->captured_p = s->P;
+            b->captured_crowded = s->crowded;
             const int rc = capture_split(b);
             if (rc) {
                 b->drop_graphs();
@@ -4872,6 +4876,7 @@ int upf_batch_step(upf_batch* b, int nsteps, int use_graph) {
         if (k < nsteps && !b->gexec[0]) {
             b->captured = s->tune;
             b->captured_p = s->P;
+            b->captured_crowded = s->crowded;
             const int cur = s->cur;
             int rc = capture_step(s, 0, &b->gexec[0]);
             if (!rc) rc = capture_step(s, 1, &b->gexec[1]);
