@@ -507,3 +507,40 @@ def test_steps_over_a_crowded_cell(gpu, method):
             sim.step(steps, method)
         _compare(sim, o, typ == upf.UPF_LIQUID, pcisph=method == upf.UPF_PCISPH_STATIC)
         sim.close()
+
+
+@pytest.mark.parametrize("method", [upf.UPF_WCSPH_STATIC, upf.UPF_SPH_STATIC])
+def test_sph_lists_with_more_jumps_than_the_code_holds(gpu, method):
+    """Thirty-one fluid particles close together whose slots lie 65,600 apart, since two million wall particles share
+    their z-index key: lists with 29 jumps of more than 16 bits.  The fused build steps like the separate kernels."""
+    p, width = _grid(64)
+    for a in range(3):  # cells of 64 h, sixteen z-index units each
+        p.scales[a] = p.block_size / (64.0 * p.support_radius)
+        p.vbox_max[a] = p.collision_max[a] = 64 * 64.0 * p.support_radius
+        p.collision_min[a] = 0.0
+    p.dt = 0.00001
+    gap = 65600
+    n = 31 + 30 * gap
+    h, unit = p.support_radius, 4.0 * p.support_radius
+    pos = np.zeros((n, 4), np.float32)
+    pos[:, :3] = 40 * unit + 3.0 * h
+    typ = np.full(n, upf.UPF_FROZEN, np.int32)
+    f = np.arange(31) * (gap + 1)
+    typ[f] = upf.UPF_LIQUID
+    pos[f, :3] = 40 * unit + (0.5 + np.random.RandomState(3).uniform(0.0, 0.5, (31, 3))) * h
+    print("list jumps: method %d, %d particles" % (method, n), flush=True)
+    assert len(np.unique(upf.device_keys(p, pos))) == 1
+    out = []
+    for fuse in (1, 0):
+        sim = upf.Simulation(p, n)
+        t = sim.tuning()
+        t.nbr_fuse = fuse
+        sim.set_tuning(t)
+        sim.upload(pos, typ)
+        sim.step(1, method)
+        s = sim.state()
+        out.append({k: s[k][f] for k in s})
+        sim.close()
+    for k in out[0]:
+        assert np.array_equal(out[0][k], out[1][k]), k
+    assert (np.abs(out[0]["force"][:, :3]).max(1) > 0.0).all()

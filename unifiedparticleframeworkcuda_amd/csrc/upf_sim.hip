@@ -465,7 +465,11 @@ __global__ void k_check_bins(float factor, const float* __restrict__ luts, uint3
 // the list is ascending, so consecutive slots mostly differ by less than
 // 2^16; larger jumps (between stencil cells far apart in Morton order) go to
 // a per-particle escape column.  Eight 16-bit increments share one 16-byte
-// load, so a reader fetches eight entries per memory round trip.
+// load, so a reader fetches eight entries per memory round trip.  A list with
+// more jumps than the column holds (cells of more than 2^16 particles) is an
+// overflow; without ctl its writer puts LIST_UNCODED in the first slot's place,
+// for a reader that then takes the row.
+constexpr uint32_t LIST_UNCODED = 0xFFFFFFFFu;
 struct ListEncoder {
     uint32_t* first;
     uint4* rows;
@@ -495,8 +499,12 @@ struct ListEncoder {
             if (d <= 65535u) {
                 w = d;
             } else {
-                if (esc < NB_ESC) e[(size_t)esc * st] = d;
-                else set_err(ctl, UPF_ERR_NBR_OVERFLOW);
+                if (esc < NB_ESC) {
+                    e[(size_t)esc * st] = d;
+                } else {
+                    w = 1;  // a reader stays below this slot
+                    if (ctl) set_err(ctl, UPF_ERR_NBR_OVERFLOW);
+                }
                 ++esc;
             }
         }
@@ -506,6 +514,7 @@ struct ListEncoder {
     __device__ void finish() {
         while (nw != 0) push(0u);
     }
+    __device__ bool whole() const { return esc <= NB_ESC; }
 };
 
 struct ListDecoder {
@@ -2309,7 +2318,7 @@ __device__ __forceinline__ void finish_density_wcsph(const StepArgs& A, const Sl
 // for the force pass.
 template <bool TAIT, bool FUSED>
 __device__ __forceinline__ void density_wcsph_slot(const StepArgs& A, const Slots& S, const Work& W, int i,
-                                                   const float* lw, const float2* th, Ctl* ctl) {
+                                                   const float* lw, const float2* th) {
     const upf_params& P = A.P;
     const float4 xi = S.pos[i];
     const float m = P.initial_mass;
@@ -2328,7 +2337,7 @@ __device__ __forceinline__ void density_wcsph_slot(const StepArgs& A, const Slot
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const int j = k + u < cnt ? (int)(e[u] >> NB_SLOT_SHIFT) : i;
-                if (k + u < cnt) enc.put(k + u, (uint32_t)j, ctl);
+                if (k + u < cnt) enc.put(k + u, (uint32_t)j, nullptr);
                 xj[u] = at_u32(S.pos, j);
             }
 #pragma unroll
@@ -2338,6 +2347,7 @@ __device__ __forceinline__ void density_wcsph_slot(const StepArgs& A, const Slot
             }
         }
         enc.finish();
+        if (!enc.whole()) W.nbf[i] = LIST_UNCODED;
     } else {
         for (int k = 0; k < cnt; ++k) rho = rho + lw[W.nbr[(size_t)k * A.stride + i] & NB_BIN_MASK] * m;
     }
@@ -2372,7 +2382,7 @@ __global__ __launch_bounds__(BLOCK) void k_density_wcsph(StepArgs A, Slots S, Wo
     for (int t = threadIdx.x; t < LUT_N; t += blockDim.x) lw[t] = luts[t];
     __syncthreads();
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < A.n) density_wcsph_slot<TAIT, false>(A, S, W, i, lw, nullptr, ctl);
+    if (i < A.n) density_wcsph_slot<TAIT, false>(A, S, W, i, lw, nullptr);
 }
 
 // The list build and the density pass in one kernel: each lane sums the
@@ -2403,13 +2413,13 @@ __global__ __launch_bounds__(64) void k_nbr_build_wcsph(StepArgs A, Slots S, Wor
         if (i >= 0) density_wcsph_lanes<TAIT, SPLIT>(A, S, W, i, (int)threadIdx.x % SPLIT, lw, th);
     } else {
         const int i = split_slot<SPLIT>(A);
-        if (i >= 0) density_wcsph_slot<TAIT, true>(A, S, W, i, lw, th, ctl);
+        if (i >= 0) density_wcsph_slot<TAIT, true>(A, S, W, i, lw, th);
     }
 }
 
 // CalculateLiquidParticleForces (:3009-3083) + gravity (:2822-2824).  CODED:
-// over the delta-coded lists of the fused build, the bins from the distances
-// (the build's positions).
+// over the delta-coded lists of the fused build (an uncoded one: the slot's row),
+// the bins from the distances (the build's positions).
 template <int CODED>
 __global__ __launch_bounds__(BLOCK) void k_force_wcsph(StepArgs A, Slots S, Work W, const float* __restrict__ luts,
                                                        Ctl* ctl) {
@@ -2439,26 +2449,34 @@ __global__ __launch_bounds__(BLOCK) void k_force_wcsph(StepArgs A, Slots S, Work
     const float invD = (float)(1.0 / (double)rho_i);
     const float pVol = m * invD;
     float fx = 0.0f, fy = 0.0f, fz = 0.0f;
-    // two 16-byte records per neighbour, four neighbours' loads in flight
-    for_each_listed<CODED, 4>(
-        W, i, (size_t)A.stride, head, [&](int j) { return PosVel{at_u32(W.xpd, j), at_u32(W.vpg, j)}; },
-        [&](int, uint32_t e, const PosVel& q) __attribute__((always_inline)) {
-            const float4& xj = q.x;
-            if (xj.w < 0.0f) return;  // not a fluid neighbour
-            const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-            const uint32_t bin = CODED ? bin_of_d2(dx * dx + dy * dy + dz * dz, A.lut_factor, th) : (e & NB_BIN_MASK);
-            const float kv = lvl[bin];
-            const float nVol = xj.w;  // m / rho_j
-            const float g = lpg[bin];
-            const float grad = p_i * invD * invD + q.v.w;  // + p_j / rho_j^2
-            fx = fx - (((dx * g) * grad) * m) * m;
-            fy = fy - (((dy * g) * grad) * m) * m;
-            fz = fz - (((dz * g) * grad) * m) * m;
-            const float vx = vi.x - q.v.x, vy = vi.y - q.v.y, vz = vi.z - q.v.z;
-            fx = fx - vx * pVol * nVol * P.visc_const * kv;
-            fy = fy - vy * pVol * nVol * P.visc_const * kv;
-            fz = fz - vz * pVol * nVol * P.visc_const * kv;
-        });
+    auto load = [&](int j) { return PosVel{at_u32(W.xpd, j), at_u32(W.vpg, j)}; };
+    auto use = [&](int, uint32_t e, const PosVel& q) __attribute__((always_inline)) {
+        const float4& xj = q.x;
+        if (xj.w < 0.0f) return;  // not a fluid neighbour
+        const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+        const uint32_t bin = CODED ? bin_of_d2(dx * dx + dy * dy + dz * dz, A.lut_factor, th) : (e & NB_BIN_MASK);
+        const float kv = lvl[bin];
+        const float nVol = xj.w;  // m / rho_j
+        const float g = lpg[bin];
+        const float grad = p_i * invD * invD + q.v.w;  // + p_j / rho_j^2
+        fx = fx - (((dx * g) * grad) * m) * m;
+        fy = fy - (((dy * g) * grad) * m) * m;
+        fz = fz - (((dz * g) * grad) * m) * m;
+        const float vx = vi.x - q.v.x, vy = vi.y - q.v.y, vz = vi.z - q.v.z;
+        fx = fx - vx * pVol * nVol * P.visc_const * kv;
+        fy = fy - vy * pVol * nVol * P.visc_const * kv;
+        fz = fz - vz * pVol * nVol * P.visc_const * kv;
+    };
+    if (CODED && head.cnt > 0 && head.first == LIST_UNCODED) {
+        const uint32_t* row = W.nbr + (size_t)i * A.nbr_ld;
+        for (int k = 0; k < head.cnt; ++k) {
+            const int j = (int)(row[k] >> NB_SLOT_SHIFT);
+            use(j, 0u, load(j));
+        }
+    } else {
+        // two 16-byte records per neighbour, four neighbours' loads in flight
+        for_each_listed<CODED, 4>(W, i, (size_t)A.stride, head, load, use);
+    }
     if (P.add_boundary_force) box_force_static(P, dom_at(A, i), xi, fx, fy, fz);
     fy = fy - P.initial_mass * P.gravity;
     W.force[i] = make_float4(fx, fy, fz, 0.0f);
