@@ -49,7 +49,9 @@ constexpr int BIN_BLOCKS = 1024;
 inline bool bins_apply(int n, uint32_t ncells) { return (uint64_t)ncells <= (1ull << 22) + 8ull * (uint64_t)n; }
 
 // Fills B.cells and B.place for keys[0..n); move_ranked gives the slots.
-hipError_t cell_bins(const uint32_t* keys, int n, const CellMap& map, const Bins& B, hipStream_t st);
+// pub: the first kernel publishes the failures so far (ctl).
+hipError_t cell_bins(const uint32_t* keys, int n, const CellMap& map, const Bins& B, hipStream_t st,
+                     const Ctl* ctl = nullptr, const Publish& pub = Publish{});
 
 // Slot of entry v of the cell whose entries are place[r.x .. r.y).
 __device__ inline uint32_t bin_slot(const uint64_t* __restrict__ place, uint64_t v, uint2 r) {

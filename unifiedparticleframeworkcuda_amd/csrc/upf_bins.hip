@@ -11,7 +11,9 @@ constexpr uint32_t BIN_TILE = 4 * BIN_THREADS;  // cells per step of a block
 // Arrival places in the cells.  Consecutive particles are mostly in the same
 // cell (the previous step's order): one atomic per run of a wave.
 __global__ __launch_bounds__(BLOCK) void k_bin_count(const uint32_t* __restrict__ keys, int n, CellMap map,
-                                                     uint32_t* __restrict__ count, uint32_t* __restrict__ at) {
+                                                     uint32_t* __restrict__ count, uint32_t* __restrict__ at,
+                                                     const Ctl* ctl, Publish pub) {
+    if (pub.m && blockIdx.x == 0 && threadIdx.x == 0) publish_failures(pub, *ctl, true);
     const int i = blockIdx.x * BLOCK + threadIdx.x, lane = threadIdx.x & 63;
     const bool in = i < n;
     const uint32_t c = in ? map(keys[i], i) : 0xFFFFFFFFu;  // no cell has this number
@@ -115,13 +117,14 @@ __global__ __launch_bounds__(BLOCK) void k_bin_place(const uint32_t* __restrict_
     count[c] = 0;
 }
 
-hipError_t cell_bins(const uint32_t* keys, int n, const CellMap& map, const Bins& B, hipStream_t st) {
+hipError_t cell_bins(const uint32_t* keys, int n, const CellMap& map, const Bins& B, hipStream_t st, const Ctl* ctl,
+                     const Publish& pub) {
     const dim3 g((unsigned)((n + BLOCK - 1) / BLOCK)), b(BLOCK);
     const uint32_t tiles = (B.ncells + BIN_TILE - 1) / BIN_TILE;
     const uint32_t per = (tiles + BIN_BLOCKS - 1) / BIN_BLOCKS, span = per * BIN_TILE;
     const dim3 gt((tiles + per - 1) / per);
     const bool direct = tiles <= 32;
-    hipLaunchKernelGGL(k_bin_count, g, b, 0, st, keys, n, map, B.count, B.at);
+    hipLaunchKernelGGL(k_bin_count, g, b, 0, st, keys, n, map, B.count, B.at, ctl, pub);
     if (!direct) hipLaunchKernelGGL(k_bin_sums, gt, dim3(BIN_THREADS), 0, st, B.count, B.ncells, span, B.sums);
     hipLaunchKernelGGL(k_bin_scan, gt, dim3(BIN_THREADS), 0, st, B.count, B.ncells, span, direct ? nullptr : B.sums, B.cells);
     hipLaunchKernelGGL(k_bin_place, g, b, 0, st, keys, n, map, B.cells, B.at, B.place, B.count);

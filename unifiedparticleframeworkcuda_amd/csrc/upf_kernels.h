@@ -98,6 +98,36 @@ struct Work {           // per-step arrays, slot order
     uint2* cells;       // dense cell table indexed by cell Morton code: [first, end)
 };
 
+// Loop state for the host: the control words and scene 0's loop state are
+// written to pinned host memory, then a sequence number the host waits for.
+struct CtlMirror {
+    Ctl ctl;
+    SceneCtl scene0;
+    uint32_t seq;
+    uint32_t pad;
+    uint64_t fail;  // failures << 32 | sequence number
+};
+struct Publish {
+    CtlMirror* m;  // null: nothing to publish
+    uint32_t seq;
+    int last;      // the last iteration enqueued: published whatever its decision
+};
+__device__ inline void publish(const Publish& pub, const Ctl& ctl, const SceneCtl& scene0) {
+    pub.m->ctl = ctl;
+    pub.m->scene0 = scene0;
+    __threadfence_system();
+    *(volatile uint32_t*)&pub.m->seq = pub.seq;
+}
+
+// Failures alone, in one store: nothing waits for it (the fence above takes as
+// long as a small kernel).  CROWDED among them: Ctl::crowded.  late: with the
+// integration's, for kernels behind it.
+constexpr uint32_t CROWDED = 1u << 31;
+__device__ inline void publish_failures(const Publish& pub, const Ctl& ctl, bool late) {
+    const uint32_t err = ctl.err | (late ? ctl.late : 0u) | (ctl.crowded ? CROWDED : 0u);
+    *(volatile uint64_t*)&pub.m->fail = (uint64_t)err << 32 | pub.seq;
+}
+
 }  // namespace upf
 
 #endif

@@ -163,37 +163,9 @@ __device__ inline int xblk_down(int remap) {
     return (blockIdx.x & 7) * per + (per - 1 - (blockIdx.x >> 3));
 }
 
-// Loop state for the host: the control words and scene 0's loop state are
-// written to pinned host memory, then a sequence number the host waits for.
-struct CtlMirror {
-    Ctl ctl;
-    SceneCtl scene0;
-    uint32_t seq;
-    uint32_t pad;
-    uint64_t fail;  // failures << 32 | sequence number
-};
-struct Publish {
-    CtlMirror* m;  // null: nothing to publish
-    uint32_t seq;
-    int last;      // the last iteration enqueued: published whatever its decision
-};
-__device__ inline void publish(const Publish& pub, const Ctl& ctl, const SceneCtl& scene0) {
-    pub.m->ctl = ctl;
-    pub.m->scene0 = scene0;
-    __threadfence_system();
-    *(volatile uint32_t*)&pub.m->seq = pub.seq;
-}
-
-// Failures alone, in one store: nothing waits for it (the fence above takes as
-// long as a small kernel).  CROWDED among them: Ctl::crowded.
-constexpr uint32_t CROWDED = 1u << 31;
-__device__ inline void publish_failures(const Publish& pub, uint32_t err, uint32_t crowded) {
-    *(volatile uint64_t*)&pub.m->fail = (uint64_t)(err | (crowded ? CROWDED : 0u)) << 32 | pub.seq;
-}
-
 // Start of a step (block 0 of the kernel that moves the state): the failures of
 // the step before, its integration's among them, for the host, if it asked for
-// them, and every scene's correction loop runs iteration 0 (the CPU loop starts with density_error_too_large_ = true) unless
+// them here, and every scene's correction loop runs iteration 0 (the CPU loop starts with density_error_too_large_ = true) unless
 // its limits are zero.  As a kernel of its own this took 4 us a step.
 struct StepBegin {
     SceneCtl* sctl;
@@ -206,10 +178,9 @@ struct StepBegin {
 __device__ inline void begin_step(const StepBegin& B) {
     if (blockIdx.x != 0) return;
     if (threadIdx.x == 0) {
-        const uint32_t err = B.ctl->err | B.ctl->late;
-        B.ctl->err = err;
+        if (B.pub.m) publish_failures(B.pub, *B.ctl, true);
+        B.ctl->err |= B.ctl->late;
         B.ctl->late = 0u;
-        if (B.pub.m) publish_failures(B.pub, err, B.ctl->crowded);
         B.ctl->want_any = B.want;
     }
     for (int sc = threadIdx.x; sc < B.n_scenes; sc += blockDim.x) B.sctl[sc] = SceneCtl{B.want, 1, 0.0f, 0};
@@ -2222,7 +2193,7 @@ __global__ __launch_bounds__(BLOCK) void k_force_lanes(int t, StepArgs A, Slots 
 __global__ void k_integrate(StepArgs A, Slots S, Work W, int pcisph, int pure_fluid_clamp, int has_bodies, Ctl* ctl,
                             Publish pub) {
     const upf_params& P = A.P;
-    if (pub.m && blockIdx.x == 0 && threadIdx.x == 0) publish_failures(pub, ctl->err, ctl->crowded);
+    if (pub.m && blockIdx.x == 0 && threadIdx.x == 0) publish_failures(pub, *ctl, false);
     for (int i = xblk(A.xcd) * blockDim.x + threadIdx.x; i < A.n; i += gstride()) {
     float4 x = S.pos[i];
     const int ti = ptype(x);
@@ -3447,7 +3418,7 @@ static void cell_table(upf_sim* s) {
 // sort + gather + cell table (the first part of every step)
 static int sort_and_bin(upf_sim* s, const Publish& pub = Publish{}) {
     const int loops = std::max(s->P.min_loops, s->P.max_loops) > 0 ? 1 : 0;
-    const StepBegin begin{s->sctl, s->ctl, s->n_scenes > 1 ? s->d_act_n : nullptr, s->n_scenes, s->n_chunks, loops, pub};
+    StepBegin begin{s->sctl, s->ctl, s->n_scenes > 1 ? s->d_act_n : nullptr, s->n_scenes, s->n_chunks, loops, pub};
     const int n = s->n;
     Work& W = s->W;
     s->prof.begin(PC_SORT, s->st);
@@ -3455,7 +3426,8 @@ static int sort_and_bin(upf_sim* s, const Publish& pub = Publish{}) {
     if (s->bins.count && !s->crowded) {
         const CellMap map{3u * s->P.block_shift, s->n_scenes > 1 ? s->d_doms : nullptr,
                           s->n_scenes > 1 ? s->d_scene_of : nullptr};
-        HIPCHK(cell_bins(W.keys, n, map, s->bins, s->st));
+        HIPCHK(cell_bins(W.keys, n, map, s->bins, s->st, s->ctl, pub));
+        begin.pub = Publish{};
         s->prof.end(s->st);
         s->prof.begin(PC_GATHER, s->st);
         hipLaunchKernelGGL(s->rigid ? k_rank_gather<true> : k_rank_gather<false>, grid_for(n), dim3(BLOCK), 0, s->st, n,
@@ -4250,7 +4222,7 @@ int upf_step(upf_sim* s, int nsteps, int method) {
     for (int k = 0; k < nsteps; ++k) {
         // The sort is enqueued while the step before still runs, then the host
         // waits for that step's failures: a WCSPH or SPH step's come from the
-        // start of this one's gather, a PCISPH step's (without its integration's,
+        // start of this one's sort, a PCISPH step's (without its integration's,
         // which the next step reports) from its integration.  After a failure the
         // sort is taken back: the call ends with the state of the step that failed.
         int rc = sort_and_bin(s, k > 0 && sph ? next_publish(s, 1) : Publish{});
