@@ -14,7 +14,6 @@
 #include <atomic>
 #include <cstddef>
 #include <cstring>
-#include <system_error>
 #include <thread>
 
 namespace upf {
@@ -75,7 +74,7 @@ class Stage {
         int started = 1;
         try {
             for (; started < t; ++started) pool[started] = std::thread(work, started);
-        } catch (const std::system_error&) {
+        } catch (...) {  // no thread, or no memory for one
         }
         work(0);
         for (int k = 1; k < started; ++k) pool[k].join();
@@ -89,15 +88,28 @@ class Stage {
         const int t = threads(total);
         // any thread may take any chunk: whole slices, unless there is one chunk
         const size_t bytes = total <= SLICE ? total : (size_t)t * SLICE;
+        for (int k = 0; k < t; ++k)
+            if (!ev_[k] && hipEventCreateWithFlags(&ev_[k], hipEventDisableTiming) != hipSuccess) return false;
         if (bytes <= cap_) return true;
         if (pin_) (void)hipHostFree(pin_);
         pin_ = nullptr;
         cap_ = 0;
         if (hipHostMalloc((void**)&pin_, bytes, hipHostMallocDefault) != hipSuccess) return false;
         cap_ = bytes;
-        for (int k = 0; k < t; ++k)
-            if (!ev_[k] && hipEventCreateWithFlags(&ev_[k], hipEventDisableTiming) != hipSuccess) return false;
         return true;
+    }
+
+    // without pinned memory
+    template <bool UP>
+    static bool copy_parts(char* dev, const StagePart* parts, int n, hipStream_t st) {
+        bool ok = true;
+        for (int p = 0; p < n && ok; ++p) {
+            char *d = dev + parts[p].off, *h = parts[p].host;
+            if (parts[p].bytes)
+                ok = hipMemcpyAsync(UP ? d : h, UP ? h : d, parts[p].bytes,
+                                    UP ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, st) == hipSuccess;
+        }
+        return hipStreamSynchronize(st) == hipSuccess && ok;
     }
 
     template <bool UP>
@@ -106,7 +118,11 @@ class Stage {
         const size_t chunks = (total + SLICE - 1) / SLICE;
         const int t = threads(total);
         int device = 0;
-        if (!reserve(total) || hipGetDevice(&device) != hipSuccess) return false;
+        if (!reserve(total)) {
+            (void)hipGetLastError();  // else a launch's check would find it
+            return copy_parts<UP>(dev, parts, n, st);
+        }
+        if (hipGetDevice(&device) != hipSuccess) return false;
         std::atomic<size_t> next{0};
         std::atomic<bool> ok{true};
         parallel(t, [&](int k) {
