@@ -1,4 +1,6 @@
 """Seeded scenes shared by the tests (generated by the library's host code)."""
+import ctypes as C
+
 import numpy as np
 
 import unifiedparticleframeworkcuda_amd as upf
@@ -30,3 +32,11 @@ def with_pile(p, pos, typ, count):
     x[mine], t[mine] = pos, typ
     x[~mine, :3] = (cell + 0.3 + rng.uniform(0.0, 0.3, (count, 3))) * width
     return x, t
+
+
+def sparse_grid(p, edge=6.0):
+    """Puts the scene of p into a virtual box of `edge` metres: a cell table far larger than the particles fill."""
+    vec = C.c_float * 3
+    upf.check("upf_params_set_domain", upf.lib().upf_params_set_domain(
+        C.byref(p), vec(edge, edge, edge), vec(*p.collision_min), vec(*p.collision_max)))
+    return p
