@@ -51,3 +51,39 @@ def test_set_tuning_rejects_unsupported_shapes_without_device():
         # a null handle is rejected first; shape checks need a handle, so only the
         # argument order is checked here and the shapes on the device test
         assert L.upf_set_tuning(None, C.byref(Tuning.from_dict(d))) == upf._abi.UPF_ERR_ARG
+
+
+def test_cache_entries_of_other_passes_are_measured_anew(tmp_path):
+    """An entry written before the passes changed: without the mark, or with another one."""
+    import json
+    path = str(tmp_path / "tuning.json")
+    old = dict(autotune.DEFAULT, nbr_rounds=8)
+    autotune.store("dam_break", 1000, old, 1.5, 9, path)
+    data = json.load(open(path))
+    for mark in (None, autotune.KERNELS - 1):
+        entry = data["dam_break:1000"]
+        entry.pop("kernels", None)
+        if mark is not None:
+            entry["kernels"] = mark
+        json.dump(data, open(path, "w"))
+        assert autotune.load("dam_break", 1000, path) is None
+    autotune.store("dam_break", 1000, old, 1.5, 9, path)
+    assert autotune.load("dam_break", 1000, path) == old
+
+
+def test_search_skips_fields_without_effect():
+    tried = []
+
+    def cost(t):
+        tried.append(t)
+        return 1.0 + t["nbr_rounds"]
+
+    best, _, trials = autotune.coordinate_search(
+        cost, ignored=lambda t: ("loop_width",) if autotune.several_lanes(5000, t) else ())
+    assert trials == len(tried) and best["nbr_rounds"] == 2
+    for t in tried:
+        if autotune.several_lanes(5000, t):
+            assert t["loop_width"] == autotune.DEFAULT["loop_width"]
+    # two rounds take the coded lists, where the width counts
+    assert any(t["loop_width"] == 4 for t in tried)
+    assert not autotune.several_lanes(196608, autotune.DEFAULT)

@@ -5,7 +5,8 @@ ahead, and the list format (packed, delta-coded, or chunk unions staged in
 LDS) and load width of the correction loop.  None of them changes results (every per-particle sum keeps its
 order), so candidates are compared on the same steps from the same initial
 state.  The best choice is kept per (workload, particle count) in a JSON
-cache: $UPF_TUNING_CACHE, else ~/.cache/upf/tuning.json.
+cache: $UPF_TUNING_CACHE, else ~/.cache/upf/tuning.json.  Entries found with
+other passes (KERNELS) are measured anew.
 """
 import ctypes as C
 import json
@@ -21,6 +22,17 @@ CANDIDATES = dict(loop_block=(64, 128, 256), grid_cap=(2048, 4096, 8192, 16384),
                   nbr_stage=(0, 32, 64), speculate=(1, 2, 4, 8), loop_list=(0, 1, 2),
                   loop_width=(4, 8), nbr_tile=(0, 256, 512), spec_first=(0, 2, 4, 8, 64),
                   xcd_remap=(0, 1), nbr_skip=(0, 1), nbr_fuse=(0, 1))
+
+
+KERNELS = 2  # raised when the passes behind the fields change
+
+
+def several_lanes(n, t):
+    """Whether a single scene of n particles runs its iterations with several
+    lanes per particle (pair_lanes in csrc/upf_sim.hip), where loop_width has
+    no effect."""
+    return (n < 196608 and t["nbr_fuse"] == 1 and t["nbr_stage"] == 0 and t["nbr_tile"] == 0 and t["loop_list"] == 1 and
+            t["nbr_rounds"] == 4 and t["nbr_skip"] == 0)
 
 
 def cache_path():
@@ -39,8 +51,9 @@ def load(workload, n, path=None):
             entry = json.load(f).get(cache_key(workload, n))
     except (OSError, ValueError):
         return None
-    # entries written before a field existed take its default
-    return None if entry is None else dict(DEFAULT, **entry["tuning"])
+    if entry is None or entry.get("kernels") != KERNELS:
+        return None
+    return dict(DEFAULT, **entry["tuning"])
 
 
 def store(workload, n, tuning, ms_per_step, trials, path=None):
@@ -50,7 +63,8 @@ def store(workload, n, tuning, ms_per_step, trials, path=None):
             data = json.load(f)
     except (OSError, ValueError):
         data = {}
-    data[cache_key(workload, n)] = {"tuning": dict(tuning), "ms_per_step": ms_per_step, "trials": trials}
+    data[cache_key(workload, n)] = {"tuning": dict(tuning), "ms_per_step": ms_per_step, "trials": trials,
+                                       "kernels": KERNELS}
     d = os.path.dirname(path)
     if d:
         os.makedirs(d, exist_ok=True)
@@ -60,15 +74,17 @@ def store(workload, n, tuning, ms_per_step, trials, path=None):
     os.replace(tmp, path)
 
 
-def coordinate_search(measure, start=None, candidates=None, sweeps=1, log=None):
+def coordinate_search(measure, start=None, candidates=None, sweeps=1, log=None, ignored=None):
     """Minimise measure(tuning dict) -> seconds one parameter at a time,
     starting from `start`; returns (best dict, best time, number of trials).
-    `log`, a list, receives (tuning, seconds) of every trial."""
+    `log`, a list, receives (tuning, seconds) of every trial; ignored(tuning)
+    names the fields without effect in it, whose values are not tried."""
     cand = candidates or CANDIDATES
     best = dict(start or DEFAULT)
     seen = {}
 
     def run(t):
+        t = dict(t, **{f: best[f] for f in (ignored(t) if ignored else ())})
         k = tuple(sorted(t.items()))
         if k not in seen:
             try:
@@ -123,7 +139,8 @@ def tune_simulation(sim, pos, types, workload, steps=4, warmup=1, settle=20, met
         hip.hipDeviceSynchronize()
         return time.perf_counter() - t0
 
-    best, sec, trials = coordinate_search(measure, log=log)
+    best, sec, trials = coordinate_search(measure, log=log,
+                                          ignored=lambda t: ("loop_width",) if several_lanes(n, t) else ())
     sim.set_tuning(Tuning.from_dict(best))
     ms = sec / steps * 1e3
     store(workload, n, best, ms, trials, path)
