@@ -42,7 +42,7 @@ def step_bytes(n, nf, ncells, k):
 # Algorithmic bytes per launch of each kernel class, from the same model.
 def class_bytes(name, n, nf, ncells):
     table = {
-        "radix_sort": 12 * n + 20 * n,          # key read + (key, perm) write, keys from integration
+        "radix_sort": 12 * n + 20 * n,          # (by cells or by key) key read + (key, perm) write, keys from integration
         "gather": 76 * n,
         "cell_table": 4 * n + 8 * ncells,
         "neighbour_lists": 20 * n + 4 * n,      # positions + keys read, counts written
@@ -60,7 +60,7 @@ def class_bytes(name, n, nf, ncells):
 # of nbr_fuse 0 have no row there)
 CLASS_KERNEL = {"pressure_force_predict": "upf::k_force<", "predicted_density": "upf::k_density<",
                 "neighbour_lists_external_force": "upf::k_nbr_build_ext<",
-                "integrate": "upf::k_integrate", "gather": "upf::k_gather", "radix_sort": "upf::rs_scatter"}
+                "integrate": "upf::k_integrate", "gather": "upf::k_rank_gather"}
 PROFILE = os.path.join(ROOT, "profiles", "pcisph_dam_break_1m_kernels.md")
 
 

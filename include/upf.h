@@ -505,15 +505,20 @@ int upf_bodies_from_particles(const upf_params* p, int n, const float* pos4, con
 /* ------------------------------------------------------ launch tuning */
 /* Launch shapes that change speed only, never results (no reference
  * counterpart; the reference fixes them at compile time).  Defaults
- * {256, 8192, 4, 0, 4, 1, 8, 0, 4, 1}.  A batch recaptures its step graph when its
- * tuning (set through its upf_batch_sim handle) changed.                   */
+ * {256, 8192, 4, 0, 4, 1, 8, 0, 4, 1, 0, 1}.  A single scene below 196,608
+ * particles with nbr_rounds 4, nbr_stage 0, loop_list 1, nbr_tile 0, nbr_skip
+ * 0 and nbr_fuse 1 runs its iterations (and the WCSPH and SPH forces) with 4
+ * or 16 lanes per particle over packed rows: loop_width, and for these passes
+ * loop_block and grid_cap, then have no effect.  A batch recaptures its step
+ * graph when its tuning (set through its upf_batch_sim handle) changed.     */
 typedef struct upf_tuning {
     int loop_block;   /* threads per block of the grid-stride passes: 64, 128, 256     */
     int grid_cap;     /* blocks of the grid-stride passes at most (>= 1)               */
     int nbr_rounds;   /* list build: candidates per lane per chunk, 2, 4 or 8 (x 64)    */
     int nbr_stage;    /* list build: entries per list staged in LDS: 0, 32 or 64       */
     int speculate;    /* host loop: iterations enqueued per read-back of the decision (1 .. 64) */
-    int loop_list;    /* correction loop reads: 0 packed 32-bit lists, 1 delta-coded,
+    int loop_list;    /* correction loop reads: 0 packed 32-bit lists, 1 delta-coded
+                         (or packed rows, see above),
                          2 the neighbours' records from LDS through per-chunk unions
                          (static PCISPH; needs loop_block 256)                     */
     int loop_width;   /* correction loop: neighbours whose loads are issued together, 4 or 8 */

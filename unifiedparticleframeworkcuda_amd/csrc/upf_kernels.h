@@ -79,7 +79,9 @@ struct Work {           // per-step arrays, slot order
     uint32_t* max_slots; // MAX_SLOTS x 32 uints: per-slot max of the predicted density (bits)
     float* rho;         // predicted density (PCISPH) / density (WCSPH)
     float* pres;        // WCSPH pressure
-    uint32_t* nbr;      // neighbour lists, column-major: nbr[k * stride + slot]
+    uint32_t* nbr;      // neighbour lists: a row of nbr_ld words per slot where the fused builds
+                        // write them (loop_list 2 apart), else column-major nbr[k * stride + slot];
+                        // between steps the way of uploads and downloads
     int* ncount;
     // the same lists for the correction loop, delta-coded: first neighbour
     // slot in nbf, then 16-bit slot increments, eight per 16-byte word of

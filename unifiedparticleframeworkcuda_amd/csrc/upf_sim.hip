@@ -1,12 +1,14 @@
 // upf_sim.hip -- the per-step particle pipeline on gfx950 and its C ABI.
 //
 // One step (PCISPH, static boundaries), all on one HIP stream:
-//   radix sort of z-index keys -> gather of the particle state into key order
-//   -> dense cell table (first/end slot per occupied cell, by boundary
-//   detection, no atomics) -> neighbour lists + external forces + first
-//   prediction (one pass over the query-box candidates) -> K x [predicted
-//   density & pressure with the convergence test on the device; correction
-//   pressure force fused with the next prediction] -> integration + new keys.
+//   sort by cells (upf_bins.h: counts, a scan that gives the dense cell table,
+//   ranks within the cells) with the particle state moved into key order --
+//   cell tables too sparse or too crowded for it: radix sort of the z-index
+//   keys, gather, cell table by boundary detection -> neighbour lists +
+//   external forces + first prediction (one pass over the query-box
+//   candidates) -> K x [predicted density & pressure with the convergence test
+//   on the device; correction pressure force fused with the next prediction]
+//   -> integration + new keys.
 //
 // Float arithmetic follows the reference CPU path (src/cpu/UnifiedPhysics.cpp)
 // operation by operation, neighbours are visited in ascending sorted order
@@ -2360,8 +2362,9 @@ __global__ __launch_bounds__(BLOCK) void k_density_wcsph(StepArgs A, Slots S, Wo
 // density of its own slot over the list its wave just wrote (as
 // k_nbr_build_ext does for the PCISPH external forces).  With column-major
 // lists, whose cache lines fill over the life of a wave, and bins in the
-// entries, a root for every 64 candidates: 417 us at 1,132,556 particles, now
-// 354; the force pass takes 113 us instead of 100 for it (bins from distances).
+// entries, a root for every 64 candidates: 417 us at 1,132,556 particles, 354
+// with rows and none (now 270, see build_wave); the force pass takes 112 us
+// instead of 100 for it (bins from distances).
 // LANES as in k_nbr_build_ext.
 template <int ROUNDS, bool TAIT, int SPLIT, bool LANES = false>
 __global__ __launch_bounds__(64) void k_nbr_build_wcsph(StepArgs A, Slots S, Work W, const float* __restrict__ luts,
@@ -3361,10 +3364,17 @@ static inline dim3 grid_persist(const upf_sim* s, int n) {
 // Waves that share a window of 64 slots in the fused builds of n slots, and
 // the grid.  A wave works through its window's cells one after the other, so
 // few windows leave most SIMDs idle behind one chain each; more waves cost a
-// set-up per cell that two of them share.  us per PCISPH / WCSPH step with 1,
-// 4 and 16 waves: 3,080 slots 159 / 110, 128 / 78, 125 / 74; 31,720 slots
-// 215 / 144, 179 / 110, 194 / 118; 143,976 slots 349 / 174, 343 / 164, 414 /
-// 230; 295,944 slots 593 / 222, 608 / 236, 774 / 382.
+// set-up per cell that two of them share.  The pair passes then take as many
+// lanes per particle (pair_lanes), one and the delta-coded lists for 1.  us per
+// step with 16, 4 and 1:
+//   slots     PCISPH           WCSPH            batch of that many (no lanes)
+//   12,400    66  77 128       39  43  79       249 253 273
+//   26,520    88  89 142       48  49  85
+//   58,752   151 121 168       72  60  88       286 267 288 (45,748)
+//  138,920   312 222 236      121  89 106       328 291 304 (90,053)
+//  173,800   402 271 264      144 100 112       395 325 324 (159,993)
+//  206,128   468 311 307      164 112 122       442 351 346 (213,734)
+//  348,440   864 546 499      260 164 170       681 499 456 (441,518)
 static int build_split(int n) {
     return n < 24576 ? 16 : n < 196608 ? 4 : 1;
 }
